@@ -55,6 +55,39 @@ def test_bits_of_the_cpu_scalar_path(backend, oracle, fmt, m, n, k):
     assert same_bits(ga, ga_w) and same_bits(gw, gw_w) and gb is None
 
 
+@pytest.mark.parametrize("m,n,k", [(9, 40, 2), (5, 3, 9), (6, 515, 1030), (3, 1100, 1001), (5, 3301, 2560), (290, 70, 3900), (1030, 67, 3300)])
+def test_every_tile_of_the_gradient_kernels(backend, oracle, m, n, k):
+    """One shape per tile size that the launch picks (rows of weights x columns per lane: 1 x 1, 4 x 1, 8 x 2, 8 x 4; token
+    tiles per wave of grad_act: 1, 2, 4), each with ragged edges. Sums and products in the CPU's order: bits."""
+    print("case vjp tiles", m, n, k, flush=True)
+    rng = np.random.default_rng(m + n + k)
+    packed = oracle.pack_matrix(ternary(rng, n, k), n, k, FMT_TQ2_0)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    sc = rng.uniform(0.05, 1.5, n).astype(np.float32)
+    gy = (rng.standard_normal((m, n)) * 10.0 ** rng.integers(-6, 3, (m, n))).astype(np.float32)
+    gy[0, :] *= np.float32(1e-38)  # products that are denormal
+    rc, ga_w, gw_w, gb_w = oracle.cpu_projected_vjp(packed, FMT_TQ2_0, act, sc, gy, m, n, k)
+    ga, gw, gb = _vjp(backend, packed, FMT_TQ2_0, act, sc, gy, m, n, k)
+    assert rc == 0 and same_bits(ga, ga_w) and same_bits(gw, gw_w) and same_bits(gb, gb_w)
+
+
+def test_product_that_overflows_under_a_zero_trit(backend, oracle):
+    """upstream * scale beyond the largest float: the CPU multiplies the scale with the trit first, so a zero trit still
+    contributes 0 and only the columns with a non-zero trit become infinite."""
+    rng = np.random.default_rng(21)
+    m, n, k = 37, 100, 700
+    packed = oracle.pack_matrix(ternary(rng, n, k), n, k, FMT_TQ2_0)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    sc = rng.uniform(0.05, 1.5, n).astype(np.float32)
+    sc[50] = np.float32(1e30)
+    gy = rng.standard_normal((m, n)).astype(np.float32)
+    gy[17, 50] = np.float32(-1e20)
+    rc, ga_w, gw_w, gb_w = oracle.cpu_projected_vjp(packed, FMT_TQ2_0, act, sc, gy, m, n, k)
+    ga, gw, gb = _vjp(backend, packed, FMT_TQ2_0, act, sc, gy, m, n, k)
+    assert rc == 0 and np.isinf(ga_w[17]).any() and np.isfinite(ga_w[17]).any()
+    assert same_bits(ga, ga_w) and same_bits(gw, gw_w) and same_bits(gb, gb_w)
+
+
 def test_non_finite_values_follow_the_host(backend, oracle):
     """Inf upstream times a zero trit is NaN on the host (upstream * (0 * scale)); so it is here."""
     rng = np.random.default_rng(12)

@@ -7,163 +7,159 @@
 //   grad_w[n,k]   = sum_m upstream[m,n] * act[m,k]                    m = 0, 1, ...
 //   grad_bias[n]  = sum_m upstream[m,n]                               m = 0, 1, ...
 //
-// Both matrix kernels are fp32 vector-ALU bound (one multiply and one add per term, kept apart for
-// the rounding). Weights are read in the device layout of the forward kernels: the 1-KiB chunk of
-// row tile t and K block kb holds, for lane group g = 0..3 and row r = 0..15, the 16 code bytes
-// g*16 .. g*16+15 of that row's block at offset g*256 + r*16; byte i of a block holds the elements
-// (i/32)*128 + s*32 + i%32 at bit pairs s = 0..3, code = trit + 1.
+// Weights are read in the device layout of the forward kernels: the 1-KiB chunk of row tile t and K
+// block kb holds, for lane group g = 0..3 and row r = 0..15, the 16 code bytes g*16 .. g*16+15 of that
+// row's block at offset g*256 + r*16; byte i of a block holds the elements (i/32)*128 + s*32 + i%32 at
+// bit pairs s = 0..3, code = trit + 1.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "tk_internal.h"
 
 #define TKV_GLOBAL __attribute__((address_space(1)))
-#ifndef TKV_ACT_TOK
-#define TKV_ACT_TOK 4  // tokens per thread of the grad_act kernel (2: 3.2 ms, 4: 2.9 ms, 8: 4.5 ms at M=2048 K=2560 N=6912)
-#endif
 
 namespace {
 
-__device__ __forceinline__ float ldg(const float *p) { return *(const TKV_GLOBAL float *)p; }
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// grad_act. A workgroup owns 4*TOK tokens x 4 K blocks; a thread owns TOK tokens x the 16 elements of
-// one code dword (piece g, dword j of its K block), the four waves are the four token groups. Per tile
-// of 16 weight rows the upstream values and scales pass through LDS (two buffers, one barrier a tile).
-template <int TOK>
+__device__ __forceinline__ float ldg(const float *p) { return *(const TKV_GLOBAL float *)p; }
+__device__ __forceinline__ f32x4 ldg4(const float *p) { return *(const TKV_GLOBAL f32x4 *)p; }
+
+// XCD-aware order of `total` workgroups: workgroups are dealt to the eight XCDs in turn, so XCD x takes the
+// x-th eighth of the index range and its L2 holds one compact part of the operands. Grids are 8 * ceil(total / 8).
+__device__ __forceinline__ unsigned xcd_index(unsigned bid, unsigned total) {
+  return (bid & 7u) * ((total + 7u) >> 3) + (bid >> 3);
+}
+
+// ---- grad_act ----
+// The term upstream * (trit * scale) is p * trit with p = upstream * scale rounded once: a trit only negates
+// or clears the product. A product with -1, 0 or 1 is exact, so ONE fused multiply-add per term rounds exactly
+// as the CPU's separate multiply and add -- and the f32 matrix instructions are chains of such fused multiply-adds:
+// v_mfma_f32_16x16x4_f32 adds its four terms in ascending order with one rounding each, denormals kept (compared with
+// fmaf chains bit for bit on the device). So the contraction runs on the matrix pipe in the CPU's order.
+// The one case where p * trit differs from the CPU's term is p overflowing to infinity from finite factors under a zero
+// trit (NaN instead of 0). Such a sum can only end as NaN or infinity, so a wave whose sums do not all end finite
+// repeats them term by term as the CPU computes them.
+//
+// A workgroup owns 16*TT tokens x the 64 columns of one bit pair of a K block; wave g takes piece g of the chunks, of which
+// four rows are the 64 contiguous bytes of one wave-wide load, and every decoded operand serves TT matrix instructions.
+// The products p of 64 weight rows pass through LDS (two buffers, one barrier per 64 rows); codes and upstream
+// values of the next 64 rows are requested before the current ones are used.
+// Bound: the f32 matrix pipe (151 TFLOP/s sustained on the device, 157 published). It shares its multipliers with the vector
+// ALU, so whatever vector work is left (decoding, the products) adds to its time.
+// M=2048 N=6912 K=2560: 0.64 ms = 113 TFLOP/s (2.9 ms as multiply and add per term on the vector ALU); M=64 N=2560
+// K=2560: 31 us (1.06 ms).
+constexpr int ACT_ROWS = 64;  // weight rows per LDS stage
+
+template <int TT>
 __global__ __launch_bounds__(256) void tk_vjp_act_kernel(const uint8_t *__restrict__ codes, int nb, int n, int k, int m,
                                                          const float *__restrict__ scales,
                                                          const float *__restrict__ grad_output,
-                                                         float *__restrict__ grad_act) {
-  constexpr int WT = 4 * TOK;            // tokens per workgroup
-  __shared__ float s_up[2][WT][16];      // [buffer][token][row of the tile]
-  __shared__ float s_sc[2][16];
-  const int tid = threadIdx.x;
-  const int set = tid >> 4, ls = tid & 15, g = ls >> 2, j = ls & 3;
-  const int kb = blockIdx.x * 4 + (set & 3), mg = set >> 2;
-  const int m0 = blockIdx.y * WT;
-  const int kbc = min(kb, nb - 1);  // blocks past the end re-read the last one; nothing of them is stored
-  const int n_tiles = (n + 15) >> 4;
-  float acc[TOK][16];
+                                                         float *__restrict__ grad_act, int wide) {
+  __shared__ float s_p[2][16 * TT][ACT_ROWS + 4];  // [buffer][token][row]; the stride keeps a wave's reads on 64 banks
+  const unsigned cols = (unsigned)nb * 4, total = cols * (unsigned)((m + 16 * TT - 1) / (16 * TT));
+  const unsigned idx = xcd_index(blockIdx.x, total);
+  if (idx >= total) return;
+  const int m0 = (int)(idx / cols) * (16 * TT), kb = (int)(idx % cols) >> 2, pair = (int)(idx & 3);
+  const int tid = threadIdx.x, g = tid >> 6, lane = tid & 63, c = lane & 15, h = lane >> 4;
+  const int n_tiles = (n + 15) >> 4, stages = (n + ACT_ROWS - 1) / ACT_ROWS;
+  // staging: a thread takes four rows of UT tokens; addresses are a uniform base per stage and a lane offset, which
+  // costs the vector ALU nothing (it shares its lanes with the f32 matrix pipe: their times add up)
+  constexpr int QUADS = ACT_ROWS / 4, TPR = 256 / QUADS, UT = 16 * TT / TPR;
+  const int ti = tid / QUADS, q = tid % QUADS * 4;
+  const float *up_base = grad_output + (size_t)m0 * n;
+  unsigned up_off[UT];
 #pragma unroll
-  for (int i = 0; i < TOK; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+  for (int t = 0; t < UT; ++t) up_off[t] = (unsigned)(min(ti + TPR * t, m - 1 - m0) * n + q);  // (past the end: not stored)
+  const unsigned code_off = (unsigned)(kb * 1024 + g * 256 + lane);
 
-  auto stage = [&](int buf, int t) {
-    if (tid < WT * 16) {
-      const int mi = m0 + (tid >> 4), ni = t * 16 + (tid & 15);
-      s_up[buf][tid >> 4][tid & 15] = (mi < m && ni < n) ? ldg(grad_output + (size_t)mi * n + ni) : 0.0f;
+  f32x4 u[UT], sc;
+  uint32_t w[ACT_ROWS / 4];
+  auto request = [&](int st) {
+    const int r = st * ACT_ROWS;
+    const float *ub = up_base + r, *sb = scales + r;
+    if (wide && r + ACT_ROWS <= n) {  // (uniform)
+#pragma unroll
+      for (int t = 0; t < UT; ++t) u[t] = ldg4(ub + up_off[t]);
+      sc = ldg4(sb + (unsigned)q);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = r + q + e < n;
+#pragma unroll
+        for (int t = 0; t < UT; ++t) u[t][e] = in ? ldg(ub + (up_off[t] + e)) : 0.0f;
+        sc[e] = in ? ldg(sb + (unsigned)(q + e)) : 0.0f;  // rows past the end: p = 0, and adding +-0 changes nothing
+      }
     }
-    if (tid < 16) s_sc[buf][tid] = (t * 16 + tid < n) ? ldg(scales + t * 16 + tid) : 0.0f;
+#pragma unroll
+    for (int t = 0; t < ACT_ROWS / 16; ++t) {
+      const uint8_t *cp = codes + (size_t)min(st * (ACT_ROWS / 16) + t, n_tiles - 1) * nb * 1024;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) w[t * 4 + x] = *(const TKV_GLOBAL uint8_t *)(cp + (code_off + x * 64));
+    }
   };
-  stage(0, 0);
-  __syncthreads();
-  for (int t = 0; t < n_tiles; ++t) {
-    const int buf = t & 1;
-    if (t + 1 < n_tiles) stage(buf ^ 1, t + 1);
-    const int rmax = min(16, n - t * 16);
-    const uint8_t *cp = codes + ((size_t)t * nb + kbc) * 1024 + g * 256 + j * 4;
-    uint32_t w[16];
+  f32x4 acc[TT];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) w[r] = *(const TKV_GLOBAL uint32_t *)(cp + r * 16);  // padding rows of the last tile exist
+  for (int t = 0; t < TT; ++t) acc[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  request(0);
+  for (int st = 0; st < stages; ++st) {
+    float(*buf)[ACT_ROWS + 4] = s_p[st & 1];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      if (r < rmax) {  // uniform
-        const float s = s_sc[buf][r];
-        float u[TOK];
+    for (int t = 0; t < UT; ++t) {
+      f32x4 p;
 #pragma unroll
-        for (int i = 0; i < TOK; ++i) u[i] = s_up[buf][mg * TOK + i][r];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          // e = b*4 + sl: byte b of the dword, bit pair sl
-          const int code = (int)((w[r] >> (8 * (e >> 2) + 2 * (e & 3))) & 3u);
-          const float projected = __fmul_rn((float)(code - 1), s);
-#pragma unroll
-          for (int i = 0; i < TOK; ++i) acc[i][e] = __fadd_rn(acc[i][e], __fmul_rn(u[i], projected));
-        }
-      }
+      for (int e = 0; e < 4; ++e) p[e] = __fmul_rn(u[t][e], sc[e]);
+      *(f32x4 *)&buf[ti + TPR * t][q] = p;
     }
+    uint32_t v[ACT_ROWS / 4];
+#pragma unroll
+    for (int x = 0; x < ACT_ROWS / 4; ++x) v[x] = w[x];
     __syncthreads();
+    if (st + 1 < stages) request(st + 1);
+#pragma unroll
+    for (int x = 0; x < ACT_ROWS / 4; ++x) {
+      const float b = (float)((v[x] >> (2 * pair)) & 3u) - 1.0f;
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(buf[16 * t + c][x * 4 + h], b, acc[t], 0, 0, 0);
+    }
   }
-  if (kb >= nb) return;
-  // byte b of this dword is byte i = g*16 + j*4 + b of the block: elements (g/2)*128 + sl*32 + (g%2)*16 + j*4 + b
-  const int e0 = kb * 256 + (g >> 1) * 128 + (g & 1) * 16 + j * 4;
+  bool finite = true;
 #pragma unroll
-  for (int i = 0; i < TOK; ++i) {
-    const int mi = m0 + mg * TOK + i;
-    if (mi >= m) continue;
-    float *row = grad_act + (size_t)mi * k;
+  for (int t = 0; t < TT; ++t)
 #pragma unroll
-    for (int sl = 0; sl < 4; ++sl)
+    for (int r = 0; r < 4; ++r) finite &= fabsf(acc[t][r]) < __builtin_inff();
+  const bool repeat = __ballot(!finite) != 0;
+  // byte c of piece g, bit pair s: element (g/2)*128 + s*32 + (g%2)*16 + c of the K block
+  const int kk = kb * 256 + (g >> 1) * 128 + pair * 32 + (g & 1) * 16 + c;
+  if (kk >= k) return;
+  if (!repeat) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int kk = e0 + sl * 32 + b;
-        if (kk < k) *(TKV_GLOBAL float *)(row + kk) = acc[i][b * 4 + sl];
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int mi = m0 + t * 16 + h * 4 + r;
+        if (mi < m) *(TKV_GLOBAL float *)(grad_act + (size_t)mi * k + kk) = acc[t][r];
       }
+    return;
+  }
+  for (int r = 0; r < 4 * TT; ++r) {
+    const int mi = m0 + (r >> 2) * 16 + h * 4 + (r & 3);
+    if (mi >= m) return;
+    float sum = 0.0f;
+    for (int row = 0; row < n; ++row) {
+      const uint32_t byte = *(const TKV_GLOBAL uint8_t *)(codes + ((size_t)(row >> 4) * nb + kb) * 1024 + g * 256 + (row & 15) * 16 + c);
+      const float trit = (float)((byte >> (2 * pair)) & 3u) - 1.0f;
+      sum = __fadd_rn(sum, __fmul_rn(ldg(grad_output + (size_t)mi * n + row), __fmul_rn(trit, ldg(scales + row))));
+    }
+    *(TKV_GLOBAL float *)(grad_act + (size_t)mi * k + kk) = sum;
   }
 }
 
-// grad_w. A workgroup owns 64 weight rows x 64 columns, a thread 4 x 4 of them; tokens pass through
-// LDS sixteen at a time (two buffers, one barrier per sixteen).
-__global__ __launch_bounds__(256) void tk_vjp_weight_kernel(int n, int k, int m, const float *__restrict__ act,
-                                                            const float *__restrict__ grad_output,
-                                                            float *__restrict__ grad_w) {
-  __shared__ __attribute__((aligned(16))) float s_act[2][16][64];
-  __shared__ __attribute__((aligned(16))) float s_up[2][16][64];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int k0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-  float acc[4][4];
-#pragma unroll
-  for (int y = 0; y < 4; ++y)
-#pragma unroll
-    for (int x = 0; x < 4; ++x) acc[y][x] = 0.0f;
-  auto stage = [&](int buf, int mt) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int idx = tid + 256 * q, i = idx >> 6, c = idx & 63;
-      const int mi = mt * 16 + i;
-      s_act[buf][i][c] = (mi < m && k0 + c < k) ? ldg(act + (size_t)mi * k + k0 + c) : 0.0f;
-      s_up[buf][i][c] = (mi < m && n0 + c < n) ? ldg(grad_output + (size_t)mi * n + n0 + c) : 0.0f;
-    }
-  };
-  const int m_tiles = (m + 15) >> 4;
-  stage(0, 0);
-  __syncthreads();
-  for (int mt = 0; mt < m_tiles; ++mt) {
-    const int buf = mt & 1;
-    if (mt + 1 < m_tiles) stage(buf ^ 1, mt + 1);
-    const int imax = min(16, m - mt * 16);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (i < imax) {  // uniform
-        const float4 a = *(const float4 *)&s_act[buf][i][tx * 4];
-        const float4 u = *(const float4 *)&s_up[buf][i][ty * 4];
-        const float av[4] = {a.x, a.y, a.z, a.w}, uv[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int y = 0; y < 4; ++y)
-#pragma unroll
-          for (int x = 0; x < 4; ++x) acc[y][x] = __fadd_rn(acc[y][x], __fmul_rn(uv[y], av[x]));
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int y = 0; y < 4; ++y) {
-    const int ni = n0 + ty * 4 + y;
-    if (ni >= n) continue;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int kk = k0 + tx * 4 + x;
-      if (kk < k) *(TKV_GLOBAL float *)(grad_w + (size_t)ni * k + kk) = acc[y][x];
-    }
-  }
-}
-
-// grad_bias. One thread per column walks the tokens in order; a wave covers 64 adjacent columns, and
-// 32 loads are in flight per thread (the additions stay in token order).
-__global__ __launch_bounds__(64) void tk_vjp_bias_kernel(int n, int m, const float *__restrict__ grad_output,
-                                                         float *__restrict__ grad_bias) {
-  const int ni = blockIdx.x * 64 + threadIdx.x;
+// ---- grad_bias ----
+// One thread per column walks the tokens in order, 32 loads in flight per thread.
+__device__ __forceinline__ void bias_column(int ni, int n, int m, const float *__restrict__ grad_output,
+                                            float *__restrict__ grad_bias) {
   if (ni >= n) return;
   float acc = 0.0f;
   int mi = 0;
@@ -178,6 +174,112 @@ __global__ __launch_bounds__(64) void tk_vjp_bias_kernel(int n, int m, const flo
   *(TKV_GLOBAL float *)(grad_bias + ni) = acc;
 }
 
+__global__ __launch_bounds__(64) void tk_vjp_bias_kernel(int n, int m, const float *__restrict__ grad_output,
+                                                         float *__restrict__ grad_bias) {
+  bias_column(blockIdx.x * 64 + threadIdx.x, n, m, grad_output, grad_bias);
+}
+
+// ---- grad_w ----
+// Here both factors are arbitrary, so a term needs its own rounded product: one multiply and one add on the vector
+// ALU (two waves per SIMD issue 69 T lane operations a second on the device; the matrix pipe as the multiplier and the
+// vector ALU as the adder measured slower: 22 against 35 T terms). A wave owns TN weight rows x 64*TK columns. Its upstream values are the
+// same for every lane: they come through scalar loads and are the multiply's scalar operand, so a token costs a lane one
+// load of TK activations for 2*TN*TK operations and nothing passes through LDS (64 x 64 tiles through LDS read two
+// 16-byte pieces per 32 operations and were held back by that). Lanes and waves past the end of a row repeat
+// the last whole piece: the same values are stored twice.
+// The first bias_blocks workgroups sum the columns of grad_bias beside the others (33 us as a launch of its own).
+// M=2048 N=6912 K=2560: 1.36 ms with the bias (1.55 + 0.03 ms with 64 x 64 tiles through LDS).
+constexpr int W_TOK = 4;  // tokens per step
+
+template <int TN, int TK>
+__global__ __launch_bounds__(256) void tk_vjp_weight_kernel(int n, int k, int m, const float *__restrict__ act,
+                                                            const float *__restrict__ grad_output,
+                                                            float *__restrict__ grad_w, float *__restrict__ grad_bias,
+                                                            int bias_blocks) {
+  typedef float piece __attribute__((ext_vector_type(TK), aligned(4)));
+  if ((int)blockIdx.x < bias_blocks) {
+    bias_column(blockIdx.x * 256 + threadIdx.x, n, m, grad_output, grad_bias);
+    return;
+  }
+  const unsigned k_tiles = (unsigned)(k + 64 * TK - 1) / (64 * TK), n_tiles = (unsigned)(n + 4 * TN - 1) / (4 * TN);
+  const unsigned idx = xcd_index(blockIdx.x - bias_blocks, k_tiles * n_tiles);
+  if (idx >= k_tiles * n_tiles) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int nw = (int)(idx / k_tiles) * (4 * TN) + wave * TN;
+  if (nw >= n) return;
+  const int n0 = min(nw, n - TN), k0 = min((int)(idx % k_tiles) * (64 * TK) + lane * TK, k - TK);
+  const float *ap = act + k0, *up = grad_output + n0;
+  float acc[TN][TK];
+#pragma unroll
+  for (int y = 0; y < TN; ++y)
+#pragma unroll
+    for (int x = 0; x < TK; ++x) acc[y][x] = 0.0f;
+  auto fold = [&](const piece &a, const float (&u)[TN]) {
+#pragma unroll
+    for (int y = 0; y < TN; ++y)
+#pragma unroll
+      for (int x = 0; x < TK; ++x) acc[y][x] = __fadd_rn(acc[y][x], __fmul_rn(u[y], a[x]));
+  };
+  auto request = [&](int mi, piece &a, float (&u)[TN]) {
+    a = *(const TKV_GLOBAL piece *)(ap + (size_t)mi * k);
+#pragma unroll
+    for (int y = 0; y < TN; ++y) u[y] = up[(size_t)mi * n + y];
+  };
+  piece a[W_TOK];
+  float u[W_TOK][TN];
+#pragma unroll
+  for (int i = 0; i < W_TOK; ++i) request(min(i, m - 1), a[i], u[i]);
+  int mi = 0;
+#pragma unroll 2
+  for (; mi + W_TOK <= m; mi += W_TOK) {
+    piece an[W_TOK];
+    float un[W_TOK][TN];
+#pragma unroll
+    for (int i = 0; i < W_TOK; ++i) request(min(mi + W_TOK + i, m - 1), an[i], un[i]);
+#pragma unroll
+    for (int i = 0; i < W_TOK; ++i) fold(a[i], u[i]);
+#pragma unroll
+    for (int i = 0; i < W_TOK; ++i) {
+      a[i] = an[i];
+#pragma unroll
+      for (int y = 0; y < TN; ++y) u[i][y] = un[i][y];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < W_TOK - 1; ++i)
+    if (mi + i < m) fold(a[i], u[i]);
+#pragma unroll
+  for (int y = 0; y < TN; ++y) {
+    piece out;
+#pragma unroll
+    for (int x = 0; x < TK; ++x) out[x] = acc[y][x];
+    *(TKV_GLOBAL piece *)(grad_w + (size_t)(n0 + y) * k + k0) = out;
+  }
+}
+
+}  // namespace
+
+namespace {
+
+constexpr size_t SIMDS = 1024;  // 256 CUs x 4
+
+template <int TT>
+void launch_act(hipStream_t s, const uint8_t *codes, size_t nb, size_t n, size_t k, size_t m, const float *scales,
+                const float *grad_output, float *grad_act, int wide) {
+  const size_t total = nb * 4 * ((m + 16 * TT - 1) / (16 * TT));
+  hipLaunchKernelGGL(tk_vjp_act_kernel<TT>, dim3((unsigned)((total + 7) / 8 * 8)), dim3(256), 0, s, codes, (int)nb,
+                     (int)n, (int)k, (int)m, scales, grad_output, grad_act, wide);
+}
+
+template <int TN, int TK>
+void launch_weight(hipStream_t s, size_t n, size_t k, size_t m, const float *act, const float *grad_output, float *grad_w,
+                   float *grad_bias) {
+  const size_t tiles = ((k + 64 * TK - 1) / (64 * TK)) * ((n + 4 * TN - 1) / (4 * TN));
+  const unsigned bias_blocks = grad_bias ? (unsigned)((n + 255) / 256) : 0;
+  hipLaunchKernelGGL((tk_vjp_weight_kernel<TN, TK>), dim3(bias_blocks + (unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, s,
+                     (int)n, (int)k, (int)m, act, grad_output, grad_w, grad_bias, (int)bias_blocks);
+}
+
 }  // namespace
 
 // m, n, k > 0 for the matrix kernels (the caller has zero-filled or skipped the degenerate shapes);
@@ -186,18 +288,27 @@ hipError_t tk_launch_projected_vjp(hipStream_t s, const uint8_t *codes, size_t n
                                    const float *scales, const float *act, const float *grad_output, float *grad_act,
                                    float *grad_w, float *grad_bias) {
   if (grad_act && m && n && k) {
-    constexpr int TOK = TKV_ACT_TOK;
-    dim3 grid((unsigned)((nb + 3) / 4), (unsigned)((m + 4 * TOK - 1) / (4 * TOK)));
-    hipLaunchKernelGGL(tk_vjp_act_kernel<TOK>, grid, dim3(256), 0, s, codes, (int)nb, (int)n, (int)k, (int)m, scales,
-                       grad_output, grad_act);
+    const int wide = n % 4 == 0 && (uintptr_t)grad_output % 16 == 0 && (uintptr_t)scales % 16 == 0;
+    // More tokens per wave share a decoded operand (vector work adds to the matrix time), fewer leave more waves. In
+    // 16 x 16 tiles of the output, tiles per wave 1 / 2 / 4, N=2560: 640 tiles 31 / 43 / 62 us, 2560 tiles 60 / 67 / 63,
+    // 10240 tiles 168 / 143 / 147; N=6912: 5120 tiles 238 / 241 / 274, 20480 tiles 871 / 732 / 640.
+    const size_t tiles = nb * 16 * ((m + 15) / 16);
+    if (tiles <= 4 * SIMDS) launch_act<1>(s, codes, nb, n, k, m, scales, grad_output, grad_act, wide);
+    else if (tiles <= 12 * SIMDS) launch_act<2>(s, codes, nb, n, k, m, scales, grad_output, grad_act, wide);
+    else launch_act<4>(s, codes, nb, n, k, m, scales, grad_output, grad_act, wide);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (grad_w && m && n && k) {
-    dim3 grid((unsigned)((k + 63) / 64), (unsigned)((n + 63) / 64));
-    hipLaunchKernelGGL(tk_vjp_weight_kernel, grid, dim3(256), 0, s, (int)n, (int)k, (int)m, act, grad_output, grad_w);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    const size_t outs = n * k;
+    // The larger the tile of a wave, the more operations per load; the launch should still have some four waves per SIMD.
+    // Rows x columns per lane 4x1 / 8x2 / 8x4: 0.5 M outputs (M=712) 57 / 79 / 108 us, 1.8 M (M=300) 64 / 38 / 50, 6.5 M
+    // (M=1024) 591 / 305 / 336, 17.7 M (M=2048) 3014 / 1455 / 1385.
+    if (n < 4) launch_weight<1, 1>(s, n, k, m, act, grad_output, grad_w, grad_bias);
+    else if (k < 4 || n < 8 || outs < (size_t)1 << 20) launch_weight<4, 1>(s, n, k, m, act, grad_output, grad_w, grad_bias);
+    else if (outs < (size_t)1 << 23) launch_weight<8, 2>(s, n, k, m, act, grad_output, grad_w, grad_bias);
+    else launch_weight<8, 4>(s, n, k, m, act, grad_output, grad_w, grad_bias);
+    return hipGetLastError();
   }
   if (grad_bias && n) {
     hipLaunchKernelGGL(tk_vjp_bias_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, (int)n, (int)m,
