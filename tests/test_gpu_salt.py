@@ -168,3 +168,35 @@ def test_every_f16_block_scale_reaches_the_kernels_exactly(backend, oracle):
     assert (~np.isfinite(got[~finite])).all()
     for a in (dact, dout, buf):
         a.free()
+
+
+@pytest.mark.parametrize("m,n,k,t_planes,dtype", [(17, 130, 256, 1, "f32"), (33, 33, 700, 2, "f32"), (64, 257, 2560, 3, "bf16"), (65, 15, 1000, 4, "f32"),
+                                                  (130, 96, 2048, 2, "bf16"), (1027, 40, 300, 1, "f32"),
+                                                  (512, 4100, 300, 1, "f32"),  # the 64-column waves
+                                                  (9, 70, 5000, 2, "f32")])    # seven such tokens fit the flow form
+def test_many_tokens_have_the_bits_of_sixteen_at_a_time(backend, oracle, m, n, k, t_planes, dtype):
+    """The many-token form adds the same exact block values in the same order as the flow form: identical bits, rows past the
+    last row tile, columns past the last pair, a token holding NaN and a second pass of tokens included."""
+    print("case salt-many", m, n, k, t_planes, dtype, flush=True)
+    rng = np.random.default_rng(m * 19 + n + k + t_planes)
+    packed, bufs = make_planes(backend, oracle, rng, n, k, t_planes)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    act[m // 2, k // 3] = np.nan
+    host = f32_to_bf16_bits(act) if dtype == "bf16" else act
+    dout = backend.empty(m * n, dtype)
+    many = backend.to_device(host, dtype)
+    backend.linear_salt(bufs, many, m, dout)
+    got = dout.to_host().reshape(m, n)
+    want = np.empty_like(got)
+    rows = np.asarray(host).reshape(m, k)
+    step = 16 if k <= 2560 else 4
+    for m0 in range(0, m, step):
+        part = rows[m0:m0 + step]
+        dact, dpart = backend.to_device(part, dtype), backend.empty(len(part) * n, dtype)
+        backend.linear_salt(bufs, dact, len(part), dpart)
+        want[m0:m0 + step] = dpart.to_host().reshape(-1, n)
+        dact.free()
+        dpart.free()
+    assert same_bits(got, want) if dtype == "f32" else (got == want).all()
+    for a in [many, dout] + bufs:
+        a.free()

@@ -1531,6 +1531,8 @@ extern "C" int tk_linear_rmsnorm_a8(tk_ctx *ctx, const tk_linear_desc *layer, co
   return run_linear(ctx, layer, TK_MODE_INT8, TK_PREP_A8, x, x_dtype, nullptr, m, out, out_dtype, norm);
 }
 
+constexpr size_t kSaltTokens = 1024;  // tokens per pass of the many-token form of the block-scale planes
+
 // Block-scale additive planes on float activations. seq != 0 forces the reference-order kernel.
 static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int act_dtype, size_t m, void *out,
                     int out_dtype, bool seq) {
@@ -1576,19 +1578,36 @@ static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int
   pr.raw_act = act;
   pr.raw_dtype = act_dtype;
   pr.out = out;
-  // More than 16 tokens: slices of 16 go through the matrix-core form one after the other (each
-  // streams the planes again; a block-scale form of the prefill kernel does not exist yet).
-  if (!seq && m > 16 && nb * 256 * 64 + nb * 64 * 4 <= kLdsFlowMax) {
-    const size_t asz = act_dtype == TK_BF16 ? 2 : 4, osz = out_dtype == TK_BF16 ? 2 : 4;
-    for (size_t m0 = 0; m0 < m; m0 += 16) {
-      const size_t mc = m - m0 < 16 ? m - m0 : 16;
+  // Up to 16 tokens whose operand rows (and their per-block sums) fit LDS take the flow form. More take the many-token form,
+  // up to kSaltTokens of them per pass (its operand rows are a workspace of 4 * k bytes a token), where the rows of four
+  // tokens would fit (K <= 9,984); beyond that the header promises the host's order. Where that workspace cannot grow now
+  // (memory, a stream that is being captured), passes of as many tokens as the flow form takes: same bits.
+  // Two planes, flow / many-token form: K=2048 N=8192 4 tokens 14.4 / 19.5 us, 8 tokens 16.5 / 20.2, 16 tokens 21.5 / 21.2; 128
+  // tokens 172 in passes of 16 / 26.5.
+  const size_t asz = act_dtype == TK_BF16 ? 2 : 4, osz = out_dtype == TK_BF16 ? 2 : 4;
+  const size_t token_lds = nb * 256 * 4 + nb * 4 * 4;
+  const size_t flow_tokens = nb ? std::min<size_t>(16, kLdsFlowMax / token_lds) : 16;
+  const bool many = !seq && flow_tokens >= 4 && m > flow_tokens;
+  bool gemm = many && nb && m <= kSaltTokens;
+  if (gemm && !(R * nb * 256 <= ctx->ap.cap && R * 4 <= ctx->rowsum.cap && m * 4 <= ctx->exps.cap && m * 4 <= ctx->flags.cap &&
+                nb * R * 4 <= ctx->blocksum.cap)) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(ctx->stream, &st));
+    gemm = st == hipStreamCaptureStatusNone && ensure(ctx, ctx->ap, R * nb * 256) == TK_OK &&
+           ensure(ctx, ctx->rowsum, R * 4) == TK_OK && ensure(ctx, ctx->exps, m * 4) == TK_OK &&
+           ensure(ctx, ctx->flags, m * 4) == TK_OK && ensure(ctx, ctx->blocksum, nb * R * 4) == TK_OK;
+  }
+  if (many && !gemm) {
+    const size_t step = m > kSaltTokens ? kSaltTokens : flow_tokens;
+    for (size_t m0 = 0; m0 < m; m0 += step) {
+      const size_t mc = m - m0 < step ? m - m0 : step;
       TKCHK(run_salt(ctx, layer, (const uint8_t *)act + m0 * k * asz, act_dtype, mc, (uint8_t *)out + m0 * n * osz,
                      out_dtype, false));
     }
     return TK_OK;
   }
   const size_t lds = nb * 256 * R + nb * R * 4;  // operand rows + their per-block sums
-  if (seq || R > 64 || lds > kLdsFlowMax) {
+  if (seq || (!gemm && m > flow_tokens)) {
     HIPCHK(tk_launch_salt_seq(ctx->stream, &pr));
     return TK_OK;
   }
@@ -1616,6 +1635,10 @@ static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int
   pr.exps = pp.exps;
   pr.flags = pp.flags;
   pr.blocksum = pp.blocksum;
+  if (gemm) {
+    HIPCHK(tk_launch_salt_gemm(ctx->stream, &pr, ctx->info.compute_units));
+    return TK_OK;
+  }
   TkLaunchCfg cfg = {};
   cfg.planes = layer->n_planes;
   cfg.rt = R <= 16 ? 1 : (R <= 32 ? 2 : 4);

@@ -134,6 +134,26 @@ __device__ __noinline__ float seq_dot_raw(const uint8_t *codes, int nb, int kdim
   return acc;
 }
 
+// Block-scale planes in the host's order, exactly: dequantize a weight (planes in order), one f32 accumulator over k
+// (crates/tritium-nn/src/layers/packed_salt.rs:585-628). For launches the matrix-core forms do not take and for tokens
+// holding NaN or Inf.
+__device__ __noinline__ float salt_exact_dot(const TkProblem &pr, int n, int tok) {
+  const int nb = pr.nb, kdim = pr.k, planes = pr.planes;
+  const size_t tile_base = (size_t)(n >> 4) * nb;
+  float acc = 0.0f;
+  for (int kb = 0; kb < nb; ++kb) {
+    float sc[TK_MAX_PLANES];
+    for (int p = 0; p < planes; ++p) sc[p] = pr.bscale[p][(tile_base + kb) * 16 + (n & 15)];
+    const int kend = min(kdim, (kb + 1) * 256);
+    for (int k = kb * 256; k < kend; ++k) {
+      float w = 0.0f;
+      for (int p = 0; p < planes; ++p) w = __fadd_rn(w, __fmul_rn(sc[p], (float)(code_at(pr.codes[p], nb, n, k) - 1)));
+      acc = __fadd_rn(acc, __fmul_rn(load_act(pr.raw_act, pr.raw_dtype, (size_t)tok * kdim + k), w));
+    }
+  }
+  return acc;
+}
+
 __device__ __forceinline__ float seq_dot(const TkProblem &pr, int p, int n, int tok, int a8) {
   const float s = a8 ? pr.aux[tok] : 0.0f;
   const int gamma_zero = a8 && pr.act_scale[tok] == 0.0f;

@@ -217,6 +217,8 @@ int tk_flow32_runs_per_wave(void);
 // reference-order kernel for everything else
 hipError_t tk_launch_salt_flow(hipStream_t s, const TkProblem *single, const TkLaunchCfg &cfg);
 hipError_t tk_launch_salt_seq(hipStream_t s, const TkProblem *single);
+// many tokens or long rows (tk_salt_gemm.hip): operand rows in memory, any K
+hipError_t tk_launch_salt_gemm(hipStream_t s, const TkProblem *single, int compute_units);
 hipError_t tk_launch_gemm(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob,
                           const TkLaunchCfg &cfg);
 // 128 x 256 prefill kernel (tk_gemm128.hip): one plane, int8 contract, f32 / bf16 rows of whole 16-byte pieces,

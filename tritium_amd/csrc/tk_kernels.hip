@@ -326,25 +326,6 @@ __global__ __launch_bounds__(TK_WG) void tk_stream_kernel(TkProblem single, cons
 // (crates/tritium-cuda/kernels/tq2_0_add.cu:640-719).
 // ------------------------------------------------------------------------------------------
 
-// The host's order, exactly: used for launches the flow form does not take and for tokens holding
-// NaN or Inf.
-__device__ __noinline__ float salt_exact_dot(const TkProblem &pr, int n, int tok) {
-  const int nb = pr.nb, kdim = pr.k, planes = pr.planes;
-  const size_t tile_base = (size_t)(n >> 4) * nb;
-  float acc = 0.0f;
-  for (int kb = 0; kb < nb; ++kb) {
-    float sc[TK_MAX_PLANES];
-    for (int p = 0; p < planes; ++p) sc[p] = pr.bscale[p][(tile_base + kb) * 16 + (n & 15)];
-    const int kend = min(kdim, (kb + 1) * 256);
-    for (int k = kb * 256; k < kend; ++k) {
-      float w = 0.0f;
-      for (int p = 0; p < planes; ++p) w = __fadd_rn(w, __fmul_rn(sc[p], (float)(code_at(pr.codes[p], nb, n, k) - 1)));
-      acc = __fadd_rn(acc, __fmul_rn(load_act(pr.raw_act, pr.raw_dtype, (size_t)tok * kdim + k), w));
-    }
-  }
-  return acc;
-}
-
 __global__ __launch_bounds__(TK_WG) void tk_salt_seq_kernel(TkProblem pr) {
   size_t idx = (size_t)blockIdx.x * TK_WG + threadIdx.x;
   size_t total = (size_t)pr.M * pr.n;
