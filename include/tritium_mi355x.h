@@ -552,7 +552,7 @@ int tk_set_fuse_tokens(tk_ctx *ctx, int tokens);
 /* Calls of this context so far that ran in that single-launch form (for tests of the dispatch). */
 int tk_get_fused_calls(tk_ctx *ctx, unsigned long long *count);
 /* Name of the contraction kernel the last single call of this context (tk_linear_*, tk_mpgemm*) took:
- * "flow", "flow32", "flow3", "stream", "ksplit_decode", "gemm64", "gemm64_ksplit", "gemm128", "gemm256";
+ * "flow", "flow32", "flow3", "stream", "ksplit_decode", "waves", "gemm64", "gemm64_ksplit", "gemm128", "gemm256";
  * "" before the first call. A static string. For tests of the dispatch; no counterpart in the reference. */
 const char *tk_last_kernel(tk_ctx *ctx);
 /* Row count of the workgroup tile for single launches of one plane under the int8 contract (f32 or bf16

@@ -744,7 +744,34 @@ struct Plan {
   size_t flow_lds;
 };
 
-enum { DECODE_AUTO = 0, DECODE_KSPLIT = 1, DECODE_STREAM = 2, DECODE_FLOW = 3, DECODE_GEMM = 4 };
+enum { DECODE_AUTO = 0, DECODE_KSPLIT = 1, DECODE_STREAM = 2, DECODE_FLOW = 3, DECODE_GEMM = 4, DECODE_WAVES = 5 };
+
+// Calls and groups that take the eight-wave kernel of small batches (tk_waves.hip) instead of `variant`: `pairs`
+// workgroups (32 columns each). It wins where they run side by side, two per CU (one for two planes beyond 32 rows), and
+// loses to the flow or prefill kernel, which reuse what they staged, once a second round begins. Call, before -> this, int8
+// rows, bf16 tokens: one plane K=2560 N=2560 4 / 16 / 32 / 64 tokens 10.1 -> 8.9 / 12.2 -> 9.3 / 14.2 -> 9.5 / 14.4 -> 10.1 us;
+// K=6912 N=2560 13.0 -> 10.8 / 16.9 -> 11.2 / 17.0 -> 11.8 / 17.5 -> 13.9; K=5120 N=10240 (320 workgroups) 3 / 16 / 64 tokens
+// two planes 14.3 -> 13.5 / 18.8 -> 14.2 / 22.0 -> 23.1, three planes 16.5 -> 16.6 / 22.4 -> 17.5; N=17408 (544) K=2560 3 / 16 / 64
+// tokens one plane 11.5 -> 10.9 / 17.6 -> 12.6 / 14.8 -> 15.8, two 12.4 -> 13.2 / 20.4 -> 14.9 / 18.1 -> 23.3, three 14.1 -> 15.9 /
+// 15.8 -> 17.0, but K=5120 8 float tokens two planes 23.8 -> 19.5, three 28.3 -> 23.4: a few workgroups beyond the round are
+// worth it for one plane or long rows. Two planes and more of short rows (K <= 1024), up to eight rows: 8.3 -> 8.7 .. 9.8 -> 8.9,
+// left alone. Groups, 48 x K=1024 N=1024 16 tokens 11.0 -> 14.9; but rows beyond LDS in one row tile, which the streaming
+// kernel would stage K slice by K slice, six of K=6912 N=6912 16 tokens 54.9 -> 28.8 (one plane), 81 -> 48 (three).
+// (a context with a kernel form forced keeps it; two int8 tokens and one float token run as one launch in the decode kernels; planes with a zero-chunk map keep the flow
+// kernel, which skips their chunks; three planes beyond 32 rows keep the K-split prefill kernel)
+static bool waves_pays(const tk_ctx *ctx, bool flow_ok, bool zskip, int planes, size_t rows, size_t tokens, size_t pairs, size_t nb,
+                       int mode, bool group) {
+  if (ctx->decode_force != DECODE_AUTO || ctx->flow_run_tiles || ctx->flow_ring || ctx->flow_mfma || ctx->flow_wg16 > 0 || !ctx->flow_swap ||
+      ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit || ctx->gemm_rows || ctx->stream_min_groups < ctx->info.compute_units ||
+      (ctx->fuse_tokens > 0 && tokens <= (size_t)ctx->fuse_tokens))
+    return false;
+  if (zskip || planes > 3 || tokens < (mode == TK_MODE_INT8 ? 3u : 2u)) return false;
+  if (rows > (planes == 3 ? 32u : 64u) || nb == 0) return false;
+  if (planes >= 2 && nb <= 4 && rows <= 8) return false;
+  if (group && !flow_ok && rows <= 16) return true;
+  const size_t round = (rows <= 32 || planes == 1 ? 2 : 1) * (size_t)ctx->info.compute_units;
+  return pairs <= round || (rows <= 32 && (planes == 1 || nb >= 16) && pairs * 16 <= round * 17);
+}
 
 static const size_t kLdsFlowMax = 160 * 1024;
 // Waves per workgroup of the flow kernels: four up to 64 KiB of operand rows, eight beyond; with two row tiles and
@@ -1209,6 +1236,7 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
   int variant = DECODE_KSPLIT, run_tiles = 1;
   unsigned flow_groups = 0;
   bool wide = false, b3 = false;
+  const bool decode = pl.skinny;
   size_t flow_lds = pl.flow_lds;
   if (pl.skinny) {
     b3 = pl.flow_ok && flow_base3(pl.pr, pl.cfg.planes, pl.cfg.rt, flow_lds);
@@ -1290,6 +1318,11 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
       plan_gemm(&pl, 4u * (unsigned)ctx->info.compute_units, ctx->gemm_tiles);
     }
   }
+  const bool waves = decode && !b3 && waves_pays(ctx, pl.flow_ok, pl.pr.zskip != 0, pl.cfg.planes, R, m, ((size_t)pl.pr.n_tiles + 1) / 2, nb, mode, false);
+  if (waves) {
+    pl.skinny = false;
+    pl.pr.rs = (int)R;
+  }
   // A single decode call of few tokens is two short dependent launches, and the gap between them costs more than
   // either: the flow kernel then builds the operand rows itself, every workgroup for itself (256 threads, at most
   // two 16-byte pieces of a token per thread, straight-line loads: whole K blocks, aligned f32 or bf16 rows).
@@ -1322,7 +1355,7 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
   const bool fused = fused_flow || fused_ksplit;
   // One plane under the int8 contract with whole 16-byte output pieces: the wide-tile prefill kernels.
   const size_t out_esz = out_dtype == TK_BF16 ? 2 : 4;
-  const bool can_wide = !pl.skinny && pl.pr.planes == 1 && mode == TK_MODE_INT8 && (out_dtype == TK_F32 || out_dtype == TK_BF16) &&
+  const bool can_wide = !pl.skinny && !waves && pl.pr.planes == 1 && mode == TK_MODE_INT8 && (out_dtype == TK_F32 || out_dtype == TK_BF16) &&
                         !residual && (n * out_esz) % 16 == 0 && ((uintptr_t)out & 15) == 0;
   int form256 = 0;
   const bool pays256 = gemm256_pays(ctx, R, (size_t)pl.pr.n_tiles, &form256);
@@ -1379,7 +1412,10 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
   } else {
     pr.act_scale = act_scale_in;
   }
-  if (pl.skinny && variant == DECODE_FLOW) {
+  if (waves) {
+    ctx->last_kernel = "waves";
+    HIPCHK(tk_launch_waves(ctx->stream, &pr, nullptr, nullptr, pl.cfg.planes, (int)R, ((unsigned)pr.n_tiles + 1) / 2));
+  } else if (pl.skinny && variant == DECODE_FLOW) {
     TkLaunchCfg cfg = pl.cfg;
     cfg.grid = flow_groups;
     cfg.lds_bytes = flow_lds;
@@ -2203,6 +2239,7 @@ struct tk_group {
   int prep_norm_pieces = 0;  // ... and the largest piece count
   unsigned prep_rows = 0;
   int variant = 1;
+  int rows_max = 0;          // operand rows of the largest member
   size_t wg_prob_off = 0;
   TkLaunchCfg cfg{};
   // a second launch: the members of a prefill-form group whose operand rows do fit in LDS go
@@ -2338,6 +2375,7 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
     if (plans[i].stream_lds > slds) slds = plans[i].stream_lds;
   }
   int variant = choose_decode(ctx, flow_ok, fgroups, sgroups);
+  const bool fits_lds = flow_ok;
   // One token for a group of more than two tiles per CU (gate,up): the flow kernel behind the prep launch, as for single
   // calls (run_linear) -- the K-split kernel would hand its workgroups several tiles each. gate,up of hidden 2560 behind
   // an RMSNorm, rotating over 30 layers: 13.4 -> 11.6 us (2 / 4 / 8 tokens 12.9 -> 12.9 / 13.9 -> 13.2 / 14.7 -> 13.8: left);
@@ -2363,6 +2401,15 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
     variant = DECODE_GEMM;
     flow_ok = false;
     for (size_t i = 0; i < count; ++i) plans[i].flow_ok = false;
+  }
+  {
+    size_t pairs = 0;
+    bool zskip = false;
+    for (size_t i = 0; i < count; ++i) {
+      pairs += ((size_t)plans[i].pr.n_tiles + 1) / 2;
+      zskip = zskip || plans[i].pr.zskip;
+    }
+    if (!b3 && waves_pays(ctx, fits_lds, zskip, planes, rows_max, tokens_max, pairs, nb_max, kmode, true)) variant = DECODE_WAVES;
   }
   std::vector<int> wg_prob;
   int group_gemm_nt = 0;
@@ -2447,7 +2494,7 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
       flow_cfg_form(&flow_cfg, pwide, false, pflds, prows_max, ztiles, pnb_max, kmode == TK_MODE_INT8 && ctx->flow_swap);
     }
   } else if (variant != DECODE_KSPLIT) {
-    const unsigned per = variant == DECODE_FLOW ? fper : tpw;
+    const unsigned per = variant == DECODE_FLOW ? fper : (variant == DECODE_WAVES ? 2u : tpw);
     for (size_t i = 0; i < count; ++i) {
       const unsigned gi = ((unsigned)plans[i].pr.n_tiles + per - 1) / per;
       plans[i].pr.group_begin = (int)groups_total;
@@ -2595,6 +2642,7 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
   g->flow_wg_prob_off = flow_wg_prob_off;
   g->flow_cfg = flow_cfg;
   g->variant = variant;
+  g->rows_max = (int)rows_max;
   g->wg_prob_off = wg_prob_off;
   g->nprobs = (int)count;
   g->nprep = (int)preps.size();
@@ -2717,6 +2765,8 @@ extern "C" int tk_group_launch_parts(tk_ctx *ctx, tk_group *g, int do_prep, int 
   }
   else if (do_main && g->variant == DECODE_GEMM)
     HIPCHK(tk_launch_gemm(ctx->stream, nullptr, probs, wg_prob, g->cfg));
+  else if (do_main && g->variant == DECODE_WAVES)
+    HIPCHK(tk_launch_waves(ctx->stream, nullptr, probs, wg_prob, g->cfg.planes, g->rows_max, g->cfg.grid));
   else if (do_main && g->variant == DECODE_FLOW && g->cfg.base3)
     HIPCHK(tk_launch_flow3(ctx->stream, nullptr, probs, wg_prob, g->cfg));
   else if (do_main && g->variant == DECODE_FLOW)

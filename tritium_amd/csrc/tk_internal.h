@@ -209,6 +209,10 @@ int tk_flow3_runs_per_wave(int planes);
 int tk_flow3_waves(int rt);  // waves per workgroup
 hipError_t tk_launch_flow3(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob,
                            const TkLaunchCfg &cfg);
+// small batches (tk_waves.hip): up to 64 operand rows (row stride as the problem says), 1..3 planes; one workgroup per two
+// tiles, `grid` of them; a table's workgroups count from the problem's group_begin
+hipError_t tk_launch_waves(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob, int planes,
+                           int rows, unsigned grid);
 int tk_gemm_tiles_per_wg(int planes);
 int tk_gemm_lds_bytes(void);
 int tk_flow_ring(const int *nbs, const double *weights, int count, int rt, int rows, int tw);
