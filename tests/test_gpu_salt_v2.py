@@ -189,3 +189,23 @@ def test_v2_upload_rejections(backend, so):
     with pytest.raises(T.UnsupportedFormat):
         up(codec=7)
     up().free()
+
+
+@pytest.mark.parametrize("codec", [S.D2, S.B3, S.S34])
+@pytest.mark.parametrize("n,k,group,m", [(17, 64 * 50, 64, 3), (16, 128 * 49, 128, 1), (5, 128 * 17, 128, 33), (33, 64, 64, 16)])
+def test_v2_matrix_form_at_its_edges(backend, so, codec, n, k, group, m):
+    """More segments than meet in LDS at once, one more than there are waves, a single one; rows and tokens past a tile of 16;
+    one to three planes mixed; activations that are denormal, zero and -0."""
+    print("case salt-v2 matrix", codec, n, k, group, m, flush=True)
+    rng = np.random.default_rng(codec + n + k + m)
+    t = S.random_v2_tensor(so, rng, codec, n, k, None, group)
+    dev = backend.salt_v2_upload(codec, group, t.payload, t.scales, t.plane_counts, n, k)
+    act = (rng.uniform(-0.75, 0.75, (m, k)) * 10.0 ** rng.integers(-42, 3, (m, k))).astype(np.float32)
+    act[:, ::7] = -0.0
+    dact, dout = backend.to_device(act, "f32"), backend.empty(m * n, "f32")
+    dev.forward(dact, m, dout)
+    rc, want = so.v2_forward(t, act, m)
+    assert rc == 0 and same_bits(dout.to_host().reshape(m, n), want)
+    for a in (dact, dout):
+        a.free()
+    dev.free()

@@ -12,18 +12,15 @@
 // so the bits are those of the CPU reference.
 //
 //
-// Rows of whole scale groups (k a multiple of the group, the usual case) take a faster form of the same
-// order, lane = weight row: a wave takes 64 rows and ONE segment index, i.e. the same columns of every row,
-// so an activation is one broadcast read for all lanes and the lanes never diverge; it folds the (up to
-// three) planes of its segment side by side, one accumulator per plane and token, and writes the scaled
-// terms to a workspace; a second kernel adds the terms of an output in the pinned order. (rows x segments
-// waves instead of rows workgroups of which half the lanes idle: 4096 x 4096, two planes: 210 -> about 20 us
-// for one token.)
+// Rows of whole scale groups (k a multiple of the group, the usual case) take a faster form of the same order on the f32
+// matrix pipe: see tk_salt_v2_exact_kernel.
 // Compiled with -ffp-contract=off; the sums use explicit round-to-nearest adds and multiplies.
 
 #include "tk_device.h"
 
 namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // bytes of one plane of `len` coefficients (crates/tritium-format/src/salt_v2.rs:160-258)
 __device__ __forceinline__ unsigned plane_bytes(unsigned codec, unsigned len) {
@@ -48,49 +45,73 @@ __device__ __forceinline__ int trit_at(const uint8_t *p, unsigned nbytes, unsign
   return (code >> (2u + sign)) & 1u ? 1 : -1;
 }
 
-// trits local .. local+15 of a plane (local a multiple of 16; all 16 lie inside the plane)
-__device__ __forceinline__ void trits16(const uint8_t *p, unsigned nbytes, unsigned local, unsigned codec, int (&tr)[16]) {
-  if (codec == TK_SALT_V2_D2) {
-    const uint8_t *q = p + (local >> 2);
-    const unsigned w = (unsigned)gload(q) | ((unsigned)gload(q + 1) << 8) | ((unsigned)gload(q + 2) << 16) | ((unsigned)gload(q + 3) << 24);
+// bytes at .. at+N-1 of a plane in the low bits (N = 4 or 8; whatever lies past the plane's end reads as 0). One load that
+// stays inside the plane: planes of whole scale groups have at least 10 bytes.
+template <typename T>
+__device__ __forceinline__ T plane_word(const uint8_t *p, unsigned nbytes, unsigned at) {
+  typedef T loose __attribute__((aligned(1)));
+  const unsigned from = min(at, nbytes - (unsigned)sizeof(T));
+  return *(const TK_GLOBAL loose *)(p + from) >> (8u * (at - from));
+}
+
+// the five digits of a B3 byte (below 243) as 2-bit fields, the first trit lowest ((b * 171) >> 9 is b / 3 exactly)
+__device__ __forceinline__ unsigned b3_fields(unsigned b) {
+  const unsigned q1 = (b * 171u) >> 9, q2 = (q1 * 171u) >> 9, q3 = (q2 * 171u) >> 9, q4 = (q3 * 171u) >> 9;
+  return (b - 3u * q1) | ((q1 - 3u * q2) << 2) | ((q2 - 3u * q3) << 4) | ((q3 - 3u * q4) << 6) | (q4 << 8);
+}
+
+// trits local .. local+15 of a plane (local a multiple of 16; all 16 lie inside the plane) as 2-bit codes trit + 1, the
+// first in the lowest bits, from the plane's bytes `raw` (the first that holds one of them lowest)
+__device__ __forceinline__ unsigned long long raw16(const uint8_t *p, unsigned nbytes, unsigned local, unsigned codec) {
+  if (codec == TK_SALT_V2_D2) return plane_word<uint32_t>(p, nbytes, local >> 2);
+  if (codec == TK_SALT_V2_B3) return plane_word<unsigned long long>(p, nbytes, local / 5u);
+  return plane_word<uint32_t>(p, nbytes, (local >> 2) * 5u >> 3);
+}
+__device__ __forceinline__ unsigned recode16(unsigned long long raw, unsigned local, unsigned codec, const uint16_t *fields) {
+  if (codec == TK_SALT_V2_D2) return (unsigned)raw;
+  if (codec == TK_SALT_V2_B3) {  // five bytes hold 25 digits, shifted to the first trit wanted
+    unsigned long long digits = 0;
 #pragma unroll
-    for (int u = 0; u < 16; ++u) tr[u] = (int)((w >> (2 * u)) & 3u) - 1;
-    return;
+    for (int i = 0; i < 5; ++i) digits |= (unsigned long long)fields[(unsigned)(raw >> (8 * i)) & 255u] << (10 * i);
+    return (unsigned)(digits >> (2u * (local % 5u)));
   }
-  if (codec == TK_SALT_V2_B3) {
-    // five bytes hold 25 digits from trit b0 * 5 on: all of them as 2-bit fields of one 64-bit word, shifted
-    // to the first trit wanted (a byte is below 243, so (b * 171) >> 9 is b / 3 exactly)
-    const unsigned b0 = local / 5u, r = local - b0 * 5u;
-    unsigned long long fields = 0;
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      const unsigned b = gload(p + min(b0 + (unsigned)i, nbytes - 1u));
-      const unsigned q1 = (b * 171u) >> 9, q2 = (q1 * 171u) >> 9, q3 = (q2 * 171u) >> 9, q4 = (q3 * 171u) >> 9;
-      const unsigned d = (b - 3u * q1) | ((q1 - 3u * q2) << 2) | ((q2 - 3u * q3) << 4) | ((q3 - 3u * q4) << 6) | (q4 << 8);
-      fields |= (unsigned long long)d << (10 * i);
-    }
-    fields >>= 2u * r;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) tr[u] = (int)((unsigned)(fields >> (2 * u)) & 3u) - 1;
-    return;
-  }
-  // S34: four groups of five bits from bit (local / 4) * 5 on (local is a multiple of 16: the offset inside the
-  // first byte is 0 or 4, so four bytes hold the twenty bits)
-  const unsigned bit = (local >> 2) * 5u, byte = bit >> 3;
-  unsigned word = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) word |= (unsigned)gload(p + min(byte + (unsigned)i, nbytes - 1u)) << (8 * i);
-  word >>= bit & 7u;
+  // S34: four groups of five bits (local is a multiple of 16: they start at bit 0 or 4 of the first byte). A group is the
+  // slot of its zero and the signs of the other three in order: their codes 2 or 0 as three fields, and code 1 put in between
+  const unsigned word = (unsigned)raw >> ((local >> 2) * 5u & 7u);
+  unsigned codes = 0;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const unsigned code = (word >> (5 * g)) & 31u, zero = code & 3u;
-#pragma unroll
-    for (int slot = 0; slot < 4; ++slot) {
-      const unsigned sign = (unsigned)slot - ((unsigned)slot > zero ? 1u : 0u);
-      const int v = (code >> (2u + sign)) & 1u ? 1 : -1;
-      tr[g * 4 + slot] = (unsigned)slot == zero ? 0 : v;
-    }
+    const unsigned code = (word >> (5 * g)) & 31u, at = 2u * (code & 3u), below = (1u << at) - 1u;
+    const unsigned signs = ((code >> 1) & 2u) | (code & 8u) | ((code << 1) & 32u);
+    codes |= ((signs & below) | (1u << at) | ((signs & ~below) << 2)) << (8 * g);
   }
+  return codes;
+}
+
+// The 4 x 4 transpose over the four 16-lane rows of a wave: register q of row h becomes register h of row q.
+__device__ __forceinline__ void transpose_rows(float (&v)[4]) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  auto bits = [](float f) { return __float_as_uint(f); };
+  const u2 a = __builtin_amdgcn_permlane32_swap(bits(v[0]), bits(v[2]), false, false);
+  const u2 b = __builtin_amdgcn_permlane32_swap(bits(v[1]), bits(v[3]), false, false);
+  const u2 e = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false);
+  const u2 o = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+  v[0] = __uint_as_float(e.x);
+  v[1] = __uint_as_float(e.y);
+  v[2] = __uint_as_float(o.x);
+  v[3] = __uint_as_float(o.y);
+}
+
+// the value of every 16-lane row of a wave in all of its lanes
+__device__ __forceinline__ void spread_rows(unsigned v, unsigned (&rows)[4]) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 half = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // rows 0 1 0 1 and 2 3 2 3
+  const u2 lo = __builtin_amdgcn_permlane16_swap(half.x, half.x, false, false);
+  const u2 hi = __builtin_amdgcn_permlane16_swap(half.y, half.y, false, false);
+  rows[0] = lo.x;
+  rows[1] = lo.y;
+  rows[2] = hi.x;
+  rows[3] = hi.y;
 }
 
 struct TileView {
@@ -174,117 +195,123 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
   if (bad) atomicOr(flag, 1u);
 }
 
-// ---- lane = row (k % group == 0) ----
-// terms[(tok * nseg * 3 + s * 3 + j) * n + row]: the product of plane j of segment s of `row` for token `tok`
-// (planes a tile does not have are left unwritten and never read).
-template <int MT>
-__global__ __launch_bounds__(64) void tk_salt_v2_terms_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned tok_begin,
-                                                              unsigned tok_end, float *__restrict__ terms,
-                                                              unsigned *__restrict__ flag) {
-  const unsigned lane = threadIdx.x, row = blockIdx.x * 64u + lane, s = blockIdx.y;
-  const unsigned tok0 = tok_begin + blockIdx.z * MT;
-  const unsigned mt = min((unsigned)MT, tok_end - tok0);
-  const bool active = row < t.n;
-  const unsigned rowc = active ? row : t.n - 1u;
-  const unsigned nseg = t.k / t.group, c0 = s * t.group;
-  const unsigned long long lo = (unsigned long long)rowc * t.k + c0;
-  const unsigned tile = (unsigned)(lo >> 8), local0 = (unsigned)(lo & 255ull);
-  const TileView tv = tile_view(t, tile);
-  const unsigned full_bytes = plane_bytes(t.codec, 256u), cur_bytes = plane_bytes(t.codec, tv.len);
-  const unsigned full_groups = 256u / t.group, cur_groups = (tv.len + t.group - 1u) / t.group;
-  const unsigned codec = t.codec, group = t.group;
-  const uint8_t *pj[3];
-#pragma unroll
-  for (int j = 0; j < 3; ++j)  // (a plane the tile does not have reads the last one it has; its sums are dropped)
-    pj[j] = t.payload + (size_t)tv.begin * full_bytes + (size_t)min((unsigned)j, tv.planes - 1u) * cur_bytes;
-  float acc[3][MT];
-#pragma unroll
-  for (int j = 0; j < 3; ++j)
-#pragma unroll
-    for (int x = 0; x < MT; ++x) acc[j][x] = 0.0f;
-  // the segment's activations, [column][token], once per workgroup (every lane reads the same ones: LDS
-  // broadcasts); the first row block checks that they are finite
-  __shared__ float sh_act[128 * MT];
+// ---- rows of whole scale groups (k % group == 0) ----
+// The fold of one segment over its columns is a chain of adds of +-activation, i.e. of fused multiply-adds with an exact
+// product (a trit times a float), and v_mfma_f32_16x16x4_f32 adds its four terms in ascending order with one rounding each,
+// denormals kept. So 16 weight rows x 16 tokens fold on the f32 matrix pipe in the pinned order; a zero trit adds +-0, which
+// changes no accumulator that started at +0. (A non-finite activation fails the call, so 0 * inf does not count.)
+// A workgroup owns 16 rows x 16 tokens; its 16 waves take every sixteenth segment: each lane recodes a quarter of the
+// segment of one row to 2-bit codes (whatever the codec), four lanes exchange them, and a step of four columns is one
+// conversion and one matrix instruction. The scaled terms of up to SV2_SLOTS segments meet in LDS (as many as fit, so that the
+// waves drift apart and one's loads hide behind another's folds), where one thread per output adds them in the pinned order. Plane counts differ by tile: a row without a plane folds its last one again and drops the term.
+// Floor: the f32 matrix pipe, 32 cycles per 16 x 16 x 4 (7 us at the size below); the recoding and the latency of the loads add to it.
+// 4096 x 4096, two planes, kernels, 8 tokens of B3: 64 us (fold with a lane per row, terms through memory) + 12 us (their sum) ->
+// 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 47 / 50 / 50 us, one token 57 / 69 / 66 -> 45 / 48 / 49, 64 tokens 302 / 389 / 353 ->
+// 111 / 122 / 126. (With the activations as 32 four-byte loads per lane and the codes as single bytes the kernel took 52 us: the
+// loads of 16 rows a few KiB apart were the bound.)
+constexpr int SV2_WAVES = 16, SV2_SLOTS = 48;
+template <int G>
+__global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
+                                                                          float *__restrict__ out, unsigned *__restrict__ flag,
+                                                                          unsigned slots) {
+  constexpr int W = G / 64;  // words of sixteen codes per lane and fold
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  uint16_t *s_fields = (uint16_t *)smem;                                   // [256], B3: the digits of a byte
+  float *s_term = (float *)(smem + 512);                                   // [slot][plane][accumulator register][lane]
+  uint8_t *s_planes = smem + 512 + (size_t)slots * 3 * 256 * sizeof(float);  // [slot][row]
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4;
+  const unsigned row = min(blockIdx.x * 16u + c, t.n - 1u), tok0 = blockIdx.y * 16u;
+  const unsigned nseg = t.k / G, codec = t.codec;
+  const unsigned full_bytes = plane_bytes(codec, 256u);
+  const float *arow = act + (size_t)min(tok0 + c, m - 1u) * t.k + h * 4;
+  const unsigned final_row = blockIdx.x * 16u + c, final_tok = tok0 + h * 4 + wave;  // of the thread that adds (waves 0..3)
+  float sum = 0.0f;
   bool bad = false;
-  const bool checks = blockIdx.x == 0;
-  for (unsigned e = lane; e < group * MT; e += 64u) {
-    const unsigned col = e / MT, x = e % MT;  // (MT is a power of two)
-    const float v = x < mt ? gload(act + (size_t)(tok0 + x) * t.k + c0 + col) : 0.0f;
-    if (checks) bad |= !(fabsf(v) <= 3.402823466e38f);
-    sh_act[e] = v;
+  if (codec == TK_SALT_V2_B3) {
+    if (threadIdx.x < 256) s_fields[threadIdx.x] = (uint16_t)b3_fields(threadIdx.x);
+    __syncthreads();
   }
-  __syncthreads();
-  // sixteen columns at a time: their codes are requested together (the loads do not depend on the sums), then
-  // folded in column order
-  for (unsigned o0 = 0; o0 < group; o0 += 16) {
-    int tr[3][16];
+  for (unsigned s0 = 0; s0 < nseg; s0 += slots) {
+    const unsigned pass = min(slots, nseg - s0);
+    for (unsigned slot = wave; slot < pass; slot += SV2_WAVES) {
+      const unsigned s = s0 + slot;
+      typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+      float a[W * 4][4];  // [sixteen columns][x]: column 4 x + h of the token, after the transpose
 #pragma unroll
-    for (int j = 0; j < 3; ++j) trits16(pj[j], cur_bytes, local0 + o0, codec, tr[j]);
+      for (int w = 0; w < W * 4; ++w) {
+        const quad v = *(const TK_GLOBAL quad *)(arow + (size_t)s * G + w * 16);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      float a[MT];
+        for (int x = 0; x < 4; ++x) a[w][x] = v[x];
+      }
+      const unsigned long long lo = (unsigned long long)row * t.k + (unsigned long long)s * G;
+      const unsigned tile = (unsigned)(lo >> 8), local = (unsigned)(lo & 255ull);
+      const TileView tv = tile_view(t, tile);
+      const unsigned cur_bytes = plane_bytes(codec, tv.len), cur_groups = tv.len / G;
+      const uint8_t *planes = t.payload + (size_t)tv.begin * full_bytes;
+      const uint16_t *scales = t.scales + (size_t)tv.begin * (256u / G) + local / G;
+      if (h == 0) s_planes[slot * 16 + c] = (uint8_t)tv.planes;
+      const unsigned most = __ballot(tv.planes >= 3u) ? 3u : (__ballot(tv.planes >= 2u) ? 2u : 1u);
+      if (blockIdx.x == 0) {  // every activation passes here
 #pragma unroll
-      for (int x = 0; x < MT; ++x) a[x] = sh_act[(o0 + u) * MT + x];
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int x = 0; x < MT; ++x) {
-          const float up = __fadd_rn(acc[j][x], a[x]), down = __fsub_rn(acc[j][x], a[x]);
-          acc[j][x] = tr[j][u] > 0 ? up : (tr[j][u] < 0 ? down : acc[j][x]);  // a zero trit skips the activation
-        }
-    }
-  }
-  if (active) {
-    const unsigned gidx = local0 / group;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      if ((unsigned)j >= tv.planes) continue;
-      const float sc = f16_to_f32(gload(t.scales + (size_t)tv.begin * full_groups + (size_t)j * cur_groups + gidx));
-#pragma unroll
-      for (int x = 0; x < MT; ++x)
-        if ((unsigned)x < mt)
-          terms[((size_t)(tok0 + x - tok_begin) * nseg * 3u + (size_t)s * 3u + j) * t.n + row] = __fmul_rn(acc[j][x], sc);
-    }
-  }
-  if (bad) atomicOr(flag, 1u);
-}
-
-// out[tok, row] = the terms of the row's segments added in the pinned order: segments ascending, planes ascending
-__global__ __launch_bounds__(TK_WG) void tk_salt_v2_sum_kernel(TkSaltV2 t, const float *__restrict__ terms, unsigned tok_begin,
-                                                               unsigned tok_end, float *__restrict__ out,
-                                                               unsigned *__restrict__ flag) {
-  const size_t idx = (size_t)blockIdx.x * TK_WG + threadIdx.x;
-  if (idx >= (size_t)(tok_end - tok_begin) * t.n) return;
-  const unsigned tl = (unsigned)(idx / t.n), row = (unsigned)(idx - (size_t)tl * t.n);
-  const unsigned nseg = t.k / t.group;
-  float accumulator = 0.0f;
-  // sixteen segments at a time: plane counts and terms are requested together, then added in order (a plane
-  // the tile does not have is not read and not added)
-  for (unsigned s0 = 0; s0 < nseg; s0 += 16) {
-    unsigned planes[16];
-    float term[16][3];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const unsigned s = min(s0 + u, nseg - 1u);
-      const unsigned tile = (unsigned)(((unsigned long long)row * t.k + (unsigned long long)s * t.group) >> 8);
-      planes[u] = s0 + u < nseg ? gload(t.tile_begin + tile + 1) - gload(t.tile_begin + tile) : 0u;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        term[u][j] = (unsigned)j < planes[u] ? gload(terms + ((size_t)tl * nseg * 3u + (size_t)(s0 + u) * 3u + j) * t.n + row) : 0.0f;
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
+        for (int x = 0; x < W * 16; ++x) bad |= !(fabsf(a[x / 4][x % 4]) <= 3.402823466e38f);
+      }
+      unsigned long long raw[3][W];
+      uint16_t scale[3];
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const float next = __fadd_rn(accumulator, term[u][j]);
-        accumulator = (unsigned)j < planes[u] ? next : accumulator;
+        if ((unsigned)j >= most) break;
+        const unsigned jc = min((unsigned)j, tv.planes - 1u);
+#pragma unroll
+        for (int i = 0; i < W; ++i) raw[j][i] = raw16(planes + (size_t)jc * cur_bytes, cur_bytes, local + (h * W + i) * 16u, codec);
+        scale[j] = gload(scales + (size_t)jc * cur_groups);
       }
+#pragma unroll
+      for (int w = 0; w < W * 4; ++w) transpose_rows(a[w]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        if ((unsigned)j >= most) break;
+        unsigned words[4 * W];
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          unsigned row_words[4];
+          spread_rows(recode16(raw[j][i], local + (h * W + i) * 16u, codec, s_fields), row_words);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) words[q * W + i] = row_words[q];
+        }
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < 4 * W; ++w) {  // sixteen columns: the word of lane group w / W; code = trit + 1 in byte x, field h
+          const unsigned word = words[w];
+          const unsigned trits = (((word >> (2u * h)) & 0x03030303u) + 0x7F7F7F7Fu) ^ 0x80808080u;  // int8 in every byte
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[w][x], (float)(int8_t)(trits >> (8 * x)), acc, 0, 0, 0);
+        }
+        const float sc = f16_to_f32(scale[j]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s_term[((slot * 3 + j) * 4 + r) * 64 + lane] = __fmul_rn(acc[r], sc);
+      }
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll 8
+      for (unsigned u = 0; u < pass; ++u) {
+        const unsigned planes = s_planes[u * 16 + c];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const float next = __fadd_rn(sum, s_term[((u * 3 + j) * 4 + wave) * 64 + lane]);  // (what a plane that is not there left is not taken)
+          sum = (unsigned)j < planes ? next : sum;
+        }
+      }
+    }
+    __syncthreads();
   }
-  // an accumulator that left the finite range never comes back (inf - inf is NaN): the end result tells
-  if (!(fabsf(accumulator) <= 3.402823466e38f)) atomicOr(flag, 1u);
-  out[(size_t)(tok_begin + tl) * t.n + row] = accumulator;
+  if (wave < 4 && final_row < t.n && final_tok < m) {
+    // an accumulator that left the finite range never comes back (inf - inf is NaN): the end result tells
+    bad |= !(fabsf(sum) <= 3.402823466e38f);
+    out[(size_t)final_tok * t.n + final_row] = sum;
+  }
+  if (bad) atomicOr(flag, 1u);
 }
 
 // The results leave the staging buffer only when no activation and no result was found non-finite.
@@ -322,37 +349,19 @@ size_t tk_salt_v2_lds_bytes(size_t k, size_t group) {
   return nseg * 3 * TK_SALT_V2_TOKENS * sizeof(float) + ((nseg + 15) & ~(size_t)15);
 }
 
-// floats of workspace per token the lane = row form needs (0: the matrix does not take that form)
-size_t tk_salt_v2_term_floats(const TkSaltV2 &t) {
-  if (!t.group || t.k % t.group != 0 || t.k / t.group > 65535u) return 0;
-  return (size_t)(t.k / t.group) * 3 * t.n;
-}
-
-// terms: workspace of term_tokens * tk_salt_v2_term_floats(t) floats (term_tokens >= 1), or null for the form
-// that needs none
-hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag,
-                                     float *terms, size_t term_tokens) {
+hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag) {
   if (!m || !t.n) return hipSuccess;
-  if (terms && term_tokens && tk_salt_v2_term_floats(t)) {
-    const unsigned nseg = t.k / t.group;
-    for (size_t b = 0; b < m; b += term_tokens) {
-      const unsigned e = (unsigned)(b + term_tokens < m ? b + term_tokens : m), cnt = e - (unsigned)b;
-      const dim3 block(64);
-      if (cnt == 1) {
-        hipLaunchKernelGGL(tk_salt_v2_terms_kernel<1>, dim3((t.n + 63) / 64, nseg, cnt), block, 0, s, t, act, (unsigned)b, e, terms, flag);
-      } else if (cnt <= 4) {
-        hipLaunchKernelGGL(tk_salt_v2_terms_kernel<4>, dim3((t.n + 63) / 64, nseg, 1), block, 0, s, t, act, (unsigned)b, e, terms, flag);
-      } else {
-        hipLaunchKernelGGL(tk_salt_v2_terms_kernel<8>, dim3((t.n + 63) / 64, nseg, (cnt + 7) / 8), block, 0, s, t, act, (unsigned)b, e, terms, flag);
-      }
-      hipError_t err = hipGetLastError();
-      if (err != hipSuccess) return err;
-      const size_t outs = (size_t)cnt * t.n;
-      hipLaunchKernelGGL(tk_salt_v2_sum_kernel, dim3((unsigned)((outs + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, t, terms, (unsigned)b, e, tmp, flag);
-      err = hipGetLastError();
-      if (err != hipSuccess) return err;
+  if (t.k && t.k % t.group == 0) {
+    const dim3 grid((t.n + 15) / 16, (unsigned)((m + 15) / 16)), block(SV2_WAVES * 64);
+    const unsigned nseg = t.k / t.group, slots = nseg < SV2_SLOTS ? nseg : SV2_SLOTS;
+    const size_t lds = 512 + (size_t)slots * (3 * 256 * sizeof(float) + 16);
+    if (lds > 64 * 1024) {
+      const hipError_t e = tk_raise_lds_limit(t.group == 128 ? (const void *)tk_salt_v2_exact_kernel<128> : (const void *)tk_salt_v2_exact_kernel<64>, 160 * 1024);
+      if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, slots);
+    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, slots);
+    return hipGetLastError();
   }
   const size_t lds = tk_salt_v2_lds_bytes(t.k, t.group);
   if (lds > 64 * 1024) {
