@@ -255,10 +255,12 @@ struct TkSaltV2 {
 // tokens one workgroup carries through a weight row, and the LDS a launch needs for rows of k columns
 #define TK_SALT_V2_TOKENS 8
 size_t tk_salt_v2_lds_bytes(size_t k, size_t group);
-// tmp receives the [m,n] results; *flag is raised when an activation or a result is not finite
-hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag);
-// out[i] = tmp[i] for i < count unless *flag is set (then nothing is written)
-hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag);
+// tmp receives the [m,n] results; *flag becomes `call` (never its value before) when an activation or a result is not finite
+hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag,
+                                     unsigned call);
+// out[i] = tmp[i] for i < count unless *flag is `call` (then nothing is written); *verdict = whether it was
+hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call,
+                                    unsigned *verdict);
 hipError_t tk_launch_salt_v2_gather(hipStream_t s, const TkSaltV2 &t, const uint32_t *rows, size_t count, float *out);
 #ifdef __cplusplus
 }

@@ -137,7 +137,7 @@ __device__ __forceinline__ float f16_to_f32(uint16_t h) {
 // LDS: float term[segments][3 planes][tokens], then one plane count per segment.
 // Segment boundaries are the multiples of the scale group (which divides the 256 of a tile).
 __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
-                                                                float *__restrict__ out, unsigned *__restrict__ flag) {
+                                                                float *__restrict__ out, unsigned *__restrict__ flag, unsigned call) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int MT = TK_SALT_V2_TOKENS;
   const unsigned row = blockIdx.x, tok0 = blockIdx.y * MT;
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
     bad |= !(fabsf(accumulator) <= 3.402823466e38f);
     out[(size_t)(tok0 + threadIdx.x) * t.n + row] = accumulator;
   }
-  if (bad) atomicOr(flag, 1u);
+  if (bad) gstore(flag, call);  // (whoever stores, stores the same)
 }
 
 // ---- rows of whole scale groups (k % group == 0) ----
@@ -213,7 +213,7 @@ constexpr int SV2_WAVES = 16, SV2_SLOTS = 48;
 template <int G>
 __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
                                                                           float *__restrict__ out, unsigned *__restrict__ flag,
-                                                                          unsigned slots) {
+                                                                          unsigned call, unsigned slots) {
   constexpr int W = G / 64;  // words of sixteen codes per lane and fold
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   uint16_t *s_fields = (uint16_t *)smem;                                   // [256], B3: the digits of a byte
@@ -311,15 +311,18 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
     bad |= !(fabsf(sum) <= 3.402823466e38f);
     out[(size_t)final_tok * t.n + final_row] = sum;
   }
-  if (bad) atomicOr(flag, 1u);
+  if (bad) gstore(flag, call);  // (whoever stores, stores the same)
 }
 
-// The results leave the staging buffer only when no activation and no result was found non-finite.
+// The results leave the staging buffer only when no activation and no result was found non-finite: the flag then holds the
+// number of an earlier call (so it is never cleared). *verdict, in host memory, says which it was.
 __global__ __launch_bounds__(TK_WG) void tk_salt_v2_commit_kernel(const float *__restrict__ tmp, float *__restrict__ out, size_t count,
-                                                                  const unsigned *__restrict__ flag) {
-  if (gload(flag)) return;
+                                                                  const unsigned *__restrict__ flag, unsigned call,
+                                                                  unsigned *__restrict__ verdict) {
+  const bool bad = gload(flag) == call;
   const size_t idx = (size_t)blockIdx.x * TK_WG + threadIdx.x;
-  if (idx < count) out[idx] = gload(tmp + idx);
+  if (idx == 0) gstore(verdict, bad ? 1u : 0u);
+  if (!bad && idx < count) gstore(out + idx, gload(tmp + idx));
 }
 
 // One thread per gathered coefficient (crates/tritium-cuda/kernels/salt_v2.cu:218-304).
@@ -349,7 +352,8 @@ size_t tk_salt_v2_lds_bytes(size_t k, size_t group) {
   return nseg * 3 * TK_SALT_V2_TOKENS * sizeof(float) + ((nseg + 15) & ~(size_t)15);
 }
 
-hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag) {
+hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag,
+                                     unsigned call) {
   if (!m || !t.n) return hipSuccess;
   if (t.k && t.k % t.group == 0) {
     const dim3 grid((t.n + 15) / 16, (unsigned)((m + 15) / 16)), block(SV2_WAVES * 64);
@@ -359,8 +363,8 @@ hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const flo
       const hipError_t e = tk_raise_lds_limit(t.group == 128 ? (const void *)tk_salt_v2_exact_kernel<128> : (const void *)tk_salt_v2_exact_kernel<64>, 160 * 1024);
       if (e != hipSuccess) return e;
     }
-    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, slots);
-    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, slots);
+    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, call, slots);
+    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, call, slots);
     return hipGetLastError();
   }
   const size_t lds = tk_salt_v2_lds_bytes(t.k, t.group);
@@ -369,13 +373,14 @@ hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const flo
     if (e != hipSuccess) return e;
   }
   const dim3 grid(t.n, (unsigned)((m + TK_SALT_V2_TOKENS - 1) / TK_SALT_V2_TOKENS));
-  hipLaunchKernelGGL(tk_salt_v2_forward_kernel, grid, dim3(64), lds, s, t, act, (unsigned)m, tmp, flag);
+  hipLaunchKernelGGL(tk_salt_v2_forward_kernel, grid, dim3(64), lds, s, t, act, (unsigned)m, tmp, flag, call);
   return hipGetLastError();
 }
 
-hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag) {
+hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call,
+                                    unsigned *verdict) {
   if (!count) return hipSuccess;
-  hipLaunchKernelGGL(tk_salt_v2_commit_kernel, dim3((unsigned)((count + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, tmp, out, count, flag);
+  hipLaunchKernelGGL(tk_salt_v2_commit_kernel, dim3((unsigned)((count + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, tmp, out, count, flag, call, verdict);
   return hipGetLastError();
 }
 
