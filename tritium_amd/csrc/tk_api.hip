@@ -91,7 +91,9 @@ struct tk_ctx {
   // it -- no copy-engine transfers (see host_call; grow-only; freed with the context)
   void *pin = nullptr;
   size_t pin_cap = 0;
-  size_t host_direct_bytes = (size_t)1 << 20;
+  // (back-to-back calls, transfers / pinned block: 48 tokens K=2560 N=6912 (1.9 MB) 138 / 111 us, K=6912 N=2560 121 / 107, 128
+  // tokens K=2560 N=2560 (2.6 MB) 169 / 148, 256 tokens K=2560 N=6912 (9.7 MB) 526 / 480; K=8192 N=8192 (16.8 MB) 752 / 756)
+  size_t host_direct_bytes = (size_t)16 << 20;
   int fuse_tokens = -1;    // single decode calls of up to this many tokens build their operand rows inside the decode kernel (-1 = chosen per call, 0 = never)
   int gemm_rows = 0;       // one-plane int8-contract prefill, single launches: 0 = tile rows chosen per launch, 64 / 128 / 256 = force
   bool gemm256_form_forced = false;  // tk_set_gemm256_form was called: automatic launches keep that form
