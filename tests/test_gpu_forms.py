@@ -3,6 +3,8 @@ with the CPU oracle: the 2-tile and 4-tile forms of the one-plane prefill kernel
 launches), the grouped prefill kernel with one, two and three planes, and the grouped flow kernel on
 the 32x32x32 matrix instruction chosen automatically. Precedent: the reference holds its tensor-core
 kernel to `to_bits` equality with its dp4a kernel (crates/tritium-cuda/src/cuda/tests.rs:2100-2190)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -670,3 +672,37 @@ def test_narrow_groups_of_several_row_tiles_take_the_prefill_kernel(backend, ora
                 layer.free()
     dx.free()
     dw.free()
+
+
+@pytest.mark.parametrize("k", [257, 1027, 2050, 4099])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("m", [40, 400])
+def test_prep_of_rows_aligned_like_an_element(backend, oracle, m, k, dtype):
+    """Rows whose starts are aligned like one element only (odd K, a base one element into a buffer): the vector loads of the
+    quantization against the oracle, and the digit split's two forms (a workgroup or a wave per token) against each other."""
+    print("case ragged prep", m, k, dtype, flush=True)
+    rng = np.random.default_rng(m + k)
+    n = 40
+    w, sc = ternary(rng, n, k, 0.4), scales(rng, n)
+    packed = T.pack_rows(w, n, k)
+    layer = backend.linear([packed], [sc], n, k)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    bits = f32_to_bf16_bits(act)
+    if dtype == "bf16":
+        act = bf16_bits_to_f32(bits).reshape(m, k)
+    host = np.concatenate([np.zeros(1, bits.dtype), bits.reshape(-1)]) if dtype == "bf16" else np.concatenate([np.zeros(1, np.float32), act.reshape(-1)])
+    whole, o, o2 = backend.to_device(host, dtype), backend.empty(m * n, "f32"), backend.empty(m * n, "f32")
+    moved = T.DeviceArray(backend, ctypes.c_void_p(whole.ptr.value + (2 if dtype == "bf16" else 4)), m * k, whole.dtype)
+    backend.linear_a8(layer, moved, m, o)
+    assert same_bits(o.to_host(), oracle.cpu_linear_a8_planes([packed], FMT_TQ2_0, [sc], act, m, n, k))
+    backend.linear_float(layer, moved, m, o)
+    backend.set_prep_team_rows(0 if m == 40 else 1000)
+    try:
+        backend.linear_float(layer, moved, m, o2)
+    finally:
+        backend.set_prep_team_rows(384)
+    assert same_bits(o.to_host(), o2.to_host())
+    assert accepts(o.to_host().reshape(m, n), oracle.cpu_mpgemm_planes([packed], FMT_TQ2_0, [sc], act, m, n, k).reshape(m, n), rel=1e-4, floor=1.0).all()
+    for a in (whole, o, o2):
+        a.free()
+    layer.free()

@@ -1493,18 +1493,20 @@ __device__ int block_sum(int v, int *sh) {
 }
 
 // Four consecutive activations starting at element e (a multiple of 4) as floats; elements at or
-// past k read as 0. `vec` says the row starts are aligned for one 8- or 16-byte load.
+// past k read as 0. `vec`: one 8- or 16-byte load where all four exist. It is aligned like an element only (rows of any k, any
+// base): global loads take that on this chip (700 bf16 tokens of K=6001, int8 contract, element by element 27.5 us, so 24.5).
 __device__ __forceinline__ void load_act4(const void *act, int dtype, size_t base, size_t e, size_t k, bool vec, float (&v)[4]) {
   if (vec && e + 4 <= k) {
     if (dtype == TK_BF16) {
-      typedef unsigned v2u __attribute__((ext_vector_type(2)));
+      typedef unsigned v2u __attribute__((ext_vector_type(2), aligned(2)));
       const v2u u = *(const TK_GLOBAL v2u *)((const uint16_t *)act + base + e);
       v[0] = __uint_as_float(u.x << 16);
       v[1] = __uint_as_float(u.x & 0xFFFF0000u);
       v[2] = __uint_as_float(u.y << 16);
       v[3] = __uint_as_float(u.y & 0xFFFF0000u);
     } else {
-      const v4u u = *(const TK_GLOBAL v4u *)((const float *)act + base + e);
+      typedef unsigned v4l __attribute__((ext_vector_type(4), aligned(4)));
+      const v4l u = *(const TK_GLOBAL v4l *)((const float *)act + base + e);
       v[0] = __uint_as_float(u.x);
       v[1] = __uint_as_float(u.y);
       v[2] = __uint_as_float(u.z);
@@ -1516,9 +1518,7 @@ __device__ __forceinline__ void load_act4(const void *act, int dtype, size_t bas
   for (int b = 0; b < 4; ++b) v[b] = e + b < k ? load_act(act, dtype, base + e + b) : 0.0f;
 }
 
-__device__ __forceinline__ bool act_rows_vectorizable(const void *act, int dtype, size_t k) {
-  return (k & 3) == 0 && (((size_t)act) & 15) == 0 && (dtype == TK_BF16 || dtype == TK_F32);
-}
+__device__ __forceinline__ bool act_rows_vectorizable(int dtype) { return dtype == TK_BF16 || dtype == TK_F32; }
 
 // gamma = max |a| with the reference's `a > gamma` rule (NaN never wins), plus a non-finite flag.
 // RMSNorm in front of the quantization (crates/tritium-nn/src/ops/rmsnorm.rs:21-96). The sum of
@@ -1678,7 +1678,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_a8_kernel(TkPrep single, const 
   const void *act = pp.act;
   const int dtype = pp.act_dtype;
   int8_t *ap = pp.ap, *qrm = pp.q_rowmajor;
-  const bool vec = act_rows_vectorizable(act, dtype, k);
+  const bool vec = act_rows_vectorizable(dtype);
   RowNorm nm = {pp.norm_kind, 0.0f, pp.norm_w};
   float *ynorm = nullptr;
   if (nm.kind) {
@@ -1727,7 +1727,8 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_a8_kernel(TkPrep single, const 
       piece[sl] = packed;
       if (qrm) {
         if (vec && e + 4 <= k) {
-          *(TK_GLOBAL uint32_t *)(qrm + base + e) = packed;
+          typedef uint32_t loose __attribute__((aligned(1)));
+          *(TK_GLOBAL loose *)(qrm + base + e) = packed;
         } else {
           for (int b = 0; b < 4; ++b)
             if (e + b < k) qrm[base + e + b] = (int8_t)(packed >> (8 * b));
@@ -1827,7 +1828,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
   const void *act = pp.act;
   const int dtype = pp.act_dtype;
   int8_t *ap = pp.ap;
-  const bool vec = act_rows_vectorizable(act, dtype, k);
+  const bool vec = act_rows_vectorizable(dtype);
   const size_t npieces = nb * 16;
   const bool resident = npieces <= (size_t)TK_PREP_HELD * TK_WG;
   float held[TK_PREP_HELD][16];
@@ -2061,7 +2062,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_a8_wave_kernel(TkPrep single, c
   const void *act = pp.act;
   const int dtype = pp.act_dtype;
   int8_t *ap = pp.ap, *qrm = pp.q_rowmajor;
-  const bool vec = act_rows_vectorizable(act, dtype, k);
+  const bool vec = act_rows_vectorizable(dtype);
   const size_t npieces = nb * 16;
   float held[HELD][16];
   float gamma;
@@ -2122,7 +2123,8 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_a8_wave_kernel(TkPrep single, c
       piece[sl] = packed;
       if (qrm) {
         if (vec && e + 4 <= k) {
-          *(TK_GLOBAL uint32_t *)(qrm + base + e) = packed;
+          typedef uint32_t loose __attribute__((aligned(1)));
+          *(TK_GLOBAL loose *)(qrm + base + e) = packed;
         } else {
           for (int b = 0; b < 4; ++b)
             if (e + b < k) qrm[base + e + b] = (int8_t)(packed >> (8 * b));
@@ -2155,7 +2157,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_wave_kernel(TkPrep singl
   const void *act = pp.act;
   const int dtype = pp.act_dtype;
   int8_t *ap = pp.ap;
-  const bool vec = act_rows_vectorizable(act, dtype, k);
+  const bool vec = act_rows_vectorizable(dtype);
   const size_t npieces = nb * 16;
   float held[HELD][16];
   float gamma;
@@ -2771,7 +2773,11 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
   if (single) pieces = (!single->norm_kind && !single->blocksum) ? single->nb * 16 : 0;
   const bool plain = pieces && (kind == TK_PREP_A8 || kind == TK_PREP_DIGITS);
   const bool team_wg = plain && fast && pieces <= 8 * (size_t)TK_WG && (rows <= (unsigned)(kind == TK_PREP_DIGITS ? g_prep_team_rows * 8 / 3 : g_prep_team_rows) || pieces > 512);
-  const bool team_wave = plain && !team_wg && rows >= 32 && pieces <= (fast ? 512u : 256u);
+  // Rows of other shapes have no straight-line form: few of them take the kernels below, which give a token the whole
+  // workgroup. Call, N=512, wave per token / workgroup per token: float contract f32 K=2050 40 / 333 / 384 tokens 25.9 / 26.7 / 26.6
+  // -> 19.0 / 20.7 / 20.8 us, 700 28.2 -> 27.0, K=1027 333 tokens 19.6 -> 17.4, 1000 tokens 21.1 -> 24.5; int8 contract bf16 K=2050
+  // 333 tokens 21.9 -> 16.4 (loads included).
+  const bool team_wave = plain && !team_wg && rows >= 32 && pieces <= (fast ? 512u : 256u) && (fast || rows > (unsigned)g_prep_team_rows);
   if (team_wg || team_wave) {
     const size_t team = team_wg ? TK_WG : 64;
     const dim3 grid(team_wg ? rows : (rows + 3) / 4), block(TK_WG);
