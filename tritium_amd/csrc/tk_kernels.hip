@@ -2776,8 +2776,10 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
   // Rows of other shapes have no straight-line form: few of them take the kernels below, which give a token the whole
   // workgroup. Call, N=512, wave per token / workgroup per token: float contract f32 K=2050 40 / 333 / 384 tokens 25.9 / 26.7 / 26.6
   // -> 19.0 / 20.7 / 20.8 us, 700 28.2 -> 27.0, K=1027 333 tokens 19.6 -> 17.4, 1000 tokens 21.1 -> 24.5; int8 contract bf16 K=2050
-  // 333 tokens 21.9 -> 16.4 (loads included).
-  const bool team_wave = plain && !team_wg && rows >= 32 && pieces <= (fast ? 512u : 256u) && (fast || rows > (unsigned)g_prep_team_rows);
+  // 333 tokens 21.9 -> 16.4 (loads included). One piece per lane (K <= 1024) stays: K=640 N=4096 106 f32 tokens, float contract
+  // 14.6 -> 15.6.
+  const bool team_wave = plain && !team_wg && rows >= 32 && pieces <= (fast ? 512u : 256u) &&
+                         (fast || pieces <= 64 || rows > (unsigned)g_prep_team_rows);
   if (team_wg || team_wave) {
     const size_t team = team_wg ? TK_WG : 64;
     const dim3 grid(team_wg ? rows : (rows + 3) / 4), block(TK_WG);
