@@ -9,7 +9,7 @@
 // The operand rows are read once per workgroup and 32 columns: they come from L2.
 // Bound: latency (launch, two or three dependent loads, the meeting in LDS). Registers are held to 128 where that is possible,
 // so that two workgroups share a CU: with 160 (two planes) N=13824 K=2560 16 rows took 15.5 us instead of 11.4. Kernel alone
-// K=2560 N=2560 32 rows: 15.5 us (prefill kernel with its K split) -> about 5; a decoder layer of hidden 2560 with 32 tokens
+// K=2560 N=2560 32 rows: 15.5 us (prefill kernel with its K split) -> about 6; a decoder layer of hidden 2560 with 32 tokens
 // (seven projections, four calls) 75 -> 48 us.
 #include "tk_device.h"
 
