@@ -108,6 +108,74 @@ def test_non_finite_values_follow_the_host(backend, oracle):
         assert (np.isnan(got) == nan).all() and same_bits(got[~nan], want[~nan])
 
 
+@pytest.mark.parametrize("m,n,k", [(37, 100, 700), (290, 70, 3900), (1030, 67, 3300)])
+def test_sums_that_leave_the_finite_range(backend, oracle, m, n, k):
+    """Every token-tile size of grad_act (1, 2 and 4 tiles of 16 per wave): infinities and NaN upstream, sums that overflow on
+    the way and meet the other infinity, products of finite factors that overflow under zero and non-zero trits, all beside
+    tokens that stay finite."""
+    print("case vjp range", m, n, k, flush=True)
+    rng = np.random.default_rng(m + 7 * n + k)
+    packed = oracle.pack_matrix(ternary(rng, n, k), n, k, FMT_TQ2_0)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    sc = rng.uniform(0.05, 1.5, n).astype(np.float32)
+    sc[50], sc[3], sc[4], sc[61] = np.float32(1e30), 1.0, 1.0, 1.0
+    base = rng.standard_normal((m, n)).astype(np.float32)
+    base[:, 50] *= np.float32(1e-25)  # (so that only the planted products overflow)
+    big = np.float32(2.5e38)
+    for rows in ((), (1, 2), (1, 2, m - 1), tuple(range(m))):
+        gy = base.copy()
+        for i, row in enumerate(rows):
+            if i % 3 == 0:
+                gy[row, 5], gy[row, 40] = np.inf, (np.nan if row % 2 else 1.0)
+            elif i % 3 == 1:
+                gy[row, [3, 4, 61]] = big, big, -big
+            else:
+                gy[row, 50] = np.float32(-1e20)
+        rc, ga_w, gw_w, gb_w = oracle.cpu_projected_vjp(packed, FMT_TQ2_0, act, sc, gy, m, n, k)
+        assert rc == 0 and np.isfinite(ga_w).all() == (not rows)
+        ga, gw, gb = _vjp(backend, packed, FMT_TQ2_0, act, sc, gy, m, n, k)
+        for got, want in ((ga, ga_w), (gw, gw_w), (gb, gb_w)):
+            nan = np.isnan(want)
+            assert (np.isnan(got) == nan).all() and same_bits(got[~nan], want[~nan]), len(rows)
+
+
+def test_non_finite_upstream_costs_no_more_than_the_unfused_sums(backend, oracle):
+    """A step of loss scaling that overflows is an ordinary step. Multiply and add per term on the vector ALU took ten times
+    the matrix form at this size, whatever the values: no call may take longer than that, whichever tokens hold an
+    infinity, a NaN or an overflowing product (measured: 1.1, 1.2 and 3.6 times the finite call)."""
+    import time
+    rng = np.random.default_rng(5)
+    m, n, k = 512, 2560, 2560
+    packed = T.pack_rows(ternary(rng, n, k), n, k)
+    buf = backend.upload_weights(packed, T.GemmShape(0, n, k), T.TernaryFormat.Tq2_0)
+    sc = rng.uniform(0.05, 1.5, n).astype(np.float32)
+    sc[50] = np.float32(1e30)
+    gy = rng.standard_normal((m, n)).astype(np.float32)
+    gy[:, 50] *= np.float32(1e-25)
+    one, nan, over = gy.copy(), gy.copy(), gy.copy()
+    one[m // 2, 7] = np.inf
+    nan[:, 7] = np.nan
+    over[:, 50] = np.float32(1e20)
+    dact, dsc, ga = backend.to_device(np.ones((m, k), np.float32), "f32"), backend.to_device(sc, "f32"), backend.empty(m * k, "f32")
+    times = {}
+    for name, up in (("finite", gy), ("one", one), ("nan", nan), ("over", over)):
+        dup = backend.to_device(up, "f32")
+        best = 1e9
+        for _ in range(4):
+            backend.sync()
+            t0 = time.perf_counter()
+            for _ in range(5):
+                backend.projected_vjp(buf, dsc, dact, dup, m, ga, None, None)
+            backend.sync()
+            best = min(best, time.perf_counter() - t0)
+        times[name] = best
+        dup.free()
+    print("vjp times", {key: round(v * 2e5, 1) for key, v in times.items()}, "us", flush=True)
+    assert max(times.values()) <= 10 * times["finite"], times
+    for a in (dact, dsc, ga, buf):
+        a.free()
+
+
 def test_device_resident_form_equals_the_host_form(backend, oracle):
     rng = np.random.default_rng(13)
     m, n, k = 40, 100, 700

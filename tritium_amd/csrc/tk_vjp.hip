@@ -37,9 +37,12 @@ __device__ __forceinline__ unsigned xcd_index(unsigned bid, unsigned total) {
 // as the CPU's separate multiply and add -- and the f32 matrix instructions are chains of such fused multiply-adds:
 // v_mfma_f32_16x16x4_f32 adds its four terms in ascending order with one rounding each, denormals kept (compared with
 // fmaf chains bit for bit on the device). So the contraction runs on the matrix pipe in the CPU's order.
-// The one case where p * trit differs from the CPU's term is p overflowing to infinity from finite factors under a zero
-// trit (NaN instead of 0). Such a sum can only end as NaN or infinity, so a wave whose sums do not all end finite
-// repeats them term by term as the CPU computes them.
+// Infinities and NaN in the upstream gradient or the scales come out the same either way (an infinite or NaN p times a zero trit is
+// NaN, as the CPU's upstream * (0 * scale) is). The one case where p * trit differs from the CPU's term is p overflowing to infinity
+// from finite factors under a zero trit (NaN instead of 0). Such a sum can only end as NaN or infinity, so a workgroup whose
+// sums do not all end finite looks for such a product among its tokens, and only where it finds one repeats its sums as the
+// CPU computes them. M=2048 N=6912 K=2560, all values finite 0.64 ms; an infinity in one token 0.75, NaN in all 0.89; such a
+// product in one token 1.8, in all 3.3 (each lane repeating its own sums of a wave: 15.9, 29.5, 16.0, 29.6).
 //
 // A workgroup owns 16*TT tokens x the 64 columns of one bit pair of a K block; wave g takes piece g of the chunks, of which
 // four rows are the 64 contiguous bytes of one wave-wide load, and every decoded operand serves TT matrix instructions.
@@ -51,18 +54,71 @@ __device__ __forceinline__ unsigned xcd_index(unsigned bid, unsigned total) {
 // K=2560: 31 us (1.06 ms).
 constexpr int ACT_ROWS = 64;  // weight rows per LDS stage
 
+// The sums of a workgroup term by term: upstream * (trit * scale) and the sum, each rounded. 64 weight rows of upstream values and
+// their scales pass through LDS as in the kernel below, whose accumulators this overwrites.
+template <int TT>
+__device__ __forceinline__ void act_repeat(const uint8_t *__restrict__ codes, int nb, int n, int n_tiles, int kb, int pair,
+                                        const float *__restrict__ scales, const float *__restrict__ up_base, int last_token,
+                                        float (*s_up)[ACT_ROWS + 4], float *s_sc, f32x4 (&acc)[TT]) {
+  int tid = threadIdx.x;
+  asm("" : "+v"(tid));  // (what follows is derived anew: the main loop's registers set the occupancy)
+  const int g = tid >> 6, lane = tid & 63, c = lane & 15, h = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < TT; ++t) acc[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  for (int r0 = 0; r0 < n; r0 += ACT_ROWS) {
+    __syncthreads();
+    const int row = r0 + (tid & 63);
+    const bool in = row < n;  // rows past the end: 0 * (trit * 0) = +-0 changes nothing
+#pragma unroll 8
+    for (int i = 0; i < 4 * TT; ++i) {
+      const int tok = i * 4 + g;
+      s_up[tok][tid & 63] = in ? ldg(up_base + (unsigned)(min(tok, last_token) * n + row)) : 0.0f;
+    }
+    if (tid < ACT_ROWS) s_sc[tid] = in ? ldg(scales + row) : 0.0f;
+    __syncthreads();
+    uint32_t w[4];
+    auto request = [&](int q) {
+      const uint8_t *cp = codes + ((size_t)min((r0 + q) >> 4, n_tiles - 1) * nb + kb) * 1024 + g * 256 + (q & 15) * 16 + c;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) w[x] = *(const TKV_GLOBAL uint8_t *)(cp + x * 16);
+    };
+    request(0);
+#pragma unroll 1
+    for (int q = 0; q < ACT_ROWS; q += 4) {
+      const f32x4 sc = *(const f32x4 *)&s_sc[q];
+      float proj[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) proj[x] = __fmul_rn((float)((w[x] >> (2 * pair)) & 3u) - 1.0f, sc[x]);
+      request(min(q + 4, ACT_ROWS - 4));
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        f32x4 up[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) up[r] = *(const f32x4 *)&s_up[16 * t + h * 4 + r][q];
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][r] = __fadd_rn(acc[t][r], __fmul_rn(up[r][x], proj[x]));
+        if (t & 1) __builtin_amdgcn_sched_barrier(0);  // (few registers: the kernel's occupancy is that of its main loop)
+      }
+    }
+  }
+}
+
 template <int TT>
 __global__ __launch_bounds__(256) void tk_vjp_act_kernel(const uint8_t *__restrict__ codes, int nb, int n, int k, int m,
                                                          const float *__restrict__ scales,
                                                          const float *__restrict__ grad_output,
                                                          float *__restrict__ grad_act, int wide) {
   __shared__ float s_p[2][16 * TT][ACT_ROWS + 4];  // [buffer][token][row]; the stride keeps a wave's reads on 64 banks
+  __shared__ int s_bad[2];  // a sum is not finite; a product of finite factors is not
   const unsigned cols = (unsigned)nb * 4, total = cols * (unsigned)((m + 16 * TT - 1) / (16 * TT));
   const unsigned idx = xcd_index(blockIdx.x, total);
   if (idx >= total) return;
   const int m0 = (int)(idx / cols) * (16 * TT), kb = (int)(idx % cols) >> 2, pair = (int)(idx & 3);
   const int tid = threadIdx.x, g = tid >> 6, lane = tid & 63, c = lane & 15, h = lane >> 4;
   const int n_tiles = (n + 15) >> 4, stages = (n + ACT_ROWS - 1) / ACT_ROWS;
+  if (tid < 2) s_bad[tid] = 0;  // (ordered by the first stage's barrier)
   // staging: a thread takes four rows of UT tokens; addresses are a uniform base per stage and a lane offset, which
   // costs the vector ALU nothing (it shares its lanes with the f32 matrix pipe: their times add up)
   constexpr int QUADS = ACT_ROWS / 4, TPR = 256 / QUADS, UT = 16 * TT / TPR;
@@ -129,31 +185,34 @@ __global__ __launch_bounds__(256) void tk_vjp_act_kernel(const uint8_t *__restri
   for (int t = 0; t < TT; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) finite &= fabsf(acc[t][r]) < __builtin_inff();
-  const bool repeat = __ballot(!finite) != 0;
-  // byte c of piece g, bit pair s: element (g/2)*128 + s*32 + (g%2)*16 + c of the K block
-  const int kk = kb * 256 + (g >> 1) * 128 + pair * 32 + (g & 1) * 16 + c;
-  if (kk >= k) return;
-  if (!repeat) {
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mi = m0 + t * 16 + h * 4 + r;
-        if (mi < m) *(TKV_GLOBAL float *)(grad_act + (size_t)mi * k + kk) = acc[t][r];
+  if (!finite) s_bad[0] = 1;
+  __syncthreads();
+  if (s_bad[0]) {
+    bool over = false;
+    for (int row = tid; row < n; row += 256) {
+      const float s = ldg(scales + row);
+#pragma unroll 4
+      for (int i = 0; i < 16 * TT; ++i) {
+        const float up = ldg(up_base + (unsigned)(min(i, m - 1 - m0) * n + row));
+        over |= fabsf(__fmul_rn(up, s)) == __builtin_inff() && fabsf(up) < __builtin_inff() && fabsf(s) < __builtin_inff();
       }
-    return;
-  }
-  for (int r = 0; r < 4 * TT; ++r) {
-    const int mi = m0 + (r >> 2) * 16 + h * 4 + (r & 3);
-    if (mi >= m) return;
-    float sum = 0.0f;
-    for (int row = 0; row < n; ++row) {
-      const uint32_t byte = *(const TKV_GLOBAL uint8_t *)(codes + ((size_t)(row >> 4) * nb + kb) * 1024 + g * 256 + (row & 15) * 16 + c);
-      const float trit = (float)((byte >> (2 * pair)) & 3u) - 1.0f;
-      sum = __fadd_rn(sum, __fmul_rn(ldg(grad_output + (size_t)mi * n + row), __fmul_rn(trit, ldg(scales + row))));
     }
-    *(TKV_GLOBAL float *)(grad_act + (size_t)mi * k + kk) = sum;
+    if (over) s_bad[1] = 1;
+    __syncthreads();
+    if (s_bad[1]) act_repeat<TT>(codes, nb, n, n_tiles, kb, pair, scales, up_base, m - 1 - m0, s_p[0], s_p[1][0], acc);
   }
+  // byte c of piece g, bit pair s: element (g/2)*128 + s*32 + (g%2)*16 + c of the K block
+  int id = threadIdx.x;
+  asm("" : "+v"(id));  // (derived anew: the main loop's registers set the occupancy)
+  const int kk = kb * 256 + (id >> 7) * 128 + pair * 32 + ((id >> 6) & 1) * 16 + (id & 15), hh = (id & 63) >> 4;
+  if (kk >= k) return;
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int mi = m0 + t * 16 + hh * 4 + r;
+      if (mi < m) *(TKV_GLOBAL float *)(grad_act + (size_t)mi * k + kk) = acc[t][r];
+    }
 }
 
 // ---- grad_bias ----
