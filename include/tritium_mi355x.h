@@ -385,10 +385,12 @@ typedef struct tk_salt_desc {
   const tk_weights *planes[TK_MAX_PLANES]; /* each from tk_upload_weights_scaled, same [n,k] */
   int n_planes;
 } tk_salt_desc;
-/* act [m,k] f32 or bf16, out [m,n] f32 or bf16. Tokens run on the matrix cores, block by block,
- * up to 1024 at a time (within 1e-4 of the host definition, normally ~1e-6); rows too long for LDS (K beyond ~9,800) and tokens holding NaN or Inf take
- * the host's order exactly (slow). A block scale that is itself infinite or NaN makes its outputs
- * non-finite here and NaN on the host (which multiplies it with the zero trits too). */
+/* act [m,k] f32 or bf16, out [m,n] f32 or bf16. Tokens run on the matrix cores, block by block, up to 1024 at a
+ * time (within 1e-4 of the host definition, normally ~1e-6, and closer to the exact sums than the host's f32 order). The host's order
+ * exactly (slow) is kept for tokens holding NaN or Inf, for tokens whose largest element is so far above the others that 31-bit
+ * fixed point would cost outputs that miss it precision, and for calls of K > 9984 whose operand rows do not fit LDS.
+ * A block scale that is itself infinite or NaN makes its outputs non-finite here and NaN on the host (which multiplies it
+ * with the zero trits too). */
 int tk_linear_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int act_dtype, size_t m,
                    void *out, int out_dtype);
 /* The host's order for every output: bit-identical to dequantize-then-fold. */

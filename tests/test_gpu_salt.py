@@ -200,3 +200,42 @@ def test_many_tokens_have_the_bits_of_sixteen_at_a_time(backend, oracle, m, n, k
     assert same_bits(got, want) if dtype == "f32" else (got == want).all()
     for a in [many, dout] + bufs:
         a.free()
+
+
+@pytest.mark.parametrize("m,n,k,t_planes", [(17, 300, 2560, 1), (16, 200, 5000, 2), (9, 130, 8192, 3), (1030, 40, 2600, 1)])
+def test_long_rows_are_no_less_exact_than_the_host_order(backend, m, n, k, t_planes):
+    """Calls whose rows do not fit the flow form stand in for the host's order, f32 sums over k: their error against float64
+    may not be larger, in any token and in the outputs that miss a token's largest element either (its weights there are
+    zero, so the values are small next to the element that sets the token's grid)."""
+    print("case salt-exactness", m, n, k, t_planes, flush=True)
+    rng = np.random.default_rng(m + n + k + t_planes)
+    nb = (k + 255) // 256
+    w64, bufs = np.zeros((n, k)), []
+    for p in range(t_planes):
+        trits = ternary(rng, n, k, (0.4, 0.7, 0.85)[p])
+        trits[: n // 2, 5] = 0
+        bits = f16_bits(rng.uniform(0.02, 1.0, (n, nb)) * (0.5 ** p))
+        packed = T.pack_rows(trits, n, k).reshape(n, nb, 66).copy()
+        packed[:, :, 64:] = bits.reshape(n, nb, 1).view(np.uint8)
+        bufs.append(backend.upload_weights_scaled(packed.reshape(-1), T.GemmShape(0, n, k)))
+        w64 += trits * np.repeat(bits.view(np.float16).astype(np.float64), 256, 1)[:, :k]
+    dout = backend.empty(m * n, "f32")
+    for name in ("normal", "log-normal", "outlier 2^6", "outlier 2^11", "outlier 2^13", "outlier 2^16", "outlier 2^20"):
+        act = rng.standard_normal((m, k))
+        if name == "log-normal":
+            act = np.sign(act) * np.exp(2 * rng.standard_normal((m, k)))
+        elif name != "normal":
+            act[:, 5] *= 2.0 ** int(name[10:])
+        act = act.astype(np.float32)
+        want = act.astype(np.float64) @ w64.T
+        dact = backend.to_device(act, "f32")
+        errors = []
+        for seq in (False, True):
+            backend.linear_salt(bufs, dact, m, dout, seq=seq)
+            d = dout.to_host().reshape(m, n) - want
+            miss = slice(0, n // 2)
+            errors.append((np.linalg.norm(d) / np.linalg.norm(want), np.linalg.norm(d[:, miss]) / np.linalg.norm(want[:, miss])))
+        assert errors[0][0] <= errors[1][0] and errors[0][1] <= errors[1][1], (name, errors)
+        dact.free()
+    for a in [dout] + bufs:
+        a.free()

@@ -1591,9 +1591,9 @@ extern "C" int tk_linear_rmsnorm_a8(tk_ctx *ctx, const tk_linear_desc *layer, co
 
 constexpr size_t kSaltTokens = 1024;  // tokens per pass of the many-token form of the block-scale planes
 
-// Block-scale additive planes on float activations. seq != 0 forces the reference-order kernel.
+// Block-scale additive planes on float activations. seq != 0 forces the reference-order kernel; strict: see below.
 static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int act_dtype, size_t m, void *out,
-                    int out_dtype, bool seq) {
+                    int out_dtype, bool seq, bool strict = false) {
   if (!layer) return tk_fail(TK_ERR_INVALID_INPUT, "null layer descriptor");
   if (layer->n_planes < 1 || layer->n_planes > TK_MAX_PLANES)
     return tk_fail(TK_ERR_INVALID_INPUT, "n_planes=%d - use 1..%d", layer->n_planes, TK_MAX_PLANES);
@@ -1647,6 +1647,12 @@ static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int
   const size_t flow_tokens = nb ? std::min<size_t>(16, kLdsFlowMax / token_lds) : 16;
   const bool many = !seq && flow_tokens >= 4 && m > flow_tokens;
   bool gemm = many && nb && m <= kSaltTokens;
+  // Rows of which fewer than 16 fit LDS (K > 2304): the other way to run such a call is the reference's order, f32 sums over k.
+  // The block form's error against float64 is a tenth to a fifth of theirs (300 outputs, K=2560 / 5000 / 8192, normal, log-normal
+  // and heavy-tailed tokens: 0.7 .. 1.6e-7 / 6.8 .. 12e-7), except in the outputs that miss the one element that sets a
+  // token's grid (2^12 times the others, f32: 17e-7 / 7e-7). Such tokens take the reference's order, well before the flow
+  // form would send them there.
+  strict = strict || (many && flow_tokens < 16);
   if (gemm && !(R * nb * 256 <= ctx->ap.cap && R * 4 <= ctx->rowsum.cap && m * 4 <= ctx->exps.cap && m * 4 <= ctx->flags.cap &&
                 nb * R * 4 <= ctx->blocksum.cap)) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -1660,7 +1666,7 @@ static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int
     for (size_t m0 = 0; m0 < m; m0 += step) {
       const size_t mc = m - m0 < step ? m - m0 : step;
       TKCHK(run_salt(ctx, layer, (const uint8_t *)act + m0 * k * asz, act_dtype, mc, (uint8_t *)out + m0 * n * osz,
-                     out_dtype, false));
+                     out_dtype, false, strict));
     }
     return TK_OK;
   }
@@ -1681,6 +1687,7 @@ static int run_salt(tk_ctx *ctx, const tk_salt_desc *layer, const void *act, int
   pp.exps = (int32_t *)ctx->exps.p;
   pp.flags = (uint32_t *)ctx->flags.p;
   pp.blocksum = (int32_t *)ctx->blocksum.p;
+  pp.strict = strict;
   pp.k = k;
   pp.nb = nb;
   pp.R = R;

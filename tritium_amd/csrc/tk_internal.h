@@ -133,6 +133,7 @@ struct TkPrep {
   // 2 = scale 1 + w). A normalized row that holds NaN or Inf is also written to ynorm [m,k] f32,
   // which the exact fallback of such rows reads in place of the raw activation.
   int32_t *blocksum;    // DIGITS, optional: [nb][R] sums of each operand row over one K block
+  int strict;           // DIGITS with blocksum: flag a token as soon as the grid costs its outputs more than f32 sums would
   int norm_kind;
   float norm_eps;
   const float *norm_w;  // [k]

@@ -1770,6 +1770,8 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_a8_kernel(TkPrep single, const 
 // An element scaled onto the grid (r = a * 2^(30-E), q = its rounding) is carried faithfully when it
 // lies on the grid or its rounding error is at most 2^-16 of it.
 __device__ __forceinline__ bool digit_poor(float r, int q) { return !(fabsf(r) >= 32768.0f || r == (float)q); }
+// Where the call stands in for sums in the reference's order (TkPrep.strict), at most 2^-21 of it.
+#define TK_DIGIT_STRICT 1048576.0f
 
 // Counts of the elements of one piece per magnitude band: band b holds 2^(30-4b-4) <= |r| < 2^(30-4b);
 // elements below the eighth band (and zeros) are not counted.
@@ -1786,8 +1788,9 @@ __device__ __forceinline__ void count_bands(const float (&v)[16], int shift, int
 #define TK_DIGITS_TRIM 96
 // Energy left without the TK_DIGITS_TRIM largest elements, in units of 2^(2E): band b counts at its
 // lower edge 2^(-4b-4). The grid does not carry the token when its rounding noise n_poor * 2^-62 / 3
-// exceeds 2^-30 of that.
-__device__ __forceinline__ bool digits_narrow(int n_poor, const int (&bands)[8]) {
+// exceeds 2^-30 of that -- or, where the call stands in for the reference's order (strict), 2^-42: amplitude 2^-21 = 4.8e-7,
+// while f32 sums over K >= 2560 in k order show 5.6e-7 and more against float64.
+__device__ __forceinline__ bool digits_narrow(int n_poor, const int (&bands)[8], bool strict = false) {
   float left = 0.0f, edge2 = 0.00390625f;  // 2^-8
   int trim = TK_DIGITS_TRIM;
 #pragma unroll
@@ -1797,7 +1800,7 @@ __device__ __forceinline__ bool digits_narrow(int n_poor, const int (&bands)[8])
     left += (float)(c - cut) * edge2;
     edge2 *= 0.00390625f;
   }
-  return n_poor > 0 && (float)n_poor > 3.0f * 4294967296.0f * left;
+  return n_poor > 0 && (float)n_poor > 3.0f * (strict ? 1048576.0f : 4294967296.0f) * left;
 }
 
 // Float token -> four balanced base-256 digit rows of round(a * 2^(30-E)), 2^(E-1) <= max|a| < 2^E.
@@ -1842,8 +1845,10 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
   if (gamma != 0.0f && !nonfinite) (void)frexpf(gamma, &E);
   const int shift = 30 - E;
   const bool live = gamma != 0.0f && !nonfinite;
-  int sums[5] = {0, 0, 0, 0, 0};  // four digit-row sums, poor elements
-  int &n_poor = sums[4];
+  const bool strict = pp.strict != 0;
+  const float carried = strict ? TK_DIGIT_STRICT : 32768.0f;  // (digit_poor)
+  int sums[6] = {0, 0, 0, 0, 0, 0};  // four digit-row sums, poor elements, elements from `carried` on
+  int &n_poor = sums[4], &n_large = sums[5];
   // split the 16 values of piece pc into their four digit rows and store those in operand order
   auto emit = [&](size_t pc, const float (&v)[16]) {
     const size_t kb = pc >> 4;
@@ -1860,7 +1865,9 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
         if (live && e + b < k) {
           const float r = ldexpf(v[sl * 4 + b], shift);
           q = __float2int_rn(r);  // |q| <= 2^30
-          n_poor += digit_poor(r, q) ? 1 : 0;
+          const bool large = fabsf(r) >= carried;
+          n_large += large ? 1 : 0;
+          n_poor += !(large || r == (float)q) ? 1 : 0;
         }
 #pragma unroll
         for (int dg = 0; dg < 4; ++dg) {
@@ -1909,11 +1916,12 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
       emit(pc, v);
     }
   }
-  block_sums<5>(sums, shi);
+  block_sums<6>(sums, shi);
   // Only a token that has poor elements needs the magnitude bands (the same answer in every thread, so
-  // the barriers inside are reached by all or by none).
+  // the barriers inside are reached by all or by none). Strict: nor does one with enough large elements, each of
+  // 2^-20 in energy (units of 2^(2E)): left >= (n_large - TK_DIGITS_TRIM) * 2^-20 answers digits_narrow.
   bool narrow = false;
-  if (sums[4] > 0) {
+  if (n_poor > 0 && !(strict && n_poor <= 3 * (n_large - TK_DIGITS_TRIM))) {
     int bands[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (resident) {
 #pragma unroll
@@ -1929,7 +1937,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
       }
     }
     block_sums<8>(bands, shi);
-    narrow = digits_narrow(sums[4], bands);
+    narrow = digits_narrow(n_poor, bands, strict);
   }
   if (threadIdx.x < 4) {
     const int t = threadIdx.x;
