@@ -538,8 +538,8 @@ int tk_set_prep_team_rows(tk_ctx *ctx, int rows);
 /* Host-slice calls (tk_mpgemm, tk_mpgemm_with_act_quant) whose operands (activation, scales, output) total at most
  * `bytes` go through a pinned host block that the context owns: one copy kernel brings activation and scales to the
  * device, the kernels write the output into the block, the call synchronizes once -- in place of four transfers from
- * and to pageable memory. Larger calls, and when no pinned memory can be had, take those transfers. Default 16 MiB;
- * 0 = never; at most 64 MiB. Identical results. A tuning and test knob. */
+ * and to pageable memory. Larger calls, calls whose activation is more than 2 MiB plus half of the output, and
+ * when no pinned memory can be had, take those transfers. Default 16 MiB; 0 = never; at most 64 MiB. Identical results. A tuning and test knob. */
 int tk_set_host_direct_bytes(tk_ctx *ctx, size_t bytes);
 /* Decode calls of very few tokens run as ONE launch: the decode kernel quantizes (or digit-splits) the tokens
  * itself, every workgroup for itself, instead of a prep launch in front of it. Single calls (tk_linear_a8,

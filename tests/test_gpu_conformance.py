@@ -128,6 +128,33 @@ def test_determinism(backend, oracle):
     assert same_bits(a, b)
 
 
+@pytest.mark.parametrize("m,n,k", [(640, 128, 4096), (896, 512, 4096), (1024, 2560, 512), (48, 6912, 2560), (8, 2560, 2560)])
+def test_host_calls_are_no_slower_for_the_pinned_block(backend, m, n, k):
+    """Left to itself, a host-slice call takes the pinned block only where that is not slower than the four transfers: large
+    activations with small outputs are (the first two cases: 1.23 and 1.18 times through the block)."""
+    import time
+    from helpers import ternary, scales as mk_scales
+    rng = np.random.default_rng(m + n + k)
+    buf = backend.upload_weights(T.pack_rows(ternary(rng, n, k, 0.4), n, k), T.GemmShape(0, n, k), T.TernaryFormat.Tq2_0)
+    out = np.zeros(m * n, np.float32)
+    call = T.MpGemm(act=rng.standard_normal(m * k).astype(np.float32), weights=buf, scales=mk_scales(rng, n),
+                    shape=T.GemmShape(m, n, k), format=T.TernaryFormat.Tq2_0, out=out)
+    best = {16 << 20: 1e9, 0: 1e9}
+    try:
+        for _ in range(6):
+            for direct in best:
+                backend.set_host_direct_bytes(direct)
+                for i in range(6):
+                    t0 = time.perf_counter()
+                    backend.mpgemm_with_act_quant(call)
+                    best[direct] = min(best[direct], time.perf_counter() - t0) if i else best[direct]
+    finally:
+        backend.set_host_direct_bytes(16 << 20)
+    print("host-direct times", m, n, k, {d: round(t * 1e6, 1) for d, t in best.items()}, "us", flush=True)
+    assert best[16 << 20] <= 1.08 * best[0], best
+    buf.free()
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 6912, 2560), (3, 300, 700), (40, 520, 1280), (1, 33, 256), (300, 1100, 512)])
 def test_host_calls_through_the_pinned_block_agree_with_the_transfers(backend, oracle, m, n, k):
     """Small host-slice calls go through the context's pinned block (one copy kernel in, the kernels write the output

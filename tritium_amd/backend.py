@@ -592,7 +592,8 @@ class Mi355xBackend:
 
     def set_host_direct_bytes(self, nbytes):
         """Host-slice calls (`mpgemm`, `mpgemm_with_act_quant`) of up to `nbytes` of operands go through the context's
-        pinned host block instead of four pageable transfers (default 1 MiB, 0 = never)."""
+        pinned host block instead of four pageable transfers, unless the activation is more than 2 MiB plus half of the
+        output (default 16 MiB, 0 = never)."""
         _check(self._lib.tk_set_host_direct_bytes(self._ctx, nbytes))
 
     def set_fuse_tokens(self, tokens):

@@ -2091,8 +2091,13 @@ static int host_call(tk_ctx *ctx, bool a8, const float *act, size_t act_len, con
   // write the output into the block themselves: two memcpy on the host, the launches and one synchronization in place
   // of four copy-engine transfers from and to pageable memory, which cost ~10 us each whatever their size.
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  // The activation's way in is a memcpy and then the copy kernel, where a transfer overlaps the two: beyond about 2 MiB the block
+  // loses some 9 us a MiB on it (11 on a host whose memcpy is slower), and gains some 8 us on each MiB of output. int8 contract,
+  // transfers / block: 640 tokens K=4096 N=128 (10 MiB in, 0.3 out) 357 / 430 us, 1024 K=2560 N=512 (10, 2) 450 / 504, 1536 K=1024 N=512
+  // (6, 3) 397 / 399 (slower memcpy 1500 K=1000 N=1000 (5.7, 5.7) 550 / 602), 768 K=1024 N=2560 (3, 7.5) 574 / 520, 128 K=4096
+  // N=2560 (2, 1.2) 184 / 170.
   const size_t a_b = al(act_len * 4), s_b = al(n * 4), o_b = al(out_len * 4);
-  if (a_b + s_b + o_b <= ctx->host_direct_bytes && (a8 || !tiny)) {
+  if (a_b + s_b + o_b <= ctx->host_direct_bytes && 2 * a_b <= ((size_t)4 << 20) + o_b && (a8 || !tiny)) {
     TKCHK(ensure_pin(ctx, a_b + s_b + o_b));
     if (ctx->pin) {  // (else the copies below)
       uint8_t *pa = (uint8_t *)ctx->pin, *ps = pa + a_b, *po = ps + s_b;
