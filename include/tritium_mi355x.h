@@ -553,9 +553,10 @@ int tk_set_host_direct_bytes(tk_ctx *ctx, size_t bytes);
 int tk_set_fuse_tokens(tk_ctx *ctx, int tokens);
 /* Calls of this context so far that ran in that single-launch form (for tests of the dispatch). */
 int tk_get_fused_calls(tk_ctx *ctx, unsigned long long *count);
-/* Name of the contraction kernel the last single call of this context (tk_linear_*, tk_mpgemm*) took:
- * "flow", "flow32", "flow3", "stream", "ksplit_decode", "waves", "gemm64", "gemm64_ksplit", "gemm128", "gemm256";
- * "" before the first call. A static string. For tests of the dispatch; no counterpart in the reference. */
+/* Name of the contraction kernel the last single call of this context (tk_linear_*, tk_mpgemm*) or the last group launch
+ * took: "flow", "flow32", "flow3", "stream", "ksplit_decode", "waves", "gemm64", "gemm64_ksplit", "gemm128", "gemm256";
+ * of groups "flow" in both of its forms, and "flow_gemm64" where the members are split over two kernels; "" before the
+ * first call. A static string. For tests of the dispatch; no counterpart in the reference. */
 const char *tk_last_kernel(tk_ctx *ctx);
 /* Row count of the workgroup tile for single launches of one plane under the int8 contract (f32 or bf16
  * rows of whole 16-byte pieces at a 16-byte aligned address, no residual): 0 = chosen per launch, 64 = the

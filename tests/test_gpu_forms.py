@@ -639,8 +639,9 @@ def test_activation_prep_forms_agree(backend, oracle, mode, k, m, copies):
 @pytest.mark.parametrize("m", [17, 20, 32, 64])
 def test_narrow_groups_of_several_row_tiles_take_the_prefill_kernel(backend, oracle, m):
     """q,k,v and gate,up of a decode step of 17..64 tokens are narrow groups (a few hundred tiles) whose rows fit LDS;
-    left to the automatic dispatch they run through the grouped prefill kernel (the K-split kernel below 20 rows for the
-    small group). Whatever is picked: the CPU oracle's bits, with and without an RMSNorm in front."""
+    left to the automatic dispatch they run through the eight-wave kernel of small batches, and through the grouped
+    prefill kernel (the K-split kernel below 20 rows for the small group) in a context that forces a form of it. Whatever
+    is picked: the CPU oracle's bits, with and without an RMSNorm in front."""
     print("case narrow-group", m, flush=True)
     rng = np.random.default_rng(900 + m)
     h, f, kv = 512, 1536, 128
@@ -660,13 +661,19 @@ def test_narrow_groups_of_several_row_tiles_take_the_prefill_kernel(backend, ora
                 out = backend.empty(m * n, "f32")
                 members.append((layer, dx, m, out))
                 keep.append((layer, out, packed, sc, n))
-            grp = backend.group(members, 1, "f32", "f32", norms=[(dw, 1e-5, False)] * len(names) if normed else None)
-            grp.launch()
-            grp.launch()
-            for layer, out, packed, sc, n in keep:
-                want = oracle.cpu_linear_a8_planes([packed], FMT_TQ2_0, [sc], y if normed else x, m, n, h)
-                assert same_bits(out.to_host(), want), (m, n, normed)
-            grp.destroy()
+            wants = [oracle.cpu_linear_a8_planes([packed], FMT_TQ2_0, [sc], y if normed else x, m, n, h) for _, _, packed, sc, n in keep]
+            for tiles, kernel in ((0, "waves"), (2, "gemm64" if m >= 20 else "ksplit_decode")):
+                backend.set_gemm_tiles(tiles)
+                try:
+                    grp = backend.group(members, 1, "f32", "f32", norms=[(dw, 1e-5, False)] * len(names) if normed else None)
+                finally:
+                    backend.set_gemm_tiles(0)
+                grp.launch()
+                grp.launch()
+                assert backend.last_kernel() == kernel, (backend.last_kernel(), kernel)
+                for (layer, out, packed, sc, n), want in zip(keep, wants):
+                    assert same_bits(out.to_host(), want), (m, n, normed, kernel)
+                grp.destroy()
             for layer, out, *_ in keep:
                 out.free()
                 layer.free()

@@ -88,6 +88,7 @@ def test_groups(backend, mode, planes, ms):
             g = backend.group(list(zip(layers, acts, ms, o)), mode, "f32", "f32", **({"norms": norms} if mode == 1 else {}))
             for _ in range(2):
                 g.launch()
+                assert backend.last_kernel() == ("ksplit_decode" if force else "waves"), backend.last_kernel()
             outs.append([x.to_host() for x in o])
             g.destroy()
             for x in o:

@@ -609,7 +609,7 @@ class Mi355xBackend:
         return int(c.value)
 
     def last_kernel(self):
-        """Name of the contraction kernel the last single call took ("flow", "gemm64_ksplit", "gemm128", ...)."""
+        """Name of the contraction kernel the last single call or group launch took ("flow", "gemm64_ksplit", "waves", ...)."""
         return self._lib.tk_last_kernel(self._ctx).decode()
 
     def set_gemm_rows(self, rows):

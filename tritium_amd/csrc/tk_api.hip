@@ -85,7 +85,7 @@ struct tk_ctx {
   int gemm_two_by_two = 0;  // one-plane prefill kernel, 64 x 128 form: 0 = four waves side by side, 1 = two by two
   int gemm_ksplit = 0;     // prefill kernel, single launches: 0 = K slices chosen per launch, 1 = never split, n = n slices
   unsigned long long fused_calls = 0;  // calls that ran as one launch (tk_get_fused_calls)
-  const char *last_kernel = "";        // contraction kernel of the last single call (tk_last_kernel)
+  const char *last_kernel = "";        // contraction kernel of the last call (tk_last_kernel)
   // Host-slice calls (tk_mpgemm, tk_mpgemm_with_act_quant) of up to host_direct_bytes of operands go through this
   // pinned host block: a copy kernel reads the activation and the scales from it, the kernels write the output into
   // it -- no copy-engine transfers (see host_call; grow-only; freed with the context)
@@ -2732,6 +2732,10 @@ extern "C" int tk_group_launch_parts(tk_ctx *ctx, tk_group *g, int do_prep, int 
   const TkProblem *probs = (const TkProblem *)g->tables;
   const TkPrep *preps = (const TkPrep *)((const uint8_t *)g->tables + (size_t)g->nprobs * sizeof(TkProblem));
   if (do_main && g->fused) ctx->fused_calls++;
+  if (do_main) {
+    static const char *const names[] = {"", "ksplit_decode", "stream", "flow", "gemm64", "waves"};  // (DECODE_*)
+    ctx->last_kernel = g->has_flow_part ? "flow_gemm64" : (g->variant == DECODE_FLOW && g->cfg.base3 ? "flow3" : names[g->variant]);
+  }
   if (do_prep && !g->fused)  // (a group that runs as one launch has no prep part)
     HIPCHK(tk_launch_prep(ctx->stream, g->prep_kind, nullptr, preps, g->nprep, g->prep_uniform_m, g->prep_rows,
                           g->prep_wave_pieces, g->prep_fast, g->prep_norm_fast, g->prep_norm_pieces));
