@@ -21,7 +21,7 @@ constexpr int WAVES = 8;
 
 // RT: 32-row tiles of operand rows (1: up to 32 rows, 2: up to 64)
 template <int P, int RT, bool TABLE>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(RT * P <= 3 && !(RT == 2 && P > 1) ? 4 : 2, RT * P <= 3 && !(RT == 2 && P > 1) ? 4 : 2))) void
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(RT * P <= 3 ? 4 : 2, RT * P <= 3 ? 4 : 2))) void
 tk_waves_kernel(const TkProblem single, const TkProblem *__restrict__ table, const int *__restrict__ wg_prob) {
   __shared__ __attribute__((aligned(16))) v4i part[WAVES][RT][4][64];  // [wave][row tile][register quad][lane]
   const TkProblem &pr = TABLE ? table[wg_prob[blockIdx.x]] : *single_problem();
@@ -38,7 +38,7 @@ tk_waves_kernel(const TkProblem single, const TkProblem *__restrict__ table, con
 #pragma unroll
   for (int t = 0; t < RT; ++t) rows[t] = pr.ap + kappa * seg + (size_t)min(t * 32 + (lane & 31), R - 1) * 16;
 
-  // a unit of work is a whole K block (one row tile) or half of one (two: their pieces would not fit the registers twice)
+  // a unit of work is a whole K block for one plane and one row tile, else half of one (the registers hold two units)
   constexpr int L = RT * P == 1 ? 2 : 1, PER = 2 / L;
   struct Unit {
     uint4 a[RT][L][4], w[P][L];
@@ -134,7 +134,7 @@ hipError_t tk_launch_waves(hipStream_t s, const TkProblem *single, const TkProbl
   switch (planes) {
     case 1: return two ? go<1, 2>(s, single, table, wg_prob, grid) : go<1, 1>(s, single, table, wg_prob, grid);
     case 2: return two ? go<2, 2>(s, single, table, wg_prob, grid) : go<2, 1>(s, single, table, wg_prob, grid);
-    case 3: return two ? go<3, 2>(s, single, table, wg_prob, grid) : go<3, 1>(s, single, table, wg_prob, grid);
+    case 3: return two ? hipErrorInvalidValue : go<3, 1>(s, single, table, wg_prob, grid);
     default: return hipErrorInvalidValue;
   }
 }
