@@ -101,3 +101,88 @@ def test_groups(backend, mode, planes, ms):
         a.free()
     for layer in layers:
         layer.free()
+
+
+# both sides of the lines of the dispatch rule: the kernel that the eight waves replace, short and long rows, within a round of
+# workgroups and beyond one
+@pytest.mark.parametrize("m,n,k,planes,kernel", [
+    (18, 17024, 256, 1, "gemm64"), (32, 16400, 256, 1, "gemm64"), (18, 16384, 256, 1, "waves"), (24, 16900, 2560, 1, "waves"),   # prefill kernel
+    (40, 16400, 512, 1, "gemm64"), (48, 16384, 300, 1, "waves"),
+    (4, 16400, 300, 1, "waves"), (12, 16400, 300, 1, "ksplit_decode"), (12, 16400, 2200, 1, "waves"),                             # K-split kernel
+    (3, 8208, 8192, 1, "ksplit_decode"), (4, 8208, 8192, 1, "waves"),
+    (4, 10560, 2816, 3, "flow"), (8, 1280, 2048, 3, "waves"), (8, 1280, 1792, 3, "flow"), (4, 2560, 1024, 2, "flow"),             # flow kernel
+    (24, 16384, 512, 3, "flow"), (24, 16384, 768, 3, "waves")])
+def test_both_sides_of_the_dispatch_rule(backend, m, n, k, planes, kernel):
+    print("case waves rule", m, n, k, planes, kernel, flush=True)
+    rng = np.random.default_rng(m + n + k + planes)
+    packed = [T.pack_rows(rng.integers(-1, 2, (n, k), dtype=np.int8), n, k) for _ in range(planes)]
+    layer = backend.linear(packed, [scales(rng, n) for _ in packed], n, k)
+    dact = backend.to_device(f32_to_bf16_bits(rng.standard_normal((m, k)).astype(np.float32)), "bf16")
+    o, o2 = backend.empty(m * n, "bf16"), backend.empty(m * n, "bf16")
+    backend.linear_a8(layer, dact, m, o)
+    assert backend.last_kernel() == kernel, backend.last_kernel()
+    forced(backend, lambda: backend.linear_a8(layer, dact, m, o2))
+    assert o.to_host().tobytes() == o2.to_host().tobytes()
+    for a in (dact, o, o2):
+        a.free()
+    layer.free()
+
+
+@pytest.mark.parametrize("m,shapes,planes,kernel", [
+    (16, [(6912, 6912)] * 6, 1, "waves"),               # rows within LDS, several workgroups of the K-split kernel per CU
+    (16, [(130, 10496), (70, 2304)], 2, "waves"),       # one member's rows beyond LDS
+    (16, [(48, 10496)] * 3, 3, "waves"),
+    (8, [(8448, 512)] * 2, 2, "flow"), (40, [(8448, 512)] * 2, 1, "gemm64")])
+def test_both_sides_of_the_dispatch_rule_in_groups(backend, m, shapes, planes, kernel):
+    print("case waves rule group", m, shapes, planes, kernel, flush=True)
+    rng = np.random.default_rng(m + len(shapes) + planes)
+    made, acts, members = {}, {}, []
+    for n, k in shapes:
+        if (n, k) not in made:
+            packed = [T.pack_rows(rng.integers(-1, 2, (n, k), dtype=np.int8), n, k) for _ in range(planes)]
+            made[(n, k)] = backend.linear(packed, [scales(rng, n) for _ in packed], n, k)
+        if k not in acts:
+            acts[k] = backend.to_device(rng.standard_normal((m, k)).astype(np.float32), "f32")
+    results = []
+    for force in (0, 1):
+        outs = [backend.empty(m * n, "f32") for n, _ in shapes]
+        backend.set_decode_kernel(force)
+        try:
+            g = backend.group([(made[s], acts[s[1]], m, o) for s, o in zip(shapes, outs)], 1, "f32", "f32")
+        finally:
+            backend.set_decode_kernel(0)
+        g.launch()
+        assert backend.last_kernel() == ("ksplit_decode" if force else kernel), backend.last_kernel()
+        results.append([o.to_host() for o in outs])
+        g.destroy()
+        for o in outs:
+            o.free()
+    for a, b in zip(*results):
+        assert same_bits(a, b)
+    for x in list(acts.values()) + list(made.values()):
+        x.free()
+
+
+def test_sparse_planes_leave_only_the_flow_kernel_its_calls(backend):
+    """Planes with a zero-chunk map: the flow kernel, which skips their chunks, keeps what it was chosen for; the K-split and the
+    prefill kernel do not read the map, and their calls go to the eight waves as any other's."""
+    rng = np.random.default_rng(3)
+    backend.set_zero_skip(2)
+    try:
+        for m, n, k, planes, kernel in ((16, 640, 2560, 1, "waves"), (32, 640, 2560, 1, "waves"), (8, 5120, 2560, 2, "flow")):
+            packed = []
+            for _ in range(planes):
+                w = rng.integers(-1, 2, (n, k), dtype=np.int8)
+                w[16:48] = 0  # whole chunks of zeros
+                packed.append(T.pack_rows(w, n, k))
+            layer = backend.linear(packed, [scales(rng, n) for _ in packed], n, k)
+            dact, o, o2 = backend.to_device(rng.standard_normal((m, k)).astype(np.float32), "f32"), backend.empty(m * n, "f32"), backend.empty(m * n, "f32")
+            backend.linear_a8(layer, dact, m, o)
+            assert backend.last_kernel() == kernel, (m, n, k, backend.last_kernel())
+            forced(backend, lambda: backend.linear_a8(layer, dact, m, o2))
+            assert same_bits(o.to_host(), o2.to_host())
+            for a in (dact, o, o2):
+                a.free()
+            layer.free()
+    finally:
+        backend.set_zero_skip(0)

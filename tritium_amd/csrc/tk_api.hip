@@ -768,31 +768,56 @@ struct Plan {
 
 enum { DECODE_AUTO = 0, DECODE_KSPLIT = 1, DECODE_STREAM = 2, DECODE_FLOW = 3, DECODE_GEMM = 4, DECODE_WAVES = 5 };
 
-// Calls and groups that take the eight-wave kernel of small batches (tk_waves.hip) instead of `variant`: `pairs`
-// workgroups (32 columns each). It wins where they run side by side, two per CU (one for two planes beyond 32 rows), and
-// loses to the flow or prefill kernel, which reuse what they staged, once a second round begins. Call, before -> this, int8
-// rows, bf16 tokens: one plane K=2560 N=2560 4 / 16 / 32 / 64 tokens 10.1 -> 8.9 / 12.2 -> 9.3 / 14.2 -> 9.5 / 14.4 -> 10.1 us;
-// K=6912 N=2560 13.0 -> 10.8 / 16.9 -> 11.2 / 17.0 -> 11.8 / 17.5 -> 13.9; K=5120 N=10240 (320 workgroups) 3 / 16 / 64 tokens
-// two planes 14.3 -> 13.5 / 18.8 -> 14.2 / 22.0 -> 23.1, three planes 16.5 -> 16.6 / 22.4 -> 17.5; N=17408 (544) K=2560 3 / 16 / 64
-// tokens one plane 11.5 -> 10.9 / 17.6 -> 12.6 / 14.8 -> 15.8, two 12.4 -> 13.2 / 20.4 -> 14.9 / 18.1 -> 23.3, three 14.1 -> 15.9 /
-// 15.8 -> 17.0, but K=5120 8 float tokens two planes 23.8 -> 19.5, three 28.3 -> 23.4: a few workgroups beyond the round are
-// worth it for one plane or long rows. Two planes and more of short rows (K <= 1024), up to eight rows: 8.3 -> 8.7 .. 9.8 -> 8.9,
-// left alone. Groups, 48 x K=1024 N=1024 16 tokens 11.0 -> 14.9; but rows beyond LDS in one row tile, which the streaming
-// kernel would stage K slice by K slice, six of K=6912 N=6912 16 tokens 54.9 -> 28.8 (one plane), 81 -> 48 (three).
-// (a context with a kernel form forced keeps it; two int8 tokens and one float token run as one launch in the decode kernels; planes with a zero-chunk map keep the flow
-// kernel, which skips their chunks; three planes beyond 32 rows keep the K-split prefill kernel)
-static bool waves_pays(const tk_ctx *ctx, bool flow_ok, bool zskip, int planes, size_t rows, size_t tokens, size_t pairs, size_t nb,
+// Whether a call or group of few tokens takes the eight-wave kernel (tk_waves.hip) instead of `old`, the kernel that the rules of
+// run_linear and group_create chose among the others. `pairs` workgroups of 32 columns go through whole K rows from L2 and memory:
+// side by side (`round`: two per CU, one for two planes beyond 32 rows) they win on latency; beyond a round they compete with
+// what the other kernels stage once and use again. Calls back to back, int8 rows, bf16 tokens, us of old / eight waves:
+// * K-split kernel, one round: K=2560 N=2560 4 / 16 tokens 10.1 / 8.9, 12.2 / 9.3; two planes K=6912 N=2560 16 tokens 20.0 / 13.0. Its own are three
+//   rows of one plane and K >= 8192 on more than a workgroup per CU, in one pass through LDS: K=8192 N=12288 13.6 / 14.8.
+//   Beyond, its workgroups stage the same rows again and again: rows of 24 KiB and more lose at any number of workgroups
+//   (tokens x K, workgroups: 12 x 2560, 896 17.4 / 13.9; 4 x 6912, 648 21.8 / 18.1; 16 x 17408, 1280 121 / 47; 16 x 6912, 1296 -- six members
+//   of N=6912 in a group -- 54.9 / 28.7, two planes 71 / 39, three 81 / 49), shorter ones are even or win (12 x 1024, 768 11.1 / 11.9;
+//   4 x 5120, 528 14.1 / 14.8) but up to eight rows of one plane and K <= 2560 (to 1.5 rounds: 4 x 1024, 768 10.3 / 9.6; 3 / 4 / 8 x
+//   2560, 544 10.7 / 10.9, 11.5 / 11.2, 12.2 / 11.3).
+// * Prefill kernel, one round: 32 tokens K=2560 N=2560 14.2 / 9.5, 64 tokens of two planes 16.6 / 11.7. Beyond, up to 32 rows: K=1024
+//   11.0 / 11.7 (768), K=2048 13.1 / 12.7 (768), K=2560 14.4 / 13.3 (640), 14.6 / 14.6 (1008), K=8192 37.1 / 35.6 (1536), 40.9 / 44.5 (2048), two
+//   planes 55.4 / 46.5, 64.3 / 63.7. 40 and 64 rows lose from the first workgroup on (K=2560, 544 14.6 / 16.1; two planes, 288 16.6 / 17.0).
+// * Flow kernel, one round. Up to eight rows of two planes: K=1024 8.8 / 9.3, K=2048 10.3 / 10.3, K=4096 14.2 / 13.4, K=17408 42.4 / 32.6; of three
+//   planes (5 rows), a workgroup per CU and less: K=1536 9.9 / 10.1, K=2048 10.8 / 10.4, K=2560 12.1 / 10.9; more: K=2560 12.4 / 12.6, K=4096
+//   15.7 / 17.2, K=8192 22.4 / 21.8, 25.2 / 25.0, K=10240 27.8 / 25.6. 12 rows of three planes: K=1536 11.0 / 12.0, K=2560 14.6 / 13.6. 17..32
+//   rows: K=256 8.7 / 9.4, K=512 9.5 / 9.6, K=1024 11.3 / 10.1. Beyond, only long rows of many tokens: 32 x 2560 15.7 / 15.5 (576), 15.8 / 16.1
+//   (768), 32 x 5120 24.1 / 20.8 (528), 24.7 / 21.8 (768), 26.1 / 25.4 (1024), three planes 29.2 / 24.7, 30.1 / 26.9; three planes
+//   16 x 5120 24.4 / 24.3, 16 x 10240 40.3 / 35.6, 4 x 10240 38.2 / 35.5; 4 x 2560 two planes 12.5 / 13.6.
+// * Streaming kernel (rows beyond LDS), groups of up to 16 rows: K=12800, 16 members of N=5120 81 / 71, four of N=17408 74 / 60, three planes
+//   186 / 144; six of them, whose codes no cache holds, 97 / 105, three planes 212 / 209. Single layers of that width go either way
+//   (N=65536 67 / 54, N=131072 107 / 128) and stay.
+// Not for: contexts with a kernel form forced; one token, and two under the int8 contract (one launch in the decode kernels);
+// planes whose zero-chunk map the flow kernel would use. Three planes beyond 32 rows keep the prefill kernel.
+static bool waves_pays(const tk_ctx *ctx, int old, bool zskip, int planes, size_t rows, size_t tokens, size_t pairs, size_t nb,
                        int mode, bool group) {
   if (ctx->decode_force != DECODE_AUTO || ctx->flow_run_tiles || ctx->flow_ring || ctx->flow_mfma || ctx->flow_wg16 > 0 || !ctx->flow_swap ||
       ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit || ctx->gemm_rows || ctx->stream_min_groups < ctx->info.compute_units ||
       (ctx->fuse_tokens > 0 && tokens <= (size_t)ctx->fuse_tokens))
     return false;
-  if (zskip || planes > 3 || tokens < (mode == TK_MODE_INT8 ? 3u : 2u)) return false;
-  if (rows > (planes == 3 ? 32u : 64u) || nb == 0) return false;
-  if (planes >= 2 && nb <= 4 && rows <= 8) return false;
-  if (group && !flow_ok && rows <= 16) return true;
-  const size_t round = (rows <= 32 || planes == 1 ? 2 : 1) * (size_t)ctx->info.compute_units;
-  return pairs <= round || (rows <= 32 && (planes == 1 || nb >= 16) && pairs * 16 <= round * 17);
+  if (planes > 3 || nb == 0 || tokens < (mode == TK_MODE_INT8 ? 3u : 2u) || rows > (planes == 3 ? 32u : 64u)) return false;
+  const size_t cus = (size_t)ctx->info.compute_units, round = (rows <= 32 || planes == 1 ? 2 : 1) * cus;
+  const size_t row_bytes = rows * nb * 256;
+  const bool one = pairs <= round, half_more = pairs * 2 <= round * 3;
+  switch (old) {
+    case DECODE_KSPLIT:
+      if (one) return !(planes == 1 && rows <= 3 && nb >= 32 && pairs > cus && row_bytes <= kLdsABudget);
+      return (rows >= 4 && row_bytes >= 24 * 1024) || (planes == 1 && rows <= 8 && nb <= 10 && half_more);
+    case DECODE_GEMM:
+      return one || (rows <= 32 && ((nb >= 8 && half_more) || (nb >= 16 && pairs <= 3 * round)));
+    case DECODE_FLOW:
+      if (zskip) return false;
+      if (one && rows > 16) return nb > 2;
+      if (one && rows > 8) return planes < 3 || nb > 6;
+      if (one) return planes < 3 ? planes == 1 || nb > 4 : (pairs <= cus ? nb >= 8 : nb > 32 || row_bytes >= 64 * 1024);
+      return rows <= 32 && half_more && ((rows > 16 && nb >= 20) || (rows > 8 && nb >= 32) || (planes == 3 && nb >= 40));
+    case DECODE_STREAM: return group && rows <= 16;
+    default: return false;
+  }
 }
 
 static const size_t kLdsFlowMax = 160 * 1024;
@@ -1260,6 +1285,9 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
   bool wide = false, b3 = false;
   const bool decode = pl.skinny;
   size_t flow_lds = pl.flow_lds;
+  // The rules of this block choose among the K-split, flow, streaming and prefill kernels, and their figures are of those among
+  // each other. Three and more tokens are then compared with the eight-wave kernel (waves_pays): what stays with these kernels
+  // are one and two tokens, four planes, base-3 streams, contexts with a form forced, and the launches that rule names.
   if (pl.skinny) {
     b3 = pl.flow_ok && flow_base3(pl.pr, pl.cfg.planes, pl.cfg.rt, flow_lds);
     wide = !b3 && pl.flow_ok && flow_wide(ctx, pl.cfg.planes, pl.cfg.rt, nb, R, mode == TK_MODE_INT8 && ctx->flow_swap);
@@ -1340,7 +1368,8 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
       plan_gemm(&pl, 4u * (unsigned)ctx->info.compute_units, ctx->gemm_tiles);
     }
   }
-  const bool waves = decode && !b3 && waves_pays(ctx, pl.flow_ok, pl.pr.zskip != 0, pl.cfg.planes, R, m, ((size_t)pl.pr.n_tiles + 1) / 2, nb, mode, false);
+  const bool waves = decode && !b3 && waves_pays(ctx, pl.skinny ? variant : DECODE_GEMM, pl.pr.zskip != 0, pl.cfg.planes, R, m,
+                                                 ((size_t)pl.pr.n_tiles + 1) / 2, nb, mode, false);
   if (waves) {
     pl.skinny = false;
     pl.pr.rs = (int)R;
@@ -2396,8 +2425,8 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
     fgroups += ((unsigned)plans[i].pr.n_tiles + fper - 1) / fper;
     if (plans[i].stream_lds > slds) slds = plans[i].stream_lds;
   }
+  // (as in run_linear: these rules choose among the other kernels, waves_pays then compares the eight-wave kernel with their choice)
   int variant = choose_decode(ctx, flow_ok, fgroups, sgroups);
-  const bool fits_lds = flow_ok;
   // One token for a group of more than two tiles per CU (gate,up): the flow kernel behind the prep launch, as for single
   // calls (run_linear) -- the K-split kernel would hand its workgroups several tiles each. gate,up of hidden 2560 behind
   // an RMSNorm, rotating over 30 layers: 13.4 -> 11.6 us (2 / 4 / 8 tokens 12.9 -> 12.9 / 13.9 -> 13.2 / 14.7 -> 13.8: left);
@@ -2431,7 +2460,7 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
       pairs += ((size_t)plans[i].pr.n_tiles + 1) / 2;
       zskip = zskip || plans[i].pr.zskip;
     }
-    if (!b3 && waves_pays(ctx, fits_lds, zskip, planes, rows_max, tokens_max, pairs, nb_max, kmode, true)) variant = DECODE_WAVES;
+    if (!b3 && waves_pays(ctx, variant, zskip, planes, rows_max, tokens_max, pairs, nb_max, kmode, true)) variant = DECODE_WAVES;
   }
   std::vector<int> wg_prob;
   int group_gemm_nt = 0;
