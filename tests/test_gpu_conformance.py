@@ -155,7 +155,9 @@ def test_host_calls_are_no_slower_for_the_pinned_block(backend, m, n, k):
     buf.free()
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 6912, 2560), (3, 300, 700), (40, 520, 1280), (1, 33, 256), (300, 1100, 512)])
+@pytest.mark.parametrize("m,n,k", [(1, 6912, 2560), (3, 300, 700), (40, 520, 1280), (1, 33, 256), (300, 1100, 512),
+                                   (70, 6001, 2050), (129, 2560, 1024), (600, 4096, 700), (900, 4096, 513),  # 2 to 16 MiB, less than the limit
+                                   (1030, 4100, 300), (400, 130, 2560)])  # beyond it in all, and in the activation
 def test_host_calls_through_the_pinned_block_agree_with_the_transfers(backend, oracle, m, n, k):
     """Small host-slice calls go through the context's pinned block (one copy kernel in, the kernels write the output
     into it); larger ones, and all of them with the knob at 0, take four transfers from and to pageable memory. Same
@@ -171,20 +173,22 @@ def test_host_calls_through_the_pinned_block_agree_with_the_transfers(backend, o
     if m >= 3:
         act[1, 3] = np.nan
     got = {}
-    for direct in (1 << 20, 0):
-        backend.set_host_direct_bytes(direct)
-        for fused in (True, False):
-            out = np.zeros(m * n, np.float32)
-            p = T.MpGemm(act=act.reshape(-1), weights=buf, scales=sc, shape=T.GemmShape(m, n, k),
-                         format=T.TernaryFormat.Tq2_0, out=out)
-            (backend.mpgemm_with_act_quant if fused else backend.mpgemm)(p)
-            got[(direct, fused)] = out
-    backend.set_host_direct_bytes(1 << 20)
+    try:
+        for direct in (16 << 20, 0):
+            backend.set_host_direct_bytes(direct)
+            for fused in (True, False):
+                out = np.zeros(m * n, np.float32)
+                p = T.MpGemm(act=act.reshape(-1), weights=buf, scales=sc, shape=T.GemmShape(m, n, k),
+                             format=T.TernaryFormat.Tq2_0, out=out)
+                (backend.mpgemm_with_act_quant if fused else backend.mpgemm)(p)
+                got[(direct, fused)] = out
+    finally:
+        backend.set_host_direct_bytes(16 << 20)
     for fused in (True, False):
-        a, b = got[(1 << 20, fused)], got[(0, fused)]
+        a, b = got[(16 << 20, fused)], got[(0, fused)]
         fin = ~np.isnan(a)
         assert (np.isnan(b) == ~fin).all() and same_bits(a[fin], b[fin]), fused
     rc, want = oracle.cpu_mpgemm_with_act_quant(packed, FMT_TQ2_0, act, sc, m, n, k)
     fin = ~np.isnan(want.reshape(-1))
-    assert same_bits(got[(1 << 20, True)][fin], want.reshape(-1)[fin])
+    assert same_bits(got[(16 << 20, True)][fin], want.reshape(-1)[fin])
     buf.free()
