@@ -4,6 +4,8 @@ The host definition (dequantize the row, planes in order; then one f32 accumulat
 crates/tritium-format/src/salt.rs:720-738, crates/tritium-nn/src/layers/packed_salt.rs:585-628) is the
 oracle. The reference-order kernel must reproduce it bit for bit; the matrix-core form is held to the
 bound the reference sets for its own GPU kernel, 1e-4 (crates/tritium-cuda/kernels/tq2_0_add.cu:651-655)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -79,8 +81,51 @@ def test_tokens_with_nan_or_inf_take_the_host_order(backend, oracle):
         a.free()
 
 
+@pytest.mark.parametrize("m,n,k", [(40, 72, 768), (9, 40, 5000)])
+def test_passes_where_the_workspace_cannot_grow(oracle, m, n, k):
+    """A context whose workspace has the size of a few tokens, under stream capture: the call may not allocate there and runs in
+    passes of as many tokens as the flow form takes (16, 16, 8; 7, 2). The bits of the call in one launch, on every replay."""
+    print("case salt-passes", m, n, k, flush=True)
+    backend = T.Mi355xBackend(0)
+    hip = C.CDLL("libamdhip64.so.7")
+    stream = C.c_void_p(backend.stream_handle())
+    rng = np.random.default_rng(m + n + k)
+    packed, bufs = make_planes(backend, oracle, rng, n, k, 2)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    act[m - 1, 3] = np.nan
+    few = min(16, 163840 // ((k + 255) // 256 * 1040))
+    dact, dout, dfew = backend.to_device(act, "f32"), backend.empty(m * n, "f32"), backend.empty(16 * n, "f32")
+    for count in (few, m % few):
+        backend.linear_salt(bufs, dact, count, dfew)
+    graph, gexec, nodes = C.c_void_p(), C.c_void_p(), C.c_size_t(0)
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    try:
+        backend.linear_salt(bufs, dact, m, dout)
+    finally:
+        rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+    assert rc == 0 and hip.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
+    assert nodes.value == 2 * ((m + few - 1) // few)  # a digit split and a flow launch per pass
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, C.c_size_t(0)) == 0
+    got = []
+    for _ in range(3):
+        dout.copy_from(np.zeros(m * n, np.float32))
+        backend.linear_salt(bufs, dact, few, dfew)
+        assert hip.hipGraphLaunch(gexec, stream) == 0
+        backend.sync()
+        got.append(dout.to_host())
+    assert hip.hipGraphExecDestroy(gexec) == 0 and hip.hipGraphDestroy(graph) == 0
+    backend.linear_salt(bufs, dact, m, dout)  # eager: the workspace grows, one launch
+    want = dout.to_host()
+    assert all(same_bits(x, want) for x in got)
+    rc, host = oracle.salt_mpgemm(packed, n, k, act, m)
+    assert accepts(want.reshape(m, n)[:-1], host[:-1], rel=SALT_REL, floor=1.0).all() and np.isnan(want.reshape(m, n)[-1]).any()
+    for a in [dact, dout, dfew] + bufs:
+        a.free()
+    backend.close()
+
+
 def test_more_than_16_tokens_run_in_slices(backend, oracle):
-    """40 tokens are three slices (16, 16, 8) of the matrix-core form, the ragged last one included."""
+    """40 tokens are one launch: three slices of 16 operand tokens (64 rows), the last one of 8 tokens."""
     rng = np.random.default_rng(41)
     m, n, k = 40, 72, 768
     packed, bufs = make_planes(backend, oracle, rng, n, k, 2)
@@ -173,7 +218,7 @@ def test_every_f16_block_scale_reaches_the_kernels_exactly(backend, oracle):
 @pytest.mark.parametrize("m,n,k,t_planes,dtype", [(17, 130, 256, 1, "f32"), (33, 33, 700, 2, "f32"), (64, 257, 2560, 3, "bf16"), (65, 15, 1000, 4, "f32"),
                                                   (130, 96, 2048, 2, "bf16"), (1027, 40, 300, 1, "f32"),
                                                   (512, 4100, 300, 1, "f32"),  # the 64-column waves
-                                                  (9, 70, 5000, 2, "f32")])    # seven such tokens fit the flow form
+                                                  (9, 70, 5000, 2, "f32")])    # seven such tokens fit the flow form (of K = 2560 fifteen)
 def test_many_tokens_have_the_bits_of_sixteen_at_a_time(backend, oracle, m, n, k, t_planes, dtype):
     """The many-token form adds the same exact block values in the same order as the flow form: identical bits, rows past the
     last row tile, columns past the last pair, a token holding NaN and a second pass of tokens included."""
@@ -189,7 +234,7 @@ def test_many_tokens_have_the_bits_of_sixteen_at_a_time(backend, oracle, m, n, k
     got = dout.to_host().reshape(m, n)
     want = np.empty_like(got)
     rows = np.asarray(host).reshape(m, k)
-    step = 16 if k <= 2560 else 4
+    step = min(16, 163840 // ((k + 255) // 256 * 1040))  # tokens that the flow form holds in LDS
     for m0 in range(0, m, step):
         part = rows[m0:m0 + step]
         dact, dpart = backend.to_device(part, dtype), backend.empty(len(part) * n, dtype)

@@ -137,8 +137,8 @@ def test_v2_refuses_non_finite_and_leaves_the_output_alone(backend, so):
 
 
 def test_v2_refusals_in_the_lane_per_row_form(backend, so):
-    """Rows of whole scale groups take the form that keeps its terms in a workspace: the same refusals there,
-    and the first row block's finiteness check covers every token."""
+    """Rows of whole scale groups take the form on the matrix pipe: the same refusals there, and the finiteness check of the
+    workgroups of the first sixteen rows covers every token."""
     one16 = 0x3C00
     fmax = np.float32(np.finfo(np.float32).max)
     trits = np.zeros((1, 256), np.int8)
