@@ -681,12 +681,13 @@ def test_narrow_groups_of_several_row_tiles_take_the_prefill_kernel(backend, ora
     dw.free()
 
 
-@pytest.mark.parametrize("k", [257, 1027, 2050, 4099])
+@pytest.mark.parametrize("k", [257, 1027, 2050, 3001, 4095, 4099])
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("m", [40, 400])
 def test_prep_of_rows_aligned_like_an_element(backend, oracle, m, k, dtype):
     """Rows whose starts are aligned like one element only (odd K, a base one element into a buffer): the vector loads of the
-    quantization against the oracle, and the digit split's two forms (a workgroup or a wave per token) against each other."""
+    quantization against the oracle, and the digit split's two forms (a workgroup or a wave per token) against each other where
+    there are two: rows of 65 to 256 pieces of 16 elements (257 has one piece per lane and keeps the wave, 4099 the workgroup)."""
     print("case ragged prep", m, k, dtype, flush=True)
     rng = np.random.default_rng(m + k)
     n = 40
