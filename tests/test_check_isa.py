@@ -112,6 +112,8 @@ amdhsa.kernels:
     bad = check_isa.check_budgets(meta, budgets)
     assert ("_Z4betaILi2EEvv", 169, 168) in bad and ("_Z5gammaILi3EEvv", 10100, 128) in bad and ("deltaILi4E", None, 64) in bad
     assert not any("alpha" in b[0] for b in bad) and len(bad) == 3
+    assert check_isa.check_budgets(meta, (("gammaILi3E", 128, 4),)) == []  # spills up to the stated number
+    assert check_isa.check_budgets(meta, (("gammaILi3E", 128, 3),)) == [("_Z5gammaILi3EEvv", 10100, 128)]
 
 
 def test_static_lds_rule():

@@ -127,7 +127,8 @@ def check_text(text, only=("tk_gemm",)):
     return found
 
 
-# Register budgets of the bandwidth kernels: (template arguments of the kernel, vector registers at most).
+# Register budgets of the bandwidth kernels: (template arguments of the kernel, vector registers at most, and registers that
+# may be spilled: none where it is left out).
 # A CU runs floor(512 / registers) waves per SIMD, in steps of 8 registers: 128 -> 4, 168 -> 3, 256 -> 2. The
 # decode kernels' rate follows the bytes their waves keep in flight, so a change that pushes one of these
 # forms over its step (a few registers are enough) costs a third or a quarter of the rate without any test
@@ -154,6 +155,20 @@ REGISTER_BUDGETS = (
     ("tk_gemm256_kernelILi0E", 512),                # prefill, 256 x 224 form, four waves (one per SIMD)
     ("tk_gemm256_kernelILi1E", 256),                # ... eight waves (two per SIMD)
     ("tk_gemm256_kernelILi2E", 256),                # ... four waves over 128 | 96 outputs, two workgroups per CU
+    ("tk_waves_kernelILi1ELi1E", 128),              # small batches: two workgroups of eight waves per CU
+    ("tk_waves_kernelILi1ELi2E", 128, 1),           # (a register outside the loop over K)
+    ("tk_waves_kernelILi2ELi1E", 128),
+    ("tk_waves_kernelILi3ELi1E", 128, 1),
+    ("tk_waves_kernelILi2ELi2E", 256),              # ... two planes beyond 32 rows: one workgroup per CU
+    ("tk_salt_gemm_kernelILi1ELi1E", 256),          # block-scale planes, many tokens: two workgroups of four waves per CU
+    ("tk_salt_gemm_kernelILi1ELi2E", 256),
+    ("tk_salt_gemm_kernelILi2ELi1E", 256),
+    ("tk_salt_v2_exact_kernelILi64E", 128),         # sixteen waves per workgroup
+    ("tk_salt_v2_exact_kernelILi128E", 128),
+    ("tk_vjp_act_kernelILi1E", 72),                 # grad_act: seven, five and four waves per SIMD
+    ("tk_vjp_act_kernelILi2E", 96),
+    ("tk_vjp_act_kernelILi4E", 128),
+    ("tk_vjp_weight_kernelILi8ELi4E", 96),          # grad_w: five waves per SIMD
 ) + tuple(  # the 32x32x32 flow forms that consult the zero-chunk maps, in both operand orders: present, no spills
     (f"tk_flow32_kernelILi{p}ELi{rt2}ELi{dr}ELb{t}ELb1ELb{sw}E", 256)
     for p in (1, 2) for rt2 in (1, 2) for dr in (2, 3, 4) for t in (0, 1) for sw in (0, 1)
@@ -161,7 +176,7 @@ REGISTER_BUDGETS = (
 
 
 def check_budgets(text, budgets=REGISTER_BUDGETS):
-    """[(kernel, registers used, budget)] for every budgeted kernel over its budget, or that spills, or that
+    """[(kernel, registers used, budget)] for every budgeted kernel over its budget, or that spills more than it may, or that
     the assembly does not contain (a renamed kernel must not drop out of the check silently)."""
     used, spills, name = {}, {}, None
     for line in text.splitlines():
@@ -175,13 +190,14 @@ def check_budgets(text, budgets=REGISTER_BUDGETS):
         if m and name:
             spills[name] = int(m.group(1))
     bad = []
-    for key, budget in budgets:
+    for key, budget, *allowed in budgets:
         names = [n for n in used if key in n]
         if not names:
             bad.append((key, None, budget))
         for n in names:
-            if used[n] > budget or spills.get(n, 0):
-                bad.append((n, used[n] + (10000 if spills.get(n, 0) else 0), budget))
+            spilled = spills.get(n, 0) > (allowed[0] if allowed else 0)
+            if used[n] > budget or spilled:
+                bad.append((n, used[n] + (10000 if spilled else 0), budget))
     return bad
 
 
