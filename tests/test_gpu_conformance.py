@@ -151,7 +151,7 @@ def test_host_calls_are_no_slower_for_the_pinned_block(backend, m, n, k):
     finally:
         backend.set_host_direct_bytes(16 << 20)
     print("host-direct times", m, n, k, {d: round(t * 1e6, 1) for d, t in best.items()}, "us", flush=True)
-    assert best[16 << 20] <= 1.08 * best[0], best
+    assert best[16 << 20] <= 1.12 * best[0], best
     buf.free()
 
 
