@@ -1820,6 +1820,8 @@ __device__ __forceinline__ bool digits_narrow(int n_poor, const int (&bands)[8],
 // top elements), the token is flagged like one holding NaN or Inf and its outputs are computed in
 // the reference's order. For every other token and every output, unconditionally,
 //   |value - exact dot product| <= n * 2^(E-31)  (+ 1.5 ulp),  n = poor elements under its non-zero trits.
+// (STRICT: TkPrep.strict; a form of its own because the count of large elements costs the others 1%)
+template <bool STRICT>
 __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, const TkPrep *__restrict__ table,
                                                                int nprep, int uniform_m) {
   __shared__ float shf[4];
@@ -1845,10 +1847,9 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
   if (gamma != 0.0f && !nonfinite) (void)frexpf(gamma, &E);
   const int shift = 30 - E;
   const bool live = gamma != 0.0f && !nonfinite;
-  const bool strict = pp.strict != 0;
-  const float carried = strict ? TK_DIGIT_STRICT : 32768.0f;  // (digit_poor)
-  int sums[6] = {0, 0, 0, 0, 0, 0};  // four digit-row sums, poor elements, elements from `carried` on
-  int &n_poor = sums[4], &n_large = sums[5];
+  constexpr int NSUMS = STRICT ? 6 : 5;
+  int sums[NSUMS] = {};  // four digit-row sums, poor elements; STRICT: elements from TK_DIGIT_STRICT on
+  int &n_poor = sums[4];
   // split the 16 values of piece pc into their four digit rows and store those in operand order
   auto emit = [&](size_t pc, const float (&v)[16]) {
     const size_t kb = pc >> 4;
@@ -1865,9 +1866,13 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
         if (live && e + b < k) {
           const float r = ldexpf(v[sl * 4 + b], shift);
           q = __float2int_rn(r);  // |q| <= 2^30
-          const bool large = fabsf(r) >= carried;
-          n_large += large ? 1 : 0;
-          n_poor += !(large || r == (float)q) ? 1 : 0;
+          if constexpr (STRICT) {
+            const bool large = fabsf(r) >= TK_DIGIT_STRICT;
+            sums[5] += large ? 1 : 0;
+            n_poor += !(large || r == (float)q) ? 1 : 0;
+          } else {
+            n_poor += digit_poor(r, q) ? 1 : 0;
+          }
         }
 #pragma unroll
         for (int dg = 0; dg < 4; ++dg) {
@@ -1916,12 +1921,13 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
       emit(pc, v);
     }
   }
-  block_sums<6>(sums, shi);
+  block_sums<NSUMS>(sums, shi);
   // Only a token that has poor elements needs the magnitude bands (the same answer in every thread, so
   // the barriers inside are reached by all or by none). Strict: nor does one with enough large elements, each of
-  // 2^-20 in energy (units of 2^(2E)): left >= (n_large - TK_DIGITS_TRIM) * 2^-20 answers digits_narrow.
-  bool narrow = false;
-  if (n_poor > 0 && !(strict && n_poor <= 3 * (n_large - TK_DIGITS_TRIM))) {
+  // 2^-20 in energy (units of 2^(2E)): left >= (their number - TK_DIGITS_TRIM) * 2^-20 answers digits_narrow.
+  bool narrow = false, bands_needed = n_poor > 0;
+  if constexpr (STRICT) bands_needed = bands_needed && n_poor > 3 * (sums[5] - TK_DIGITS_TRIM);
+  if (bands_needed) {
     int bands[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (resident) {
 #pragma unroll
@@ -1937,7 +1943,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
       }
     }
     block_sums<8>(bands, shi);
-    narrow = digits_narrow(n_poor, bands, strict);
+    narrow = digits_narrow(n_poor, bands, STRICT);
   }
   if (threadIdx.x < 4) {
     const int t = threadIdx.x;
@@ -2828,7 +2834,10 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
       else
         hipLaunchKernelGGL(tk_prep_a8_kernel<TK_PREP_HELD>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
       break;
-    case TK_PREP_DIGITS: hipLaunchKernelGGL(tk_prep_digits_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m); break;
+    case TK_PREP_DIGITS:
+      if (single && single->strict) hipLaunchKernelGGL(tk_prep_digits_kernel<true>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
+      else hipLaunchKernelGGL(tk_prep_digits_kernel<false>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
+      break;
     case TK_PREP_I8: hipLaunchKernelGGL(tk_prep_i8_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m); break;
     default: return hipErrorInvalidValue;
   }
