@@ -210,7 +210,7 @@ int tk_flow3_runs_per_wave(int planes);
 int tk_flow3_waves(int rt);  // waves per workgroup
 hipError_t tk_launch_flow3(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob,
                            const TkLaunchCfg &cfg);
-// small batches (tk_waves.hip): up to 64 operand rows (row stride as the problem says), 1..3 planes; one workgroup per two
+// small batches (tk_waves.hip): 1 or 2 planes and up to 64 operand rows, 3 and up to 32 (row stride as the problem says); one workgroup per two
 // tiles, `grid` of them; a table's workgroups count from the problem's group_begin
 hipError_t tk_launch_waves(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob, int planes,
                            int rows, unsigned grid);

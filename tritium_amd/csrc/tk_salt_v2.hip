@@ -206,8 +206,8 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
 // waves drift apart and one's loads hide behind another's folds), where one thread per output adds them in the pinned order. Plane counts differ by tile: a row without a plane folds its last one again and drops the term.
 // Floor: the f32 matrix pipe, 32 cycles per 16 x 16 x 4 (7 us at the size below); the recoding and the latency of the loads add to it.
 // 4096 x 4096, two planes, kernels, 8 tokens of B3: 64 us (fold with a lane per row, terms through memory) + 12 us (their sum) ->
-// 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 47 / 50 / 50 us, one token 57 / 69 / 66 -> 45 / 48 / 49, 64 tokens 302 / 389 / 353 ->
-// 111 / 122 / 126. (With the activations as 32 four-byte loads per lane and the codes as single bytes the kernel took 52 us: the
+// 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 35 / 37 / 38 us, one token 57 / 69 / 66 -> 33 / 36 / 37, 64 tokens 302 / 389 / 353 ->
+// 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory). (With the activations as 32 four-byte loads per lane and the codes as single bytes the kernel took 52 us: the
 // loads of 16 rows a few KiB apart were the bound.)
 constexpr int SV2_WAVES = 16, SV2_SLOTS = 48;
 template <int G>
