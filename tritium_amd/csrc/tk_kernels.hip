@@ -1494,7 +1494,7 @@ __device__ int block_sum(int v, int *sh) {
 
 // Four consecutive activations starting at element e (a multiple of 4) as floats; elements at or
 // past k read as 0. `vec`: one 8- or 16-byte load where all four exist. It is aligned like an element only (rows of any k, any
-// base): global loads take that on this chip (700 bf16 tokens of K=6001, int8 contract, element by element 27.5 us, so 24.5).
+// base): global loads take that on this chip (700 bf16 tokens of K=6001, int8 contract, element by element 27.8 us, so 24.8).
 __device__ __forceinline__ void load_act4(const void *act, int dtype, size_t base, size_t e, size_t k, bool vec, float (&v)[4]) {
   if (vec && e + 4 <= k) {
     if (dtype == TK_BF16) {
@@ -2788,10 +2788,10 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
   const bool plain = pieces && (kind == TK_PREP_A8 || kind == TK_PREP_DIGITS);
   const bool team_wg = plain && fast && pieces <= 8 * (size_t)TK_WG && (rows <= (unsigned)(kind == TK_PREP_DIGITS ? g_prep_team_rows * 8 / 3 : g_prep_team_rows) || pieces > 512);
   // Rows of other shapes have no straight-line form: few of them take the kernels below, which give a token the whole
-  // workgroup. Call, N=512, wave per token / workgroup per token: float contract f32 K=2050 40 / 333 / 384 tokens 25.9 / 26.7 / 26.6
-  // -> 19.0 / 20.7 / 20.8 us, 700 28.2 -> 27.0, K=1027 333 tokens 19.6 -> 17.4, 1000 tokens 21.1 -> 24.5; int8 contract bf16 K=2050
-  // 333 tokens 21.9 -> 16.4 (loads included). One piece per lane (K <= 1024) stays: K=640 N=4096 106 f32 tokens, float contract
-  // 14.6 -> 15.6.
+  // workgroup. Call, N=512, wave per token element by element / with the vector loads of load_act4 / workgroup per token with them: float
+  // contract f32 K=2050 40 / 333 / 384 / 700 tokens 25.7, 26.6, 26.6, 28.5 / 23.5, 24.5, 24.6, 26.3 / 19.0, 20.7, 20.8, 27.0 us, K=1027 333 / 1000
+  // tokens 19.4, 21.2 / 18.4, 20.2 / 17.2, 24.5; int8 contract K=2050 333 tokens bf16 21.8 / 19.1 / 16.3, f32 20.6 / 18.7 / 16.2. One piece
+  // per lane (K <= 1024) stays: K=640 N=4096 106 f32 tokens, float contract 14.8 / 14.8 / 15.6.
   const bool team_wave = plain && !team_wg && rows >= 32 && pieces <= (fast ? 512u : 256u) &&
                          (fast || pieces <= 64 || rows > (unsigned)g_prep_team_rows);
   if (team_wg || team_wave) {
