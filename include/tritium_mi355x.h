@@ -558,11 +558,11 @@ int tk_get_fused_calls(tk_ctx *ctx, unsigned long long *count);
  * of groups "flow" in both of its forms, and "flow_gemm64" where the members are split over two kernels; "" before the
  * first call. A static string. For tests of the dispatch; no counterpart in the reference. */
 const char *tk_last_kernel(tk_ctx *ctx);
-/* Row count of the workgroup tile for single launches of one plane under the int8 contract (f32 or bf16
- * rows of whole 16-byte pieces at a 16-byte aligned address, no residual): 0 = chosen per launch, 64 = the
- * 64-row kernels, 128 = the 128 x 256 kernel, which shares both operands through LDS, 256 = the 256-row kernel,
- * which expands the weight tile to int8 once per workgroup, in LDS. Other launches take the 64-row kernels
- * whatever this says. A tuning and test knob: identical bits. */
+/* Row count of the workgroup tile of single prefill launches: 0 = chosen per launch, 64 = the 64-row kernels, 128 = the
+ * 128-row kernel (96 rows for three planes; one to three planes, both contracts), 256 = the 256-row kernel, which expands the
+ * weight tile to int8 once per workgroup, in LDS (one plane under the int8 contract, f32 or bf16 rows of whole 16-byte pieces at a
+ * 16-byte aligned address, no residual). Launches that the named kernel does not take go to the 64-row kernels. A tuning
+ * and test knob: identical bits. */
 int tk_set_gemm_rows(tk_ctx *ctx, int rows);
 /* Form of the 256-row kernel: 0 = four waves of 64 rows over a column block of 224 outputs, one workgroup per CU; 1 =
  * eight waves of 32 rows; 2 = four waves over a part of the column block (128 or 96 outputs), two workgroups per CU;

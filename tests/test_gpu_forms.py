@@ -131,6 +131,62 @@ def test_prefill_kernel_128_rows(backend, oracle, m, n, k):
     layer.free()
 
 
+@pytest.mark.parametrize("planes", [1, 2, 3])
+@pytest.mark.parametrize("m,n,k", [(65, 8, 100), (96, 128, 200), (97, 129, 256), (128, 250, 300), (129, 272, 640), (193, 260, 1000),
+                                   (300, 515, 1153), (1030, 136, 768)])
+def test_prefill_kernel_128_rows_planes_and_contracts(backend, oracle, m, n, k, planes):
+    """tk_gemm128_kernel with one to three planes under both contracts, with a residual and raw int32 results: one to ten half
+    blocks of K (a last block of at most and of more than 128 elements), row blocks of 96 and 128 filled and not, output
+    rows of whole 16-byte pieces and others, NaN and Inf tokens. The int8 contract against the CPU oracle, the float contract
+    against the 64-row kernels (identical bits) and float64 (1e-5 of the largest output: f32 sums of the planes)."""
+    print("case gemm-128 planes", m, n, k, planes, flush=True)
+    rng = np.random.default_rng(128128 + m + n + k + planes)
+    ws, scs, packed = _planes(rng, n, k, planes)
+    layer = backend.linear(packed, scs, n, k)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    exact = sum((act.astype(np.float64) @ w.astype(np.float64).T) * sc[None, :].astype(np.float64) for w, sc in zip(ws, scs))
+    act[m // 2] = 0.0
+    exact[m // 2] = 0.0
+    act[1, k // 3] = np.nan
+    act[m - 1, 0] = np.inf
+    plain = np.ones(m, bool)
+    plain[[1, m - 1]] = False
+    dact, dres = backend.to_device(act, "f32"), backend.to_device(res, "f32")
+    want = oracle.cpu_linear_a8_planes(packed, FMT_TQ2_0, scs, act, m, n, k)
+    nan = np.isnan(want)
+    got = {}
+    for rows in (128, 64):
+        backend.set_gemm_rows(rows)
+        out, outb = backend.empty(m * n, "f32"), backend.empty(m * n, "bf16")
+        backend.linear_a8(layer, dact, m, out)
+        assert backend.last_kernel().split("_")[0] == f"gemm{rows}", backend.last_kernel()
+        g = out.to_host().reshape(m, n)
+        assert (np.isnan(g) == nan).all() and same_bits(g[~nan], want[~nan])
+        backend.linear_a8(layer, dact, m, outb)
+        assert (outb.to_host().reshape(m, n)[~nan] == f32_to_bf16_bits(want)[~nan]).all()
+        backend.linear_a8_residual(layer, dact, m, dres, out)
+        assert same_bits(out.to_host().reshape(m, n)[~nan], (res + want)[~nan])
+        backend.linear_float(layer, dact, m, out)
+        assert backend.last_kernel().split("_")[0] == f"gemm{rows}", backend.last_kernel()
+        got[rows] = out.to_host().reshape(m, n)
+        assert np.abs(got[rows][plain] - exact[plain]).max() <= 1e-5 * np.abs(exact).max()
+        out.free()
+        outb.free()
+    assert (got[64].view(np.uint32) == got[128].view(np.uint32)).all()
+    if planes == 1:
+        backend.set_gemm_rows(128)
+        q = rng.integers(-128, 128, (m, k)).astype(np.int8)
+        dq, dacc = backend.to_device(q, "i8"), backend.empty(m * n, "i32")
+        backend.linear_i8(layer, dq, None, m, dacc)
+        assert (dacc.to_host().reshape(m, n) == oracle.int8_accumulators(packed[0], FMT_TQ2_0, q, m, n, k)).all()
+        for a in (dq, dacc):
+            a.free()
+    for a in (dact, dres):
+        a.free()
+    layer.free()
+
+
 @pytest.mark.parametrize("form", [0, 1, 2])
 @pytest.mark.parametrize("m,n,k", [(65, 8, 256), (257, 232, 512), (300, 456, 300), (256, 1040, 2560), (520, 2104, 768),
                                    (1030, 4104, 256), (640, 520, 1280), (700, 240, 4096)])

@@ -30,7 +30,7 @@ def hipcc():
 # hand-issued loads (the prefill kernels), register budgets, and kernels that need an empty static LDS segment.
 ASM_SOURCES = ["tk_kernels.hip", "tk_flow_a8.hip", "tk_zskip.hip", "tk_gemm128.hip", "tk_gemm256.hip", "tk_base3.hip", "tk_waves.hip",
                "tk_salt_gemm.hip", "tk_salt_v2.hip", "tk_vjp.hip"]
-HAZARD_SOURCES = ["tk_kernels.hip", "tk_gemm256.hip"]
+HAZARD_SOURCES = ["tk_kernels.hip", "tk_gemm128.hip", "tk_gemm256.hip"]
 
 
 def build_library(verbose=True):

@@ -1082,12 +1082,13 @@ static void plan_gemm(Plan *pl, unsigned fill = 0, int force_nt = 0) {
   }
 }
 
-// The 128 x 256 kernel's grid: row blocks of 128 operand rows, column blocks of 16 tiles, split over the
-// XCDs like plan_gemm's (the operand-row stride plan_gemm chose stays).
+// The 128-row kernel's grid: row blocks of 128 operand rows (96 for three planes), column blocks of 256 (one plane) or 128
+// outputs, split over the XCDs like plan_gemm's (the operand-row stride plan_gemm chose stays).
 static void plan_gemm128(Plan *pl) {
   TkProblem &pr = pl->pr;
-  pl->grid_m = (unsigned)(((size_t)pr.R + 127) / 128);
-  pl->grid_n = ((unsigned)pr.n_tiles + 15u) / 16u;
+  const int rows = tk_gemm128_rows(pr.planes), tiles = tk_gemm128_tiles(pr.planes);
+  pl->grid_m = (unsigned)((pr.R + rows - 1) / rows);
+  pl->grid_n = (unsigned)((pr.n_tiles + tiles - 1) / tiles);
   pr.grid_m = (int)pl->grid_m;
   pr.grid_n = (int)pl->grid_n;
   pr.ksplit = 0;
@@ -1095,7 +1096,7 @@ static void plan_gemm128(Plan *pl) {
   for (int xr = 1; xr <= 8; xr *= 2) {
     const int xc = 8 / xr;
     const int sm = ((int)pl->grid_m + xr - 1) / xr, sn = ((int)pl->grid_n + xc - 1) / xc;
-    const size_t cost = (size_t)128 * sm + (size_t)64 * sn;  // bytes touched per XCD and unit of K
+    const size_t cost = (size_t)rows * sm + (size_t)4 * tiles * pr.planes * sn;  // bytes touched per XCD and unit of K
     const size_t waste = (size_t)8 * sm * sn;
     const size_t score = cost * 1024 + waste;
     if (score < best) {
@@ -1133,16 +1134,34 @@ static void plan_gemm256(Plan *pl) {
   }
 }
 
-// Where the 128 x 256 kernel is chosen over the 64-row forms: launches it finishes in one round of its 512
-// resident workgroups (two per CU) and that still give most CUs one. A/B on one box, int8 rows in, bf16 out,
-// call incl. the operand re-ordering launch, 64-row kernels -> 128 x 256: 2048 x 2560 -> 6912 (432 blocks)
-// 47.9 -> 44.7 us; 1024 tokens (216) 30.0 -> 28.2; 512 tokens (108) 17.6 -> 24.8; 256 tokens 13.8 -> 23.6;
-// 2048 x 6912 -> 2560 (160) 52.0 -> 56.8; 2048 x 2560 -> 2560 (160) 27.7 -> 30.0; and with several rounds:
-// 8192 x 2560 -> 6912 (1728) 135 -> 140; 4096 x 5120 -> 17408 (2176) 288 -> 302; 4096 x 17408 -> 5120 (640)
-// 294 -> 330.
-static bool gemm128_pays(const tk_ctx *ctx, size_t rows, size_t blocks128) {
-  const size_t cus = (size_t)ctx->info.compute_units;
-  return rows >= 1024 && blocks128 * 4 >= cus * 3 && blocks128 <= 2 * cus;
+// Time per K block (us at the clock these launches hold) of a prefill launch with x workgroups per CU. A CU runs two (64 rows
+// of one and two planes: three) at a time, so what counts is the CU with the most of them: `full[c - 1]` with c workgroups on
+// every CU, repeating with the slots; a launch that gives only some CUs the last one is a little faster (an eighth at most).
+static double prefill_cost(double x, const double *full, int slots) {
+  const int c = x > 0.0 ? (int)x + (x > (double)(int)x ? 1 : 0) : 1;
+  const double whole = (double)((c - 1) / slots) * full[slots - 1] + full[(c - 1) % slots];
+  const double part = whole * (c > 1 ? 1.0 - 0.12 * ((double)c - x) : 1.0), even = x * full[slots - 1] / slots;
+  return part > even ? part : even;
+}
+// Where the 128-row kernel is chosen over the 64-row one. It moves and expands less per operation, but its tiles are larger: a
+// workgroup takes 256 (three planes: 96 x 384) plane columns x 128 rows where the other takes half of that, a call pays 2.5 us more for its first
+// loads and last stores, and 1.1 workgroups per CU cost as much as two. The figures are the slopes and offsets of calls of 768
+// int8 tokens over K = 2048 and 6144, N = 1024 .. 40960 (64 rows / 128 rows, us at K=6144; 64-row workgroups per CU): one plane
+// 1.9 58 / 53, 2.3 65 / 75, 3.8 98 / 83, 4.5 103 / 115, 6 129 / 125, 7.5 161 / 154; two planes 1.1 46 / 49, 2.3 64 / 74, 3.8 87 / 81, 6 125 / 120;
+// three planes 0.8 43 / 53, 1.1 58 / 52, 1.9 64 / 79, 2.3 90 / 81, 3 93 / 88, 3.8 115 / 120, 4.5 141 / 125, 6 174 / 164, 7.5 226 / 204.
+// One plane of float digit rows loses in every launch measured (512 tokens K=2560 N=6912 44.6 / 46.5, 1024 K=6912 N=2560 76 / 91).
+static bool gemm128_pays(const tk_ctx *ctx, int planes, int mode, size_t rows, size_t n_tiles, size_t k) {
+  if (planes > 3 || (planes == 1 && mode == TK_MODE_DIGITS) || ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit) return false;
+  static const double rows64[3][3] = {{0.0, 0.0, 0.0}, {1.18, 1.72, 2.43}, {1.42, 2.27, 0.0}};
+  static const double rows128[3][2] = {{1.64, 2.9}, {1.6, 2.85}, {1.8, 3.175}};
+  const double cus = (double)ctx->info.compute_units;
+  const size_t tiles = (size_t)tk_gemm128_tiles(planes), tall = (size_t)tk_gemm128_rows(planes);
+  const size_t cols = (n_tiles + tiles - 1) / tiles;
+  const double x64 = (double)(((rows + 63) / 64) * cols) / cus, x128 = (double)(((rows + tall - 1) / tall) * cols) / cus;
+  const double blocks = (double)((k + 127) / 128) * 0.5;  // (the 64-row kernel takes whole K blocks)
+  // one plane, 64 rows: two and four tiles per wave together are nearly linear in the work
+  const double c64 = planes == 1 ? (x64 < 4.0 ? 0.55 + 0.78 * x64 : 0.807 * x64) : prefill_cost(x64, rows64[planes - 1], planes == 2 ? 3 : 2);
+  return (double)num_blocks(k) * c64 > blocks * prefill_cost(x128, rows128[planes - 1], 2) + 2.5;
 }
 
 // Where the 256-row kernel (weight tile expanded once per workgroup) is chosen: launches of 1024 rows or more that give
@@ -1505,9 +1524,7 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
     ctx->last_kernel = "ksplit_decode";
     HIPCHK(tk_launch_skinny(ctx->stream, &pr, nullptr, 0, pl.cfg));
   } else {
-    // One plane under the int8 contract with whole 16-byte output pieces: the 128 x 256 kernel moves a third
-    // of the bytes per op through the CU's memory path (both operands shared through LDS).
-    const bool can128 = can_wide;
+    const bool can128 = pr.planes <= 3 && nb >= 1 && (size_t)pr.n_tiles * nb * TK_CHUNK_BYTES < (size_t)1 << 32 && (size_t)pr.rs * 256 < (size_t)1 << 32;
     if (use256) {
       ctx->last_kernel = "gemm256";
       const hipError_t le = tk_launch_gemm256(ctx->stream, &pr, form256);
@@ -1516,8 +1533,7 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
       }
       return TK_OK;
     }
-    const size_t blocks128 = ((R + 127) / 128) * (((size_t)pr.n_tiles + 15) / 16);
-    const bool want128 = ctx->gemm_rows == 128 || (ctx->gemm_rows == 0 && gemm128_pays(ctx, R, blocks128));
+    const bool want128 = ctx->gemm_rows == 128 || (ctx->gemm_rows == 0 && gemm128_pays(ctx, pr.planes, mode, R, (size_t)pr.n_tiles, k));
     if (can128 && want128) {
       plan_gemm128(&pl);
       ctx->last_kernel = "gemm128";

@@ -1,249 +1,337 @@
-// gfx950 prefill GEMM, 128 x 256 outputs per workgroup, one plane, int8 contract.
+// gfx950 prefill GEMM, 128 operand rows (96 for three planes) per workgroup, one to three planes, both contracts.
 //
-// The 64-row prefill kernels (tk_kernels.hip) are held back by the CU's vector-memory path, not by the
-// matrix pipe: every wave loads its own weight chunks into registers and the four waves of a workgroup
-// share one 64-row A block, 24-32 KiB of loads per 4-8 MOP. Here eight waves (two row groups of 64 rows x
-// four column groups of 64 outputs) share both operands through LDS: per half K block (128 k) a workgroup
-// brings in 16 KiB of A rows and 8 KiB of 2-bit weight chunks, all by LDS-DMA (three wave-wide 16-byte
-// loads per wave), for 16.8 MOP -- 1.4 KiB per MOP where the 64 x 256 form moves 3.8. A wave computes
-// 64 x 64 outputs with v_mfma_i32_32x32x32_i8 (two 32-row A tiles x two pairs of weight tiles: 64
-// accumulator registers), reads its A pieces and its 16-byte weight pieces from LDS and expands the 2-bit
-// codes exactly as the other kernels do, so the accumulators are the same integers and the outputs carry
-// the same bits. (A wave over all 128 rows of 32 outputs -- half the expansion work, 1.7 times the LDS reads --
-// measured 4-8% slower.)
+// The 64-row prefill kernel (tk_kernels.hip) is held back by the CU's vector-memory path and by the expansion of the 2-bit
+// codes: every wave expands the codes of its own columns, seven vector instructions for an operand that two matrix
+// instructions use, and a K block of 64 rows x 384 plane columns brings in 40 KiB. Here a workgroup is four waves side by
+// side over 128 rows x 128 plane columns and more: an expanded operand serves four matrix instructions (three for three
+// planes: 96 rows, whose 144 accumulators leave room for two waves per SIMD), and a byte that comes in serves a quarter to a
+// third more of them. The operand rows come to LDS by DMA in HALF K blocks (128 k: 16 KiB, three slots, two half blocks
+// ahead), so that two workgroups still share a CU; the weight codes go straight to registers, one 16-byte piece per lane,
+// pair of tiles and half block; one barrier per half block (32 or 36 matrix instructions per wave).
+// Lane maps are those of the 64-row kernel (v_mfma_i32_32x32x32_i8): lane L = 32 kappa + 16 h + r takes piece g = 2 l + kappa
+// of row r of tile h of a pair, l = the half of the K block; dword j of the piece is the operand of k step j. The codes are
+// trit + 1, so the accumulators start at minus the row sums. Same integers, same epilogue arithmetic: identical bits.
+// A K whose last block holds at most 128 elements has one half block less (its operand rows are zero there).
 //
-// LDS: three stages of 24 KiB (A: 8 segments (j, kappa) x 128 rows x 16 B; W: 16 tiles x 512 B = the half
-// of each 1-KiB chunk that belongs to this half block), two half blocks in flight, one barrier per half
-// block; 1.5 KiB of row constants behind the stages. Two workgroups per CU (four waves per SIMD, at most
-// 128 registers). The epilogue stages finished rows through the (then free) stage memory and writes whole
-// 16-byte pieces of contiguous row segments, like the 64-row kernels.
-//
-// Takes: one plane, int8 operand rows (W1.58A8 or int8 input), f32 or bf16 output whose rows are 16-byte
-// multiples at a 16-byte aligned address, no residual. Everything else stays with the 64-row kernels.
+// Bound: in long launches the chip's power -- registers full of gaussian int8 rows and codes, nothing but matrix instructions,
+// hold 4.0 POPS of the 5.0 that all-zero operands reach (and 3.5 with the weights as the first operand: so activations go first),
+// and interleaving the expansion with the matrix instructions one by one changed nothing. Otherwise the number of workgroups
+// on the CU that has most (gemm128_pays in tk_api.hip). Calls incl. quantization, 64 rows -> 128: 4096 tokens K=5120 N=17408 three
+// planes 759 -> 738 us, 1024 tokens K=5120 N=5120 79 -> 72, 200 tokens N=17408 73 -> 65; 768 tokens K=6144 N=20480 one plane 98 -> 83,
+// two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 -> 41.1. One workgroup alone on a CU runs its
+// loop at 0.58 of the matrix rate, two at 0.70.
+
+#include <type_traits>
 
 #include "tk_device.h"
 
 typedef int v16i_g __attribute__((ext_vector_type(16)));
 
-#define TK_G128_THREADS 512
-#define TK_G128_HALF_A 16384
-#define TK_G128_HALF_W 8192
-#define TK_G128_STAGE (TK_G128_HALF_A + TK_G128_HALF_W)
-#define TK_G128_STAGES 3
-#define TK_G128_CST (TK_G128_STAGES * TK_G128_STAGE)
-#define TK_G128_BAND 4
+namespace {
 
-__global__ __launch_bounds__(TK_G128_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void tk_gemm128_kernel(const TkProblem single) {
+constexpr int WAVES = 4, SLOTS = 3, BAND = 4;
+
+// P planes, NT tiles of 16 outputs per wave and plane, RT 32-row tiles of operand rows per workgroup
+template <int P>
+struct Form {
+  static constexpr int NT = P == 1 ? 4 : 2, RT = P == 3 ? 3 : 4, ROWS = 32 * RT;
+  static constexpr int SLOT = ROWS * 128;             // bytes of a half block of operand rows
+  static constexpr int CST = SLOTS * SLOT;            // float act_scale[128] | int exps[64] | uint flags[128]
+  static constexpr int LDS = CST + 512 + 256 + 512;
+};
+
+template <int P>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void tk_gemm128_kernel(const TkProblem single) {
+  using F = Form<P>;
+  constexpr int NT = F::NT, RT = F::RT, ROWS = F::ROWS, HP = NT / 2, NP = HP * P;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const TkProblem &pr = *single_problem();
   const TkHot hot = make_hot(pr);
-  const int tid = (int)threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int r16 = lane & 15, h = (lane >> 4) & 1, kappa = lane >> 5;
-  const int rg = wave >> 2, cg = wave & 3;  // row group (64 rows), column group (64 outputs)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, h = (lane >> 4) & 1, r32 = lane & 31, kappa = lane >> 5;
   const int nb = pr.nb, R = pr.R, n_tiles = pr.n_tiles, rs = pr.rs;
-  const uint8_t *codes = pr.codes[0];
-  const int8_t *ap = pr.ap;
+  const int H = 2 * nb - (((pr.k - 1) & 255) < 128 ? 1 : 0);  // half blocks that hold elements
 
-  // XCD x = id % 8 owns a compact sub-grid of sub_m x sub_n tiles and walks it in bands of TK_G128_BAND
-  // row tiles, down the band first (as the 64-row kernels do)
-  const unsigned wg = blockIdx.x;
-  const int xcd = (int)(wg & 7u), slot = (int)(wg >> 3);
+  // XCD x = id % 8 owns a compact sub-grid of sub_m x sub_n workgroups and walks it in bands of BAND row blocks, down the
+  // band first (as the 64-row kernel does)
+  const int xcd = (int)(blockIdx.x & 7u), at = (int)(blockIdx.x >> 3);
   const int sub_m = pr.sub_m, sub_n = pr.sub_n;
-  const int band_sz = TK_G128_BAND * sub_n;
-  const int band = slot / band_sz, in_band = slot - band * band_sz;
-  const int band_rows = min(TK_G128_BAND, sub_m - band * TK_G128_BAND);
+  const int band = at / (BAND * sub_n), in_band = at - band * (BAND * sub_n);
+  const int band_rows = min(BAND, sub_m - band * BAND);
   if (band_rows <= 0) return;
-  const int lm = band * TK_G128_BAND + in_band % band_rows, ln = in_band / band_rows;
+  const int lm = band * BAND + in_band % band_rows, ln = in_band / band_rows;
   const int bm = (xcd % pr.xr) * sub_m + lm, bn = (xcd / pr.xr) * sub_n + ln;
-  if (lm >= sub_m || ln >= sub_n || bm >= pr.grid_m || bn >= pr.grid_n) return;
-  const int row0 = bm * 128, tile0 = bn * 16;
+  if (ln >= sub_n || bm >= pr.grid_m || bn >= pr.grid_n) return;
+  const int row0 = bm * ROWS, tile0 = (bn * WAVES + wave) * NT;
 
-  // this wave's three DMA instructions of a half block: ids 3*wave .. 3*wave+2 of [A0..A15, W0..W7].
-  // A id i: segment i >> 1 (j = seg >> 1, kappa = seg & 1), rows (i & 1) * 64 + lane.
-  // W id w: tiles 2w and 2w+1, lane -> tile 2w + (lane >> 5), 16-byte piece lane & 31 of its half chunk.
-  const uint8_t *gsrc[3];   // lane address for half block 0 (K block 0, l = 0)
-  unsigned kb_step[3];      // bytes from one K block to the next
-  unsigned l_step[3];       // bytes from half 0 to half 1 of a K block
-  unsigned lds_dst[3];      // wave-uniform offset inside a stage
+  // ---- operand addresses ----
+  // weights: lane offset of pair z, the same in every plane (tiles past the end re-read the last one; results dropped)
+  unsigned w_off[HP];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const int id = wave * 3 + i;
-    if (id < 16) {
-      const int seg = id >> 1, j = seg >> 1, kap = seg & 1;
-      const int row = min(row0 + (id & 1) * 64 + lane, R - 1);
-      gsrc[i] = (const uint8_t *)ap + ((size_t)(j * 4 + kap) * (size_t)rs + (size_t)row) * 16;
-      kb_step[i] = (unsigned)rs * 256u;  // 16 segments of rs rows of 16 bytes
-      l_step[i] = (unsigned)rs * 32u;    // g = 2l + kappa: two segments further
-      lds_dst[i] = (unsigned)((seg * 128 + (id & 1) * 64) * 16);
-    } else {
-      const int w = id - 16;
-      const int tile = min(tile0 + 2 * w + (lane >> 5), n_tiles - 1);
-      gsrc[i] = codes + (size_t)tile * (size_t)nb * 1024 + (size_t)(lane & 31) * 16;
-      kb_step[i] = 1024u;
-      l_step[i] = 512u;
-      lds_dst[i] = (unsigned)(TK_G128_HALF_A + w * 1024);
-    }
+  for (int z = 0; z < HP; ++z)
+    w_off[z] = (unsigned)min(tile0 + 2 * z + h, n_tiles - 1) * (unsigned)nb * 1024u + (unsigned)(kappa * 16 + r16) * 16u;
+  // operand rows: a half block is 8 segments (j, kappa) of ROWS pieces, cut into 4 RT wave-wide DMA loads, RT per wave
+  unsigned a_off[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int idx = (wave * RT + i) * 64 + lane, seg = idx / ROWS, row = idx - seg * ROWS;
+    a_off[i] = (unsigned)((seg >> 1) * 4 + (seg & 1)) * (unsigned)rs * 16u + (unsigned)min(row0 + row, R - 1) * 16u;
   }
-  auto issue = [&](int hb, int stage) {
-    const unsigned kb = (unsigned)hb >> 1, l = (unsigned)hb & 1u;
+  auto load_w = [&](v4i (&w)[NP], int hb) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gsrc[i] + (size_t)kb * kb_step[i] + l * l_step[i]),
-                                       (__attribute__((address_space(3))) void *)(smem + (size_t)stage * TK_G128_STAGE + lds_dst[i]),
-                                       16, 0, 0);
+    for (int p = 0; p < P; ++p) {
+      const uint8_t *base = pr.codes[p] + (size_t)(unsigned)hb * 512u;  // wave-uniform
+#pragma unroll
+      for (int z = 0; z < HP; ++z)
+        asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(w[p * HP + z]) : "v"(w_off[z]), "s"(base));
+    }
+  };
+  auto dma = [&](int hb, int slot) {
+    const uint8_t *base = (const uint8_t *)pr.ap + ((size_t)(hb >> 1) * 16 + (hb & 1) * 2) * (size_t)rs * 16;  // wave-uniform
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(base + a_off[i]),
+                                       (__attribute__((address_space(3))) void *)(smem + slot * F::SLOT + (wave * RT + i) * 1024), 16, 0, 0);
   };
 
-  // row constants behind the stages: int rowsum[128] | float act_scale[128]
-  int *cst_rs = (int *)(smem + TK_G128_CST);
-  float *cst_as = (float *)(smem + TK_G128_CST + 512);
-  if (tid < 128) {
-    const int row = min(row0 + tid, R - 1);
-    cst_rs[tid] = gload(hot.rowsum + row);
-    cst_as[tid] = hot.act_scale ? gload(hot.act_scale + row) : 1.0f;
+  // ---- prologue: constants, minus the row sums, the first two half blocks ----
+  const bool int8_in = hot.mode == TK_MODE_INT8;
+  {
+    const void *src = nullptr;
+    int last = 0, first = 0, n64 = 0, dst = 0;
+    if (wave == 0 && int8_in && hot.act_scale) src = hot.act_scale, first = row0, last = R - 1, n64 = 2, dst = 0;
+    if (wave == 1 && !int8_in) src = hot.exps, first = row0 >> 2, last = hot.M - 1, n64 = 1, dst = 512;
+    if (wave == 2 && hot.flags) src = hot.flags, first = int8_in ? row0 : row0 >> 2, last = int8_in ? R - 1 : hot.M - 1, n64 = int8_in ? 2 : 1, dst = 768;
+    for (int i = 0; i < n64; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)((const uint32_t *)src + min(first + i * 64 + lane, last)),
+                                       (__attribute__((address_space(3))) void *)(smem + F::CST + dst + i * 256), 4, 0, 0);
+  }
+  float sc[HP][P];
+#pragma unroll
+  for (int z = 0; z < HP; ++z) {
+    const int n = (tile0 + 2 * z + h) * 16 + r16;
+#pragma unroll
+    for (int p = 0; p < P; ++p) sc[z][p] = hot.out_dtype == TK_I32 ? 0.0f : gload(pr.scales[p] + min(n, hot.n - 1));
+  }
+  // (requested before the row sums are waited for: one trip to memory, not two)
+  v4i wset[SLOTS][NP], a[2][RT];
+  load_w(wset[0], 0);
+  dma(0, 0);
+  if (H > 1) {
+    load_w(wset[1], 1);
+    dma(1, 1);
+  }
+  v16i_g acc[RT][NP];
+  if (row0 + ROWS <= R) {
+    v4i rs4[RT][4];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) rs4[rt][q] = *(const TK_GLOBAL v4i *)(hot.rowsum + row0 + rt * 32 + 8 * q + 4 * kappa);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int y = 0; y < NP; ++y) acc[rt][y][e] = -rs4[rt][e >> 2][e & 3];
+  } else {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int neg = -gload(hot.rowsum + min(row0 + rt * 32 + 8 * (e >> 2) + 4 * kappa + (e & 3), R - 1));
+#pragma unroll
+        for (int y = 0; y < NP; ++y) acc[rt][y][e] = neg;
+      }
   }
 
-  const int HB = 2 * nb;
-  issue(0, 0);
-  issue(1, 1);  // nb >= 1: a K block has two halves
+  // wait until at most `ahead` of the youngest half blocks are still in flight
+  auto wait_blocks = [&](int ahead) {
+    if (ahead <= 0) asm volatile("s_waitcnt vmcnt(0)");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RT + NP));
+  };
+  auto tie_w = [&](v4i (&w)[NP]) {
+#pragma unroll
+    for (int y = 0; y < NP; ++y) asm volatile("" : "+v"(w[y]));
+  };
+  const unsigned lds_lane = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t *)smem + (unsigned)(kappa * ROWS + r32) * 16u;
+  auto lds_read = [&](v4i (&d)[RT], int off) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(d[rt]) : "v"(lds_lane), "n"(off + rt * 512));
+  };
+  // LDS reads return in order: wait until only those of the next k step (or none) are in flight
+  auto lds_wait = [&](v4i (&d)[RT], bool ahead) {
+    if (ahead) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(RT));
+    else asm volatile("s_waitcnt lgkmcnt(0)");
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) asm volatile("" : "+v"(d[rt]));
+  };
+  wait_blocks(0);
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) tie_w(wset[s]);
+  __builtin_amdgcn_s_barrier();
 
-  v16i_g acc[2][2];
-#pragma unroll
-  for (int rt2 = 0; rt2 < 2; ++rt2)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int c = 0; c < 16; ++c) acc[rt2][y][c] = 0;
-
-  asm volatile("s_waitcnt vmcnt(3)" ::: "memory");  // half block 0 has landed (this wave's part)
-  __syncthreads();  // (also publishes the row constants)
-
-  // lane offsets inside a stage: A piece (j, kappa) of row rg*64 + rt2*32 + (lane & 31); weight piece
-  // (kappa, r16) of tile cg*4 + 2y + h
-  const unsigned a_lane = (unsigned)((kappa * 128 + rg * 64 + (lane & 31)) * 16);
-  const unsigned w_lane = (unsigned)(TK_G128_HALF_A + (cg * 4 + h) * 512 + (kappa * 16 + r16) * 16);
-  int stage = 0;
-  for (int hb = 0; hb < HB; ++hb) {
-    const bool more = hb + 2 < HB;
-    if (more) issue(hb + 2, stage == 0 ? 2 : stage - 1);  // the stage half block hb-1 just left
-    const uint8_t *sb = smem + (size_t)stage * TK_G128_STAGE;
-    v4i wp[2];
-#pragma unroll
-    for (int y = 0; y < 2; ++y) wp[y] = *(const v4i *)(sb + w_lane + y * 1024);
-    v4i a_cur[2], a_nxt[2];
-#pragma unroll
-    for (int rt2 = 0; rt2 < 2; ++rt2) a_cur[rt2] = *(const v4i *)(sb + a_lane + rt2 * 512);
+  // ---- half block hb in slot `cur`; block hb + 2 goes where block hb - 1 was ----
+  auto block = [&](auto cur_c, int hb) {
+    constexpr int cur = decltype(cur_c)::value, prev = (cur + 2) % SLOTS, next = (cur + 1) % SLOTS;
+    if (hb + 2 < H) {
+      load_w(wset[prev], hb + 2);
+      dma(hb + 2, prev);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (j < 3) {
+      if (j < 3) lds_read(a[(j + 1) & 1], cur * F::SLOT + (j + 1) * 2 * ROWS * 16);
+      lds_wait(a[j & 1], j < 3);
 #pragma unroll
-        for (int rt2 = 0; rt2 < 2; ++rt2) a_nxt[rt2] = *(const v4i *)(sb + a_lane + (j + 1) * 4096 + rt2 * 512);
-      }
+      for (int y = 0; y < NP; ++y) {
+        const v4i b = expand_codes((uint32_t)wset[cur][y][j]);
 #pragma unroll
-      for (int y = 0; y < 2; ++y) {
-        const v4i b = expand_codes((uint32_t)wp[y][j]);
-#pragma unroll
-        for (int rt2 = 0; rt2 < 2; ++rt2)
-          acc[rt2][y] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_cur[rt2], b, acc[rt2][y], 0, 0, 0);
-      }
-      if (j < 3) {
-#pragma unroll
-        for (int rt2 = 0; rt2 < 2; ++rt2) a_cur[rt2] = a_nxt[rt2];
+        for (int rt = 0; rt < RT; ++rt) acc[rt][y] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[j & 1][rt], b, acc[rt][y], 0, 0, 0);
       }
     }
-    // half block hb+1 must have landed; the one issued above may stay in flight.
-    // (A bare barrier: __syncthreads() would also drain the loads in flight. Every wave has consumed its
-    // LDS reads of this stage in matrix instructions issued above, so the stage may be overwritten. Moving
-    // the barrier in front of the last k step, with the next half block's first reads behind it, measured
-    // no faster here and 2-4% slower in the 64-row kernels.)
-    if (more) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_blocks(min(hb + 2, H - 1) - (hb + 1));  // block hb + 1 has landed
+    tie_w(wset[next]);
     __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");  // no LDS read of the next half block moves above the barrier
-    stage = stage == 2 ? 0 : stage + 1;
+    lds_read(a[0], next * F::SLOT);  // (behind the last block: stale rows, waited for below)
+  };
+  lds_read(a[0], 0);
+  int hb = 0;
+  for (; hb + SLOTS <= H; hb += SLOTS) {  // one exit only: the accumulators keep their registers
+    block(std::integral_constant<int, 0>{}, hb);
+    block(std::integral_constant<int, 1>{}, hb + 1);
+    block(std::integral_constant<int, 2>{}, hb + 2);
   }
+  if (hb < H) {
+    block(std::integral_constant<int, 0>{}, hb);
+    if (hb + 1 < H) block(std::integral_constant<int, 1>{}, hb + 1);
+  }
+  lds_wait(a[0], false);
 
-  // ---- epilogue: out[m,n] = ((float)(acc - rowsum[m]) * scale[n]) * act_scale[m] ----
+  // ---- epilogue ----
+  const float *cst_as = (const float *)(smem + F::CST);
+  const int *cst_exp = (const int *)(smem + F::CST + 512);
+  const uint32_t *cst_flag = (const uint32_t *)(smem + F::CST + 768);
+  const int tid = (int)threadIdx.x;
   unsigned my_flag = 0;
-  if (hot.flags && tid < 128 && row0 + tid < R) my_flag = gload(hot.flags + row0 + tid) ? 1u : 0u;
-  const int wg_flag = __syncthreads_or((int)my_flag);
-  const bool has_as = hot.act_scale != nullptr;
-  float sc[2][1];
-  int ncol[2];
+  if (hot.flags && tid < ROWS && (int8_in ? row0 + tid < R : (tid < ROWS / 4 && (row0 >> 2) + tid < hot.M))) my_flag = cst_flag[tid] ? 1u : 0u;
+  const int wg_flag = __syncthreads_or((int)my_flag);  // (also: every wave is done with the slots)
+  const bool has_as = int8_in && hot.act_scale;
+  auto consts = [&](int rl) {  // of the 4 rows rl .. rl + 3 of the workgroup
+    RowConst rc = {};
+    const float4 as4 = *(const float4 *)(cst_as + rl);
+    rc.as[0] = as4.x; rc.as[1] = as4.y; rc.as[2] = as4.z; rc.as[3] = as4.w;
+    rc.exp = cst_exp[rl >> 2];
+    if (wg_flag) {
+      if (int8_in) {
 #pragma unroll
-  for (int y = 0; y < 2; ++y) {
-    ncol[y] = (tile0 + cg * 4 + 2 * y + h) * 16 + r16;
-    sc[y][0] = ncol[y] < hot.n ? gload(pr.scales[0] + ncol[y]) : 0.0f;
-  }
-  const int col0 = bn * 256;
-  auto finish = [&](auto esz_c) {
-    constexpr int ESZ = decltype(esz_c)::value;
-    constexpr int HALVES = ESZ == 4 ? 2 : 1, SROWS = 128 / HALVES;  // staging rows per pass
-    constexpr int STRIDE = 256 * ESZ + 16, PIECES_ROW = 256 * ESZ / 16, PER16 = 16 / ESZ;
-    static_assert(SROWS * STRIDE <= TK_G128_CST, "the staging area is the stage memory");
-    uint8_t *lane_base = smem + (size_t)(4 * kappa) * STRIDE + (size_t)((cg * 4 + h) * 16 + r16) * ESZ;
+        for (int r = 0; r < 4; ++r) rc.flag |= cst_flag[rl + r] ? 1u << r : 0u;
+      } else {
+        rc.flag = cst_flag[rl >> 2] ? 1u : 0u;
+      }
+    }
+    return rc;
+  };
+  auto quad = [&](int rt, int q, int z, v4i (&av)[P]) {
 #pragma unroll
-    for (int hh = 0; hh < HALVES; ++hh) {
-      if (hh > 0) __syncthreads();
+    for (int p = 0; p < P; ++p) {
+      const v16i_g &c = acc[rt][p * HP + z];
+      av[p] = v4i{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+    }
+  };
+  // int8 contract, output rows of whole 16-byte pieces, no residual: a wave stages 32 rows of its columns in its own piece of
+  // LDS and writes them as whole segments
+  auto staged = [&](auto esz_c) {
+    constexpr int ESZ = decltype(esz_c)::value, COLS = NT * 16, STRIDE = COLS * ESZ + 16, PPR = COLS * ESZ / 16, RPI = 64 / PPR;
+    static_assert(WAVES * 32 * STRIDE <= F::CST, "the staging areas fit the slots");
+    uint8_t *wl = smem + wave * (32 * STRIDE);
+    uint8_t *lane_base = wl + (4 * kappa) * STRIDE + (h * 16 + r16) * ESZ;
+    const int piece = lane % PPR, srow = lane / PPR, c = tile0 * 16 + piece * (16 / ESZ);
 #pragma unroll
-      for (int rt2 = 0; rt2 < 2; ++rt2) {
-        if (HALVES == 2 && rt2 != hh) continue;
+    for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int rl = rg * 64 + rt2 * 32 + 8 * q + 4 * kappa;             // first of this lane's 4 rows, tile-local
-          const int sl = (HALVES == 2 ? rg * 32 : rg * 64 + rt2 * 32) + 8 * q;  // staging row less 4 * kappa
-          RowConst rc;
-          const v4i rs4 = *(const v4i *)(cst_rs + rl);
-          const float4 as4 = *(const float4 *)(cst_as + rl);
-          rc.rs[0] = rs4.x; rc.rs[1] = rs4.y; rc.rs[2] = rs4.z; rc.rs[3] = rs4.w;
-          rc.as[0] = as4.x; rc.as[1] = as4.y; rc.as[2] = as4.z; rc.as[3] = as4.w;
+      for (int q = 0; q < 4; ++q) {
+        const float4 as4 = *(const float4 *)(cst_as + rt * 32 + 8 * q + 4 * kappa);
+        RowConst rc = {};
+        rc.as[0] = as4.x; rc.as[1] = as4.y; rc.as[2] = as4.z; rc.as[3] = as4.w;
 #pragma unroll
-          for (int y = 0; y < 2; ++y) {
-            const v4i av[1] = {v4i{acc[rt2][y][4 * q], acc[rt2][y][4 * q + 1], acc[rt2][y][4 * q + 2], acc[rt2][y][4 * q + 3]}};
+        for (int z = 0; z < HP; ++z) {
+          v4i av[P];
+          quad(rt, q, z, av);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float f = int8_value<1>(av, r, sc[y], rc, has_as);
-              uint8_t *dst = lane_base + (size_t)(sl + r) * STRIDE + y * 32 * ESZ;
-              if (ESZ == 2) *(uint16_t *)dst = f32_to_bf16_hw(f); else *(float *)dst = f;
-            }
+          for (int r = 0; r < 4; ++r) {
+            const float f = int8_value<P>(av, r, sc[z], rc, has_as);
+            uint8_t *dst = lane_base + (8 * q + r) * STRIDE + z * 32 * ESZ;
+            if (ESZ == 2) *(uint16_t *)dst = f32_to_bf16_hw(f); else *(float *)dst = f;
           }
         }
       }
-      __syncthreads();
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (c < hot.n) {
 #pragma unroll
-      for (int it = 0; it < SROWS * PIECES_ROW / TK_G128_THREADS; ++it) {
-        const int pc = it * TK_G128_THREADS + tid;
-        const int srow = pc / PIECES_ROW, piece = pc % PIECES_ROW;
-        const int orow = row0 + (HALVES == 2 ? (srow >> 5) * 64 + hh * 32 + (srow & 31) : srow);
-        const int c = col0 + piece * PER16;
-        if (orow >= R || c >= hot.n) continue;
-        if (wg_flag && gload(hot.flags + orow)) continue;  // written by exact_rows below
-        *(TK_GLOBAL v4u *)((uint8_t *)hot.out + ((size_t)orow * hot.n + c) * ESZ) = *(const v4u *)(smem + (size_t)srow * STRIDE + piece * 16);
+        for (int it = 0; it < 32 / RPI; ++it) {
+          const int rl = it * RPI + srow, orow = row0 + rt * 32 + rl;
+          if (orow < R && !(wg_flag && cst_flag[rt * 32 + rl]))  // (flagged rows: exact_rows below)
+            *(TK_GLOBAL v4u *)((uint8_t *)hot.out + ((size_t)orow * hot.n + c) * ESZ) = *(const v4u *)(wl + rl * STRIDE + piece * 16);
+        }
       }
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   };
-  if (hot.out_dtype == TK_BF16) finish(std::integral_constant<int, 2>{});
-  else finish(std::integral_constant<int, 4>{});
+  const int esz = hot.out_dtype == TK_BF16 ? 2 : 4;
+  if (int8_in && hot.out_dtype != TK_I32 && (((size_t)hot.n * esz) & 15) == 0 && ((uintptr_t)hot.out & 15) == 0 && !hot.residual) {
+    if (esz == 2) staged(std::integral_constant<int, 2>{});
+    else staged(std::integral_constant<int, 4>{});
+  } else {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int rl = rt * 32 + 8 * q + 4 * kappa;
+        const RowConst rc = consts(rl);
+#pragma unroll
+        for (int z = 0; z < HP; ++z) {
+          const int n = (tile0 + 2 * z + h) * 16 + r16;
+          if (n >= hot.n) continue;
+          v4i av[P];
+          quad(rt, q, z, av);
+          flow_epilogue<P>(hot, n, row0 + rl, av, sc[z], rc);
+        }
+      }
+  }
   if (wg_flag) {
-    for (int y = 0; y < 2; ++y) {
-      if (ncol[y] >= pr.n) continue;
-      for (int rt2 = 0; rt2 < 2; ++rt2)
+    for (int z = 0; z < HP; ++z) {
+      const int n = (tile0 + 2 * z + h) * 16 + r16;
+      if (n >= pr.n) continue;
+      for (int rt = 0; rt < RT; ++rt)
         for (int q = 0; q < 4; ++q) {
-          const int rowbase = row0 + rg * 64 + rt2 * 32 + 8 * q + 4 * kappa;
+          const int rowbase = row0 + rt * 32 + 8 * q + 4 * kappa;
           const unsigned fl = row_flags(pr, rowbase);
-          if (fl) exact_rows(pr, ncol[y], rowbase, fl);
+          if (fl) exact_rows(pr, n, rowbase, fl);
         }
     }
   }
 }
 
-int tk_gemm128_lds_bytes(void) { return TK_G128_CST + 1536; }
+template <int P>
+hipError_t go(hipStream_t s, const TkProblem *single, unsigned wgs) {
+  hipLaunchKernelGGL(tk_gemm128_kernel<P>, dim3(wgs), dim3(WAVES * 64), (size_t)Form<P>::LDS, s, *single);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+int tk_gemm128_rows(int planes) { return planes == 3 ? Form<3>::ROWS : Form<1>::ROWS; }
+int tk_gemm128_tiles(int planes) { return WAVES * (planes == 1 ? Form<1>::NT : Form<2>::NT); }
 
 hipError_t tk_launch_gemm128(hipStream_t s, const TkProblem *single) {
   const unsigned wgs = 8u * (unsigned)single->sub_m * (unsigned)single->sub_n;
   if (!wgs) return hipSuccess;
-  hipError_t e = tk_raise_lds_limit((const void *)tk_gemm128_kernel, 128 * 1024);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(tk_gemm128_kernel, dim3(wgs), dim3(TK_G128_THREADS), (size_t)tk_gemm128_lds_bytes(), s, *single);
-  return hipGetLastError();
+  switch (single->planes) {
+    case 1: return go<1>(s, single, wgs);
+    case 2: return go<2>(s, single, wgs);
+    case 3: return go<3>(s, single, wgs);
+    default: return hipErrorInvalidValue;
+  }
 }

@@ -226,11 +226,12 @@ hipError_t tk_launch_salt_seq(hipStream_t s, const TkProblem *single);
 hipError_t tk_launch_salt_gemm(hipStream_t s, const TkProblem *single, int compute_units);
 hipError_t tk_launch_gemm(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob,
                           const TkLaunchCfg &cfg);
-// 128 x 256 prefill kernel (tk_gemm128.hip): one plane, int8 contract, f32 / bf16 rows of whole 16-byte pieces,
-// no residual; grid from the problem's XCD split over 128-row x 16-tile blocks
-int tk_gemm128_lds_bytes(void);
+// 128-row prefill kernel (tk_gemm128.hip): one to three planes, both contracts, planes of less than 4 GiB of codes and at
+// least one K block; grid from the problem's XCD split over blocks of tk_gemm128_rows operand rows x tk_gemm128_tiles tiles
+int tk_gemm128_rows(int planes);
+int tk_gemm128_tiles(int planes);
 hipError_t tk_launch_gemm128(hipStream_t s, const TkProblem *single);
-// 256 x 224 prefill kernel (tk_gemm256.hip): the same launches as the 128 x 256 kernel; the weight tile is expanded to
+// 256 x 224 prefill kernel (tk_gemm256.hip): one plane, int8 contract, f32 / bf16 rows of whole 16-byte pieces, no residual; the weight tile is expanded to
 // int8 once per workgroup, in LDS. form 0: four waves of 64 rows over the whole column block (224 outputs); 1: eight
 // waves of 32 rows; 2: four waves over a part of the column block (128 or 96 outputs), two workgroups per CU. Grid from
 // the problem's XCD split over 256-row x 14-tile blocks.
