@@ -770,3 +770,39 @@ def test_prep_of_rows_aligned_like_an_element(backend, oracle, m, k, dtype):
     for a in (whole, o, o2):
         a.free()
     layer.free()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("m", [3, 40, 1100])
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 31, 130, 255, 256, 257, 515, 770])
+def test_activation_prep_of_ragged_rows_places_every_element(backend, oracle, k, m, dt):
+    """Rows of any length and (from the second row on) any address, a workgroup and a wave per token: a layer of one non-zero trit per
+    output shows every element on its own. Float contract: the element on the token's 31-bit grid, |out - a| at most half
+    a step (2^-30 of the row's maximum and a power of two at most: 2^-29) and 1.5 ulp of the recombination; the int8 contract: the oracle's bits.
+    Rows of NaN, of zeros, and of magnitudes whose scale 127 / max overflows (zeros among them) included."""
+    print("case ragged-prep", k, m, dt, flush=True)
+    rng = np.random.default_rng(k * 3 + m)
+    w = np.zeros((k, k), np.int8)
+    w[np.arange(k), rng.permutation(k)] = rng.choice([-1, 1], k)
+    packed, ones = T.pack_rows(w, k, k), np.ones(k, np.float32)
+    layer = backend.linear([packed], [ones], k, k)
+    a = (rng.standard_normal((m, k)) * 10.0 ** rng.integers(-3, 3, (m, 1))).astype(np.float32)
+    a[0] = rng.choice(np.float32([1e-37, -1e-37, 0.0, 3e-38, -2e-38]), k)
+    a[1, k // 2] = np.nan
+    a[2] = 0.0
+    host = f32_to_bf16_bits(a) if dt == "bf16" else a
+    seen = bf16_bits_to_f32(host).reshape(m, k) if dt == "bf16" else a
+    act, out = backend.to_device(host, dt), backend.empty(m * k, "f32")
+    backend.linear_a8(layer, act, m, out)
+    got, want = out.to_host().reshape(m, k), oracle.cpu_linear_a8_planes([packed], FMT_TQ2_0, [ones], seen, m, k, k).reshape(m, k)
+    fin = ~np.isnan(want)
+    assert (np.isnan(got) == ~fin).all() and same_bits(got[fin], want[fin])
+    backend.linear_float(layer, act, m, out)
+    got = out.to_host().reshape(m, k)
+    want = seen.astype(np.float64) @ w.T.astype(np.float64)
+    plain = np.arange(m) != 1
+    top = np.abs(seen).max(axis=1, keepdims=True)
+    assert (np.abs(got - want) <= top * 2.0 ** -29 + np.abs(want) * 2e-7 + 1e-44)[plain].all()
+    for x in (act, out):
+        x.free()
+    layer.free()

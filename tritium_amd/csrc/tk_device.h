@@ -492,11 +492,6 @@ __device__ __forceinline__ size_t piece_offset(size_t kb, int q, size_t R, size_
   return (((kb * 4 + j) * 4 + g) * R + row) * 16;
 }
 
-__device__ __forceinline__ int wave_sum(int v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
 // Rows of whole K blocks, 16-byte aligned, of one element type (FAST 1 = f32, 2 = bf16): the 16 elements of the piece
 // that starts at element e0 of the row at `base`, without bound, alignment or type tests.
 template <int FAST>

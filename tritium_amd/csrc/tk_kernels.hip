@@ -1447,56 +1447,88 @@ __global__ void tk_decode_trits_kernel(const uint8_t *__restrict__ codes, size_t
 }
 
 // ------------------------------------------------------------------------------------------
-// activation prep: one workgroup per token
+// activation prep. A thread builds whole 16-byte operand pieces and keeps them in registers between the pass that finds the
+// row maximum and the pass that quantizes, so that a row is read once. These launches are a token's chain -- load, maximum,
+// reduction, quantization, stores -- on few waves, so the instructions of the chain and the trips to memory in it are what they
+// cost: every load of a token is issued before the first is used (a piece past the row's end re-reads the last one), the
+// maximum is an integer one on the magnitude bits (which shows NaN and Inf as well), a rounding to an integer is one add
+// (1.5 * 2^23 leaves the int8 in the low byte), the four balanced digits of a float are one add and one exclusive or, bytes
+// are gathered by v_perm and summed by v_dot4, and reductions go through DPP and lane swaps instead of LDS.
+// About 6 vector instructions per element of the int8 quantization and 17 of the digit split (17 and 40 element by element). Kernels, before
+// -> now: digit split of 128 bf16 tokens K=2048 with block sums 7.5 -> 4.9 us, of 333 f32 tokens K=2050 11.9 -> 7.2; quantization of 32
+// bf16 tokens K=2560 4.1 -> 3.4, K=6912 4.8 -> 4.0, behind an RMSNorm 5.5 -> 4.5; of 2048 tokens K=2560 9.9 -> 9.5, which is near the
+// rate of a copy (15.7 MB; 4096 tokens K=5120 move 3.7 TB/s in 20.6 us). There, eight tokens to a workgroup with token = lane % 8, so that a
+// store fills whole lines, was no faster (2048 tokens K=2560, call with N=64 17.8 us either way; 400 tokens 14.1 -> 15.6).
 // ------------------------------------------------------------------------------------------
 
-// Row maximum and "any lane saw NaN/Inf" in one pass through LDS (one barrier pair instead of two).
-__device__ void block_max_any(float &v, int &flag, float *sh, int *shi) {
-  for (int o = 32; o > 0; o >>= 1) {
-    v = fmaxf(v, __shfl_xor(v, o));
-    flag |= __shfl_xor(flag, o);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    sh[threadIdx.x >> 6] = v;
-    shi[threadIdx.x >> 6] = flag;
-  }
-  __syncthreads();
-  v = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
-  flag = shi[0] | shi[1] | shi[2] | shi[3];
-  __syncthreads();
+// ---- reductions: every lane receives the result ----
+template <int CTRL>
+__device__ __forceinline__ unsigned lane_dpp(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
 }
-
-// NV block sums at once (the four digit rows of a token, and its two element counts); sh holds
-// 4 * NV ints.
-template <int NV>
-__device__ void block_sums(int (&v)[NV], int *sh) {
-#pragma unroll
-  for (int d = 0; d < NV; ++d)
-    for (int o = 32; o > 0; o >>= 1) v[d] += __shfl_xor(v[d], o);
-  if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-    for (int d = 0; d < NV; ++d) sh[(threadIdx.x >> 6) * NV + d] = v[d];
+typedef unsigned tk_u2 __attribute__((ext_vector_type(2)));
+// over the 16 lanes of a row: neighbours, pairs, then the mirrored half row and the mirrored row
+__device__ __forceinline__ int row16_sum(int v) {
+  v += (int)lane_dpp<0xB1>((unsigned)v);
+  v += (int)lane_dpp<0x4E>((unsigned)v);
+  v += (int)lane_dpp<0x141>((unsigned)v);
+  return v + (int)lane_dpp<0x140>((unsigned)v);
+}
+__device__ __forceinline__ int lanes_sum(int v) {
+  v = row16_sum(v);
+  const tk_u2 a = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+  v = (int)(a.x + a.y);
+  const tk_u2 b = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+  return (int)(b.x + b.y);
+}
+__device__ __forceinline__ unsigned lanes_max(unsigned v) {
+  v = max(v, lane_dpp<0xB1>(v));
+  v = max(v, lane_dpp<0x4E>(v));
+  v = max(v, lane_dpp<0x141>(v));
+  v = max(v, lane_dpp<0x140>(v));
+  const tk_u2 a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = max(a.x, a.y);
+  const tk_u2 b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return max(b.x, b.y);
+}
+// Over a team: a wave (64), or the four waves of the workgroup (256) through `sh`, one barrier. Nothing may still read `sh`
+// from an earlier use that no barrier has followed: a kernel uses one array per reduction and alternates between them.
+template <int TEAM>
+__device__ __forceinline__ unsigned team_max(unsigned v, unsigned *sh) {
+  v = lanes_max(v);
+  if constexpr (TEAM != 64) {
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = max(max(sh[0], sh[1]), max(sh[2], sh[3]));
   }
-  __syncthreads();
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)v);  // (uniform: the branches on it are scalar)
+}
+template <int TEAM, int NV>
+__device__ __forceinline__ void team_sums(int (&v)[NV], int *sh) {
 #pragma unroll
-  for (int d = 0; d < NV; ++d) v[d] = sh[d] + sh[NV + d] + sh[2 * NV + d] + sh[3 * NV + d];
-  __syncthreads();
+  for (int d = 0; d < NV; ++d) v[d] = lanes_sum(v[d]);
+  if constexpr (TEAM != 64) {
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+      for (int d = 0; d < NV; ++d) sh[(threadIdx.x >> 6) * NV + d] = v[d];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < NV; ++d) v[d] = sh[d] + sh[NV + d] + sh[2 * NV + d] + sh[3 * NV + d];
+  }
+#pragma unroll
+  for (int d = 0; d < NV; ++d) v[d] = __builtin_amdgcn_readfirstlane(v[d]);
 }
-
-__device__ int block_sum(int v, int *sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
-  int r = sh[0] + sh[1] + sh[2] + sh[3];
-  __syncthreads();
-  return r;
-}
+struct TkPrepShared {  // LDS of a team of 256: one array per reduction
+  unsigned peak[4], peak2[4];
+  int sums[24], bands[32];
+};
 
 // Four consecutive activations starting at element e (a multiple of 4) as floats; elements at or
-// past k read as 0. `vec`: one 8- or 16-byte load where all four exist. It is aligned like an element only (rows of any k, any
+// past k read as 0. One 8- or 16-byte load where all four exist. It is aligned like an element only (rows of any k, any
 // base): global loads take that on this chip (700 bf16 tokens of K=6001, int8 contract, element by element 27.8 us, so 24.8).
-__device__ __forceinline__ void load_act4(const void *act, int dtype, size_t base, size_t e, size_t k, bool vec, float (&v)[4]) {
-  if (vec && e + 4 <= k) {
+__device__ __forceinline__ void load_act4(const void *act, int dtype, size_t base, size_t e, size_t k, float (&v)[4]) {
+  if (e + 4 <= k) {
     if (dtype == TK_BF16) {
       typedef unsigned v2u __attribute__((ext_vector_type(2), aligned(2)));
       const v2u u = *(const TK_GLOBAL v2u *)((const uint16_t *)act + base + e);
@@ -1518,9 +1550,6 @@ __device__ __forceinline__ void load_act4(const void *act, int dtype, size_t bas
   for (int b = 0; b < 4; ++b) v[b] = e + b < k ? load_act(act, dtype, base + e + b) : 0.0f;
 }
 
-__device__ __forceinline__ bool act_rows_vectorizable(int dtype) { return dtype == TK_BF16 || dtype == TK_F32; }
-
-// gamma = max |a| with the reference's `a > gamma` rule (NaN never wins), plus a non-finite flag.
 // RMSNorm in front of the quantization (crates/tritium-nn/src/ops/rmsnorm.rs:21-96). The sum of
 // squares folds in the reference's canonical order: slot t (= thread t of the 256) takes x[t],
 // x[t+256], ... in ascending order, multiply then add, and a power-of-two tree (off = 128 .. 1)
@@ -1573,26 +1602,6 @@ __device__ __forceinline__ void apply_norm4(const RowNorm &nm, size_t e, size_t 
   }
 }
 
-__device__ void row_absmax(const void *act, int dtype, size_t base, size_t k, bool vec, float *sh, float &gamma,
-                           int &nonfinite, int *shi, const RowNorm &nm = RowNorm{0, 0.0f, nullptr}) {
-  float g = 0.0f;
-  int nf = 0;
-  for (size_t e = (size_t)threadIdx.x * 4; e < k; e += TK_WG * 4) {
-    float v[4];
-    load_act4(act, dtype, base, e, k, vec, v);
-    apply_norm4(nm, e, k, v);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const float a = fabsf(v[b]);
-      if (a > g) g = a;
-      nf |= !(a <= 3.402823466e38f);  // NaN or Inf
-    }
-  }
-  block_max_any(g, nf, sh, shi);
-  gamma = g;
-  nonfinite = nf != 0;
-}
-
 // uniform_m > 0: every tensor of the table has that many tokens, so the entry follows from the
 // workgroup index without the chain of dependent loads the search costs.
 __device__ __forceinline__ const TkPrep &find_prep(const TkPrep &single, const TkPrep *table, int nprep, int uniform_m,
@@ -1623,347 +1632,6 @@ __device__ __forceinline__ const TkPrep &find_prep(const TkPrep &single, const T
   row = blockIdx.x - table[lo].row_begin;
   return table[lo];
 }
-
-// The 16 elements of operand piece (kb, q16) of a row: four groups of four, 32 elements apart.
-__device__ __forceinline__ void load_piece(const void *act, int dtype, size_t base, size_t e0, size_t k, bool vec,
-                                           float (&v)[16]) {
-#pragma unroll
-  for (int sl = 0; sl < 4; ++sl) {
-    float t[4];
-    load_act4(act, dtype, base, e0 + (size_t)sl * 32, k, vec, t);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) v[sl * 4 + b] = t[b];
-  }
-}
-
-// Rows of up to TK_PREP_HELD * 256 pieces (K <= 16384) are read from memory once: every thread keeps
-// its pieces in registers between the pass that finds the row maximum and the pass that quantizes.
-#define TK_PREP_HELD 4
-template <int HELD>
-__device__ __forceinline__ void row_absmax_held(const void *act, int dtype, size_t base, size_t k, size_t npieces,
-                                                bool vec, float (&held)[HELD][16], float *sh, float &gamma,
-                                                int &nonfinite, int *shi) {
-  float g = 0.0f;
-  int nf = 0;
-#pragma unroll
-  for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)threadIdx.x + (size_t)it * TK_WG;
-    if (pc < npieces) {
-      load_piece(act, dtype, base, piece_elem0(pc >> 4, (int)(pc & 15)), k, vec, held[it]);
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        const float a = fabsf(held[it][x]);  // elements past k were loaded as 0
-        if (a > g) g = a;
-        nf |= !(a <= 3.402823466e38f);
-      }
-    }
-  }
-  block_max_any(g, nf, sh, shi);
-  gamma = g;
-  nonfinite = nf != 0;
-}
-
-// Per-token int8 absmax quant (crates/tritium-spec/src/lib.rs:351-378) straight into operand order.
-// HELD = pieces a thread keeps in registers: 1 for rows of up to 256 pieces (K <= 4096), 2 up to 512:
-// the registers saved double the resident workgroups, so that 2048 tokens run as one round.
-template <int HELD>
-__global__ __launch_bounds__(TK_WG) void tk_prep_a8_kernel(TkPrep single, const TkPrep *__restrict__ table,
-                                                           int nprep, int uniform_m) {
-  __shared__ float shf[4];
-  __shared__ int shi[4];
-  int rowi;
-  const TkPrep &pp = find_prep(single, table, nprep, uniform_m, rowi);
-  const size_t row = rowi, k = pp.k, nb = pp.nb, R = pp.rs;
-  const size_t base = row * k;
-  const void *act = pp.act;
-  const int dtype = pp.act_dtype;
-  int8_t *ap = pp.ap, *qrm = pp.q_rowmajor;
-  const bool vec = act_rows_vectorizable(dtype);
-  RowNorm nm = {pp.norm_kind, 0.0f, pp.norm_w};
-  float *ynorm = nullptr;
-  if (nm.kind) {
-    __shared__ float part[TK_WG];
-    nm.inv = row_inv_rms(act, dtype, base, k, pp.norm_eps, part);
-  }
-  const size_t npieces = nb * 16;
-  const bool resident = !nm.kind && npieces <= (size_t)HELD * TK_WG;
-  float held[HELD][16];
-  float gamma;
-  int nonfinite;
-  if (resident)
-    row_absmax_held(act, dtype, base, k, npieces, vec, held, shf, gamma, nonfinite, shi);
-  else
-    row_absmax(act, dtype, base, k, vec, shf, gamma, nonfinite, shi, nm);
-  if (nm.kind && nonfinite) ynorm = pp.ynorm;  // only the exact fallback reads the normalized row
-  const float s = gamma == 0.0f ? 0.0f : __fdiv_rn(127.0f, gamma);  // one divide
-  const bool live = gamma != 0.0f && !nonfinite;
-  int sum = 0;
-  // quantize the 16 values of piece pc and store them in operand order (and row-major, if asked)
-  auto emit = [&](size_t pc, const float (&v)[16]) {
-    const size_t kb = pc >> 4;
-    const int q16 = (int)(pc & 15);
-    const size_t e0 = piece_elem0(kb, q16);
-    v4u piece;
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      const size_t e = e0 + (size_t)sl * 32;
-      if (ynorm) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          if (e + b < k) gstore(ynorm + base + e + b, v[sl * 4 + b]);
-      }
-      uint32_t packed = 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        int q = 0;
-        if (live && e + b < k) {
-          float r = rintf(__fmul_rn(v[sl * 4 + b], s));  // one multiply, ties to even
-          r = r < -128.0f ? -128.0f : (r > 127.0f ? 127.0f : r);
-          q = (int)r;
-        }
-        sum += q;
-        packed |= ((uint32_t)q & 0xFFu) << (8 * b);
-      }
-      piece[sl] = packed;
-      if (qrm) {
-        if (vec && e + 4 <= k) {
-          typedef uint32_t loose __attribute__((aligned(1)));
-          *(TK_GLOBAL loose *)(qrm + base + e) = packed;
-        } else {
-          for (int b = 0; b < 4; ++b)
-            if (e + b < k) qrm[base + e + b] = (int8_t)(packed >> (8 * b));
-        }
-      }
-    }
-    if (ap) *(TK_GLOBAL v4u *)(ap + piece_offset(kb, q16, R, row)) = piece;
-  };
-  if (resident) {
-#pragma unroll
-    for (int it = 0; it < HELD; ++it) {
-      const size_t pc = (size_t)threadIdx.x + (size_t)it * TK_WG;
-      if (pc < npieces) emit(pc, held[it]);
-    }
-  } else {
-    for (size_t pc = threadIdx.x; pc < npieces; pc += TK_WG) {
-      float v[16];
-      const size_t e0 = piece_elem0(pc >> 4, (int)(pc & 15));
-      load_piece(act, dtype, base, e0, k, vec, v);
-#pragma unroll
-      for (int sl = 0; sl < 4; ++sl) {
-        float t[4] = {v[sl * 4], v[sl * 4 + 1], v[sl * 4 + 2], v[sl * 4 + 3]};
-        apply_norm4(nm, e0 + (size_t)sl * 32, k, t);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) v[sl * 4 + b] = t[b];
-      }
-      emit(pc, v);
-    }
-  }
-  sum = block_sum(sum, shi);
-  if (threadIdx.x == 0) {
-    if (pp.rowsum) pp.rowsum[row] = sum;
-    pp.act_scale[row] = gamma == 0.0f ? 0.0f : __fdiv_rn(gamma, 127.0f);
-    if (pp.aux) pp.aux[row] = s;
-    if (pp.flags) pp.flags[row] = nonfinite ? 1u : 0u;
-  }
-}
-
-// An element scaled onto the grid (r = a * 2^(30-E), q = its rounding) is carried faithfully when it
-// lies on the grid or its rounding error is at most 2^-16 of it.
-__device__ __forceinline__ bool digit_poor(float r, int q) { return !(fabsf(r) >= 32768.0f || r == (float)q); }
-// Where the call stands in for sums in the reference's order (TkPrep.strict), at most 2^-21 of it.
-#define TK_DIGIT_STRICT 1048576.0f
-
-// Counts of the elements of one piece per magnitude band: band b holds 2^(30-4b-4) <= |r| < 2^(30-4b);
-// elements below the eighth band (and zeros) are not counted.
-__device__ __forceinline__ void count_bands(const float (&v)[16], int shift, int (&bands)[8]) {
-#pragma unroll
-  for (int x = 0; x < 16; ++x) {
-    const float r = ldexpf(v[x], shift);
-    const int band = (156 - (int)((__float_as_uint(r) >> 23) & 0xFFu)) >> 2;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) bands[b] += band == b ? 1 : 0;
-  }
-}
-
-#define TK_DIGITS_TRIM 96
-// Energy left without the TK_DIGITS_TRIM largest elements, in units of 2^(2E): band b counts at its
-// lower edge 2^(-4b-4). The grid does not carry the token when its rounding noise n_poor * 2^-62 / 3
-// exceeds 2^-30 of that -- or, where the call stands in for the reference's order (strict), 2^-42: amplitude 2^-21 = 4.8e-7,
-// while f32 sums over K >= 2560 in k order show 5.6e-7 and more against float64.
-__device__ __forceinline__ bool digits_narrow(int n_poor, const int (&bands)[8], bool strict = false) {
-  float left = 0.0f, edge2 = 0.00390625f;  // 2^-8
-  int trim = TK_DIGITS_TRIM;
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    const int c = bands[b], cut = c < trim ? c : trim;
-    trim -= cut;
-    left += (float)(c - cut) * edge2;
-    edge2 *= 0.00390625f;
-  }
-  return n_poor > 0 && (float)n_poor > 3.0f * (strict ? 1048576.0f : 4294967296.0f) * left;
-}
-
-// Float token -> four balanced base-256 digit rows of round(a * 2^(30-E)), 2^(E-1) <= max|a| < 2^E.
-// Scaling a float by a power of two is exact, so the rounding to an integer happens once, in
-// single precision.
-//
-// Dynamic range. The grid is 2^(E-30) wide against the token's own maximum. An element that lies on
-// the grid exactly, or is at least 2^(E-15) in magnitude (rounding error at most 2^-16 of itself), is
-// carried faithfully; any other ("poor") element is rounded by up to 2^(E-31), which can be all of
-// it. The reference's k-ordered f32 fold skips an activation under a zero trit
-// (crates/tritium-core/src/reference.rs:42-51), so an output can miss the largest elements of a token
-// and consist of small ones only: its value is then small next to the token's maximum, and the
-// rounding of the poor elements shows. The prep therefore compares the rounding noise of a token,
-// n_poor * 2^(2(E-31)) / 3, with the energy that is left when its TK_DIGITS_TRIM largest elements
-// are all skipped (a lower bound from counts per 4-bit magnitude band below 2^E): where the noise
-// exceeds 2^-30 of that energy (2^-15 in amplitude, i.e. 3e-5 of a typical output that misses the
-// top elements), the token is flagged like one holding NaN or Inf and its outputs are computed in
-// the reference's order. For every other token and every output, unconditionally,
-//   |value - exact dot product| <= n * 2^(E-31)  (+ 1.5 ulp),  n = poor elements under its non-zero trits.
-// (STRICT: TkPrep.strict; a form of its own because the count of large elements costs the others 1%)
-template <bool STRICT>
-__global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, const TkPrep *__restrict__ table,
-                                                               int nprep, int uniform_m) {
-  __shared__ float shf[4];
-  __shared__ int shi[32];
-  int rowi;
-  const TkPrep &pp = find_prep(single, table, nprep, uniform_m, rowi);
-  const size_t tok = rowi, k = pp.k, nb = pp.nb, R = pp.rs;
-  const size_t base = tok * k;
-  const void *act = pp.act;
-  const int dtype = pp.act_dtype;
-  int8_t *ap = pp.ap;
-  const bool vec = act_rows_vectorizable(dtype);
-  const size_t npieces = nb * 16;
-  const bool resident = npieces <= (size_t)TK_PREP_HELD * TK_WG;
-  float held[TK_PREP_HELD][16];
-  float gamma;
-  int nonfinite;
-  if (resident)
-    row_absmax_held(act, dtype, base, k, npieces, vec, held, shf, gamma, nonfinite, shi);
-  else
-    row_absmax(act, dtype, base, k, vec, shf, gamma, nonfinite, shi);
-  int E = 0;
-  if (gamma != 0.0f && !nonfinite) (void)frexpf(gamma, &E);
-  const int shift = 30 - E;
-  const bool live = gamma != 0.0f && !nonfinite;
-  constexpr int NSUMS = STRICT ? 6 : 5;
-  int sums[NSUMS] = {};  // four digit-row sums, poor elements; STRICT: elements from TK_DIGIT_STRICT on
-  int &n_poor = sums[4];
-  // split the 16 values of piece pc into their four digit rows and store those in operand order
-  auto emit = [&](size_t pc, const float (&v)[16]) {
-    const size_t kb = pc >> 4;
-    const int q16 = (int)(pc & 15);
-    const size_t e0 = piece_elem0(kb, q16);
-    v4u piece[4];
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      const size_t e = e0 + (size_t)sl * 32;
-      uint32_t packed[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        int q = 0;
-        if (live && e + b < k) {
-          const float r = ldexpf(v[sl * 4 + b], shift);
-          q = __float2int_rn(r);  // |q| <= 2^30
-          if constexpr (STRICT) {
-            const bool large = fabsf(r) >= TK_DIGIT_STRICT;
-            sums[5] += large ? 1 : 0;
-            n_poor += !(large || r == (float)q) ? 1 : 0;
-          } else {
-            n_poor += digit_poor(r, q) ? 1 : 0;
-          }
-        }
-#pragma unroll
-        for (int dg = 0; dg < 4; ++dg) {
-          int dv = dg == 3 ? q : (((q + 128) & 0xFF) - 128);  // balanced digit in [-128,127]
-          q = (q - dv) >> 8;
-          sums[dg] += dv;
-          packed[dg] |= ((uint32_t)dv & 0xFFu) << (8 * b);
-        }
-      }
-#pragma unroll
-      for (int dg = 0; dg < 4; ++dg) piece[dg][sl] = packed[dg];
-    }
-#pragma unroll
-    for (int dg = 0; dg < 4; ++dg) *(TK_GLOBAL v4u *)(ap + piece_offset(kb, q16, R, tok * 4 + dg)) = piece[dg];
-    if (pp.blocksum) {
-      // sums of each digit row over this K block alone (the 16 pieces of a block sit in 16
-      // consecutive lanes): entry [kb][row], row stride = the operand row count
-      int bs[4];
-#pragma unroll
-      for (int dg = 0; dg < 4; ++dg) {
-        int t = 0;
-#pragma unroll
-        for (int sl = 0; sl < 4; ++sl) {
-          const uint32_t u = piece[dg][sl];
-          t += (int)(int8_t)(u & 0xFF) + (int)(int8_t)((u >> 8) & 0xFF) + (int)(int8_t)((u >> 16) & 0xFF) + (int)(int8_t)(u >> 24);
-        }
-        for (int o = 8; o > 0; o >>= 1) t += __shfl_xor(t, o);
-        bs[dg] = t;
-      }
-      if (q16 == 0) {
-#pragma unroll
-        for (int dg = 0; dg < 4; ++dg) pp.blocksum[kb * pp.R + tok * 4 + dg] = bs[dg];
-      }
-    }
-  };
-  if (resident) {
-#pragma unroll
-    for (int it = 0; it < TK_PREP_HELD; ++it) {
-      const size_t pc = (size_t)threadIdx.x + (size_t)it * TK_WG;
-      if (pc < npieces) emit(pc, held[it]);
-    }
-  } else {
-    for (size_t pc = threadIdx.x; pc < npieces; pc += TK_WG) {
-      float v[16];
-      load_piece(act, dtype, base, piece_elem0(pc >> 4, (int)(pc & 15)), k, vec, v);
-      emit(pc, v);
-    }
-  }
-  block_sums<NSUMS>(sums, shi);
-  // Only a token that has poor elements needs the magnitude bands (the same answer in every thread, so
-  // the barriers inside are reached by all or by none). Strict: nor does one with enough large elements, each of
-  // 2^-20 in energy (units of 2^(2E)): left >= (their number - TK_DIGITS_TRIM) * 2^-20 answers digits_narrow.
-  bool narrow = false, bands_needed = n_poor > 0;
-  if constexpr (STRICT) bands_needed = bands_needed && n_poor > 3 * (sums[5] - TK_DIGITS_TRIM);
-  if (bands_needed) {
-    int bands[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (resident) {
-#pragma unroll
-      for (int it = 0; it < TK_PREP_HELD; ++it) {
-        const size_t pc = (size_t)threadIdx.x + (size_t)it * TK_WG;
-        if (pc < npieces) count_bands(held[it], shift, bands);
-      }
-    } else {
-      for (size_t pc = threadIdx.x; pc < npieces; pc += TK_WG) {
-        float v[16];
-        load_piece(act, dtype, base, piece_elem0(pc >> 4, (int)(pc & 15)), k, vec, v);
-        count_bands(v, shift, bands);
-      }
-    }
-    block_sums<8>(bands, shi);
-    narrow = digits_narrow(n_poor, bands, STRICT);
-  }
-  if (threadIdx.x < 4) {
-    const int t = threadIdx.x;
-    pp.rowsum[tok * 4 + t] = t == 0 ? sums[0] : t == 1 ? sums[1] : t == 2 ? sums[2] : sums[3];
-  }
-  if (threadIdx.x == 0) {
-    pp.exps[tok] = -shift;
-    pp.flags[tok] = (nonfinite || narrow) ? 1u : 0u;
-  }
-}
-
-// ------------------------------------------------------------------------------------------
-// activation prep, one WAVE per token: rows of up to HELD * 64 pieces (K <= 4096 at HELD = 4). Same
-// arithmetic and the same bytes out as the one-workgroup-per-token kernels above; what changes is the
-// shape of the work: a token's pieces sit in the registers of one wave, the row maximum and the row
-// sums are wave shuffles, nothing waits at a barrier, every lane has pieces to work on (a K = 2048
-// row has 128 pieces: half a workgroup's threads idle), and a launch has a quarter of the workgroups.
-// Not for rows that are normalized first (the canonical sum of squares has 256 slots) nor for the
-// per-block row sums of the block-scale planes.
-// ------------------------------------------------------------------------------------------
 
 // The token a wave works on, and its tensor. Single tensor, workgroup count a multiple of 16: eight
 // consecutive rows share every 128-byte line of the operand layout, and workgroups go to the 8 XCDs
@@ -2023,232 +1691,508 @@ __device__ __forceinline__ const TkPrep &find_prep_wave(const TkPrep &single, co
   return table[lo];
 }
 
-// FAST != 0: the launch's rows are whole K blocks (k a multiple of 256), 16-byte aligned, of one element type
-// (1 = f32, 2 = bf16) and only the operand rows are wanted: no bound, alignment or type is tested per
-// element, which is most of what the general form executes (a wave works through its token alone, one
-// dependent instruction after the other: the instruction count is the launch's time).
-template <int HELD, int FAST = 0, int TEAM = 64>
-__device__ __forceinline__ void wave_absmax_held(const void *act, int dtype, size_t base, size_t k, size_t npieces, bool vec,
-                                                 int lane, float (&held)[HELD][16], float &gamma, int &nonfinite,
-                                                 float *shf = nullptr, int *shi = nullptr) {
-  float g = 0.0f;
-  int nf = 0;
+// ---- pieces of a row ----
+// The piece that starts at element e0 of a row of any length and address, zeros past its end: four loads that stay inside the
+// row (of at least four elements), aligned like an element; what a load at the row's end brings too early is shifted out.
+template <int DT>
+__device__ __forceinline__ void load_piece_ragged(const void *act, size_t base, unsigned e0, unsigned k, float (&v)[16]) {
+  int over[4];  // elements that group sl's load starts before the group
+  if constexpr (DT == TK_BF16) {
+    typedef unsigned v2l __attribute__((ext_vector_type(2), aligned(2)));
+    v2l u[4];
 #pragma unroll
-  for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * TEAM;
-    if (pc < npieces) {
-      if constexpr (FAST != 0) load_piece_fast<FAST>(act, base, piece_elem0(pc >> 4, (int)(pc & 15)), held[it]);
-      else load_piece(act, dtype, base, piece_elem0(pc >> 4, (int)(pc & 15)), k, vec, held[it]);
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        const float a = fabsf(held[it][x]);  // elements past k were loaded as 0
-        if (a > g) g = a;                    // NaN never wins (crates/tritium-spec/src/lib.rs:351-360)
-        nf |= !(a <= 3.402823466e38f);
-      }
+    for (int sl = 0; sl < 4; ++sl) {
+      const unsigned e = e0 + sl * 32, at = min(e, k - 4);
+      over[sl] = (int)(e - at);
+      u[sl] = *(const TK_GLOBAL v2l *)((const uint16_t *)act + base + at);
     }
-  }
-  if constexpr (TEAM == 64) {
-    for (int o = 32; o > 0; o >>= 1) {
-      g = fmaxf(g, __shfl_xor(g, o));
-      nf |= __shfl_xor(nf, o);
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl) {
+      v[sl * 4 + 0] = __uint_as_float(u[sl].x << 16);
+      v[sl * 4 + 1] = __uint_as_float(u[sl].x & 0xFFFF0000u);
+      v[sl * 4 + 2] = __uint_as_float(u[sl].y << 16);
+      v[sl * 4 + 3] = __uint_as_float(u[sl].y & 0xFFFF0000u);
     }
   } else {
-    block_max_any(g, nf, shf, shi);
+    typedef unsigned v4l __attribute__((ext_vector_type(4), aligned(4)));
+    v4l u[4];
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl) {
+      const unsigned e = e0 + sl * 32, at = min(e, k - 4);
+      over[sl] = (int)(e - at);
+      u[sl] = *(const TK_GLOBAL v4l *)((const float *)act + base + at);
+    }
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) v[sl * 4 + b] = __uint_as_float(u[sl][b]);
   }
-  gamma = g;
-  nonfinite = nf != 0;
+  if (__any(over[3] > 0)) {  // (the groups of a piece ascend)
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl) {
+      float *g = v + sl * 4;
+      const int d = over[sl];
+      const bool one = d & 1, two = d & 2;
+      g[0] = one ? g[1] : g[0];
+      g[1] = one ? g[2] : g[1];
+      g[2] = one ? g[3] : g[2];
+      g[3] = one ? 0.0f : g[3];
+      g[0] = two ? g[2] : g[0];
+      g[1] = two ? g[3] : g[1];
+      g[2] = two ? 0.0f : g[2];
+      g[3] = two ? 0.0f : g[3];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) g[b] = d >= 4 ? 0.0f : g[b];
+    }
+  }
+}
+// the same for rows of fewer than four elements too, and an element type known at run time (uniform)
+__device__ __forceinline__ void load_piece(const void *act, int dtype, size_t base, size_t e0, size_t k, float (&v)[16]) {
+  if (k < 4) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) v[x] = 0.0f;
+    if (e0 == 0) {
+#pragma unroll
+      for (int b = 0; b < 3; ++b) v[b] = (size_t)b < k ? load_act(act, dtype, base + b) : 0.0f;
+    }
+  } else if (dtype == TK_BF16) {
+    load_piece_ragged<TK_BF16>(act, base, (unsigned)e0, (unsigned)k, v);
+  } else {
+    load_piece_ragged<TK_F32>(act, base, (unsigned)e0, (unsigned)k, v);
+  }
+}
+// The pieces lane, lane + TEAM, ... of a row. FAST: rows of whole K blocks, 16-byte aligned, of one element type (1 = f32, 2 = bf16).
+template <int HELD, int FAST, int TEAM>
+__device__ __forceinline__ void load_held(const void *act, int dtype, size_t base, size_t k, int npieces, int lane,
+                                          float (&held)[HELD][16]) {
+#pragma unroll
+  for (int it = 0; it < HELD; ++it) {
+    if (it > 0 && it * TEAM >= npieces) {  // (uniform)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) held[it][x] = 0.0f;
+      continue;
+    }
+    const int pc = min(lane + it * TEAM, npieces - 1);
+    const size_t e0 = piece_elem0((size_t)(pc >> 4), pc & 15);
+    if constexpr (FAST != 0) load_piece_fast<FAST>(act, base, e0, held[it]);
+    else load_piece(act, dtype, base, e0, k, held[it]);
+  }
+}
+__device__ __forceinline__ unsigned magnitude_bits(float x) { return __float_as_uint(x) & 0x7FFFFFFFu; }
+constexpr unsigned TK_INF_BITS = 0x7F800000u;
+
+// max |a| of a row from the largest magnitude bits its team found. The reference's rule is `a > gamma` (NaN never wins:
+// crates/tritium-spec/src/lib.rs:351-360): where the bits are a NaN's, `again` gives the largest that are not.
+template <int HELD, int TEAM>
+__device__ __forceinline__ float held_peak(const float (&held)[HELD][16], bool &nonfinite, unsigned *sh, unsigned *sh2) {
+  unsigned m = 0;
+#pragma unroll
+  for (int it = 0; it < HELD; ++it)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) m = max(m, magnitude_bits(held[it][x]));
+  m = team_max<TEAM>(m, sh);
+  nonfinite = m >= TK_INF_BITS;
+  if (m > TK_INF_BITS) {
+    m = 0;
+#pragma unroll
+    for (int it = 0; it < HELD; ++it)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        float a = held[it][x];
+        asm("" : "+v"(a));  // (the magnitudes are formed anew: kept from above they would double the registers)
+        const unsigned b = magnitude_bits(a);
+        m = max(m, b > TK_INF_BITS ? 0u : b);
+      }
+    m = team_max<TEAM>(m, sh2);
+  }
+  return __uint_as_float(m);
 }
 
-// TEAM = 64: a wave per token, four tokens per workgroup, no barrier. TEAM = 256: the workgroup per token (the
-// maximum and the sums cross its waves through LDS): a quarter of the instructions per thread, for launches
-// of few tokens, whose time is one token's chain.
-template <int HELD, int FAST = 0, int TEAM = 64>
-__global__ __launch_bounds__(TK_WG) void tk_prep_a8_wave_kernel(TkPrep single, const TkPrep *__restrict__ table, int nprep,
-                                                                int uniform_m, unsigned rows) {
-  __shared__ float shf[4];
-  __shared__ int shi[4];
-  const int wave = threadIdx.x >> 6, lane = TEAM == 64 ? (threadIdx.x & 63) : threadIdx.x;
-  int rowi, gt;
-  const TkPrep &pp = find_prep_wave(single, table, nprep, uniform_m, wave, rowi, gt, TEAM);
-  if ((unsigned)gt >= rows) return;  // (a whole team leaves together: the barriers below stay uniform)
+// ---- the int8 quantization (crates/tritium-spec/src/lib.rs:351-378) ----
+// scale of a row: s = 127 / gamma, one divide. odd: 1 = the row quantizes to zeros (no maximum, or NaN / Inf), 2 = s overflows
+// (gamma below 3.8e-37): every element but zero saturates, and a zero times s is NaN, which the host carries on as NaN -- so such a
+// row takes the exact fallback (`exact`) like one that holds NaN or Inf; as an int8 it is 0.
+struct RowScale {
+  float s, mul;
+  int odd;
+  bool exact;
+};
+__device__ __forceinline__ RowScale row_scale(float gamma, bool nonfinite) {
+  RowScale rs;
+  rs.s = gamma == 0.0f ? 0.0f : __fdiv_rn(127.0f, gamma);
+  rs.odd = (gamma == 0.0f || nonfinite) ? 1 : (rs.s > 3.402823466e38f ? 2 : 0);
+  rs.exact = nonfinite || rs.odd == 2;
+  rs.mul = rs.odd == 0 ? rs.s : (rs.odd == 1 ? 0.0f : 127.0f);
+  return rs;
+}
+__device__ __forceinline__ void odd_row(float (&v)[16], int odd) {
+  const float above = odd == 1 ? 0.0f : 1.0f, below = odd == 1 ? 0.0f : -128.0f / 127.0f;
+#pragma unroll
+  for (int x = 0; x < 16; ++x) v[x] = v[x] > 0.0f ? above : (v[x] < 0.0f ? below : 0.0f);
+}
+// A piece of int8 values and their sum: one multiply, then to nearest even. |a| <= gamma, so the product rounds to 127 at most
+// (rows with scale.odd have been through odd_row).
+__device__ __forceinline__ v4u quantize_piece(const float (&v)[16], const RowScale &rs, int &sum) {
+  v4u piece;
+#pragma unroll
+  for (int sl = 0; sl < 4; ++sl) {
+    unsigned u[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) u[b] = __float_as_uint(__fadd_rn(__fmul_rn(v[sl * 4 + b], rs.mul), 12582912.0f));
+    piece[sl] = __builtin_amdgcn_perm(u[1], u[0], 0x0C0C0400u) | __builtin_amdgcn_perm(u[3], u[2], 0x04000C0Cu);
+    sum = __builtin_amdgcn_sdot4((int)piece[sl], 0x01010101, sum, false);
+  }
+  return piece;
+}
+__device__ __forceinline__ float gamma_over_127(float gamma) { return gamma == 0.0f ? 0.0f : __fdiv_rn(gamma, 127.0f); }
+
+// ---- the digit split ----
+// An element scaled onto the grid (r = a * 2^(30-E), rounded to q) is carried faithfully when it lies on the grid or its
+// rounding error is at most 2^-16 of it; where the call stands in for sums in the reference's order (TkPrep.strict), 2^-21.
+constexpr float TK_DIGIT_LARGE = 32768.0f, TK_DIGIT_STRICT = 1048576.0f;
+
+// Counts of the elements of one piece per magnitude band: band b holds 2^(30-4b-4) <= |r| < 2^(30-4b);
+// elements below the eighth band (and zeros) are not counted.
+__device__ __forceinline__ void count_bands(const float (&v)[16], int shift, int (&bands)[8]) {
+  unsigned lo = 0, hi = 0;  // a byte per band
+#pragma unroll
+  for (int x = 0; x < 16; ++x) {
+    const float r = ldexpf(v[x], shift);
+    const int band = (156 - (int)((__float_as_uint(r) >> 23) & 0xFFu)) >> 2;
+    const unsigned one = 1u << ((band & 3) * 8);
+    lo += band < 4 ? one : 0u;
+    hi += (band & ~3) == 4 ? one : 0u;
+  }
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    bands[b] += (int)((lo >> (8 * b)) & 255u);
+    bands[4 + b] += (int)((hi >> (8 * b)) & 255u);
+  }
+}
+
+#define TK_DIGITS_TRIM 96
+// Energy left without the TK_DIGITS_TRIM largest elements, in units of 2^(2E): band b counts at its
+// lower edge 2^(-4b-4). The grid does not carry the token when its rounding noise n_poor * 2^-62 / 3
+// exceeds 2^-30 of that -- or, where the call stands in for the reference's order (strict), 2^-42: amplitude 2^-21 = 4.8e-7,
+// while f32 sums over K >= 2560 in k order show 5.6e-7 and more against float64.
+__device__ __forceinline__ bool digits_narrow(int n_poor, const int (&bands)[8], bool strict = false) {
+  float left = 0.0f, edge2 = 0.00390625f;  // 2^-8
+  int trim = TK_DIGITS_TRIM;
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int c = bands[b], cut = c < trim ? c : trim;
+    trim -= cut;
+    left += (float)(c - cut) * edge2;
+    edge2 *= 0.00390625f;
+  }
+  return n_poor > 0 && (float)n_poor > 3.0f * (strict ? 1048576.0f : 4294967296.0f) * left;
+}
+
+// Float token -> four balanced base-256 digit rows of round(a * 2^(30-E)), 2^(E-1) <= max|a| < 2^E.
+// Scaling a float by a power of two is exact, so the rounding to an integer happens once, in
+// single precision. With q + 0x808080 the three lower bytes hold their digit plus 128 and the carries have gone on, so an
+// exclusive or with the same constant leaves the four digits as int8.
+//
+// Dynamic range. The grid is 2^(E-30) wide against the token's own maximum. An element that lies on
+// the grid exactly, or is at least 2^(E-15) in magnitude (rounding error at most 2^-16 of itself), is
+// carried faithfully; any other ("poor") element is rounded by up to 2^(E-31), which can be all of
+// it. The reference's k-ordered f32 fold skips an activation under a zero trit
+// (crates/tritium-core/src/reference.rs:42-51), so an output can miss the largest elements of a token
+// and consist of small ones only: its value is then small next to the token's maximum, and the
+// rounding of the poor elements shows. The prep therefore compares the rounding noise of a token,
+// n_poor * 2^(2(E-31)) / 3, with the energy that is left when its TK_DIGITS_TRIM largest elements
+// are all skipped (a lower bound from counts per 4-bit magnitude band below 2^E): where the noise
+// exceeds 2^-30 of that energy (2^-15 in amplitude, i.e. 3e-5 of a typical output that misses the
+// top elements), the token is flagged like one holding NaN or Inf and its outputs are computed in
+// the reference's order. For every other token and every output, unconditionally,
+//   |value - exact dot product| <= n * 2^(E-31)  (+ 1.5 ulp),  n = poor elements under its non-zero trits.
+// counts[0]: elements not carried faithfully; counts[1]: elements of `large` and more.
+__device__ __forceinline__ void split_piece(const float (&v)[16], int shift, float large, v4u (&piece)[4], int (&counts)[2]) {
+#pragma unroll
+  for (int sl = 0; sl < 4; ++sl) {
+    unsigned u[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const float r = ldexpf(v[sl * 4 + b], shift), t = rintf(r);  // |t| <= 2^30
+      const float small = __builtin_amdgcn_fmed3f(r, -large, large);  // (a large element becomes an integer)
+      counts[0] += (int)min(magnitude_bits(small - rintf(small)), 1u);
+      counts[1] += (int)((__float_as_uint(large) - 1u - magnitude_bits(r)) >> 31);
+      u[b] = ((unsigned)(int)t + 0x00808080u) ^ 0x00808080u;
+    }
+    const unsigned lo01 = __builtin_amdgcn_perm(u[1], u[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(u[1], u[0], 0x07030602u);
+    const unsigned lo23 = __builtin_amdgcn_perm(u[3], u[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(u[3], u[2], 0x07030602u);
+    piece[0][sl] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+    piece[1][sl] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+    piece[2][sl] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+    piece[3][sl] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+  }
+}
+__device__ __forceinline__ int piece_sum(const v4u &piece) {
+  int t = 0;
+#pragma unroll
+  for (int sl = 0; sl < 4; ++sl) t = __builtin_amdgcn_sdot4((int)piece[sl], 0x01010101, t, false);
+  return t;
+}
+// the grid of a row: shift = 30 - E (a row without a finite maximum splits zeros)
+__device__ __forceinline__ int grid_shift(float gamma, bool live) {
+  int E = 0;
+  if (live) (void)frexpf(gamma, &E);
+  return 30 - E;
+}
+// Whether the token is finished in the reference's order. The magnitude bands are needed only where the two counts do not answer
+// (the same in every thread of the team, so the barriers are reached by all or by none): an element of 2^15 and more lies in band 3
+// or above, so left >= (their number - TK_DIGITS_TRIM) * 2^-32 and 3 * 2^32 * left exceeds twice that number; strict, an element of 2^20
+// and more is of 2^-20 in energy (units of 2^(2E)). `each(f)` calls f with every piece of this thread.
+template <int TEAM, bool STRICT, typename E>
+__device__ __forceinline__ bool token_narrow(int poor, int large, int shift, TkPrepShared &sh, E &&each) {
+  if (poor == 0 || poor <= (STRICT ? 3 : 2) * (large - TK_DIGITS_TRIM)) return false;
+  int bands[8] = {};
+  each([&](const float (&p)[16]) { count_bands(p, shift, bands); });
+  team_sums<TEAM, 8>(bands, sh.bands);
+  return digits_narrow(poor, bands, STRICT);
+}
+
+// ---- kernels ----
+// Rows of any form: with an RMSNorm of a shape the one-pass kernel does not take, a row-major copy, or more pieces than a team holds
+// (re-read from memory for the quantization). HELD = pieces a thread keeps in registers where all fit.
+#define TK_PREP_HELD 4
+__global__ __launch_bounds__(TK_WG) void tk_prep_a8_kernel(TkPrep single, const TkPrep *__restrict__ table, int nprep, int uniform_m) {
+  __shared__ TkPrepShared sh;
+  int rowi;
+  const TkPrep &pp = find_prep(single, table, nprep, uniform_m, rowi);
   const size_t row = rowi, k = pp.k, nb = pp.nb, R = pp.rs;
   const size_t base = row * k;
   const void *act = pp.act;
   const int dtype = pp.act_dtype;
   int8_t *ap = pp.ap, *qrm = pp.q_rowmajor;
-  const bool vec = act_rows_vectorizable(dtype);
-  const size_t npieces = nb * 16;
-  float held[HELD][16];
+  RowNorm nm = {pp.norm_kind, 0.0f, pp.norm_w};
+  if (nm.kind) {
+    __shared__ float part[TK_WG];
+    nm.inv = row_inv_rms(act, dtype, base, k, pp.norm_eps, part);
+  }
+  const int npieces = (int)(nb * 16), tid = threadIdx.x;
+  const bool resident = !nm.kind && npieces <= TK_PREP_HELD * TK_WG;
+  float held[TK_PREP_HELD][16];
   float gamma;
-  int nonfinite;
-  wave_absmax_held<HELD, FAST, TEAM>(act, dtype, base, k, npieces, vec, lane, held, gamma, nonfinite, shf, shi);
-  const float s = gamma == 0.0f ? 0.0f : __fdiv_rn(127.0f, gamma);  // one divide
-  const bool live = gamma != 0.0f && !nonfinite;
-  int sum = 0;
-  if constexpr (FAST != 0) {
-    // a multiply by 0 stands in for the tests of `live` (a row without a finite maximum quantizes to zeros)
-    const float sl_ = live ? s : 0.0f;
-#pragma unroll
-    for (int it = 0; it < HELD; ++it) {
-      const size_t pc = (size_t)lane + (size_t)it * TEAM;
-      if (pc >= npieces) continue;
-      v4u piece;
-#pragma unroll
-      for (int sl = 0; sl < 4; ++sl) {
-        uint32_t packed = 0;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          float x = held[it][sl * 4 + b];
-          if (!live) x = 0.0f;  // (a NaN or Inf times zero would not be zero)
-          float r = rintf(__fmul_rn(x, sl_));  // one multiply, ties to even
-          r = __builtin_fminf(__builtin_fmaxf(r, -128.0f), 127.0f);
-          const int q = (int)r;
-          sum += q;
-          packed |= ((uint32_t)q & 0xFFu) << (8 * b);
-        }
-        piece[sl] = packed;
-      }
-      *(TK_GLOBAL v4u *)(ap + piece_offset(pc >> 4, (int)(pc & 15), R, row)) = piece;
-    }
-  } else
-#pragma unroll
-  for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * TEAM;
-    if (pc >= npieces) continue;
-    const size_t kb = pc >> 4;
-    const int q16 = (int)(pc & 15);
-    const size_t e0 = piece_elem0(kb, q16);
-    v4u piece;
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      const size_t e = e0 + (size_t)sl * 32;
-      uint32_t packed = 0;
+  bool nonfinite;
+  if (resident) {
+    load_held<TK_PREP_HELD, 0, TK_WG>(act, dtype, base, k, npieces, tid, held);
+    gamma = held_peak<TK_PREP_HELD, TK_WG>(held, nonfinite, sh.peak, sh.peak2);
+  } else {
+    unsigned m = 0, m2 = 0;  // of all elements, and of those that are not NaN
+    for (size_t e = (size_t)tid * 4; e < k; e += TK_WG * 4) {
+      float v[4];
+      load_act4(act, dtype, base, e, k, v);
+      apply_norm4(nm, e, k, v);
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        int q = 0;
-        if (live && e + b < k) {
-          float r = rintf(__fmul_rn(held[it][sl * 4 + b], s));  // one multiply, ties to even
-          r = r < -128.0f ? -128.0f : (r > 127.0f ? 127.0f : r);
-          q = (int)r;
-        }
-        sum += q;
-        packed |= ((uint32_t)q & 0xFFu) << (8 * b);
+        const unsigned u = magnitude_bits(v[b]);
+        m = max(m, u);
+        m2 = max(m2, u > TK_INF_BITS ? 0u : u);
       }
-      piece[sl] = packed;
-      if (qrm) {
-        if (vec && e + 4 <= k) {
+    }
+    nonfinite = team_max<TK_WG>(m, sh.peak) >= TK_INF_BITS;
+    gamma = __uint_as_float(team_max<TK_WG>(m2, sh.peak2));
+  }
+  const RowScale scale = row_scale(gamma, nonfinite);
+  float *ynorm = nm.kind && scale.exact ? pp.ynorm : nullptr;  // only the exact fallback reads the normalized row
+  int sum[1] = {0};
+  // quantize the 16 values of piece pc and store them in operand order (and row-major, if asked)
+  auto emit = [&](int pc, float (&v)[16]) {
+    const size_t e0 = piece_elem0((size_t)(pc >> 4), pc & 15);
+    if (ynorm) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        const size_t e = e0 + (size_t)(x >> 2) * 32 + (x & 3);
+        if (e < k) gstore(ynorm + base + e, v[x]);
+      }
+    }
+    if (scale.odd) odd_row(v, scale.odd);
+    const v4u piece = quantize_piece(v, scale, sum[0]);
+    if (qrm) {
+#pragma unroll
+      for (int sl = 0; sl < 4; ++sl) {
+        const size_t e = e0 + (size_t)sl * 32;
+        if (e + 4 <= k) {
           typedef uint32_t loose __attribute__((aligned(1)));
-          *(TK_GLOBAL loose *)(qrm + base + e) = packed;
+          *(TK_GLOBAL loose *)(qrm + base + e) = piece[sl];
         } else {
           for (int b = 0; b < 4; ++b)
-            if (e + b < k) qrm[base + e + b] = (int8_t)(packed >> (8 * b));
+            if (e + b < k) qrm[base + e + b] = (int8_t)(piece[sl] >> (8 * b));
         }
       }
     }
-    if (ap) *(TK_GLOBAL v4u *)(ap + piece_offset(kb, q16, R, row)) = piece;
+    if (ap) *(TK_GLOBAL v4u *)(ap + piece_offset((size_t)(pc >> 4), pc & 15, R, row)) = piece;
+  };
+  if (resident) {
+#pragma unroll
+    for (int it = 0; it < TK_PREP_HELD; ++it)
+      if (tid + it * TK_WG < npieces) emit(tid + it * TK_WG, held[it]);
+  } else {
+    for (int pc = tid; pc < npieces; pc += TK_WG) {
+      float v[16];
+      const size_t e0 = piece_elem0((size_t)(pc >> 4), pc & 15);
+      load_piece(act, dtype, base, e0, k, v);
+#pragma unroll
+      for (int sl = 0; sl < 4; ++sl) {
+        float t[4] = {v[sl * 4], v[sl * 4 + 1], v[sl * 4 + 2], v[sl * 4 + 3]};
+        apply_norm4(nm, e0 + (size_t)sl * 32, k, t);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) v[sl * 4 + b] = t[b];
+      }
+      emit(pc, v);
+    }
   }
-  if constexpr (TEAM == 64) sum = wave_sum(sum);
-  else sum = block_sum(sum, shi);
-  if (lane == 0) {
-    if (pp.rowsum) pp.rowsum[row] = sum;
-    pp.act_scale[row] = gamma == 0.0f ? 0.0f : __fdiv_rn(gamma, 127.0f);
-    if (pp.aux) pp.aux[row] = s;
-    if (pp.flags) pp.flags[row] = nonfinite ? 1u : 0u;
+  team_sums<TK_WG, 1>(sum, sh.sums);
+  if (tid == 0) {
+    if (pp.rowsum) pp.rowsum[row] = sum[0];
+    pp.act_scale[row] = gamma_over_127(gamma);
+    if (pp.aux) pp.aux[row] = scale.s;
+    if (pp.flags) pp.flags[row] = (ap ? scale.exact : nonfinite) ? 1u : 0u;  // (a row-major copy reports NaN and Inf)
   }
 }
 
-template <int HELD, int FAST = 0, int TEAM = 64>
+// The four digit rows of one piece in operand order, and the sums of its K block (the 16 pieces of a block sit in 16 consecutive
+// lanes): entry [kb][row] of blocksum, row stride = the operand row count.
+template <bool STRICT>
+__device__ __forceinline__ void emit_digits(const TkPrep &pp, size_t tok, int pc, const float (&v)[16], int shift, int (&sums)[4], int (&counts)[2]) {
+  v4u piece[4];
+  split_piece(v, shift, STRICT ? TK_DIGIT_STRICT : TK_DIGIT_LARGE, piece, counts);
+  v4i t;
+#pragma unroll
+  for (int dg = 0; dg < 4; ++dg) {
+    *(TK_GLOBAL v4u *)(pp.ap + piece_offset((size_t)(pc >> 4), pc & 15, pp.rs, tok * 4 + dg)) = piece[dg];
+    t[dg] = piece_sum(piece[dg]);
+    sums[dg] += t[dg];
+  }
+  if (pp.blocksum) {  // (uniform)
+#pragma unroll
+    for (int dg = 0; dg < 4; ++dg) t[dg] = row16_sum(t[dg]);
+    if ((pc & 15) == 0) *(TK_GLOBAL v4i *)(pp.blocksum + (size_t)(pc >> 4) * pp.R + tok * 4) = t;
+  }
+}
+
+// Rows of more pieces than a team holds: read twice. (STRICT: TkPrep.strict.)
+template <bool STRICT>
+__global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, const TkPrep *__restrict__ table, int nprep, int uniform_m) {
+  __shared__ TkPrepShared sh;
+  int rowi;
+  const TkPrep &pp = find_prep(single, table, nprep, uniform_m, rowi);
+  const size_t tok = rowi, k = pp.k, base = tok * k;
+  const int npieces = (int)(pp.nb * 16), tid = threadIdx.x;
+  auto each = [&](auto &&f) {
+    for (int pc = tid; pc < npieces; pc += TK_WG) {
+      float v[16];
+      load_piece(pp.act, pp.act_dtype, base, piece_elem0((size_t)(pc >> 4), pc & 15), k, v);
+      f(v);
+    }
+  };
+  unsigned m = 0;
+  each([&](const float (&v)[16]) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) m = max(m, magnitude_bits(v[x]));
+  });
+  m = team_max<TK_WG>(m, sh.peak);
+  const bool nonfinite = m >= TK_INF_BITS, live = m != 0 && !nonfinite;
+  const int shift = grid_shift(__uint_as_float(m), live);
+  int sums[4] = {}, counts[2] = {};
+  int pc = tid;
+  each([&](float (&v)[16]) {
+    if (!live) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) v[x] = 0.0f;
+    }
+    emit_digits<STRICT>(pp, tok, pc, v, shift, sums, counts);
+    pc += TK_WG;
+  });
+  int six[6] = {sums[0], sums[1], sums[2], sums[3], counts[0], counts[1]};
+  team_sums<TK_WG, 6>(six, sh.sums);
+  const bool narrow = token_narrow<TK_WG, STRICT>(six[4], six[5], shift, sh, each);
+  if (tid == 0) {
+    *(TK_GLOBAL v4i *)(pp.rowsum + tok * 4) = v4i{six[0], six[1], six[2], six[3]};
+    pp.exps[tok] = -shift;
+    pp.flags[tok] = (nonfinite || narrow) ? 1u : 0u;
+  }
+}
+
+// Rows whose pieces the threads working on a token keep in registers (HELD each). TEAM = 64: a wave per token, four tokens per
+// workgroup, no barrier. TEAM = 256: the workgroup per token, for launches of few tokens, whose time is one token's chain, and
+// for long rows. FAST: see load_held.
+template <int HELD, int FAST, int TEAM>
+__global__ __launch_bounds__(TK_WG) void tk_prep_a8_wave_kernel(TkPrep single, const TkPrep *__restrict__ table, int nprep,
+                                                                int uniform_m, unsigned rows) {
+  __shared__ TkPrepShared sh;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = TEAM == 64 ? (threadIdx.x & 63) : threadIdx.x;
+  int rowi, gt;
+  const TkPrep &pp = find_prep_wave(single, table, nprep, uniform_m, wave, rowi, gt, TEAM);
+  if ((unsigned)gt >= rows) return;  // (a whole team leaves together: the barriers below stay uniform)
+  const size_t row = rowi, k = pp.k;
+  const int npieces = (int)(pp.nb * 16);
+  float held[HELD][16];
+  load_held<HELD, FAST, TEAM>(pp.act, pp.act_dtype, row * k, k, npieces, lane, held);
+  bool nonfinite;
+  const float gamma = held_peak<HELD, TEAM>(held, nonfinite, sh.peak, sh.peak2);
+  const RowScale scale = row_scale(gamma, nonfinite);
+  if (scale.odd) {
+#pragma unroll
+    for (int it = 0; it < HELD; ++it) odd_row(held[it], scale.odd);
+  }
+  int sum[1] = {0};
+#pragma unroll
+  for (int it = 0; it < HELD; ++it) {
+    const int pc = lane + it * TEAM;
+    if (pc < npieces) *(TK_GLOBAL v4u *)(pp.ap + piece_offset((size_t)(pc >> 4), pc & 15, pp.rs, row)) = quantize_piece(held[it], scale, sum[0]);
+  }
+  team_sums<TEAM, 1>(sum, sh.sums);
+  if (lane == 0) {
+    if (pp.rowsum) pp.rowsum[row] = sum[0];
+    pp.act_scale[row] = gamma_over_127(gamma);
+    if (pp.aux) pp.aux[row] = scale.s;
+    if (pp.flags) pp.flags[row] = scale.exact ? 1u : 0u;
+  }
+}
+
+template <int HELD, int FAST, int TEAM, bool STRICT = false>
 __global__ __launch_bounds__(TK_WG) void tk_prep_digits_wave_kernel(TkPrep single, const TkPrep *__restrict__ table,
                                                                     int nprep, int uniform_m, unsigned rows) {
-  __shared__ float shf[4];
-  __shared__ int shi[32];
-  const int wave = threadIdx.x >> 6, lane = TEAM == 64 ? (threadIdx.x & 63) : threadIdx.x;
+  __shared__ TkPrepShared sh;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = TEAM == 64 ? (threadIdx.x & 63) : threadIdx.x;
   int rowi, gt;
   const TkPrep &pp = find_prep_wave(single, table, nprep, uniform_m, wave, rowi, gt, TEAM);
   if ((unsigned)gt >= rows) return;
-  const size_t tok = rowi, k = pp.k, nb = pp.nb, R = pp.rs;
-  const size_t base = tok * k;
-  const void *act = pp.act;
-  const int dtype = pp.act_dtype;
-  int8_t *ap = pp.ap;
-  const bool vec = act_rows_vectorizable(dtype);
-  const size_t npieces = nb * 16;
+  const size_t tok = rowi, k = pp.k;
+  const int npieces = (int)(pp.nb * 16);
   float held[HELD][16];
-  float gamma;
-  int nonfinite;
-  wave_absmax_held<HELD, FAST, TEAM>(act, dtype, base, k, npieces, vec, lane, held, gamma, nonfinite, shf, shi);
-  int E = 0;
-  if (gamma != 0.0f && !nonfinite) (void)frexpf(gamma, &E);
-  const int shift = 30 - E;
-  const bool live = gamma != 0.0f && !nonfinite;
-  int sums[4] = {0, 0, 0, 0}, n_poor = 0;
+  load_held<HELD, FAST, TEAM>(pp.act, pp.act_dtype, tok * k, k, npieces, lane, held);
+  unsigned m = 0;
+#pragma unroll
+  for (int it = 0; it < HELD; ++it)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) m = max(m, magnitude_bits(held[it][x]));
+  m = team_max<TEAM>(m, sh.peak);
+  const bool nonfinite = m >= TK_INF_BITS, live = m != 0 && !nonfinite;
+  if (!live) {
+#pragma unroll
+    for (int it = 0; it < HELD; ++it)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) held[it][x] = 0.0f;
+  }
+  const int shift = grid_shift(__uint_as_float(m), live);
+  int sums[4] = {}, counts[2] = {};
 #pragma unroll
   for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * TEAM;
-    if (pc >= npieces) continue;
-    const size_t kb = pc >> 4;
-    const int q16 = (int)(pc & 15);
-    const size_t e0 = piece_elem0(kb, q16);
-    v4u piece[4];
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      const size_t e = e0 + (size_t)sl * 32;
-      uint32_t packed[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        int q = 0;
-        if constexpr (FAST != 0) {  // every element is inside the row; a row without a finite maximum splits zeros
-          const float r = ldexpf(live ? held[it][sl * 4 + b] : 0.0f, shift);
-          q = __float2int_rn(r);  // |q| <= 2^30
-          n_poor += digit_poor(r, q) ? 1 : 0;
-        } else if (live && e + b < k) {
-          const float r = ldexpf(held[it][sl * 4 + b], shift);
-          q = __float2int_rn(r);  // |q| <= 2^30
-          n_poor += digit_poor(r, q) ? 1 : 0;
-        }
-#pragma unroll
-        for (int dg = 0; dg < 4; ++dg) {
-          int dv = dg == 3 ? q : (((q + 128) & 0xFF) - 128);  // balanced digit in [-128,127]
-          q = (q - dv) >> 8;
-          sums[dg] += dv;
-          packed[dg] |= ((uint32_t)dv & 0xFFu) << (8 * b);
-        }
-      }
-#pragma unroll
-      for (int dg = 0; dg < 4; ++dg) piece[dg][sl] = packed[dg];
-    }
-#pragma unroll
-    for (int dg = 0; dg < 4; ++dg) *(TK_GLOBAL v4u *)(ap + piece_offset(kb, q16, R, tok * 4 + dg)) = piece[dg];
+    const int pc = lane + it * TEAM;
+    if (pc < npieces) emit_digits<STRICT>(pp, tok, pc, held[it], shift, sums, counts);
   }
-  if constexpr (TEAM == 64) {
+  int six[6] = {sums[0], sums[1], sums[2], sums[3], counts[0], counts[1]};
+  team_sums<TEAM, 6>(six, sh.sums);
+  const bool narrow = token_narrow<TEAM, STRICT>(six[4], six[5], shift, sh, [&](auto &&f) {
 #pragma unroll
-    for (int dg = 0; dg < 4; ++dg) sums[dg] = wave_sum(sums[dg]);
-    n_poor = wave_sum(n_poor);
-  } else {
-    int five[5] = {sums[0], sums[1], sums[2], sums[3], n_poor};
-    block_sums<5>(five, shi);
-#pragma unroll
-    for (int dg = 0; dg < 4; ++dg) sums[dg] = five[dg];
-    n_poor = five[4];
-  }
-  bool narrow = false;
-  if (n_poor > 0) {  // uniform over the team
-    int bands[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int it = 0; it < HELD; ++it) {
-      const size_t pc = (size_t)lane + (size_t)it * TEAM;
-      if (pc < npieces) count_bands(held[it], shift, bands);
-    }
-    if constexpr (TEAM == 64) {
-#pragma unroll
-      for (int b = 0; b < 8; ++b) bands[b] = wave_sum(bands[b]);
-    } else {
-      block_sums<8>(bands, shi);
-    }
-    narrow = digits_narrow(n_poor, bands);
-  }
-  if (lane < 4) pp.rowsum[tok * 4 + lane] = lane == 0 ? sums[0] : lane == 1 ? sums[1] : lane == 2 ? sums[2] : sums[3];
+    for (int it = 0; it < HELD; ++it)
+      if (lane + it * TEAM < npieces) f(held[it]);
+  });
   if (lane == 0) {
+    *(TK_GLOBAL v4i *)(pp.rowsum + tok * 4) = v4i{six[0], six[1], six[2], six[3]};
     pp.exps[tok] = -shift;
     pp.flags[tok] = (nonfinite || narrow) ? 1u : 0u;
   }
@@ -2259,24 +2203,19 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_wave_kernel(TkPrep singl
 // xs and part are free again on return.
 template <int HELD>
 __device__ __forceinline__ void norm_held_pieces(float (&held)[HELD][16], const float *norm_w, int norm_kind, float eps,
-                                                 size_t k, size_t npieces, float *xs, float *part) {
+                                                 size_t k, int npieces, float *xs, float *part) {
   const int tid = threadIdx.x;
   float w[HELD][16];
+  load_held<HELD, 1, TK_WG>(norm_w, 0, 0, k, npieces, tid, w);
 #pragma unroll
   for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)tid + (size_t)it * TK_WG;
+    const int pc = tid + it * TK_WG;
     if (pc >= npieces) continue;
-    const size_t e0 = piece_elem0(pc >> 4, (int)(pc & 15));
+    const size_t e0 = piece_elem0((size_t)(pc >> 4), pc & 15);
 #pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      const v4u u = *(const TK_GLOBAL v4u *)(norm_w + e0 + (size_t)sl * 32);
-      w[it][sl * 4 + 0] = __uint_as_float(u.x);
-      w[it][sl * 4 + 1] = __uint_as_float(u.y);
-      w[it][sl * 4 + 2] = __uint_as_float(u.z);
-      w[it][sl * 4 + 3] = __uint_as_float(u.w);
+    for (int sl = 0; sl < 4; ++sl)
       *(float4 *)(xs + e0 + (size_t)sl * 32) =
           make_float4(held[it][sl * 4], held[it][sl * 4 + 1], held[it][sl * 4 + 2], held[it][sl * 4 + 3]);
-    }
   }
   __syncthreads();
   float acc = 0.0f;
@@ -2319,190 +2258,133 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_a8_norm_kernel(TkPrep single, c
   static_assert(TK_WG == 256, "the canonical reduction has 256 slots");
   __shared__ __attribute__((aligned(16))) float xs[HELD * 256 * 16];
   __shared__ float part[TK_WG];
-  __shared__ float shf[4];
-  __shared__ int shi[4];
+  __shared__ TkPrepShared sh;
   int rowi;
   const TkPrep &pp = find_prep(single, table, nprep, uniform_m, rowi);
-  const size_t row = rowi, k = pp.k, nb = pp.nb, R = pp.rs;
-  const size_t base = row * k, npieces = nb * 16;
-  const int tid = threadIdx.x;
+  const size_t row = rowi, k = pp.k, base = row * k;
+  const int npieces = (int)(pp.nb * 16), tid = threadIdx.x;
   float held[HELD][16];
-#pragma unroll
-  for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)tid + (size_t)it * TK_WG;
-    if (pc < npieces) load_piece_fast<FAST>(pp.act, base, piece_elem0(pc >> 4, (int)(pc & 15)), held[it]);
-  }
+  load_held<HELD, FAST, TK_WG>(pp.act, 0, base, k, npieces, tid, held);
   if (pp.norm_kind) norm_held_pieces<HELD>(held, pp.norm_w, pp.norm_kind, pp.norm_eps, k, npieces, xs, part);  // uniform over the workgroup
-  float g = 0.0f;
-  int nf = 0;
+  bool nonfinite;
+  const float gamma = held_peak<HELD, TK_WG>(held, nonfinite, sh.peak, sh.peak2);
+  const RowScale scale = row_scale(gamma, nonfinite);
+  if (pp.norm_kind && scale.exact) {  // only the exact fallback reads the normalized row
 #pragma unroll
-  for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)tid + (size_t)it * TK_WG;
-    if (pc >= npieces) continue;
+    for (int it = 0; it < HELD; ++it) {
+      const int pc = tid + it * TK_WG;
+      if (pc >= npieces) continue;
+      const size_t e0 = piece_elem0((size_t)(pc >> 4), pc & 15);
 #pragma unroll
-    for (int x = 0; x < 16; ++x) {
-      const float a = fabsf(held[it][x]);
-      if (a > g) g = a;  // NaN never wins (crates/tritium-spec/src/lib.rs:351-360)
-      nf |= !(a <= 3.402823466e38f);
+      for (int x = 0; x < 16; ++x) gstore(pp.ynorm + base + e0 + (size_t)(x >> 2) * 32 + (x & 3), held[it][x]);
     }
   }
-  block_max_any(g, nf, shf, shi);
-  const float gamma = g;
-  const bool nonfinite = nf != 0;
-  const float s = gamma == 0.0f ? 0.0f : __fdiv_rn(127.0f, gamma);  // one divide
-  const bool live = gamma != 0.0f && !nonfinite;
-  const float sl_ = live ? s : 0.0f;
-  float *ynorm = (pp.norm_kind && nonfinite) ? pp.ynorm : nullptr;  // only the exact fallback reads the normalized row
-  int sum = 0;
+  if (scale.odd) {
+#pragma unroll
+    for (int it = 0; it < HELD; ++it) odd_row(held[it], scale.odd);
+  }
+  int sum[1] = {0};
 #pragma unroll
   for (int it = 0; it < HELD; ++it) {
-    const size_t pc = (size_t)tid + (size_t)it * TK_WG;
-    if (pc >= npieces) continue;
-    const size_t e0 = piece_elem0(pc >> 4, (int)(pc & 15));
-    v4u piece;
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      if (ynorm) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) gstore(ynorm + base + e0 + (size_t)sl * 32 + b, held[it][sl * 4 + b]);
-      }
-      uint32_t packed = 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        float x = held[it][sl * 4 + b];
-        if (!live) x = 0.0f;  // (a NaN or Inf times zero would not be zero)
-        float r = rintf(__fmul_rn(x, sl_));  // one multiply, ties to even
-        r = __builtin_fminf(__builtin_fmaxf(r, -128.0f), 127.0f);
-        const int q = (int)r;
-        sum += q;
-        packed |= ((uint32_t)q & 0xFFu) << (8 * b);
-      }
-      piece[sl] = packed;
-    }
-    *(TK_GLOBAL v4u *)(pp.ap + piece_offset(pc >> 4, (int)(pc & 15), R, row)) = piece;
+    const int pc = tid + it * TK_WG;
+    if (pc < npieces) *(TK_GLOBAL v4u *)(pp.ap + piece_offset((size_t)(pc >> 4), pc & 15, pp.rs, row)) = quantize_piece(held[it], scale, sum[0]);
   }
-  sum = block_sum(sum, shi);
+  team_sums<TK_WG, 1>(sum, sh.sums);
   if (tid == 0) {
-    if (pp.rowsum) pp.rowsum[row] = sum;
-    pp.act_scale[row] = gamma == 0.0f ? 0.0f : __fdiv_rn(gamma, 127.0f);
-    if (pp.aux) pp.aux[row] = s;
-    if (pp.flags) pp.flags[row] = nonfinite ? 1u : 0u;
+    if (pp.rowsum) pp.rowsum[row] = sum[0];
+    pp.act_scale[row] = gamma_over_127(gamma);
+    if (pp.aux) pp.aux[row] = scale.s;
+    if (pp.flags) pp.flags[row] = scale.exact ? 1u : 0u;
   }
 }
 
 // ------------------------------------------------------------------------------------------
-// Decode in one launch: the flow kernel builds the operand rows of its one to four tokens itself. Every workgroup
+// Decode in one launch: the decode kernel builds the operand rows of its one to four tokens itself. Every workgroup
 // repeats the prep kernels' work for all tokens -- a few elements per thread -- in place of a second launch in
-// front of every call, which costs more than the kernel itself on a single layer. The arithmetic is that of
-// tk_prep_a8_wave_kernel / tk_prep_digits_wave_kernel in their straight-line form with the workgroup as the team
-// (whole K blocks, 16-byte aligned rows of f32 or bf16, at most two pieces per thread of the 256), statement for
-// statement, so rows, row sums, scales, exponents and flags carry the same bits. They go to LDS: the rows in
+// front of every call, which costs more than the kernel itself on a single layer. The pieces are made by the functions of the
+// prep kernels with the workgroup as the team (whole K blocks, 16-byte aligned rows of f32 or bf16, at most two pieces per thread
+// of the 256), so rows, row sums, scales, exponents and flags carry the same bits. They go to LDS: the rows in
 // operand order at `rows`, the constants at `cst` (int rowsum[64] | float scale or int exponent [64] |
-// uint flag[64] | float 127/gamma [64]).
+// uint flag[64] | float 127/gamma [64]). The tokens are taken one after the other (a version with the loads and reductions of
+// four tokens at once was slower for one token and no faster for four).
 // ------------------------------------------------------------------------------------------
-// The tokens are taken one after the other (a version with the loads and reductions of four tokens at once was
-// slower for one token and no faster for four: the kernel's code grows fourfold, and what a token costs is its
-// arithmetic, about 25 instructions per element under the float contract, repeated by every workgroup).
 #define TK_FUSED_HELD 2
-template <int FAST>
-__device__ __forceinline__ void fused_token_a8(const void *act, int tok, size_t k, size_t nb, size_t R, uint4 *rows,
-                                               uint8_t *cst, float *shf, int *shi) {
+// quantize the held pieces of a token into `rows` and leave its constants
+__device__ __forceinline__ void fused_emit_a8(float (&held)[TK_FUSED_HELD][16], float gamma, const RowScale &scale, int tok, int npieces,
+                                              size_t R, uint4 *rows, uint8_t *cst, TkPrepShared &sh) {
   const int lane = threadIdx.x;
-  const size_t npieces = nb * 16, base = (size_t)tok * k;
-  float held[TK_FUSED_HELD][16];
-  float gamma;
-  int nonfinite;
-  wave_absmax_held<TK_FUSED_HELD, FAST, 256>(act, 0, base, k, npieces, true, lane, held, gamma, nonfinite, shf, shi);
-  const float s = gamma == 0.0f ? 0.0f : __fdiv_rn(127.0f, gamma);  // one divide
-  const bool live = gamma != 0.0f && !nonfinite;
-  const float sl_ = live ? s : 0.0f;
-  int sum = 0;
+  if (scale.odd) {
+#pragma unroll
+    for (int it = 0; it < TK_FUSED_HELD; ++it) odd_row(held[it], scale.odd);
+  }
+  int sum[1] = {0};
 #pragma unroll
   for (int it = 0; it < TK_FUSED_HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * 256;
-    if (pc >= npieces) continue;
-    uint4 piece;
-    uint32_t *pw = (uint32_t *)&piece;
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      uint32_t packed = 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        float x = held[it][sl * 4 + b];
-        if (!live) x = 0.0f;  // (a NaN or Inf times zero would not be zero)
-        float r = rintf(__fmul_rn(x, sl_));  // one multiply, ties to even
-        r = __builtin_fminf(__builtin_fmaxf(r, -128.0f), 127.0f);
-        const int q = (int)r;
-        sum += q;
-        packed |= ((uint32_t)q & 0xFFu) << (8 * b);
-      }
-      pw[sl] = packed;
-    }
-    rows[piece_offset(pc >> 4, (int)(pc & 15), R, (size_t)tok) >> 4] = piece;
+    const int pc = lane + it * 256;
+    if (pc < npieces) *(v4u *)&rows[piece_offset((size_t)(pc >> 4), pc & 15, R, (size_t)tok) >> 4] = quantize_piece(held[it], scale, sum[0]);
   }
-  sum = block_sum(sum, shi);
+  team_sums<256, 1>(sum, sh.sums);
   if (lane == 0) {
-    ((int *)cst)[tok] = sum;
-    ((float *)(cst + 256))[tok] = gamma == 0.0f ? 0.0f : __fdiv_rn(gamma, 127.0f);
-    ((uint32_t *)(cst + 512))[tok] = nonfinite ? 1u : 0u;
-    ((float *)(cst + 768))[tok] = s;
+    ((int *)cst)[tok] = sum[0];
+    ((float *)(cst + 256))[tok] = gamma_over_127(gamma);
+    ((uint32_t *)(cst + 512))[tok] = scale.exact ? 1u : 0u;
+    ((float *)(cst + 768))[tok] = scale.s;
   }
+}
+
+template <int FAST>
+__device__ __forceinline__ void fused_token_a8(const void *act, int tok, size_t k, size_t nb, size_t R, uint4 *rows,
+                                               uint8_t *cst, TkPrepShared &sh) {
+  const int npieces = (int)(nb * 16);
+  float held[TK_FUSED_HELD][16];
+  load_held<TK_FUSED_HELD, FAST, 256>(act, 0, (size_t)tok * k, k, npieces, threadIdx.x, held);
+  bool nonfinite;
+  const float gamma = held_peak<TK_FUSED_HELD, 256>(held, nonfinite, sh.peak, sh.peak2);
+  fused_emit_a8(held, gamma, row_scale(gamma, nonfinite), tok, npieces, R, rows, cst, sh);
 }
 
 template <int FAST>
 __device__ __forceinline__ void fused_token_digits(const void *act, int tok, size_t k, size_t nb, size_t R, uint4 *rows,
-                                                   uint8_t *cst, float *shf, int *shi) {
-  const int lane = threadIdx.x;
-  const size_t npieces = nb * 16, base = (size_t)tok * k;
+                                                   uint8_t *cst, TkPrepShared &sh) {
+  const int lane = threadIdx.x, npieces = (int)(nb * 16);
   float held[TK_FUSED_HELD][16];
-  float gamma;
-  int nonfinite;
-  wave_absmax_held<TK_FUSED_HELD, FAST, 256>(act, 0, base, k, npieces, true, lane, held, gamma, nonfinite, shf, shi);
-  int E = 0;
-  if (gamma != 0.0f && !nonfinite) (void)frexpf(gamma, &E);
-  const int shift = 30 - E;
-  const bool live = gamma != 0.0f && !nonfinite;
-  int five[5] = {0, 0, 0, 0, 0};  // four digit-row sums, poor elements
+  load_held<TK_FUSED_HELD, FAST, 256>(act, 0, (size_t)tok * k, k, npieces, lane, held);
+  unsigned m = 0;
+#pragma unroll
+  for (int it = 0; it < TK_FUSED_HELD; ++it)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) m = max(m, magnitude_bits(held[it][x]));
+  m = team_max<256>(m, sh.peak);
+  const bool nonfinite = m >= TK_INF_BITS, live = m != 0 && !nonfinite;
+  if (!live) {
+#pragma unroll
+    for (int it = 0; it < TK_FUSED_HELD; ++it)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) held[it][x] = 0.0f;
+  }
+  const int shift = grid_shift(__uint_as_float(m), live);
+  int six[6] = {}, counts[2] = {};  // four digit-row sums and the two counts
 #pragma unroll
   for (int it = 0; it < TK_FUSED_HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * 256;
+    const int pc = lane + it * 256;
     if (pc >= npieces) continue;
-    uint4 piece[4];
+    v4u piece[4];
+    split_piece(held[it], shift, TK_DIGIT_LARGE, piece, counts);
 #pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      uint32_t packed[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const float r = ldexpf(live ? held[it][sl * 4 + b] : 0.0f, shift);
-        int q = __float2int_rn(r);  // |q| <= 2^30
-        five[4] += digit_poor(r, q) ? 1 : 0;
-#pragma unroll
-        for (int dg = 0; dg < 4; ++dg) {
-          int dv = dg == 3 ? q : (((q + 128) & 0xFF) - 128);  // balanced digit in [-128,127]
-          q = (q - dv) >> 8;
-          five[dg] += dv;
-          packed[dg] |= ((uint32_t)dv & 0xFFu) << (8 * b);
-        }
-      }
-#pragma unroll
-      for (int dg = 0; dg < 4; ++dg) ((uint32_t *)&piece[dg])[sl] = packed[dg];
+    for (int dg = 0; dg < 4; ++dg) {
+      *(v4u *)&rows[piece_offset((size_t)(pc >> 4), pc & 15, R, (size_t)tok * 4 + dg) >> 4] = piece[dg];
+      six[dg] += piece_sum(piece[dg]);
     }
-#pragma unroll
-    for (int dg = 0; dg < 4; ++dg) rows[piece_offset(pc >> 4, (int)(pc & 15), R, (size_t)tok * 4 + dg) >> 4] = piece[dg];
   }
-  block_sums<5>(five, shi);
-  bool narrow = false;
-  if (five[4] > 0) {  // uniform over the workgroup
-    int bands[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  six[4] = counts[0];
+  six[5] = counts[1];
+  team_sums<256, 6>(six, sh.sums);
+  const bool narrow = token_narrow<256, false>(six[4], six[5], shift, sh, [&](auto &&f) {
 #pragma unroll
-    for (int it = 0; it < TK_FUSED_HELD; ++it) {
-      const size_t pc = (size_t)lane + (size_t)it * 256;
-      if (pc < npieces) count_bands(held[it], shift, bands);
-    }
-    block_sums<8>(bands, shi);
-    narrow = digits_narrow(five[4], bands);
-  }
-  if (lane < 4) ((int *)cst)[tok * 4 + lane] = lane == 0 ? five[0] : lane == 1 ? five[1] : lane == 2 ? five[2] : five[3];
+    for (int it = 0; it < TK_FUSED_HELD; ++it)
+      if (lane + it * 256 < npieces) f(held[it]);
+  });
+  if (lane < 4) ((int *)cst)[tok * 4 + lane] = lane == 0 ? six[0] : lane == 1 ? six[1] : lane == 2 ? six[2] : six[3];
   if (lane == 0) {
     ((int *)(cst + 256))[tok] = -shift;
     ((uint32_t *)(cst + 512))[tok] = (nonfinite || narrow) ? 1u : 0u;
@@ -2512,77 +2394,36 @@ __device__ __forceinline__ void fused_token_digits(const void *act, int tok, siz
 // One token whose quantization has an RMSNorm in front (the int8 contract): xs [k] and part [256] floats of LDS lie
 // behind the row constants. A normalized row that holds NaN or Inf stays in xs, where the exact fallback reads it.
 template <int FAST>
-__device__ __forceinline__ void fused_token_a8_normed(const TkProblem &pr, uint4 *rows, uint8_t *cst, float *shf, int *shi) {
+__device__ __forceinline__ void fused_token_a8_normed(const TkProblem &pr, uint4 *rows, uint8_t *cst, TkPrepShared &sh) {
   const int lane = threadIdx.x;
-  const size_t k = (size_t)pr.k, nb = (size_t)pr.nb, R = (size_t)pr.R, npieces = nb * 16;
+  const size_t k = (size_t)pr.k;
+  const int npieces = pr.nb * 16;
   float *xs = (float *)(cst + 1024), *part = xs + k;
   float held[TK_FUSED_HELD][16];
-#pragma unroll
-  for (int it = 0; it < TK_FUSED_HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * 256;
-    if (pc < npieces) load_piece_fast<FAST>(pr.raw_act, 0, piece_elem0(pc >> 4, (int)(pc & 15)), held[it]);
-  }
+  load_held<TK_FUSED_HELD, FAST, 256>(pr.raw_act, 0, 0, k, npieces, lane, held);
   norm_held_pieces<TK_FUSED_HELD>(held, pr.norm_w, pr.norm_kind, pr.norm_eps, k, npieces, xs, part);
-  float gamma = 0.0f;
-  int nonfinite = 0;
+  bool nonfinite;
+  const float gamma = held_peak<TK_FUSED_HELD, 256>(held, nonfinite, sh.peak, sh.peak2);
+  const RowScale scale = row_scale(gamma, nonfinite);
+  if (scale.exact) {  // uniform
 #pragma unroll
-  for (int it = 0; it < TK_FUSED_HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * 256;
-    if (pc >= npieces) continue;
+    for (int it = 0; it < TK_FUSED_HELD; ++it) {
+      const int pc = lane + it * 256;
+      if (pc >= npieces) continue;
+      const size_t e0 = piece_elem0((size_t)(pc >> 4), pc & 15);
 #pragma unroll
-    for (int x = 0; x < 16; ++x) {
-      const float a = fabsf(held[it][x]);
-      if (a > gamma) gamma = a;  // NaN never wins (crates/tritium-spec/src/lib.rs:351-360)
-      nonfinite |= !(a <= 3.402823466e38f);
+      for (int sl = 0; sl < 4; ++sl)
+        *(float4 *)(xs + e0 + (size_t)sl * 32) = make_float4(held[it][sl * 4], held[it][sl * 4 + 1], held[it][sl * 4 + 2], held[it][sl * 4 + 3]);
     }
   }
-  block_max_any(gamma, nonfinite, shf, shi);
-  const float s = gamma == 0.0f ? 0.0f : __fdiv_rn(127.0f, gamma);  // one divide
-  const bool live = gamma != 0.0f && !nonfinite;
-  const float sl_ = live ? s : 0.0f;
-  int sum = 0;
-#pragma unroll
-  for (int it = 0; it < TK_FUSED_HELD; ++it) {
-    const size_t pc = (size_t)lane + (size_t)it * 256;
-    if (pc >= npieces) continue;
-    const size_t e0 = piece_elem0(pc >> 4, (int)(pc & 15));
-    uint4 piece;
-    uint32_t *pw = (uint32_t *)&piece;
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      if (nonfinite)  // uniform
-        *(float4 *)(xs + e0 + (size_t)sl * 32) =
-            make_float4(held[it][sl * 4], held[it][sl * 4 + 1], held[it][sl * 4 + 2], held[it][sl * 4 + 3]);
-      uint32_t packed = 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        float x = held[it][sl * 4 + b];
-        if (!live) x = 0.0f;  // (a NaN or Inf times zero would not be zero)
-        float r = rintf(__fmul_rn(x, sl_));  // one multiply, ties to even
-        r = __builtin_fminf(__builtin_fmaxf(r, -128.0f), 127.0f);
-        const int q = (int)r;
-        sum += q;
-        packed |= ((uint32_t)q & 0xFFu) << (8 * b);
-      }
-      pw[sl] = packed;
-    }
-    rows[piece_offset(pc >> 4, (int)(pc & 15), R, 0) >> 4] = piece;
-  }
-  sum = block_sum(sum, shi);
-  if (lane == 0) {
-    ((int *)cst)[0] = sum;
-    ((float *)(cst + 256))[0] = gamma == 0.0f ? 0.0f : __fdiv_rn(gamma, 127.0f);
-    ((uint32_t *)(cst + 512))[0] = nonfinite ? 1u : 0u;
-    ((float *)(cst + 768))[0] = s;
-  }
+  fused_emit_a8(held, gamma, scale, 0, npieces, (size_t)pr.R, rows, cst, sh);
 }
 
 __device__ __forceinline__ void fused_stage_rows(const TkProblem &pr, uint4 *rows, uint8_t *cst) {
-  __shared__ float shf[4];
-  __shared__ int shi[32];
+  __shared__ TkPrepShared sh;
   if (pr.norm_kind) {  // (one token under the int8 contract: the host's rule)
-    if (pr.raw_dtype == TK_BF16) fused_token_a8_normed<2>(pr, rows, cst, shf, shi);
-    else fused_token_a8_normed<1>(pr, rows, cst, shf, shi);
+    if (pr.raw_dtype == TK_BF16) fused_token_a8_normed<2>(pr, rows, cst, sh);
+    else fused_token_a8_normed<1>(pr, rows, cst, sh);
     __syncthreads();
     return;
   }
@@ -2592,11 +2433,11 @@ __device__ __forceinline__ void fused_stage_rows(const TkProblem &pr, uint4 *row
   const bool bf16 = pr.raw_dtype == TK_BF16;
   for (int tok = 0; tok < M; ++tok) {
     if (pr.mode == TK_MODE_INT8) {
-      if (bf16) fused_token_a8<2>(act, tok, k, nb, R, rows, cst, shf, shi);
-      else fused_token_a8<1>(act, tok, k, nb, R, rows, cst, shf, shi);
+      if (bf16) fused_token_a8<2>(act, tok, k, nb, R, rows, cst, sh);
+      else fused_token_a8<1>(act, tok, k, nb, R, rows, cst, sh);
     } else {
-      if (bf16) fused_token_digits<2>(act, tok, k, nb, R, rows, cst, shf, shi);
-      else fused_token_digits<1>(act, tok, k, nb, R, rows, cst, shf, shi);
+      if (bf16) fused_token_digits<2>(act, tok, k, nb, R, rows, cst, sh);
+      else fused_token_digits<1>(act, tok, k, nb, R, rows, cst, sh);
     }
   }
   __syncthreads();
@@ -2647,7 +2488,7 @@ __device__ __forceinline__ void exact_rows_fused(const TkProblem &pr, int n, int
 // Already-quantized int8 rows -> operand order + row sums.
 __global__ __launch_bounds__(TK_WG) void tk_prep_i8_kernel(TkPrep single, const TkPrep *__restrict__ table,
                                                            int nprep, int uniform_m) {
-  __shared__ int shi[4];
+  __shared__ int sh[4];
   int rowi;
   const TkPrep &pp = find_prep(single, table, nprep, uniform_m, rowi);
   const size_t row = rowi, k = pp.k, nb = pp.nb, R = pp.rs;
@@ -2655,7 +2496,7 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_i8_kernel(TkPrep single, const 
   int8_t *ap = pp.ap;
   const size_t base = row * k;
   const bool vec = (k & 3) == 0 && (((size_t)q) & 3) == 0;
-  int sum = 0;
+  int sum[1] = {0};
   for (size_t pc = threadIdx.x; pc < nb * 16; pc += TK_WG) {
     const size_t kb = pc >> 4;
     const int q16 = (int)(pc & 15);
@@ -2671,13 +2512,13 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_i8_kernel(TkPrep single, const 
         for (int b = 0; b < 4; ++b)
           if (e + b < k) packed |= ((uint32_t)q[base + e + b] & 0xFFu) << (8 * b);
       }
-      sum += (int)(int8_t)(packed) + (int)(int8_t)(packed >> 8) + (int)(int8_t)(packed >> 16) + (int)(int8_t)(packed >> 24);
+      sum[0] = __builtin_amdgcn_sdot4((int)packed, 0x01010101, sum[0], false);
       piece[sl] = packed;
     }
     *(TK_GLOBAL v4u *)(ap + piece_offset(kb, q16, R, row)) = piece;
   }
-  sum = block_sum(sum, shi);
-  if (threadIdx.x == 0) pp.rowsum[row] = sum;
+  team_sums<TK_WG, 1>(sum, sh);
+  if (threadIdx.x == 0) pp.rowsum[row] = sum[0];
 }
 
 // One wave per 1-KiB chunk of a re-laid-out plane: the chunk is zero when all of its bytes are 0x55
@@ -2744,7 +2585,7 @@ hipError_t tk_launch_decode_trits(hipStream_t s, const uint8_t *codes, size_t n,
 static int g_prep_team_rows = 384;
 void tk_prep_set_team_rows(int rows) { g_prep_team_rows = rows < 0 ? 0 : rows; }
 int tk_prep_fast(const TkPrep &pp) {
-  const bool ok = pp.k % 256 == 0 && (((size_t)pp.act) & 15) == 0 && pp.ap && !pp.q_rowmajor && !pp.norm_kind && !pp.blocksum;
+  const bool ok = pp.k % 256 == 0 && (((size_t)pp.act) & 15) == 0 && pp.ap && !pp.q_rowmajor && !pp.norm_kind;
   if (!ok) return 0;
   return pp.act_dtype == TK_F32 ? 1 : (pp.act_dtype == TK_BF16 ? 2 : 0);
 }
@@ -2776,47 +2617,43 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
     }
     return hipGetLastError();
   }
-  // Rows that need neither a norm nor per-block sums, whose pieces the threads working on a token can keep
-  // in registers. Team = the threads of one token: a wave (four tokens per workgroup, no barrier), up to 4
-  // pieces per lane (K <= 4096) or 8 in the straight-line form (whole K blocks, aligned rows of one element
-  // type, operand rows only), whose registers hold little else; or, in the straight-line form, the whole
-  // workgroup (up to 8 pieces per thread: K <= 32768), where few tokens make the launch one token's chain of
-  // instructions (g_prep_team_rows tokens and fewer).
+  // Rows that need no norm and no row-major copy, whose pieces the threads working on a token can keep in registers. Team = the
+  // threads of one token: a wave (four tokens per workgroup, no barrier), up to 8 pieces per lane; or the whole workgroup (up to 8 pieces
+  // per thread: K <= 32768), where few tokens make the launch one token's chain of instructions (g_prep_team_rows tokens and
+  // fewer). fast: straight-line loads (whole K blocks, aligned rows of one element type).
   const int fast = single ? tk_prep_fast(*single) : table_fast;
   size_t pieces = (size_t)(table_wave_pieces > 0 ? table_wave_pieces : 0);
-  if (single) pieces = (!single->norm_kind && !single->blocksum) ? single->nb * 16 : 0;
-  const bool plain = pieces && (kind == TK_PREP_A8 || kind == TK_PREP_DIGITS);
-  const bool team_wg = plain && fast && pieces <= 8 * (size_t)TK_WG && (rows <= (unsigned)(kind == TK_PREP_DIGITS ? g_prep_team_rows * 8 / 3 : g_prep_team_rows) || pieces > 512);
-  // Rows of other shapes have no straight-line form: few of them take the kernels below, which give a token the whole
-  // workgroup. Call, N=512, wave per token element by element / with the vector loads of load_act4 / workgroup per token with them: float
-  // contract f32 K=2050 40 / 333 / 384 / 700 tokens 25.7, 26.6, 26.6, 28.5 / 23.5, 24.5, 24.6, 26.3 / 19.0, 20.7, 20.8, 27.0 us, K=1027 333 / 1000
-  // tokens 19.4, 21.2 / 18.4, 20.2 / 17.2, 24.5; int8 contract K=2050 333 tokens bf16 21.8 / 19.1 / 16.3, f32 20.6 / 18.7 / 16.2. One piece
-  // per lane (K <= 1024) stays: K=640 N=4096 106 f32 tokens, float contract 14.8 / 14.8 / 15.6.
-  const bool team_wave = plain && !team_wg && rows >= 32 && pieces <= (fast ? 512u : 256u) &&
-                         (fast || pieces <= 64 || rows > (unsigned)g_prep_team_rows);
-  if (team_wg || team_wave) {
+  if (single) pieces = (!single->norm_kind && !single->q_rowmajor && single->ap) ? single->nb * 16 : 0;
+  const bool strict = single && single->strict;
+  const bool plain = pieces && pieces <= 8 * (size_t)TK_WG && (kind == TK_PREP_A8 || kind == TK_PREP_DIGITS);
+  const bool team_wg = plain && (rows < 32 || rows <= (unsigned)(kind == TK_PREP_DIGITS ? g_prep_team_rows * 8 / 3 : g_prep_team_rows) || pieces > 512 || strict);
+  if (plain) {
     const size_t team = team_wg ? TK_WG : 64;
     const dim3 grid(team_wg ? rows : (rows + 3) / 4), block(TK_WG);
     const size_t per = (pieces + team - 1) / team;
     const int held = per <= 1 ? 1 : (per <= 2 ? 2 : (per <= 4 ? 4 : 8));
-#define TK_WAVE_PREP(KERNEL, H, F, T) hipLaunchKernelGGL((KERNEL<H, F, T>), grid, block, 0, s, sg, table, nprep, uniform_m, rows)
-#define TK_WAVE_PREP_H(KERNEL, F, T)                    \
-  switch (held) {                                       \
-    case 1: TK_WAVE_PREP(KERNEL, 1, F, T); break;       \
-    case 2: TK_WAVE_PREP(KERNEL, 2, F, T); break;       \
-    case 4: TK_WAVE_PREP(KERNEL, 4, F, T); break;       \
-    default: TK_WAVE_PREP(KERNEL, 8, F, T); break;      \
+#define TK_WAVE_PREP(...) hipLaunchKernelGGL((__VA_ARGS__), grid, block, 0, s, sg, table, nprep, uniform_m, rows)
+#define TK_WAVE_PREP_H(KERNEL, ...)                          \
+  switch (held) {                                            \
+    case 1: TK_WAVE_PREP(KERNEL<1, __VA_ARGS__>); break;     \
+    case 2: TK_WAVE_PREP(KERNEL<2, __VA_ARGS__>); break;     \
+    case 4: TK_WAVE_PREP(KERNEL<4, __VA_ARGS__>); break;     \
+    default: TK_WAVE_PREP(KERNEL<8, __VA_ARGS__>); break;    \
   }
-#define TK_WAVE_PREP_K(KERNEL)                                                         \
-  if (team_wg) {                                                                       \
-    if (fast == 2) { TK_WAVE_PREP_H(KERNEL, 2, 256) } else { TK_WAVE_PREP_H(KERNEL, 1, 256) } \
-  } else if (fast == 2) { TK_WAVE_PREP_H(KERNEL, 2, 64) }                              \
-  else if (fast == 1) { TK_WAVE_PREP_H(KERNEL, 1, 64) }                                \
-  else if (held == 1) TK_WAVE_PREP(KERNEL, 1, 0, 64);                                  \
-  else if (held == 2) TK_WAVE_PREP(KERNEL, 2, 0, 64);                                  \
-  else TK_WAVE_PREP(KERNEL, 4, 0, 64)
+#define TK_WAVE_PREP_K(KERNEL)                                                  \
+  if (team_wg) {                                                                \
+    if (fast == 2) { TK_WAVE_PREP_H(KERNEL, 2, 256) }                           \
+    else if (fast == 1) { TK_WAVE_PREP_H(KERNEL, 1, 256) }                      \
+    else { TK_WAVE_PREP_H(KERNEL, 0, 256) }                                     \
+  } else if (fast == 2) { TK_WAVE_PREP_H(KERNEL, 2, 64) }                       \
+  else if (fast == 1) { TK_WAVE_PREP_H(KERNEL, 1, 64) }                         \
+  else { TK_WAVE_PREP_H(KERNEL, 0, 64) }
     if (kind == TK_PREP_A8) {
       TK_WAVE_PREP_K(tk_prep_a8_wave_kernel);
+    } else if (strict) {
+      if (fast == 2) { TK_WAVE_PREP_H(tk_prep_digits_wave_kernel, 2, 256, true) }
+      else if (fast == 1) { TK_WAVE_PREP_H(tk_prep_digits_wave_kernel, 1, 256, true) }
+      else { TK_WAVE_PREP_H(tk_prep_digits_wave_kernel, 0, 256, true) }
     } else {
       TK_WAVE_PREP_K(tk_prep_digits_wave_kernel);
     }
@@ -2826,16 +2663,9 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
     return hipGetLastError();
   }
   switch (kind) {
-    case TK_PREP_A8:
-      if (single && single->nb * 16 <= (size_t)TK_WG)
-        hipLaunchKernelGGL(tk_prep_a8_kernel<1>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
-      else if (single && single->nb * 16 <= 2 * (size_t)TK_WG)
-        hipLaunchKernelGGL(tk_prep_a8_kernel<2>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
-      else
-        hipLaunchKernelGGL(tk_prep_a8_kernel<TK_PREP_HELD>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
-      break;
+    case TK_PREP_A8: hipLaunchKernelGGL(tk_prep_a8_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m); break;
     case TK_PREP_DIGITS:
-      if (single && single->strict) hipLaunchKernelGGL(tk_prep_digits_kernel<true>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
+      if (strict) hipLaunchKernelGGL(tk_prep_digits_kernel<true>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
       else hipLaunchKernelGGL(tk_prep_digits_kernel<false>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
       break;
     case TK_PREP_I8: hipLaunchKernelGGL(tk_prep_i8_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m); break;
