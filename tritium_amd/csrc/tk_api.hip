@@ -986,7 +986,11 @@ static int flow_run_tiles(const tk_ctx *ctx, unsigned total_tiles, int planes, i
   // where two workgroups share a CU: a CU's time follows the number of workgroups it is handed (two planes K=5120 N=5120
   // 16 rows, 32 copies, runs of 1 / 2 / 4 / 8: 86 / 94 / 77 / 123 us, rule: 2; three planes N=17408 370 / 364 / 387 / 425,
   // rule: 4).
-  bool use_model = !b3 && waves >= 8 && (rt == 1 || (rt >= 2 && lds_bytes > kLdsFlowMax / 2));
+  // The 32x32x32 form in eight-wave workgroups (25..32 rows of up to 64 KiB; its registers leave a CU one workgroup): likewise. 32 digit rows
+  // of eight float tokens / 32 int8 rows, two planes K=2048 N=8192, 48 copies, runs of 1 / 2 / 4 / 6 pairs: 84 / 82.7 / 86 / 112 and 95 / 92 / 99 /
+  // 136 us (4 fill one and a half rounds); 128 copies 209 / 206 / 201 / 209 (4: four rounds; the rule's and the model's choice); one plane
+  // N=6912, 48 copies 44.5 / 41.6 / 41.9 / -.
+  bool use_model = !b3 && waves >= 8 && (rt == 1 || (rt >= 2 && (wide || lds_bytes > kLdsFlowMax / 2)));
   if (use_model && rt > 2) {
     const double wgs = (double)((total_tiles + per_s * s - 1) / (per_s * s)), cus = (double)ctx->info.compute_units;
     const double rounds = (double)(size_t)((wgs + cus - 1.0) / cus);
@@ -1003,7 +1007,8 @@ static int flow_run_tiles(const tk_ctx *ctx, unsigned total_tiles, int planes, i
       const double cost = rounds * ((double)c * (double)per_s * (double)tile_bytes + 2.0 * (double)lds_bytes);
       // (equal costs are common, the terms being powers of two: one row tile then measured better with the longer run
       // -- K=5120 N=5120 16 rows 48 vs 42 us, K=8192 N=8192 105 vs 97 --, two row tiles with the shorter)
-      if (c == 1 || cost < best || (rt == 1 && cost <= best)) {
+      // (the 32x32x32 form with the longer run where that still fills the CUs: 32 copies of N=8192, runs of 2 / 4 56.8 vs 54.0)
+      if (c == 1 || cost < best || (rt == 1 && cost <= best) || (wide && cost <= best && wgs >= 0.95 * cus)) {
         best = cost;
         best_s = c;
       }
