@@ -209,3 +209,34 @@ def test_v2_matrix_form_at_its_edges(backend, so, codec, n, k, group, m):
     for a in (dact, dout):
         a.free()
     dev.free()
+
+
+@pytest.mark.parametrize("m,bad", [(3, False), (20, False), (3, True), (20, True)])
+def test_v2_output_over_the_activations(backend, so, m, bad):
+    """Results go straight to the output and a refused call puts back what it held; an output that is the activation tensor itself is
+    staged: the bits of a call with its own output, and the activations untouched by a refused one."""
+    rng = np.random.default_rng(m)
+    n = k = 256
+    tiles = n * k // 256
+    planes = [rng.integers(-1, 2, (tiles, 256)).astype(np.int8) for _ in range(2)]
+    t = S.V2Tensor(so, S.D2, 128, n, k, [(np.stack([planes[0][i], planes[1][i]]), rng.uniform(0.1, 1.0, (2, 2)).astype(np.float16).view(np.uint16)) for i in range(tiles)])
+    dev = backend.salt_v2_upload(S.D2, 128, t.payload, t.scales, t.plane_counts, n, k)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    if bad:
+        act[m - 1, 7] = np.inf
+    held = rng.standard_normal(m * n).astype(np.float32)
+    dact, dout = backend.to_device(act, "f32"), backend.to_device(held, "f32")
+    if bad:
+        for out in (dout, dact):
+            with pytest.raises(T.InvalidInput):
+                dev.forward(dact, m, out)
+        assert (dout.to_host().view(np.uint32) == held.view(np.uint32)).all()
+        assert (dact.to_host().view(np.uint32) == act.reshape(-1).view(np.uint32)).all()
+    else:
+        dev.forward(dact, m, dout)
+        want = dout.to_host()
+        dev.forward(dact, m, dact)
+        assert (dact.to_host().view(np.uint32) == want.view(np.uint32)).all()
+    for x in (dact, dout):
+        x.free()
+    dev.free()

@@ -16,6 +16,8 @@
 // matrix pipe: see tk_salt_v2_exact_kernel.
 // Compiled with -ffp-contract=off; the sums use explicit round-to-nearest adds and multiplies.
 
+#include <type_traits>
+
 #include "tk_device.h"
 
 namespace {
@@ -137,7 +139,8 @@ __device__ __forceinline__ float f16_to_f32(uint16_t h) {
 // LDS: float term[segments][3 planes][tokens], then one plane count per segment.
 // Segment boundaries are the multiples of the scale group (which divides the 256 of a tile).
 __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
-                                                                float *__restrict__ out, unsigned *__restrict__ flag, unsigned call) {
+                                                                float *__restrict__ out, float *__restrict__ keep, unsigned *__restrict__ flag,
+                                                                unsigned call) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int MT = TK_SALT_V2_TOKENS;
   const unsigned row = blockIdx.x, tok0 = blockIdx.y * MT;
@@ -190,7 +193,9 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
       for (unsigned j = 0; j < seg_planes[s]; ++j) accumulator = __fadd_rn(accumulator, term[((size_t)s * 3 + j) * MT + threadIdx.x]);
     // an accumulator that left the finite range never comes back (inf - inf is NaN): the end result tells
     bad |= !(fabsf(accumulator) <= 3.402823466e38f);
-    out[(size_t)(tok0 + threadIdx.x) * t.n + row] = accumulator;
+    const size_t at = (size_t)(tok0 + threadIdx.x) * t.n + row;
+    if (keep) gstore(keep + at, gload(out + at));
+    out[at] = accumulator;
   }
   if (bad) gstore(flag, call);  // (whoever stores, stores the same)
 }
@@ -207,63 +212,81 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
 // Floor: the f32 matrix pipe, 32 cycles per 16 x 16 x 4 (7 us at the size below); the recoding and the latency of the loads add to it.
 // 4096 x 4096, two planes, kernels, 8 tokens of B3: 64 us (fold with a lane per row, terms through memory) + 12 us (their sum) ->
 // 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 35 / 37 / 38 us, one token 57 / 69 / 66 -> 33 / 36 / 37, 64 tokens 302 / 389 / 353 ->
-// 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory). (With the activations as 32 four-byte loads per lane and the codes as single bytes the kernel took 52 us: the
+// 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory), without a launch that commits the results 33 / 35 us (D2 / B3). (A segment's codes
+// and activations requested ahead of the fold before it: 38.8 against 35.5 for B3.) (With the activations as 32 four-byte loads per lane and the codes as single bytes the kernel took 52 us: the
 // loads of 16 rows a few KiB apart were the bound.)
-constexpr int SV2_WAVES = 16, SV2_SLOTS = 48;
+constexpr int SV2_WAVES = 16, SV2_SLOTS = 48, SV2_HEAD = 528;
 template <int G>
 __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
-                                                                          float *__restrict__ out, unsigned *__restrict__ flag,
-                                                                          unsigned call, unsigned slots) {
+                                                                          float *__restrict__ out, float *__restrict__ keep,
+                                                                          unsigned *__restrict__ flag, unsigned call, unsigned slots) {
   constexpr int W = G / 64;  // words of sixteen codes per lane and fold
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   uint16_t *s_fields = (uint16_t *)smem;                                   // [256], B3: the digits of a byte
-  float *s_term = (float *)(smem + 512);                                   // [slot][plane][accumulator register][lane]
-  uint8_t *s_planes = smem + 512 + (size_t)slots * 3 * 256 * sizeof(float);  // [slot][row]
+  int *s_three = (int *)(smem + 512);                                      // some tile of the workgroup has three planes
+  float *s_term = (float *)(smem + SV2_HEAD);                              // [slot][plane][accumulator register][lane]
+  uint8_t *s_planes = smem + SV2_HEAD + (size_t)slots * 3 * 256 * sizeof(float);  // [slot][row]
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4;
   const unsigned row = min(blockIdx.x * 16u + c, t.n - 1u), tok0 = blockIdx.y * 16u;
   const unsigned nseg = t.k / G, codec = t.codec;
   const unsigned full_bytes = plane_bytes(codec, 256u);
   const float *arow = act + (size_t)min(tok0 + c, m - 1u) * t.k + h * 4;
   const unsigned final_row = blockIdx.x * 16u + c, final_tok = tok0 + h * 4 + wave;  // of the thread that adds (waves 0..3)
+  const size_t final_at = (size_t)min(final_tok, m - 1u) * t.n + min(final_row, t.n - 1u);
+  const bool ends = wave < 4 && final_row < t.n && final_tok < m;
+  float before = 0.0f;  // what a bad call puts back
+  if (keep && ends) before = gload(out + final_at);
   float sum = 0.0f;
   bool bad = false;
-  if (codec == TK_SALT_V2_B3) {
-    if (threadIdx.x < 256) s_fields[threadIdx.x] = (uint16_t)b3_fields(threadIdx.x);
-    __syncthreads();
-  }
+  if (threadIdx.x == 0) *s_three = 0;
+  if (codec == TK_SALT_V2_B3 && threadIdx.x < 256) s_fields[threadIdx.x] = (uint16_t)b3_fields(threadIdx.x);
+  __syncthreads();
+  typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+  struct Codes {
+    unsigned long long raw[3][W];
+    uint16_t scale[3];
+    unsigned planes, most, local;
+  };
+  float a[W * 4][4];  // [sixteen columns][x]: column 4 x + h of the token, after the transpose
+  auto request_act = [&](unsigned s) {
+#pragma unroll
+    for (int w = 0; w < W * 4; ++w) {
+      const quad v = *(const TK_GLOBAL quad *)(arow + (size_t)s * G + w * 16);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) a[w][x] = v[x];
+    }
+  };
+  auto request_codes = [&](unsigned s, Codes &d) {
+    const unsigned long long lo = (unsigned long long)row * t.k + (unsigned long long)s * G;
+    const unsigned tile = (unsigned)(lo >> 8);
+    d.local = (unsigned)(lo & 255ull);
+    const TileView tv = tile_view(t, tile);
+    const unsigned cur_bytes = plane_bytes(codec, tv.len), cur_groups = tv.len / G;
+    const uint8_t *planes = t.payload + (size_t)tv.begin * full_bytes;
+    const uint16_t *scales = t.scales + (size_t)tv.begin * (256u / G) + d.local / G;
+    d.planes = tv.planes;
+    d.most = __ballot(tv.planes >= 3u) ? 3u : (__ballot(tv.planes >= 2u) ? 2u : 1u);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      if ((unsigned)j >= d.most) break;
+      const unsigned jc = min((unsigned)j, tv.planes - 1u);
+#pragma unroll
+      for (int i = 0; i < W; ++i) d.raw[j][i] = raw16(planes + (size_t)jc * cur_bytes, cur_bytes, d.local + (h * W + i) * 16u, codec);
+      d.scale[j] = gload(scales + (size_t)jc * cur_groups);
+    }
+  };
   for (unsigned s0 = 0; s0 < nseg; s0 += slots) {
     const unsigned pass = min(slots, nseg - s0);
     for (unsigned slot = wave; slot < pass; slot += SV2_WAVES) {
-      const unsigned s = s0 + slot;
-      typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
-      float a[W * 4][4];  // [sixteen columns][x]: column 4 x + h of the token, after the transpose
-#pragma unroll
-      for (int w = 0; w < W * 4; ++w) {
-        const quad v = *(const TK_GLOBAL quad *)(arow + (size_t)s * G + w * 16);
-#pragma unroll
-        for (int x = 0; x < 4; ++x) a[w][x] = v[x];
-      }
-      const unsigned long long lo = (unsigned long long)row * t.k + (unsigned long long)s * G;
-      const unsigned tile = (unsigned)(lo >> 8), local = (unsigned)(lo & 255ull);
-      const TileView tv = tile_view(t, tile);
-      const unsigned cur_bytes = plane_bytes(codec, tv.len), cur_groups = tv.len / G;
-      const uint8_t *planes = t.payload + (size_t)tv.begin * full_bytes;
-      const uint16_t *scales = t.scales + (size_t)tv.begin * (256u / G) + local / G;
-      if (h == 0) s_planes[slot * 16 + c] = (uint8_t)tv.planes;
-      const unsigned most = __ballot(tv.planes >= 3u) ? 3u : (__ballot(tv.planes >= 2u) ? 2u : 1u);
+      Codes cur = {};
+      request_act(s0 + slot);
+      request_codes(s0 + slot, cur);
+      const unsigned local = cur.local, most = cur.most;
+      if (h == 0) s_planes[slot * 16 + c] = (uint8_t)cur.planes;
+      if (most == 3u && lane == 0) *s_three = 1;
       if (blockIdx.x == 0) {  // every activation passes here
 #pragma unroll
         for (int x = 0; x < W * 16; ++x) bad |= !(fabsf(a[x / 4][x % 4]) <= 3.402823466e38f);
-      }
-      unsigned long long raw[3][W];
-      uint16_t scale[3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        if ((unsigned)j >= most) break;
-        const unsigned jc = min((unsigned)j, tv.planes - 1u);
-#pragma unroll
-        for (int i = 0; i < W; ++i) raw[j][i] = raw16(planes + (size_t)jc * cur_bytes, cur_bytes, local + (h * W + i) * 16u, codec);
-        scale[j] = gload(scales + (size_t)jc * cur_groups);
       }
 #pragma unroll
       for (int w = 0; w < W * 4; ++w) transpose_rows(a[w]);
@@ -274,7 +297,7 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
 #pragma unroll
         for (int i = 0; i < W; ++i) {
           unsigned row_words[4];
-          spread_rows(recode16(raw[j][i], local + (h * W + i) * 16u, codec, s_fields), row_words);
+          spread_rows(recode16(cur.raw[j][i], local + (h * W + i) * 16u, codec, s_fields), row_words);
 #pragma unroll
           for (int q = 0; q < 4; ++q) words[q * W + i] = row_words[q];
         }
@@ -287,42 +310,45 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
           for (int x = 0; x < 4; ++x)
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[w][x], (float)(int8_t)(trits >> (8 * x)), acc, 0, 0, 0);
         }
-        const float sc = f16_to_f32(scale[j]);
+        const float sc = f16_to_f32(cur.scale[j]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) s_term[((slot * 3 + j) * 4 + r) * 64 + lane] = __fmul_rn(acc[r], sc);
       }
     }
     __syncthreads();
     if (wave < 4) {
+      auto add = [&](auto np_c) {
+        constexpr int NP = decltype(np_c)::value;
 #pragma unroll 8
-      for (unsigned u = 0; u < pass; ++u) {
-        const unsigned planes = s_planes[u * 16 + c];
+        for (unsigned u = 0; u < pass; ++u) {
+          const unsigned planes = s_planes[u * 16 + c];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const float next = __fadd_rn(sum, s_term[((u * 3 + j) * 4 + wave) * 64 + lane]);  // (what a plane that is not there left is not taken)
-          sum = (unsigned)j < planes ? next : sum;
+          for (int j = 0; j < NP; ++j) {
+            const float next = __fadd_rn(sum, s_term[((u * 3 + j) * 4 + wave) * 64 + lane]);  // (what a plane that is not there left is not taken)
+            sum = (unsigned)j < planes ? next : sum;
+          }
         }
-      }
+      };
+      if (*s_three) add(std::integral_constant<int, 3>{});
+      else add(std::integral_constant<int, 2>{});
     }
     __syncthreads();
   }
-  if (wave < 4 && final_row < t.n && final_tok < m) {
+  if (ends) {
     // an accumulator that left the finite range never comes back (inf - inf is NaN): the end result tells
     bad |= !(fabsf(sum) <= 3.402823466e38f);
-    out[(size_t)final_tok * t.n + final_row] = sum;
+    if (keep) gstore(keep + final_at, before);
+    gstore(out + final_at, sum);
   }
   if (bad) gstore(flag, call);  // (whoever stores, stores the same)
 }
 
-// The results leave the staging buffer only when no activation and no result was found non-finite: the flag then holds the
-// number of an earlier call (so it is never cleared). *verdict, in host memory, says which it was.
+// out[i] = tmp[i] unless *flag is `call`: the results of a call whose output overlaps its activations leave the staging buffer
+// this way; without a flag the values that a bad call replaced go back.
 __global__ __launch_bounds__(TK_WG) void tk_salt_v2_commit_kernel(const float *__restrict__ tmp, float *__restrict__ out, size_t count,
-                                                                  const unsigned *__restrict__ flag, unsigned call,
-                                                                  unsigned *__restrict__ verdict) {
-  const bool bad = gload(flag) == call;
+                                                                  const unsigned *__restrict__ flag, unsigned call) {
   const size_t idx = (size_t)blockIdx.x * TK_WG + threadIdx.x;
-  if (idx == 0) gstore(verdict, bad ? 1u : 0u);
-  if (!bad && idx < count) gstore(out + idx, gload(tmp + idx));
+  if (idx < count && !(flag && gload(flag) == call)) gstore(out + idx, gload(tmp + idx));
 }
 
 // One thread per gathered coefficient (crates/tritium-cuda/kernels/salt_v2.cu:218-304).
@@ -352,19 +378,19 @@ size_t tk_salt_v2_lds_bytes(size_t k, size_t group) {
   return nseg * 3 * TK_SALT_V2_TOKENS * sizeof(float) + ((nseg + 15) & ~(size_t)15);
 }
 
-hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *tmp, unsigned *flag,
+hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *out, float *keep, unsigned *flag,
                                      unsigned call) {
   if (!m || !t.n) return hipSuccess;
   if (t.k && t.k % t.group == 0) {
     const dim3 grid((t.n + 15) / 16, (unsigned)((m + 15) / 16)), block(SV2_WAVES * 64);
     const unsigned nseg = t.k / t.group, slots = nseg < SV2_SLOTS ? nseg : SV2_SLOTS;
-    const size_t lds = 512 + (size_t)slots * (3 * 256 * sizeof(float) + 16);
+    const size_t lds = SV2_HEAD + (size_t)slots * (3 * 256 * sizeof(float) + 16);
     if (lds > 64 * 1024) {
       const hipError_t e = tk_raise_lds_limit(t.group == 128 ? (const void *)tk_salt_v2_exact_kernel<128> : (const void *)tk_salt_v2_exact_kernel<64>, 160 * 1024);
       if (e != hipSuccess) return e;
     }
-    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, call, slots);
-    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, tmp, flag, call, slots);
+    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, out, keep, flag, call, slots);
+    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, out, keep, flag, call, slots);
     return hipGetLastError();
   }
   const size_t lds = tk_salt_v2_lds_bytes(t.k, t.group);
@@ -373,14 +399,13 @@ hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const flo
     if (e != hipSuccess) return e;
   }
   const dim3 grid(t.n, (unsigned)((m + TK_SALT_V2_TOKENS - 1) / TK_SALT_V2_TOKENS));
-  hipLaunchKernelGGL(tk_salt_v2_forward_kernel, grid, dim3(64), lds, s, t, act, (unsigned)m, tmp, flag, call);
+  hipLaunchKernelGGL(tk_salt_v2_forward_kernel, grid, dim3(64), lds, s, t, act, (unsigned)m, out, keep, flag, call);
   return hipGetLastError();
 }
 
-hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call,
-                                    unsigned *verdict) {
+hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call) {
   if (!count) return hipSuccess;
-  hipLaunchKernelGGL(tk_salt_v2_commit_kernel, dim3((unsigned)((count + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, tmp, out, count, flag, call, verdict);
+  hipLaunchKernelGGL(tk_salt_v2_commit_kernel, dim3((unsigned)((count + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, tmp, out, count, flag, call);
   return hipGetLastError();
 }
 
