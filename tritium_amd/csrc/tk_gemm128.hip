@@ -18,7 +18,7 @@
 // and interleaving the expansion with the matrix instructions one by one changed nothing. Otherwise the number of workgroups
 // on the CU that has most (gemm128_pays in tk_api.hip). Calls incl. quantization, 64 rows -> 128: 4096 tokens K=5120 N=17408 three
 // planes 759 -> 738 us, 1024 tokens K=5120 N=5120 79 -> 72, 200 tokens N=17408 73 -> 65; 768 tokens K=6144 N=20480 one plane 98 -> 83,
-// two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 -> 41.1. One workgroup alone on a CU runs its
+// two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 -> 41.1 (35.7 with the epilogue and the digit split of now). One workgroup alone on a CU runs its
 // loop at 0.58 of the matrix rate, two at 0.70.
 
 #include <type_traits>
@@ -283,6 +283,37 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
   if (int8_in && hot.out_dtype != TK_I32 && (((size_t)hot.n * esz) & 15) == 0 && ((uintptr_t)hot.out & 15) == 0 && !hot.residual) {
     if (esz == 2) staged(std::integral_constant<int, 2>{});
     else staged(std::integral_constant<int, 4>{});
+  } else if (!int8_in && !hot.residual && !wg_flag) {
+    // float contract: token 8 rt + 2 q + kappa of the workgroup, one output per accumulator quad; a store is 32 adjacent columns of
+    // two tokens (straight-line: one address per column, stepped by two tokens, where flow_epilogue decides per output: 333 f32 tokens K=2050 N=5003
+    // two planes, call 37.3 -> 35.7 us)
+    auto plain = [&](auto esz_c) {
+      constexpr int ESZ = decltype(esz_c)::value;
+      const size_t step = (size_t)hot.n * (2 * ESZ);
+      const int tok0 = (row0 >> 2) + kappa;
+#pragma unroll
+      for (int z = 0; z < HP; ++z) {
+        const int n = (tile0 + 2 * z + h) * 16 + r16;
+        uint8_t *dst = (uint8_t *)hot.out + ((size_t)tok0 * hot.n + n) * ESZ;
+        const bool in = n < hot.n;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            RowConst rc = {};
+            rc.exp = cst_exp[rt * 8 + 2 * q + kappa];
+            v4i av[P];
+            quad(rt, q, z, av);
+            const float f = digits_value<P>(av, sc[z], rc);
+            if (in && tok0 + rt * 8 + 2 * q < hot.M) {
+              if (ESZ == 2) gstore((uint16_t *)dst, f32_to_bf16_hw(f)); else gstore((float *)dst, f);
+            }
+            dst += step;
+          }
+      }
+    };
+    if (esz == 2) plain(std::integral_constant<int, 2>{});
+    else plain(std::integral_constant<int, 4>{});
   } else {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
