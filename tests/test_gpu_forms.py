@@ -171,6 +171,8 @@ def test_prefill_kernel_128_rows_planes_and_contracts(backend, oracle, m, n, k, 
         assert backend.last_kernel().split("_")[0] == f"gemm{rows}", backend.last_kernel()
         got[rows] = out.to_host().reshape(m, n)
         assert np.abs(got[rows][plain] - exact[plain]).max() <= 1e-5 * np.abs(exact).max()
+        backend.linear_float(layer, dact, m, outb)
+        assert (outb.to_host().reshape(m, n)[plain] == f32_to_bf16_bits(got[rows])[plain]).all()
         out.free()
         outb.free()
     assert (got[64].view(np.uint32) == got[128].view(np.uint32)).all()
