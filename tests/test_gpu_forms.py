@@ -808,3 +808,48 @@ def test_activation_prep_of_ragged_rows_places_every_element(backend, oracle, k,
     for x in (act, out):
         x.free()
     layer.free()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("m,n,planes", [(1, 40, 1), (2, 40, 2), (3, 40, 1), (1, 9600, 1), (1, 9600, 2), (70, 40, 1)])
+def test_layers_without_inputs(backend, m, n, planes, dt):
+    """K = 0 is accepted and gives zeros (a sum of nothing, +0 times positive scales), plus the residual: both contracts, behind an
+    RMSNorm, alone and as a member of a group beside one with inputs. No form may read an activation or a norm weight: such rows
+    have none, so the one-launch forms and the straight-line loads, whose lanes past a row's end read its last piece again, are not for them."""
+    print("case no-inputs", m, n, planes, dt, flush=True)
+    rng = np.random.default_rng(m + n + planes)
+    empty = backend.linear([np.zeros(0, np.uint8)] * planes, [scales(rng, n) for _ in range(planes)], n, 0)
+    k = 256
+    ws, scs, packed = _planes(rng, 48, k, planes)
+    layer = backend.linear(packed, scs, 48, k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    act = backend.to_device(f32_to_bf16_bits(x) if dt == "bf16" else x, dt)
+    weight = backend.to_device(rng.uniform(0.5, 1.5, k).astype(np.float32), "f32")
+    out, other, alone = backend.empty(m * n, "f32"), backend.empty(m * 48, "f32"), backend.empty(m * 48, "f32")
+    held = rng.standard_normal(m * n).astype(np.float32)
+    res = backend.to_device(held, "f32")
+    calls = {"a8": lambda: backend.linear_a8(empty, act, m, out), "float": lambda: backend.linear_float(empty, act, m, out),
+             "normed": lambda: backend.linear_rmsnorm_a8(empty, act, weight, 1e-5, m, out)}
+    for name, call in calls.items():
+        backend.linear_a8_residual(empty, act, m, res, out)  # (leaves the residual there)
+        call()
+        assert (out.to_host().view(np.uint32) == 0).all(), name
+    backend.linear_a8_residual(empty, act, m, res, out)
+    assert same_bits(out.to_host(), held)
+    for mode, normed in ((1, False), (1, True), (0, False)):
+        if m * (1 if mode else 4) > 64:  # groups take at most 64 operand rows
+            continue
+        if normed:
+            backend.linear_rmsnorm_a8(layer, act, weight, 1e-5, m, alone)
+        else:
+            (backend.linear_a8 if mode else backend.linear_float)(layer, act, m, alone)
+        grp = backend.group([(empty, act, m, out), (layer, act, m, other)], mode, dt, "f32", norms=[(weight, 1e-5, False)] * 2 if normed else None)
+        backend.linear_a8_residual(empty, act, m, res, out)
+        grp.launch()
+        assert (out.to_host().view(np.uint32) == 0).all(), (mode, normed)
+        assert same_bits(other.to_host(), alone.to_host()), (mode, normed)
+        grp.destroy()
+    for a in (act, weight, out, other, alone, res):
+        a.free()
+    layer.free()
+    empty.free()

@@ -1334,7 +1334,7 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
     // two and three planes of K <= 4096 gain 10-20%, one plane of K=8192 loses 20%) and stay.
     if (ctx->decode_force == DECODE_AUTO && variant == DECODE_KSPLIT && pl.flow_ok && !wide && !b3 && m == 1 &&
         ctx->fuse_tokens != 0 && (unsigned)pl.pr.n_tiles > 2u * (unsigned)ctx->info.compute_units && pl.cfg.rt == 1 &&
-        (prep_kind == TK_PREP_A8 || prep_kind == TK_PREP_DIGITS) && nb * 16 <= 512 && k % 256 == 0 &&
+        (prep_kind == TK_PREP_A8 || prep_kind == TK_PREP_DIGITS) && nb && nb * 16 <= 512 && k % 256 == 0 &&
         ((uintptr_t)act & 15) == 0 && (act_dtype == TK_F32 || act_dtype == TK_BF16) &&
         (!norm || ((uintptr_t)norm->weight & 15) == 0) &&
         flow_lds + 1024 + (norm ? k * 4 + 1024 : 0) + 1024 <= 64 * 1024)
@@ -1415,7 +1415,7 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
   // 1 KiB behind the row constants).
   const size_t fuse_lds = 1024 + (norm ? k * 4 + 1024 : 0);
   const bool fuse_rows = pl.skinny && pl.cfg.rt == 1 && (prep_kind == TK_PREP_A8 || prep_kind == TK_PREP_DIGITS) &&
-                         m <= (size_t)fuse_limit && nb * 16 <= 512 && k % 256 == 0 && ((uintptr_t)act & 15) == 0 &&
+                         m <= (size_t)fuse_limit && nb && nb * 16 <= 512 && k % 256 == 0 && ((uintptr_t)act & 15) == 0 &&
                          (act_dtype == TK_F32 || act_dtype == TK_BF16) &&
                          (!norm || (m == 1 && fuse_limit >= 1 && ((uintptr_t)norm->weight & 15) == 0));
   const bool fused_flow = fuse_rows && variant == DECODE_FLOW && !wide && !b3 && flow_lds + fuse_lds + 1024 <= 64 * 1024;
@@ -2610,7 +2610,7 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
     for (size_t i = 0; i < count && gfused; ++i) {
       const TkPrep &pp = preps[prep_of[i]];
       const size_t k = (size_t)plans[i].pr.k, nb = (size_t)plans[i].pr.nb;
-      gfused = (size_t)members[i].m <= glimit && nb * 16 <= 512 && k % 256 == 0 && ((uintptr_t)members[i].act & 15) == 0 &&
+      gfused = (size_t)members[i].m <= glimit && nb && nb * 16 <= 512 && k % 256 == 0 && ((uintptr_t)members[i].act & 15) == 0 &&
                (size_t)plans[i].pr.kc >= nb &&
                (!pp.norm_kind || (members[i].m == 1 && ((uintptr_t)pp.norm_w & 15) == 0));
       const size_t need = nb * 256 * (size_t)plans[i].pr.R + 1024 + (pp.norm_kind ? k * 4 + 1024 : 0) + (size_t)4096 * planes;
@@ -2641,7 +2641,7 @@ static int group_create(tk_ctx *ctx, const tk_group_member *members, const tk_rm
   for (size_t i = 0; i < count && gfused_flow; ++i) {
     const TkPrep &pp = preps[prep_of[i]];
     const size_t k = (size_t)plans[i].pr.k, nb = (size_t)plans[i].pr.nb;
-    gfused_flow = members[i].m == 1 && nb * 16 <= 512 && k % 256 == 0 && ((uintptr_t)members[i].act & 15) == 0 &&
+    gfused_flow = members[i].m == 1 && nb && nb * 16 <= 512 && k % 256 == 0 && ((uintptr_t)members[i].act & 15) == 0 &&
                   (!pp.norm_kind || ((uintptr_t)pp.norm_w & 15) == 0);
     if (pp.norm_kind && 1024 + k * 4 + 1024 > fuse_flow_extra) fuse_flow_extra = 1024 + k * 4 + 1024;
   }

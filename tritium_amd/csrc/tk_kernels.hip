@@ -1803,7 +1803,9 @@ __device__ __forceinline__ void load_piece(const void *act, int dtype, size_t ba
     load_piece_ragged<TK_F32>(act, base, (unsigned)e0, (unsigned)k, v);
   }
 }
-// The pieces lane, lane + TEAM, ... of a row. FAST: rows of whole K blocks, 16-byte aligned, of one element type (1 = f32, 2 = bf16).
+// The pieces lane, lane + TEAM, ... of a row. FAST: rows of whole K blocks, 16-byte aligned, of one element type (1 = f32, 2 = bf16),
+// and at least one block: in a row without any, the piece that a lane past the end re-reads does not exist (the host's rules keep K = 0 off
+// every kernel that loads this way; FAST = 0 reads nothing of such a row).
 template <int HELD, int FAST, int TEAM>
 __device__ __forceinline__ void load_held(const void *act, int dtype, size_t base, size_t k, int npieces, int lane,
                                           float (&held)[HELD][16]) {
@@ -2627,14 +2629,14 @@ hipError_t tk_launch_decode_trits(hipStream_t s, const uint8_t *codes, size_t n,
 static int g_prep_team_rows = 384;
 void tk_prep_set_team_rows(int rows) { g_prep_team_rows = rows < 0 ? 0 : rows; }
 int tk_prep_fast(const TkPrep &pp) {
-  const bool ok = pp.k % 256 == 0 && (((size_t)pp.act) & 15) == 0 && pp.ap && !pp.q_rowmajor && !pp.norm_kind;
+  const bool ok = pp.nb && pp.k % 256 == 0 && (((size_t)pp.act) & 15) == 0 && pp.ap && !pp.q_rowmajor && !pp.norm_kind;
   if (!ok) return 0;
   return pp.act_dtype == TK_F32 ? 1 : (pp.act_dtype == TK_BF16 ? 2 : 0);
 }
 // ... the same for the one-pass RMSNorm + quantization kernel, which takes entries with and without a norm (at most
 // 512 pieces, i.e. K <= 8192; aligned norm weights): 1 (f32) or 2 (bf16), else 0
 int tk_prep_norm_fast(const TkPrep &pp) {
-  const bool ok = pp.k % 256 == 0 && (((size_t)pp.act) & 15) == 0 && pp.ap && !pp.q_rowmajor && !pp.blocksum &&
+  const bool ok = pp.nb && pp.k % 256 == 0 && (((size_t)pp.act) & 15) == 0 && pp.ap && !pp.q_rowmajor && !pp.blocksum &&
                   pp.nb * 16 <= 2 * (size_t)TK_WG && (!pp.norm_kind || (pp.norm_w && (((size_t)pp.norm_w) & 15) == 0));
   if (!ok) return 0;
   return pp.act_dtype == TK_F32 ? 1 : (pp.act_dtype == TK_BF16 ? 2 : 0);
