@@ -811,7 +811,7 @@ def test_activation_prep_of_ragged_rows_places_every_element(backend, oracle, k,
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
-@pytest.mark.parametrize("m,n,planes", [(1, 40, 1), (2, 40, 2), (3, 40, 1), (1, 9600, 1), (1, 9600, 2), (70, 40, 1)])
+@pytest.mark.parametrize("m,n,planes", [(1, 40, 1), (2, 40, 2), (3, 40, 1), (1, 9600, 1), (1, 9600, 2), (70, 40, 1), (1100, 9600, 1)])
 def test_layers_without_inputs(backend, m, n, planes, dt):
     """K = 0 is accepted and gives zeros (a sum of nothing, +0 times positive scales), plus the residual: both contracts, behind an
     RMSNorm, alone and as a member of a group beside one with inputs. No form may read an activation or a norm weight: such rows

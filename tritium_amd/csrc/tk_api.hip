@@ -1428,9 +1428,10 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
   const bool fused_ksplit = fuse_rows && variant == DECODE_KSPLIT && (size_t)pl.pr.kc >= nb && fused_ksplit_lds + 1024 <= 64 * 1024 &&
                             fuse_tpw <= 4;
   const bool fused = fused_flow || fused_ksplit;
-  // One plane under the int8 contract with whole 16-byte output pieces: the wide-tile prefill kernels.
+  // One plane under the int8 contract with whole 16-byte output pieces: the 256-row prefill kernel (which requests a K block
+  // before it looks how many there are).
   const size_t out_esz = out_dtype == TK_BF16 ? 2 : 4;
-  const bool can_wide = !pl.skinny && !waves && pl.pr.planes == 1 && mode == TK_MODE_INT8 && (out_dtype == TK_F32 || out_dtype == TK_BF16) &&
+  const bool can_wide = nb && !pl.skinny && !waves && pl.pr.planes == 1 && mode == TK_MODE_INT8 && (out_dtype == TK_F32 || out_dtype == TK_BF16) &&
                         !residual && (n * out_esz) % 16 == 0 && ((uintptr_t)out & 15) == 0;
   int form256 = 0;
   const bool pays256 = gemm256_pays(ctx, R, (size_t)pl.pr.n_tiles, &form256);
