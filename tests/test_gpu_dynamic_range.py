@@ -129,3 +129,80 @@ def test_plain_and_integer_tokens_stay_on_the_fast_path(backend, oracle, dtype):
     dact.free()
     dout.free()
     layer.free()
+
+
+def _small_rows(rng, k):
+    """Rows around the smallest scales of the int8 contract: 127 / max overflows below 3.8e-37, and max / 127 is zero up to 8.8e-44.
+    An infinite 127 / max makes every element saturate and a zero NaN, which the host carries on; a row without one gives outputs
+    that are zero with the sign of the sum."""
+    def row(top, zeros=False):
+        a = (rng.uniform(0.25, 1.0, k) * rng.choice([-1.0, 1.0], k)).astype(np.float64) * top
+        a = a.astype(np.float32)
+        a[a == 0] = np.float32(top)
+        if zeros:
+            a[rng.choice(k, 3, replace=False)] = 0.0
+        return a
+    return np.stack([row(1e-37), row(1e-37, True), row(4e-44), row(4e-44, True), np.full(k, -4e-44, np.float32), row(5e-45, True),
+                     np.zeros(k, np.float32), row(3.9e-37, True)])
+
+
+def _same_with_nan(got, want):
+    got, want = got.reshape(want.shape), np.asarray(want, np.float32)
+    nan = np.isnan(want)
+    return (np.isnan(got) == nan).all() and (got.view(np.uint32) == want.view(np.uint32))[~nan].all()
+
+
+@pytest.mark.parametrize("n,planes,k", [(48, 1, 256), (48, 1, 300), (48, 1, 2560), (64, 2, 256), (64, 2, 300), (64, 2, 2560), (9600, 1, 256), (9600, 1, 300)])
+def test_rows_whose_scale_overflows(backend, oracle, n, planes, k):
+    """The int8 contract's bits (signs of zeros and places of NaN among them) for rows whose 127 / max overflows, in every form: one and
+    two tokens built by the decode kernels themselves, the small-batch, decode and prefill kernels behind a quantization launch, the same behind
+    an RMSNorm whose weights make the row that small, and groups. 9600 outputs: more than two tiles per CU (flow kernel)."""
+    print("case small-rows", n, planes, k, flush=True)
+    rng = np.random.default_rng(n + k + planes)
+    ws = [ternary(rng, n, k, 0.4) for _ in range(planes)]
+    ws[0][0] = -1
+    ws[0][1] = 1
+    ws[0][2] = 0
+    scs = [scales(rng, n) for _ in range(planes)]
+    packed = [T.pack_rows(w, n, k) for w in ws]
+    layer = backend.linear(packed, scs, n, k)
+    rows = _small_rows(rng, k)
+    want = oracle.cpu_linear_a8_planes(packed, FMT_TQ2_0, scs, rows, len(rows), n, k).reshape(len(rows), n)
+    assert np.signbit(want[4][want[4] == 0]).any() and np.isnan(want[1]).any()  # (what the rows are for)
+
+    def calls(acts, wants, m, norm=None):
+        """acts [m, k] on the device through a call, a residual call and a group"""
+        act, out, res = backend.to_device(acts, "f32"), backend.empty(m * n, "f32"), backend.to_device(np.full(m * n, -0.0, np.float32), "f32")
+        if norm is None:
+            backend.linear_a8(layer, act, m, out)
+        else:
+            backend.linear_rmsnorm_a8(layer, act, norm, 1e-5, m, out)
+        assert _same_with_nan(out.to_host(), wants), (m, "call", backend.last_kernel())
+        if norm is None:
+            backend.linear_a8_residual(layer, act, m, res, out)
+            assert _same_with_nan(out.to_host(), np.float32(-0.0) + wants), (m, "residual")
+        if m <= 64:
+            grp = backend.group([(layer, act, m, out)] * 2, 1, "f32", "f32", norms=None if norm is None else [(norm, 1e-5, False)] * 2)
+            grp.launch()
+            assert _same_with_nan(out.to_host(), wants), (m, "group", backend.last_kernel())
+            grp.destroy()
+        for a in (act, out, res):
+            a.free()
+
+    for r in range(len(rows)):
+        calls(rows[r:r + 1], want[r:r + 1], 1)
+    for r in range(0, len(rows), 2):
+        calls(rows[r:r + 2], want[r:r + 2], 2)
+    for m in (3, 8, 24, 70) if n < 9600 else (8,):
+        which = np.arange(m) % len(rows)
+        calls(rows[which], want[which], m)
+    # behind an RMSNorm: the token is +-1 throughout (rms 1 / (1 + eps)), so its normalized row is the weights
+    for r in (0, 2, 3, 5):
+        x = rng.choice(np.float32([-1.0, 1.0]), (3, k))
+        y = np.stack([oracle.rmsnorm(t, rows[r], 1e-5) for t in x])
+        wn = oracle.cpu_linear_a8_planes(packed, FMT_TQ2_0, scs, y, 3, n, k).reshape(3, n)
+        norm = backend.to_device(rows[r], "f32")
+        for m in (1, 3):
+            calls(x[:m], wn[:m], m, norm)
+        norm.free()
+    layer.free()

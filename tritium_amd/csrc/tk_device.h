@@ -154,9 +154,13 @@ __device__ __noinline__ float salt_exact_dot(const TkProblem &pr, int n, int tok
   return acc;
 }
 
+// Whether a token has no largest element (then it quantizes to zeros) from its scale max / 127 and 127 / max: both are zero. The scale
+// alone underflows to zero for a largest element of up to 8.8e-44, whose 127 / max is infinite, and 127 / max alone is zero for Inf.
+__device__ __forceinline__ bool no_maximum(float act_scale, float s) { return act_scale == 0.0f && s == 0.0f; }
+
 __device__ __forceinline__ float seq_dot(const TkProblem &pr, int p, int n, int tok, int a8) {
   const float s = a8 ? pr.aux[tok] : 0.0f;
-  const int gamma_zero = a8 && pr.act_scale[tok] == 0.0f;
+  const int gamma_zero = a8 && no_maximum(pr.act_scale[tok], s);
   return seq_dot_raw(pr.codes[p], pr.nb, pr.k, pr.raw_act, pr.raw_dtype, n, tok, a8, s, gamma_zero);
 }
 

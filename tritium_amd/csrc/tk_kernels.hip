@@ -2519,8 +2519,8 @@ __device__ __forceinline__ void exact_rows_fused(const TkProblem &pr, int n, int
     float f = 0.0f;
     for (int p = 0; p < pr.planes; ++p) {
       // behind an RMSNorm (one token) the row to re-quantize is the normalized one, left in LDS by the staging
-      const float dot = pr.norm_kind ? seq_dot_a8_lds(pr.codes[p], pr.nb, pr.k, (const float *)(cst + 1024), n, s, as == 0.0f)
-                                     : seq_dot_raw(pr.codes[p], pr.nb, pr.k, pr.raw_act, pr.raw_dtype, n, m, a8 ? 1 : 0, s, a8 && as == 0.0f);
+      const float dot = pr.norm_kind ? seq_dot_a8_lds(pr.codes[p], pr.nb, pr.k, (const float *)(cst + 1024), n, s, no_maximum(as, s))
+                                     : seq_dot_raw(pr.codes[p], pr.nb, pr.k, pr.raw_act, pr.raw_dtype, n, m, a8 ? 1 : 0, s, a8 && no_maximum(as, s));
       float t = __fmul_rn(dot, pr.scales[p][n]);
       f = p == 0 ? t : __fadd_rn(f, t);
     }
