@@ -4,6 +4,9 @@ dequantize-then-fold within the reference's 1e-4 (crates/tritium-cuda/kernels/tq
 exact forward and the row gather must carry the bits of the CPU reference's pinned order
 (crates/tritium-cpu/src/salt_v2.rs:10-23,316-423), for all three codecs, ragged tiles and both scale groups;
 non-finite inputs or results are refused and leave the output untouched (crates/tritium-cuda/src/cuda/tests.rs:246-280)."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -213,8 +216,8 @@ def test_v2_matrix_form_at_its_edges(backend, so, codec, n, k, group, m):
 
 @pytest.mark.parametrize("m,bad", [(3, False), (20, False), (3, True), (20, True)])
 def test_v2_output_over_the_activations(backend, so, m, bad):
-    """Results go straight to the output and a refused call puts back what it held; an output that is the activation tensor itself is
-    staged: the bits of a call with its own output, and the activations untouched by a refused one."""
+    """An output that is the activation tensor itself: the bits of a call with its own output, and the activations untouched by a
+    refused one."""
     rng = np.random.default_rng(m)
     n = k = 256
     tiles = n * k // 256
@@ -239,4 +242,98 @@ def test_v2_output_over_the_activations(backend, so, m, bad):
         assert (dact.to_host().view(np.uint32) == want.view(np.uint32)).all()
     for x in (dact, dout):
         x.free()
+    dev.free()
+
+
+def _v2_rows(so, rng, n, k, scale=None):
+    """Two planes of D2 in every tile, scale groups of 128; scale: the f16 bits of every scale instead of random ones"""
+    return S.V2Tensor(so, S.D2, 128, n, k, [(rng.integers(-1, 2, (2, 256)).astype(np.int8),
+                                             np.full((2, 2), scale, np.uint16) if scale else rng.uniform(0.1, 1.0, (2, 2)).astype(np.float16).view(np.uint16))
+                                            for _ in range(n * k // 256)])
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 33])
+def test_v2_results_that_may_not_be_finite(backend, so, m):
+    """Up to 16 tokens of moderate size write their results at once; activations beyond 2^64, from which a result may overflow, and
+    tensors with a scale that is not finite are staged, as are more tokens: the reference's bits where the call is good, a refusal and an untouched output
+    where it is not. Activations on both sides of 2^64, one alone among small ones."""
+    print("case salt-v2 large", m, flush=True)
+    rng = np.random.default_rng(m)
+    n, k = 40, 512
+    t, inf_scale = _v2_rows(so, rng, n, k), _v2_rows(so, rng, n, k, 0x7C00)
+    dev = backend.salt_v2_upload(S.D2, 128, t.payload, t.scales, t.plane_counts, n, k)
+    dev_inf = backend.salt_v2_upload(S.D2, 128, inf_scale.payload, inf_scale.scales, inf_scale.plane_counts, n, k)
+    small = rng.standard_normal((m, k)).astype(np.float32)
+    held = rng.standard_normal(m * n).astype(np.float32)
+    held[::5] = np.nan
+    dact, dout = backend.to_device(small, "f32"), backend.to_device(held, "f32")
+    edge = np.float32(2.0 ** 64)
+    good = [small, small * np.float32(1e30)]
+    for v in (edge, np.nextafter(edge, np.float32(np.inf)), -np.float32(1e33)):
+        a = small.copy()
+        a[m - 1, k - 3] = v
+        good.append(a)
+    for act in good:
+        rc, want = so.v2_forward(t, act, m)
+        assert rc == 0
+        dact.copy_from(act)
+        dev.forward(dact, m, dout)
+        assert same_bits(dout.to_host().reshape(m, n), want)
+    over = small.copy()
+    over[m - 1] = np.float32(3e38)
+    nan = small.copy()
+    nan[0, 1] = np.nan
+    dout.copy_from(held)
+    for tensor, act in ((dev, over), (dev, nan), (dev_inf, small)):
+        dact.copy_from(act)
+        with pytest.raises(T.InvalidInput):
+            tensor.forward(dact, m, dout)
+        assert (dout.to_host().view(np.uint32) == held.view(np.uint32)).all()
+    for x in (dact, dout):
+        x.free()
+    dev.free()
+    dev_inf.free()
+
+
+@pytest.mark.parametrize("m", [16, 64])
+def test_v2_refused_calls_never_write_the_output(backend, so, m):
+    """What a refused call leaves untouched is untouched throughout: the output lies in host memory, and another thread looks at it
+    while calls with one bad activation come back refused."""
+    print("case salt-v2 untouched", m, flush=True)
+    rng = np.random.default_rng(m)
+    n, k = 2048, 512
+    t = _v2_rows(so, rng, n, k)
+    dev = backend.salt_v2_upload(S.D2, 128, t.payload, t.scales, t.plane_counts, n, k)
+    act = rng.standard_normal((m, k)).astype(np.float32)
+    act[m - 1, k - 1] = np.inf
+    dact = backend.to_device(act, "f32")
+    hip = ctypes.CDLL("libamdhip64.so.7")  # (the runtime that the library has loaded)
+    memory = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(memory), ctypes.c_size_t(m * n * 4), 0) == 0
+    view = np.frombuffer((ctypes.c_float * (m * n)).from_address(memory.value), np.float32)
+    view[:] = 19.0
+    out = T.DeviceArray(backend, memory, m * n, T.backend.DTYPES["f32"])
+    refused, done = [], threading.Event()
+
+    def caller():
+        try:
+            for _ in range(60):
+                try:
+                    dev.forward(dact, m, out)
+                except T.InvalidInput:
+                    refused.append(True)
+        finally:
+            done.set()
+
+    looks, intact = 0, True
+    thread = threading.Thread(target=caller)
+    thread.start()
+    while not done.is_set():
+        intact = intact and bool((view == np.float32(19.0)).all())
+        looks += 1
+    thread.join()
+    assert len(refused) == 60 and looks > 60
+    assert intact and (view == np.float32(19.0)).all()
+    assert hip.hipHostFree(memory) == 0
+    dact.free()
     dev.free()

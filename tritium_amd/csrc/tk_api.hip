@@ -103,7 +103,7 @@ struct tk_ctx {
   int flow_swap = 1;       // flow kernel, int8 contract: 1 = weights as the first operand of the matrix instruction (one wide store per lane), 0 = activations first
   int base3 = 0;           // uploads: 0 = no base-3 stream, 1 = TQ1_0 uploads keep one beside the 2-bit codes, 2 = every upload
   unsigned *d_count = nullptr;  // a device counter for the uploads
-  unsigned *d_salt = nullptr;   // SALT V2: the flag of a call where no pinned memory is to be had
+  unsigned *d_salt = nullptr;   // SALT V2: [0] the number of the last staged call that met a non-finite value, [1] a call's verdict where no pinned memory is to be had
   unsigned salt_calls = 0;
 
   uint8_t *static_scratch = nullptr;  // this device's copy of `scratch` (below), resolved at tk_init
@@ -1858,6 +1858,7 @@ struct tk_salt_v2 {
   tk_ctx *ctx;
   void *payload, *scales, *tile_begin;
   TkSaltV2 dev;
+  bool finite_scales;  // no scale is Inf or NaN
 };
 
 extern "C" int tk_salt_v2_upload(tk_ctx *ctx, int codec, size_t scale_group, const uint8_t *payload, size_t payload_len,
@@ -1941,6 +1942,8 @@ extern "C" int tk_salt_v2_upload(tk_ctx *ctx, int codec, size_t scale_group, con
   w->dev.group = (unsigned)scale_group;
   w->dev.tiles = (unsigned)tiles;
   w->dev.total = total;
+  w->finite_scales = true;
+  for (size_t i = 0; i < scale_count; ++i) w->finite_scales = w->finite_scales && (scales_f16[i] & 0x7C00u) != 0x7C00u;
   ctx->refs.fetch_add(1);
   *out = w;
   return TK_OK;
@@ -1961,6 +1964,8 @@ extern "C" void tk_salt_v2_free(tk_salt_v2 *t) {
   ctx_release(ctx);
 }
 
+static const char *const kSaltV2NotFinite = "SALT V2 forward: a non-finite activation or result; the output was not written";
+
 extern "C" int tk_salt_v2_forward(tk_ctx *ctx, const tk_salt_v2 *t, const float *act, size_t m, float *out) {
   if (!ctx || !t) return tk_fail(TK_ERR_INVALID_INPUT, "tk_salt_v2_forward: null pointer");
   if (t->ctx != ctx) return tk_fail(TK_ERR_INVALID_INPUT, "tensor belongs to another context");
@@ -1971,28 +1976,38 @@ extern "C" int tk_salt_v2_forward(tk_ctx *ctx, const tk_salt_v2 *t, const float 
   HIPCHK(hipSetDevice(ctx->device));
   const size_t bytes = m * (size_t)t->dev.n * sizeof(float);
   TKCHK(ensure(ctx, ctx->tmp, bytes));
-  // The results go straight to `out`, and what it held to the workspace: a bad call (a non-finite activation or result; it leaves its
-  // own number in the flag, so nothing is cleared in front) puts that back before it returns. The flag is a word of the pinned block:
-  // nothing is copied behind. (Results staged and copied by a second launch: 37.6 us for 4096 x 4096, B3, 8 tokens, so 34.8.) An output
-  // that overlaps the activations is staged.
-  if (++ctx->salt_calls == 0) ctx->salt_calls = 1;  // numbers start over
-  (void)ensure_pin(ctx, sizeof(unsigned));
+  (void)ensure_pin(ctx, 2 * sizeof(unsigned));
   const size_t count = m * (size_t)t->dev.n;
   const uintptr_t a0 = (uintptr_t)act, a1 = a0 + m * (size_t)t->dev.k * 4, o0 = (uintptr_t)out, o1 = o0 + bytes;
-  const bool staged = a0 < o1 && o0 < a1;
-  unsigned flag = 0, *verdict = ctx->pin ? (unsigned *)ctx->pin : ctx->d_salt;
-  if (ctx->pin) *(volatile unsigned *)verdict = 0;
-  else HIPCHK(hipMemsetAsync(verdict, 0, sizeof(unsigned), ctx->stream));
-  HIPCHK(tk_launch_salt_v2_forward(ctx->stream, t->dev, act, m, staged ? (float *)ctx->tmp.p : out, staged ? nullptr : (float *)ctx->tmp.p, verdict, ctx->salt_calls));
-  if (staged) HIPCHK(tk_launch_salt_v2_commit(ctx->stream, (const float *)ctx->tmp.p, out, count, verdict, ctx->salt_calls));
+  if (ctx->pin && t->finite_scales && tk_salt_v2_direct(t->dev, m) && !(a0 < o1 && o0 < a1)) {
+    // One block of tokens: every workgroup sees all activations, and unless one of them is so large that a result may not be finite, the
+    // results go straight to `out` (a second launch that moves them: 4096 x 4096, B3, 8 tokens 37.6 us, so 34.8). Otherwise they are
+    // staged, and moved when the call is known to be good: `out` is never written by a call that is refused.
+    volatile unsigned *const word = (volatile unsigned *)ctx->pin;  // [0] not finite, [1] staged
+    word[0] = word[1] = 0;
+    HIPCHK(tk_launch_salt_v2_forward(ctx->stream, t->dev, act, m, out, (float *)ctx->tmp.p, (unsigned *)ctx->pin, 1u, (unsigned *)ctx->pin + 1));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (word[0]) return tk_fail(TK_ERR_INVALID_INPUT, "%s", kSaltV2NotFinite);
+    if (word[1]) {
+      HIPCHK(tk_launch_salt_v2_commit(ctx->stream, (const float *)ctx->tmp.p, out, count, nullptr, 0, nullptr));
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
+    return TK_OK;
+  }
+  // The verdict comes back through the pinned block, and a bad call leaves its own number: no clearing launch in front and
+  // no copy behind (4096 x 4096, B3, 8 tokens, call 50 -> 38 us)
+  if (++ctx->salt_calls == 0) {  // numbers start over
+    HIPCHK(hipMemsetAsync(ctx->d_salt, 0, sizeof(unsigned), ctx->stream));
+    ctx->salt_calls = 1;
+  }
+  unsigned flag = 0, *verdict = ctx->pin ? (unsigned *)ctx->pin : ctx->d_salt + 1;
+  HIPCHK(tk_launch_salt_v2_forward(ctx->stream, t->dev, act, m, nullptr, (float *)ctx->tmp.p, ctx->d_salt, ctx->salt_calls, nullptr));
+  // the device commits the results only when the flag stayed clear: one synchronization per call
+  HIPCHK(tk_launch_salt_v2_commit(ctx->stream, (const float *)ctx->tmp.p, out, count, ctx->d_salt, ctx->salt_calls, verdict));
   if (!ctx->pin) HIPCHK(hipMemcpyAsync(&flag, verdict, sizeof flag, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   if (ctx->pin) flag = *(volatile unsigned *)verdict;
-  if (flag && !staged) {
-    HIPCHK(tk_launch_salt_v2_commit(ctx->stream, (const float *)ctx->tmp.p, out, count, nullptr, 0));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-  }
-  if (flag) return tk_fail(TK_ERR_INVALID_INPUT, "SALT V2 forward: a non-finite activation or result; the output was not written");
+  if (flag) return tk_fail(TK_ERR_INVALID_INPUT, "%s", kSaltV2NotFinite);
   return TK_OK;
 }
 

@@ -257,12 +257,15 @@ struct TkSaltV2 {
 // tokens one workgroup carries through a weight row, and the LDS a launch needs for rows of k columns
 #define TK_SALT_V2_TOKENS 8
 size_t tk_salt_v2_lds_bytes(size_t k, size_t group);
-// out receives the [m,n] results; *flag becomes `call` (never its value before) when an activation or a result is not finite. keep, if
-// not null, receives what `out` held before (which the caller then puts back)
-hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *out, float *keep, unsigned *flag,
-                                     unsigned call);
-// out[i] = tmp[i] for i < count unless *flag is `call` (flag may be null: always)
-hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call);
+// tmp receives the [m,n] results; *flag becomes `call` (never its value before) when an activation or a result is not finite.
+// out, where tk_salt_v2_direct allows it and every scale is finite, receives them instead if no call with such activations can be
+// refused; where it may be, *spill becomes 1 and they are in tmp. out must not overlap the activations.
+bool tk_salt_v2_direct(const TkSaltV2 &t, size_t m);
+hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *out, float *tmp, unsigned *flag,
+                                     unsigned call, unsigned *spill);
+// out[i] = tmp[i] for i < count unless *flag is `call` (then nothing is written); *verdict = whether it was. flag null: always
+hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call,
+                                    unsigned *verdict);
 hipError_t tk_launch_salt_v2_gather(hipStream_t s, const TkSaltV2 &t, const uint32_t *rows, size_t count, float *out);
 #ifdef __cplusplus
 }

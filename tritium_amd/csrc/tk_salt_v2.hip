@@ -139,8 +139,7 @@ __device__ __forceinline__ float f16_to_f32(uint16_t h) {
 // LDS: float term[segments][3 planes][tokens], then one plane count per segment.
 // Segment boundaries are the multiples of the scale group (which divides the 256 of a tile).
 __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
-                                                                float *__restrict__ out, float *__restrict__ keep, unsigned *__restrict__ flag,
-                                                                unsigned call) {
+                                                                float *__restrict__ out, unsigned *__restrict__ flag, unsigned call) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int MT = TK_SALT_V2_TOKENS;
   const unsigned row = blockIdx.x, tok0 = blockIdx.y * MT;
@@ -193,9 +192,7 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
       for (unsigned j = 0; j < seg_planes[s]; ++j) accumulator = __fadd_rn(accumulator, term[((size_t)s * 3 + j) * MT + threadIdx.x]);
     // an accumulator that left the finite range never comes back (inf - inf is NaN): the end result tells
     bad |= !(fabsf(accumulator) <= 3.402823466e38f);
-    const size_t at = (size_t)(tok0 + threadIdx.x) * t.n + row;
-    if (keep) gstore(keep + at, gload(out + at));
-    out[at] = accumulator;
+    out[(size_t)(tok0 + threadIdx.x) * t.n + row] = accumulator;
   }
   if (bad) gstore(flag, call);  // (whoever stores, stores the same)
 }
@@ -212,18 +209,25 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
 // Floor: the f32 matrix pipe, 32 cycles per 16 x 16 x 4 (7 us at the size below); the recoding and the latency of the loads add to it.
 // 4096 x 4096, two planes, kernels, 8 tokens of B3: 64 us (fold with a lane per row, terms through memory) + 12 us (their sum) ->
 // 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 35 / 37 / 38 us, one token 57 / 69 / 66 -> 33 / 36 / 37, 64 tokens 302 / 389 / 353 ->
-// 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory), without a launch that commits the results 33 / 35 us (D2 / B3). (A segment's codes
-// and activations requested ahead of the fold before it: 38.8 against 35.5 for B3.) (With the activations as 32 four-byte loads per lane and the codes as single bytes the kernel took 52 us: the
-// loads of 16 rows a few KiB apart were the bound.)
+// 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory); up to 16 tokens of moderate size, whose results
+// need no launch that commits them, 35 / 37 -> 32 / 34 (D2 / B3, 8 tokens). A segment's codes and activations requested ahead of the
+// fold before it: 38.8 against 35.5 for B3. With the activations as 32 four-byte loads per lane and the codes as single bytes the
+// kernel took 52 us: the loads of 16 rows a few KiB apart were the bound.
 constexpr int SV2_WAVES = 16, SV2_SLOTS = 48, SV2_HEAD = 528;
+// out (null: not asked for): a call of one block of tokens writes its results there at once if none of its activations exceeds
+// SV2_TAME in magnitude, else to tmp, and says so in *spill. With finite scales (the host's condition) results of such activations are below
+// 3 k * SV2_TAME * 2^16, which is finite for every k that is staged, and every workgroup reads all activations: none can
+// refuse the call once one has written.
+constexpr float SV2_TAME = 18446744073709551616.0f;  // 2^64
 template <int G>
 __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
-                                                                          float *__restrict__ out, float *__restrict__ keep,
-                                                                          unsigned *__restrict__ flag, unsigned call, unsigned slots) {
+                                                                          float *__restrict__ out, float *__restrict__ tmp,
+                                                                          unsigned *__restrict__ flag, unsigned call,
+                                                                          unsigned *__restrict__ spill, unsigned slots) {
   constexpr int W = G / 64;  // words of sixteen codes per lane and fold
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   uint16_t *s_fields = (uint16_t *)smem;                                   // [256], B3: the digits of a byte
-  int *s_three = (int *)(smem + 512);                                      // some tile of the workgroup has three planes
+  int *s_three = (int *)(smem + 512), *s_wild = s_three + 1;               // some tile has three planes; some activation is beyond SV2_TAME
   float *s_term = (float *)(smem + SV2_HEAD);                              // [slot][plane][accumulator register][lane]
   uint8_t *s_planes = smem + SV2_HEAD + (size_t)slots * 3 * 256 * sizeof(float);  // [slot][row]
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4;
@@ -234,11 +238,8 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
   const unsigned final_row = blockIdx.x * 16u + c, final_tok = tok0 + h * 4 + wave;  // of the thread that adds (waves 0..3)
   const size_t final_at = (size_t)min(final_tok, m - 1u) * t.n + min(final_row, t.n - 1u);
   const bool ends = wave < 4 && final_row < t.n && final_tok < m;
-  float before = 0.0f;  // what a bad call puts back
-  if (keep && ends) before = gload(out + final_at);
-  float sum = 0.0f;
-  bool bad = false;
-  if (threadIdx.x == 0) *s_three = 0;
+  float sum = 0.0f, top = 0.0f;  // (top: the largest magnitude this lane has seen; NaN stays)
+  if (threadIdx.x == 0) *s_three = *s_wild = 0;
   if (codec == TK_SALT_V2_B3 && threadIdx.x < 256) s_fields[threadIdx.x] = (uint16_t)b3_fields(threadIdx.x);
   __syncthreads();
   typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
@@ -284,10 +285,8 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
       const unsigned local = cur.local, most = cur.most;
       if (h == 0) s_planes[slot * 16 + c] = (uint8_t)cur.planes;
       if (most == 3u && lane == 0) *s_three = 1;
-      if (blockIdx.x == 0) {  // every activation passes here
 #pragma unroll
-        for (int x = 0; x < W * 16; ++x) bad |= !(fabsf(a[x / 4][x % 4]) <= 3.402823466e38f);
-      }
+      for (int x = 0; x < W * 16; ++x) top = __builtin_elementwise_maximum(top, fabsf(a[x / 4][x % 4]));
 #pragma unroll
       for (int w = 0; w < W * 4; ++w) transpose_rows(a[w]);
 #pragma unroll
@@ -315,6 +314,7 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
         for (int r = 0; r < 4; ++r) s_term[((slot * 3 + j) * 4 + r) * 64 + lane] = __fmul_rn(acc[r], sc);
       }
     }
+    if (!(top <= SV2_TAME)) *s_wild = 1;
     __syncthreads();
     if (wave < 4) {
       auto add = [&](auto np_c) {
@@ -334,21 +334,27 @@ __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSalt
     }
     __syncthreads();
   }
+  const bool wild = *s_wild;
+  bool bad = !(top <= 3.402823466e38f);
   if (ends) {
     // an accumulator that left the finite range never comes back (inf - inf is NaN): the end result tells
     bad |= !(fabsf(sum) <= 3.402823466e38f);
-    if (keep) gstore(keep + final_at, before);
-    gstore(out + final_at, sum);
+    gstore((out && !wild ? out : tmp) + final_at, sum);
   }
+  if (out && wild && threadIdx.x == 0) gstore(spill, 1u);
   if (bad) gstore(flag, call);  // (whoever stores, stores the same)
 }
 
-// out[i] = tmp[i] unless *flag is `call`: the results of a call whose output overlaps its activations leave the staging buffer
-// this way; without a flag the values that a bad call replaced go back.
+// The results leave the staging buffer only when no activation and no result was found non-finite: the flag then holds the
+// number of an earlier call (so it is never cleared). *verdict, in host memory, says which it was. Without a flag (the host has
+// looked): always.
 __global__ __launch_bounds__(TK_WG) void tk_salt_v2_commit_kernel(const float *__restrict__ tmp, float *__restrict__ out, size_t count,
-                                                                  const unsigned *__restrict__ flag, unsigned call) {
+                                                                  const unsigned *__restrict__ flag, unsigned call,
+                                                                  unsigned *__restrict__ verdict) {
+  const bool bad = flag && gload(flag) == call;
   const size_t idx = (size_t)blockIdx.x * TK_WG + threadIdx.x;
-  if (idx < count && !(flag && gload(flag) == call)) gstore(out + idx, gload(tmp + idx));
+  if (flag && idx == 0) gstore(verdict, bad ? 1u : 0u);
+  if (!bad && idx < count) gstore(out + idx, gload(tmp + idx));
 }
 
 // One thread per gathered coefficient (crates/tritium-cuda/kernels/salt_v2.cu:218-304).
@@ -378,9 +384,12 @@ size_t tk_salt_v2_lds_bytes(size_t k, size_t group) {
   return nseg * 3 * TK_SALT_V2_TOKENS * sizeof(float) + ((nseg + 15) & ~(size_t)15);
 }
 
-hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *out, float *keep, unsigned *flag,
-                                     unsigned call) {
+bool tk_salt_v2_direct(const TkSaltV2 &t, size_t m) { return t.k && t.k % t.group == 0 && m <= 16; }
+
+hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const float *act, size_t m, float *out, float *tmp, unsigned *flag,
+                                     unsigned call, unsigned *spill) {
   if (!m || !t.n) return hipSuccess;
+  if (out && !tk_salt_v2_direct(t, m)) return hipErrorInvalidValue;
   if (t.k && t.k % t.group == 0) {
     const dim3 grid((t.n + 15) / 16, (unsigned)((m + 15) / 16)), block(SV2_WAVES * 64);
     const unsigned nseg = t.k / t.group, slots = nseg < SV2_SLOTS ? nseg : SV2_SLOTS;
@@ -389,23 +398,24 @@ hipError_t tk_launch_salt_v2_forward(hipStream_t s, const TkSaltV2 &t, const flo
       const hipError_t e = tk_raise_lds_limit(t.group == 128 ? (const void *)tk_salt_v2_exact_kernel<128> : (const void *)tk_salt_v2_exact_kernel<64>, 160 * 1024);
       if (e != hipSuccess) return e;
     }
-    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, out, keep, flag, call, slots);
-    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, out, keep, flag, call, slots);
+    if (t.group == 128) hipLaunchKernelGGL(tk_salt_v2_exact_kernel<128>, grid, block, lds, s, t, act, (unsigned)m, out, tmp, flag, call, spill, slots);
+    else hipLaunchKernelGGL(tk_salt_v2_exact_kernel<64>, grid, block, lds, s, t, act, (unsigned)m, out, tmp, flag, call, spill, slots);
     return hipGetLastError();
   }
   const size_t lds = tk_salt_v2_lds_bytes(t.k, t.group);
   if (lds > 64 * 1024) {
-    hipError_t e = tk_raise_lds_limit((const void *)tk_salt_v2_forward_kernel, 160 * 1024);
+    const hipError_t e = tk_raise_lds_limit((const void *)tk_salt_v2_forward_kernel, 160 * 1024);
     if (e != hipSuccess) return e;
   }
   const dim3 grid(t.n, (unsigned)((m + TK_SALT_V2_TOKENS - 1) / TK_SALT_V2_TOKENS));
-  hipLaunchKernelGGL(tk_salt_v2_forward_kernel, grid, dim3(64), lds, s, t, act, (unsigned)m, out, keep, flag, call);
+  hipLaunchKernelGGL(tk_salt_v2_forward_kernel, grid, dim3(64), lds, s, t, act, (unsigned)m, tmp, flag, call);
   return hipGetLastError();
 }
 
-hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call) {
+hipError_t tk_launch_salt_v2_commit(hipStream_t s, const float *tmp, float *out, size_t count, const unsigned *flag, unsigned call,
+                                    unsigned *verdict) {
   if (!count) return hipSuccess;
-  hipLaunchKernelGGL(tk_salt_v2_commit_kernel, dim3((unsigned)((count + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, tmp, out, count, flag, call);
+  hipLaunchKernelGGL(tk_salt_v2_commit_kernel, dim3((unsigned)((count + TK_WG - 1) / TK_WG)), dim3(TK_WG), 0, s, tmp, out, count, flag, call, verdict);
   return hipGetLastError();
 }
 
