@@ -103,7 +103,7 @@ def test_prefill_kernel_128_rows(backend, oracle, m, n, k):
     want = oracle.cpu_linear_a8_planes(packed, FMT_TQ2_0, scs, act, m, n, k)
     nan = np.isnan(want)
     got = {}
-    for rows in (128, 64):
+    for rows in (132, 136, 64):  # 128 rows on four and on eight waves
         backend.set_gemm_rows(rows)
         dout = backend.empty(m * n, "f32")
         backend.linear_a8(layer, dact, m, dout)
@@ -117,15 +117,16 @@ def test_prefill_kernel_128_rows(backend, oracle, m, n, k):
         dout.free()
         dob.free()
     # int8 rows in, with and without per-token scales
-    backend.set_gemm_rows(128)
     q = rng.integers(-128, 128, (m, k)).astype(np.int8)
     asc = rng.uniform(0.01, 0.2, m).astype(np.float32)
     dq, dsc, do = backend.to_device(q, "i8"), backend.to_device(asc, "f32"), backend.empty(m * n, "f32")
     acc = oracle.int8_accumulators(packed[0], FMT_TQ2_0, q, m, n, k).astype(np.float32)
-    backend.linear_i8(layer, dq, dsc, m, do)
-    assert same_bits(do.to_host().reshape(m, n), (acc * scs[0][None, :]) * asc[:, None])
-    backend.linear_i8(layer, dq, None, m, do)
-    assert same_bits(do.to_host().reshape(m, n), acc * scs[0][None, :])
+    for rows in (132, 136):
+        backend.set_gemm_rows(rows)
+        backend.linear_i8(layer, dq, dsc, m, do)
+        assert same_bits(do.to_host().reshape(m, n), (acc * scs[0][None, :]) * asc[:, None])
+        backend.linear_i8(layer, dq, None, m, do)
+        assert same_bits(do.to_host().reshape(m, n), acc * scs[0][None, :])
     for a in (dact, dq, dsc, do):
         a.free()
     layer.free()
@@ -156,11 +157,12 @@ def test_prefill_kernel_128_rows_planes_and_contracts(backend, oracle, m, n, k, 
     want = oracle.cpu_linear_a8_planes(packed, FMT_TQ2_0, scs, act, m, n, k)
     nan = np.isnan(want)
     got = {}
-    for rows in (128, 64):
+    for rows in (132, 136, 64) if planes == 1 else (128, 64):
         backend.set_gemm_rows(rows)
+        kernel = "gemm64" if rows == 64 else "gemm128"
         out, outb = backend.empty(m * n, "f32"), backend.empty(m * n, "bf16")
         backend.linear_a8(layer, dact, m, out)
-        assert backend.last_kernel().split("_")[0] == f"gemm{rows}", backend.last_kernel()
+        assert backend.last_kernel().split("_")[0] == kernel, backend.last_kernel()
         g = out.to_host().reshape(m, n)
         assert (np.isnan(g) == nan).all() and same_bits(g[~nan], want[~nan])
         backend.linear_a8(layer, dact, m, outb)
@@ -168,23 +170,48 @@ def test_prefill_kernel_128_rows_planes_and_contracts(backend, oracle, m, n, k, 
         backend.linear_a8_residual(layer, dact, m, dres, out)
         assert same_bits(out.to_host().reshape(m, n)[~nan], (res + want)[~nan])
         backend.linear_float(layer, dact, m, out)
-        assert backend.last_kernel().split("_")[0] == f"gemm{rows}", backend.last_kernel()
+        assert backend.last_kernel().split("_")[0] == kernel, backend.last_kernel()
         got[rows] = out.to_host().reshape(m, n)
         assert np.abs(got[rows][plain] - exact[plain]).max() <= 1e-5 * np.abs(exact).max()
         backend.linear_float(layer, dact, m, outb)
         assert (outb.to_host().reshape(m, n)[plain] == f32_to_bf16_bits(got[rows])[plain]).all()
         out.free()
         outb.free()
-    assert (got[64].view(np.uint32) == got[128].view(np.uint32)).all()
+    for rows in got:
+        assert (got[64].view(np.uint32) == got[rows].view(np.uint32)).all()
     if planes == 1:
-        backend.set_gemm_rows(128)
         q = rng.integers(-128, 128, (m, k)).astype(np.int8)
         dq, dacc = backend.to_device(q, "i8"), backend.empty(m * n, "i32")
-        backend.linear_i8(layer, dq, None, m, dacc)
-        assert (dacc.to_host().reshape(m, n) == oracle.int8_accumulators(packed[0], FMT_TQ2_0, q, m, n, k)).all()
+        for rows in (132, 136):
+            backend.set_gemm_rows(rows)
+            backend.linear_i8(layer, dq, None, m, dacc)
+            assert (dacc.to_host().reshape(m, n) == oracle.int8_accumulators(packed[0], FMT_TQ2_0, q, m, n, k)).all()
         for a in (dq, dacc):
             a.free()
     for a in (dact, dres):
+        a.free()
+    layer.free()
+
+
+@pytest.mark.parametrize("m,n,k,planes,kernel", [(768, 10880, 2048, 2, "gemm64"), (768, 9600, 2048, 2, "gemm128"), (1024, 15360, 1024, 1, "gemm128"),
+                                                 (2048, 3328, 2048, 1, "gemm128"), (1024, 6144, 1024, 1, "gemm64")])
+def test_prefill_kernel_by_the_fullest_xcd(backend, m, n, k, planes, kernel):
+    """An XCD takes a sub-grid of a prefill launch as a whole: 85 column blocks of two planes are eleven on seven XCDs, 66 workgroups
+    of the 128-row kernel for 64 places, and the launch a third round (47 us against 41 through the 64-row kernel). And launches of one
+    plane that the 128-row kernel finishes in one round, on short rows as well (K=1024 N=15360 26.5 us against 29.4)."""
+    print("case prefill-dispatch", m, n, k, planes, flush=True)
+    if backend.info.compute_units != 256:
+        pytest.skip("counts of a chip of 256 CUs")
+    rng = np.random.default_rng(n)
+    packed = [T.pack_rows(rng.integers(-1, 2, (n, k)).astype(np.int8), n, k) for _ in range(planes)]
+    layer = backend.linear(packed, [scales(rng, n) for _ in range(planes)], n, k)
+    act, out, ref = backend.to_device(rng.standard_normal((m, k)).astype(np.float32), "f32"), backend.empty(m * n, "f32"), backend.empty(m * n, "f32")
+    backend.linear_a8(layer, act, m, out)
+    assert backend.last_kernel() == kernel
+    backend.set_gemm_rows(64)
+    backend.linear_a8(layer, act, m, ref)
+    assert same_bits(out.to_host(), ref.to_host())
+    for a in (act, out, ref):
         a.free()
     layer.free()
 

@@ -613,7 +613,8 @@ class Mi355xBackend:
         return self._lib.tk_last_kernel(self._ctx).decode()
 
     def set_gemm_rows(self, rows):
-        """0 = automatic, 64 / 128 / 256 = rows of the workgroup tile of single prefill launches (256: one plane, int8 contract)."""
+        """0 = automatic, 64 / 128 / 256 = rows of the workgroup tile of single prefill launches (256: one plane, int8 contract;
+        132 / 136: 128 rows, one plane on four / eight waves)."""
         _check(self._lib.tk_set_gemm_rows(self._ctx, rows))
 
     def set_gemm256_form(self, form):

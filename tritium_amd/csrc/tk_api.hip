@@ -95,7 +95,7 @@ struct tk_ctx {
   // tokens K=2560 N=2560 (2.6 MB) 169 / 148, 256 tokens K=2560 N=6912 (9.7 MB) 526 / 480; K=8192 N=8192 (16.8 MB) 752 / 756)
   size_t host_direct_bytes = (size_t)16 << 20;
   int fuse_tokens = -1;    // single decode calls of up to this many tokens build their operand rows inside the decode kernel (-1 = chosen per call, 0 = never)
-  int gemm_rows = 0;       // one-plane int8-contract prefill, single launches: 0 = tile rows chosen per launch, 64 / 128 / 256 = force
+  int gemm_rows = 0;       // prefill, single launches: 0 = tile rows chosen per launch, 64 / 128 / 256 = force (tk_set_gemm_rows)
   bool gemm256_form_forced = false;  // tk_set_gemm256_form was called: automatic launches keep that form
   int gemm256_form = 0;    // the 256-row kernel: 0 = 4 waves x 224 outputs, 1 = 8 waves x 224, 2 = 4 waves x (128 | 96), two workgroups per CU
   int zero_skip = 0;       // uploads: 0 = keep a zero-chunk map when at least 0.5% of the chunks are zero, 1 = never, 2 = always
@@ -427,8 +427,8 @@ extern "C" const char *tk_last_kernel(tk_ctx *ctx) {
 
 extern "C" int tk_set_gemm_rows(tk_ctx *ctx, int rows) {
   if (!ctx) return tk_fail(TK_ERR_INVALID_INPUT, "tk_set_gemm_rows: null context");
-  if (rows != 0 && rows != 64 && rows != 128 && rows != 256)
-    return tk_fail(TK_ERR_INVALID_INPUT, "gemm_rows=%d - use 0 (automatic), 64, 128 or 256", rows);
+  if (rows != 0 && rows != 64 && rows != 128 && rows != 132 && rows != 136 && rows != 256)
+    return tk_fail(TK_ERR_INVALID_INPUT, "gemm_rows=%d - use 0 (automatic), 64, 128 (132, 136: on four or eight waves) or 256", rows);
   std::lock_guard<std::mutex> lk(ctx->mu);
   ctx->gemm_rows = rows;
   return TK_OK;
@@ -1139,44 +1139,61 @@ static void plan_gemm256(Plan *pl) {
   }
 }
 
-// Time per K block (us at the clock these launches hold) of a prefill launch with x workgroups per CU. A CU runs two (64 rows
-// of one and two planes: three) at a time, so what counts is the CU with the most of them: `full[c - 1]` with c workgroups on
-// every CU, repeating with the slots; a launch that gives only some CUs the last one is a little faster (an eighth at most).
-static double prefill_cost(double x, const double *full, int slots) {
-  const int c = x > 0.0 ? (int)x + (x > (double)(int)x ? 1 : 0) : 1;
-  const double whole = (double)((c - 1) / slots) * full[slots - 1] + full[(c - 1) % slots];
-  const double part = whole * (c > 1 ? 1.0 - 0.12 * ((double)c - x) : 1.0), even = x * full[slots - 1] / slots;
-  return part > even ? part : even;
+// workgroups per CU of a planned prefill launch on its fullest XCD
+static double workgroups_per_cu(const tk_ctx *ctx, const TkProblem &pr) { return 8.0 * (double)pr.sub_m * (double)pr.sub_n / (double)ctx->info.compute_units; }
+
+// What a prefill launch costs (us at the clock these launches hold) apart from what both kernels pay, for x workgroups per CU on
+// the fullest XCD (an XCD takes a sub-grid as a whole: 85 column blocks are eleven on seven XCDs and eight on the last). A CU runs
+// `slots` of them at a time, so what counts is the CU with the most: a K block takes full[c - 1] with c workgroups on every CU,
+// repeating with the slots, and a little less (`part`) where only some CUs have the last one. Every round of workgroups pays
+// `round` for its first loads and last stores.
+struct PrefillCost {
+  int slots;
+  double full[3], part, round;
+};
+static double prefill_cost(const PrefillCost &f, double x, double k_blocks) {
+  const int c = x > 1.0 ? (int)x + (x > (double)(int)x ? 1 : 0) : 1;
+  const double whole = (double)((c - 1) / f.slots) * f.full[f.slots - 1] + f.full[(c - 1) % f.slots];
+  const double part = whole * (1.0 - (c > 1 ? f.part * ((double)c - x) : 0.0)), even = x * f.full[f.slots - 1] / f.slots;
+  return k_blocks * (part > even ? part : even) + f.round * (double)((c - 1) / f.slots + 1);
 }
-// Where the 128-row kernel is chosen over the 64-row one. It moves and expands less per operation, but its tiles are larger: a
-// workgroup takes 256 (three planes: 96 x 384) plane columns x 128 rows where the other takes half of that, a call pays 2.5 us more for its first
-// loads and last stores, and 1.1 workgroups per CU cost as much as two. The figures are the slopes and offsets of calls of 768
-// int8 tokens over K = 2048 and 6144, N = 1024 .. 40960 (64 rows / 128 rows, us at K=6144; 64-row workgroups per CU): one plane
-// 1.9 58 / 53, 2.3 65 / 75, 3.8 98 / 83, 4.5 103 / 115, 6 129 / 125, 7.5 161 / 154; two planes 1.1 46 / 49, 2.3 64 / 74, 3.8 87 / 81, 6 125 / 120;
-// three planes 0.8 43 / 53, 1.1 58 / 52, 1.9 64 / 79, 2.3 90 / 81, 3 93 / 88, 3.8 115 / 120, 4.5 141 / 125, 6 174 / 164, 7.5 226 / 204.
-// One plane of float digit rows loses in every launch measured (512 tokens K=2560 N=6912 44.6 / 46.5, 1024 K=6912 N=2560 76 / 91).
-static bool gemm128_pays(const tk_ctx *ctx, int planes, int mode, size_t rows, size_t n_tiles, size_t k) {
-  if (planes > 3 || (planes == 1 && mode == TK_MODE_DIGITS) || ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit) return false;
-  static const double rows64[3][3] = {{0.0, 0.0, 0.0}, {1.18, 1.72, 2.43}, {1.42, 2.27, 0.0}};
-  static const double rows128[3][2] = {{1.64, 2.9}, {1.6, 2.85}, {1.8, 3.175}};
-  const double cus = (double)ctx->info.compute_units;
-  const size_t tiles = (size_t)tk_gemm128_tiles(planes), tall = (size_t)tk_gemm128_rows(planes);
-  const size_t cols = (n_tiles + tiles - 1) / tiles;
-  const double x64 = (double)(((rows + 63) / 64) * cols) / cus, x128 = (double)(((rows + tall - 1) / tall) * cols) / cus;
-  const double blocks = (double)((k + 127) / 128) * 0.5;  // (the 64-row kernel takes whole K blocks)
-  // one plane, 64 rows: two and four tiles per wave together are nearly linear in the work
-  const double c64 = planes == 1 ? (x64 < 4.0 ? 0.55 + 0.78 * x64 : 0.807 * x64) : prefill_cost(x64, rows64[planes - 1], planes == 2 ? 3 : 2);
-  return (double)num_blocks(k) * c64 > blocks * prefill_cost(x128, rows128[planes - 1], 2) + 2.5;
+// Where the 128-row kernel is chosen over the 64-row one: it moves and expands less per operation, but its tiles are larger and
+// its rounds dearer, so it wins where its workgroups fall better on the CUs. The figures are fitted to 1007 pairs of calls (65 to
+// 4096 tokens, N = 512 .. 32768, K = 512 .. 17408; one to three planes of int8 rows, two and three of float ones): the rule's choice
+// is 0.07% behind the faster kernel on average and more than 4% in three calls, all of K <= 640 and float digits of three planes
+// (1184 tokens K=512 N=14336 111 us against 99). 64 rows / 128 rows, us: one plane, 1024 tokens K=1024, N=6144 16.3 / 18.1, 7680
+// 19.4 / 19.0, 9216 21.8 / 24.4, 15360 29.4 / 26.5, 16384 27.6 / 26.8, 17408 29.6 / 34.8; two planes, 768 tokens K=2048, N=8192
+// 30.5 / 34.5, 9600 36.0 / 35.4, 10880 (85 column blocks) 40.6 / 46.4, 16384 49.3 / 48.8; three planes N=2688 24.9 / 24.1, 5504
+// 36.4 / 34.0, 10880 53.3 / 48.5. One plane of float digit rows loses in every launch measured (512 tokens K=2560 N=6912
+// 44.6 / 46.5, 1024 tokens K=6912 N=2560 76 / 91).
+static bool gemm128_pays(const tk_ctx *ctx, const TkProblem &pr64, int gemm_nt, const TkProblem &pr128) {
+  static const PrefillCost rows64[4] = {{3, {0.372, 0.646, 1.133}, 0.072, 1.32},   // one plane, two tiles per wave
+                                        {3, {0.748, 1.645, 2.43}, 0.058, 1.14},    // one plane, four
+                                        {3, {0.672, 1.174, 1.894}, 0.077, 0.85},   // two planes
+                                        {2, {0.818, 1.5}, 0.0, 1.57}};             // three
+  static const PrefillCost rows128[4] = {{2, {1.119, 2.357}, 0.097, 3.72},
+                                         {2, {1.412, 3.004}, 0.052, 2.97},
+                                         {2, {1.127, 2.216}, 0.066, 2.81},
+                                         {2, {1.196, 2.026}, 0.016, 2.97}};
+  const int planes = pr64.planes;
+  if ((planes == 1 && pr64.mode == TK_MODE_DIGITS) || ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit) return false;
+  const int row = planes == 1 ? (gemm_nt == 2 ? 0 : 1) : planes;
+  const double halves = (double)(((size_t)pr64.k + 127) / 128) * 0.5;  // (the 64-row kernel takes whole K blocks)
+  return prefill_cost(rows64[row], workgroups_per_cu(ctx, pr64), (double)pr64.nb) > prefill_cost(rows128[row], workgroups_per_cu(ctx, pr128), halves);
 }
+// One plane: eight waves of 32 columns where no CU gets a second workgroup (one of four waves leaves each SIMD a single wave),
+// four of 64 elsewhere. 1024 tokens, four / eight waves: K=2048 N=6656 27.3 / 25.7 us, 7680 27.8 / 26.5; K=6912 N=6912 58.4 / 55.4; two
+// workgroups per CU: K=2048 N=15360 38.4 / 39.2.
+static bool gemm128_eight_waves(const tk_ctx *ctx, const TkProblem &pr) { return pr.planes == 1 && workgroups_per_cu(ctx, pr) <= 1.0; }
 
 // Where the 256-row kernel (weight tile expanded once per workgroup) is chosen: launches of 1024 rows or more that give
-// 0.7 .. 1 workgroups per CU, as eight waves of 32 rows over whole 224-output column blocks. A/B on one box, bf16 rows
-// in and out, call incl. quantization, best of the 64-row / 128-row kernels -> this form: 2048 x 2560 -> 6912 (248
-// blocks) 45.6 -> 41.6 us; 1536 x 2560 -> 6912 (186) 40.4 -> 38.9; 2048 x 5120 -> 5120 (184) 62.6 -> 59.8; 4096 x 2560 ->
-// 2560 (192) 42.2 -> 40.8. Outside that window it loses -- one workgroup per CU leaves every round's prologue and
-// epilogue in the open: 1024 x 2048 -> 8192 (148 blocks) 26.7 -> 31.2; 3072 x 2560 -> 6912 (372) 61.8 -> 64.5; 4096 x 17408
-// -> 5120 320 -> 360 -- and the form with two workgroups per CU over 128 | 96 outputs is within 1-2% of the 64-row
-// kernels either way (e.g. 4096 x 5120 -> 17408 282 -> 276, 1024 x 2048 -> 8192 26.7 -> 30.9): not chosen by itself.
+// 0.7 .. 1 workgroups per CU, as eight waves of 32 rows over whole 224-output column blocks. bf16 rows in and out, call incl.
+// quantization, 64 rows / 128 rows / this form: 2048 x 2560 -> 6144 46.2 / 45.8 / 42.2 us; 1536 x 2560 -> 6912 42.2 / 43.3 / 38.5;
+// 1024 x 2560 -> 14336 48.6 / 44.8 / 42.1; 4096 x 2560 -> 2560 42.8 / 46.1 / 41.0; 2048 x 6912 -> 6144 98.5 / 94.3 / 87.0; on short rows it
+// is even at worst by 4% (1024 x 1024 -> 10240 22.1 / 24.4 / 21.9; 2444 x 768 -> 3968 20.6 / 23.1 / 21.5). Outside that window it loses --
+// one workgroup per CU leaves every round's prologue and epilogue in the open: 1024 x 2560 -> 8192 (148 blocks) 33.1 / 32.6 / 36.1;
+// 2048 x 2560 -> 8192 (296) 51.1 / 50.1 / 66.4; 3072 x 6912 -> 5120 (276) 125.6 / 106.5 / 148.9 -- and the form with two workgroups per CU
+// over 128 | 96 outputs was within 1-2% of the 64-row kernels either way: not chosen by itself.
 static bool gemm256_pays(const tk_ctx *ctx, size_t rows, size_t n_tiles, int *form) {
   const size_t cus = (size_t)ctx->info.compute_units;
   const size_t blocks = ((rows + 255) / 256) * ((n_tiles + 13) / 14);
@@ -1539,12 +1556,15 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
       }
       return TK_OK;
     }
-    const bool want128 = ctx->gemm_rows == 128 || (ctx->gemm_rows == 0 && gemm128_pays(ctx, pr.planes, mode, R, (size_t)pr.n_tiles, k));
-    if (can128 && want128) {
-      plan_gemm128(&pl);
-      ctx->last_kernel = "gemm128";
-      HIPCHK(tk_launch_gemm128(ctx->stream, &pr));
-      return TK_OK;
+    const int forced = ctx->gemm_rows;
+    if (can128 && (forced == 0 || (forced >= 128 && forced <= 136))) {
+      Plan tall = pl;
+      plan_gemm128(&tall);
+      if (forced || gemm128_pays(ctx, pr, pl.cfg.gemm_nt, tall.pr)) {
+        ctx->last_kernel = "gemm128";
+        HIPCHK(tk_launch_gemm128(ctx->stream, &tall.pr, forced == 136 || (forced != 132 && gemm128_eight_waves(ctx, tall.pr))));
+        return TK_OK;
+      }
     }
     // A single launch with few workgroups is a latency chain over K per workgroup: cut K into slices.
     // The partial sums cost 4 bytes per accumulator and slice, so few slices: measured, call incl.

@@ -13,13 +13,16 @@
 // trit + 1, so the accumulators start at minus the row sums. Same integers, same epilogue arithmetic: identical bits.
 // A K whose last block holds at most 128 elements has one half block less (its operand rows are zero there).
 //
+// One plane has a second form, eight waves of 32 columns in 128 registers: where a CU has one workgroup, four waves leave every
+// SIMD a single one to hide its loads behind (gemm128_eight_waves in tk_api.hip).
+//
 // Bound: in long launches the chip's power -- registers full of gaussian int8 rows and codes, nothing but matrix instructions,
 // hold 4.0 POPS of the 5.0 that all-zero operands reach (and 3.5 with the weights as the first operand: so activations go first),
 // and interleaving the expansion with the matrix instructions one by one changed nothing. Otherwise the number of workgroups
 // on the CU that has most (gemm128_pays in tk_api.hip). Calls incl. quantization, 64 rows -> 128: 4096 tokens K=5120 N=17408 three
-// planes 759 -> 738 us, 1024 tokens K=5120 N=5120 79 -> 72, 200 tokens N=17408 73 -> 65; 768 tokens K=6144 N=20480 one plane 98 -> 83,
-// two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 -> 41.1 (35.7 with the epilogue and the digit split of now). One workgroup alone on a CU runs its
-// loop at 0.58 of the matrix rate, two at 0.70.
+// planes 759 -> 738 us, 1024 tokens K=5120 N=5120 79 -> 72, 200 tokens N=17408 73 -> 65; 768 tokens K=6144 N=20480 one plane
+// 98 -> 83, two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 -> 41.1 (35.7 with the
+// epilogue and the digit split of now). One workgroup alone on a CU runs its loop at 0.58 of the matrix rate, two at 0.70.
 
 #include <type_traits>
 
@@ -29,21 +32,22 @@ typedef int v16i_g __attribute__((ext_vector_type(16)));
 
 namespace {
 
-constexpr int WAVES = 4, SLOTS = 3, BAND = 4;
+constexpr int SLOTS = 3, BAND = 4;
 
-// P planes, NT tiles of 16 outputs per wave and plane, RT 32-row tiles of operand rows per workgroup
-template <int P>
+// P planes, W waves, NT tiles of 16 outputs per wave and plane, RT 32-row tiles of operand rows per workgroup
+template <int P, int W>
 struct Form {
-  static constexpr int NT = P == 1 ? 4 : 2, RT = P == 3 ? 3 : 4, ROWS = 32 * RT;
+  static constexpr int NT = P == 1 && W == 4 ? 4 : 2, RT = P == 3 ? 3 : 4, ROWS = 32 * RT;
+  static constexpr int LOADS = 4 * RT / W;            // wave-wide DMA loads per wave and half block
   static constexpr int SLOT = ROWS * 128;             // bytes of a half block of operand rows
   static constexpr int CST = SLOTS * SLOT;            // float act_scale[128] | int exps[64] | uint flags[128]
   static constexpr int LDS = CST + 512 + 256 + 512;
 };
 
-template <int P>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void tk_gemm128_kernel(const TkProblem single) {
-  using F = Form<P>;
-  constexpr int NT = F::NT, RT = F::RT, ROWS = F::ROWS, HP = NT / 2, NP = HP * P;
+template <int P, int W>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W / 2, W / 2))) void tk_gemm128_kernel(const TkProblem single) {
+  using F = Form<P, W>;
+  constexpr int WAVES = W, LOADS = F::LOADS, NT = F::NT, RT = F::RT, ROWS = F::ROWS, HP = NT / 2, NP = HP * P;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const TkProblem &pr = *single_problem();
   const TkHot hot = make_hot(pr);
@@ -70,11 +74,11 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
   for (int z = 0; z < HP; ++z)
     w_off[z] = (unsigned)min(tile0 + 2 * z + h, n_tiles - 1) * (unsigned)nb * 1024u + (unsigned)(kappa * 16 + r16) * 16u;
-  // operand rows: a half block is 8 segments (j, kappa) of ROWS pieces, cut into 4 RT wave-wide DMA loads, RT per wave
-  unsigned a_off[RT];
+  // operand rows: a half block is 8 segments (j, kappa) of ROWS pieces, cut into 4 RT wave-wide DMA loads
+  unsigned a_off[LOADS];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const int idx = (wave * RT + i) * 64 + lane, seg = idx / ROWS, row = idx - seg * ROWS;
+  for (int i = 0; i < LOADS; ++i) {
+    const int idx = (wave * LOADS + i) * 64 + lane, seg = idx / ROWS, row = idx - seg * ROWS;
     a_off[i] = (unsigned)((seg >> 1) * 4 + (seg & 1)) * (unsigned)rs * 16u + (unsigned)min(row0 + row, R - 1) * 16u;
   }
   auto load_w = [&](v4i (&w)[NP], int hb) {
@@ -89,9 +93,9 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
   auto dma = [&](int hb, int slot) {
     const uint8_t *base = (const uint8_t *)pr.ap + ((size_t)(hb >> 1) * 16 + (hb & 1) * 2) * (size_t)rs * 16;  // wave-uniform
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
+    for (int i = 0; i < LOADS; ++i)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(base + a_off[i]),
-                                       (__attribute__((address_space(3))) void *)(smem + slot * F::SLOT + (wave * RT + i) * 1024), 16, 0, 0);
+                                       (__attribute__((address_space(3))) void *)(smem + slot * F::SLOT + (wave * LOADS + i) * 1024), 16, 0, 0);
   };
 
   // ---- prologue: constants, minus the row sums, the first two half blocks ----
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
   // wait until at most `ahead` of the youngest half blocks are still in flight
   auto wait_blocks = [&](int ahead) {
     if (ahead <= 0) asm volatile("s_waitcnt vmcnt(0)");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RT + NP));
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + NP));
   };
   auto tie_w = [&](v4i (&w)[NP]) {
 #pragma unroll
@@ -345,24 +349,24 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
   }
 }
 
-template <int P>
+template <int P, int W>
 hipError_t go(hipStream_t s, const TkProblem *single, unsigned wgs) {
-  hipLaunchKernelGGL(tk_gemm128_kernel<P>, dim3(wgs), dim3(WAVES * 64), (size_t)Form<P>::LDS, s, *single);
+  hipLaunchKernelGGL((tk_gemm128_kernel<P, W>), dim3(wgs), dim3(W * 64), (size_t)(Form<P, W>::LDS), s, *single);
   return hipGetLastError();
 }
 
 }  // namespace
 
-int tk_gemm128_rows(int planes) { return planes == 3 ? Form<3>::ROWS : Form<1>::ROWS; }
-int tk_gemm128_tiles(int planes) { return WAVES * (planes == 1 ? Form<1>::NT : Form<2>::NT); }
+int tk_gemm128_rows(int planes) { return planes == 3 ? Form<3, 4>::ROWS : Form<1, 4>::ROWS; }
+int tk_gemm128_tiles(int planes) { return 4 * (planes == 1 ? Form<1, 4>::NT : Form<2, 4>::NT); }
 
-hipError_t tk_launch_gemm128(hipStream_t s, const TkProblem *single) {
+hipError_t tk_launch_gemm128(hipStream_t s, const TkProblem *single, bool eight_waves) {
   const unsigned wgs = 8u * (unsigned)single->sub_m * (unsigned)single->sub_n;
   if (!wgs) return hipSuccess;
   switch (single->planes) {
-    case 1: return go<1>(s, single, wgs);
-    case 2: return go<2>(s, single, wgs);
-    case 3: return go<3>(s, single, wgs);
+    case 1: return eight_waves ? go<1, 8>(s, single, wgs) : go<1, 4>(s, single, wgs);
+    case 2: return go<2, 4>(s, single, wgs);
+    case 3: return go<3, 4>(s, single, wgs);
     default: return hipErrorInvalidValue;
   }
 }
