@@ -559,8 +559,8 @@ int tk_get_fused_calls(tk_ctx *ctx, unsigned long long *count);
  * first call. A static string. For tests of the dispatch; no counterpart in the reference. */
 const char *tk_last_kernel(tk_ctx *ctx);
 /* Row count of the workgroup tile of single prefill launches: 0 = chosen per launch, 64 = the 64-row kernels, 128 = the
- * 128-row kernel (96 rows for three planes; one to three planes, both contracts; one plane on four or eight waves per workgroup
- * as the launch goes, 132 = always four, 136 = always eight), 256 = the 256-row kernel, which expands the
+ * 128-row kernel (96 rows for three planes; one plane under the int8 contract, two and three under both; one plane on four or eight
+ * waves per workgroup as the launch goes, 132 = always four, 136 = always eight), 256 = the 256-row kernel, which expands the
  * weight tile to int8 once per workgroup, in LDS (one plane under the int8 contract, f32 or bf16 rows of whole 16-byte pieces at a
  * 16-byte aligned address, no residual). Launches that the named kernel does not take go to the 64-row kernels. A tuning
  * and test knob: identical bits. */

@@ -1164,8 +1164,7 @@ static double prefill_cost(const PrefillCost &f, double x, double k_blocks) {
 // (1184 tokens K=512 N=14336 111 us against 99). 64 rows / 128 rows, us: one plane, 1024 tokens K=1024, N=6144 16.3 / 18.1, 7680
 // 19.4 / 19.0, 9216 21.8 / 24.4, 15360 29.4 / 26.5, 16384 27.6 / 26.8, 17408 29.6 / 34.8; two planes, 768 tokens K=2048, N=8192
 // 30.5 / 34.5, 9600 36.0 / 35.4, 10880 (85 column blocks) 40.6 / 46.4, 16384 49.3 / 48.8; three planes N=2688 24.9 / 24.1, 5504
-// 36.4 / 34.0, 10880 53.3 / 48.5. One plane of float digit rows loses in every launch measured (512 tokens K=2560 N=6912
-// 44.6 / 46.5, 1024 tokens K=6912 N=2560 76 / 91).
+// 36.4 / 34.0, 10880 53.3 / 48.5.
 static bool gemm128_pays(const tk_ctx *ctx, const TkProblem &pr64, int gemm_nt, const TkProblem &pr128) {
   static const PrefillCost rows64[4] = {{3, {0.372, 0.646, 1.133}, 0.072, 1.32},   // one plane, two tiles per wave
                                         {3, {0.748, 1.645, 2.43}, 0.058, 1.14},    // one plane, four
@@ -1176,7 +1175,7 @@ static bool gemm128_pays(const tk_ctx *ctx, const TkProblem &pr64, int gemm_nt, 
                                          {2, {1.127, 2.216}, 0.066, 2.81},
                                          {2, {1.196, 2.026}, 0.016, 2.97}};
   const int planes = pr64.planes;
-  if ((planes == 1 && pr64.mode == TK_MODE_DIGITS) || ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit) return false;
+  if (ctx->gemm_tiles || ctx->gemm_two_by_two || ctx->gemm_ksplit) return false;
   const int row = planes == 1 ? (gemm_nt == 2 ? 0 : 1) : planes;
   const double halves = (double)(((size_t)pr64.k + 127) / 128) * 0.5;  // (the 64-row kernel takes whole K blocks)
   return prefill_cost(rows64[row], workgroups_per_cu(ctx, pr64), (double)pr64.nb) > prefill_cost(rows128[row], workgroups_per_cu(ctx, pr128), halves);
@@ -1547,7 +1546,9 @@ static int run_linear(tk_ctx *ctx, const tk_linear_desc *layer, int mode, int pr
     ctx->last_kernel = "ksplit_decode";
     HIPCHK(tk_launch_skinny(ctx->stream, &pr, nullptr, 0, pl.cfg));
   } else {
-    const bool can128 = pr.planes <= 3 && nb >= 1 && (size_t)pr.n_tiles * nb * TK_CHUNK_BYTES < (size_t)1 << 32 && (size_t)pr.rs * 256 < (size_t)1 << 32;
+    // (one plane of float digit rows loses in every launch measured: 512 tokens K=2560 N=6912 44.6 us through the 64-row kernel, 46.5
+    // through this one, 1024 tokens K=6912 N=2560 76 / 91. The kernel has no such form.)
+    const bool can128 = pr.planes <= 3 && !(pr.planes == 1 && mode == TK_MODE_DIGITS) && nb >= 1 && (size_t)pr.n_tiles * nb * TK_CHUNK_BYTES < (size_t)1 << 32 && (size_t)pr.rs * 256 < (size_t)1 << 32;
     if (use256) {
       ctx->last_kernel = "gemm256";
       const hipError_t le = tk_launch_gemm256(ctx->stream, &pr, form256);

@@ -1,4 +1,5 @@
-// gfx950 prefill GEMM, 128 operand rows (96 for three planes) per workgroup, one to three planes, both contracts.
+// gfx950 prefill GEMM, 128 operand rows (96 for three planes) per workgroup: one to three planes under the int8 contract, two and
+// three under the float contract.
 //
 // The 64-row prefill kernel (tk_kernels.hip) is held back by the CU's vector-memory path and by the expansion of the 2-bit
 // codes: every wave expands the codes of its own columns, seven vector instructions for an operand that two matrix
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W / 2, W
   };
 
   // ---- prologue: constants, minus the row sums, the first two half blocks ----
-  const bool int8_in = hot.mode == TK_MODE_INT8;
+  const bool int8_in = P == 1 || hot.mode == TK_MODE_INT8;  // (one plane: the int8 contract only)
   {
     const void *src = nullptr;
     int last = 0, first = 0, n64 = 0, dst = 0;

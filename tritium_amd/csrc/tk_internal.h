@@ -226,8 +226,8 @@ hipError_t tk_launch_salt_seq(hipStream_t s, const TkProblem *single);
 hipError_t tk_launch_salt_gemm(hipStream_t s, const TkProblem *single, int compute_units);
 hipError_t tk_launch_gemm(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob,
                           const TkLaunchCfg &cfg);
-// 128-row prefill kernel (tk_gemm128.hip): one to three planes, both contracts, planes of less than 4 GiB of codes and at
-// least one K block; grid from the problem's XCD split over blocks of tk_gemm128_rows operand rows x tk_gemm128_tiles tiles.
+// 128-row prefill kernel (tk_gemm128.hip): one to three planes of int8 rows, two and three of float digit rows, planes of less than
+// 4 GiB of codes and at least one K block; grid from the problem's XCD split over blocks of tk_gemm128_rows operand rows x tk_gemm128_tiles tiles.
 // eight_waves: the form of one plane with eight waves per workgroup
 int tk_gemm128_rows(int planes);
 int tk_gemm128_tiles(int planes);
