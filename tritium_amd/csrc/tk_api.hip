@@ -2348,7 +2348,7 @@ struct tk_group {
   void *tables = nullptr;    // TkProblem[count], TkPrep[nprep], then int wg_prob[] (streaming form)
   int nprobs = 0, nprep = 0, prep_kind = 0;
   int prep_uniform_m = 0;    // > 0: prep entry j starts at token j * prep_uniform_m
-  int prep_wave_pieces = 0;  // > 0: every entry fits the one-wave-per-token prep kernels; the largest piece count
+  int prep_wave_pieces = 0;  // > 0: no entry has a norm; the largest piece count (tk_launch_prep)
   int prep_fast = 0;         // tk_prep_fast of every entry when they agree
   bool fused = false;        // the K-split kernel builds the operand rows itself: no prep launch (decided at creation)
   int prep_norm_fast = 0;    // some entry has an RMSNorm and tk_prep_norm_fast agrees for every entry: that value

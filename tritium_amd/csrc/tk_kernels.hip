@@ -1998,7 +1998,7 @@ __device__ __forceinline__ bool token_narrow(int poor, int large, int shift, TkP
 
 // ---- kernels ----
 // Rows of any form: with an RMSNorm of a shape the one-pass kernel does not take, a row-major copy, or more pieces than a team holds
-// (re-read from memory for the quantization). HELD = pieces a thread keeps in registers where all fit.
+// (re-read from memory for the quantization). A thread keeps up to TK_PREP_HELD pieces in registers where all of a row fit.
 #define TK_PREP_HELD 4
 __global__ __launch_bounds__(TK_WG) void tk_prep_a8_kernel(TkPrep single, const TkPrep *__restrict__ table, int nprep, int uniform_m) {
   __shared__ TkPrepShared sh;
@@ -2116,8 +2116,7 @@ __device__ __forceinline__ void emit_digits(const TkPrep &pp, size_t tok, int pc
   }
 }
 
-// Rows of more pieces than a team holds: read twice. (STRICT: TkPrep.strict.)
-template <bool STRICT>
+// Rows of more pieces than a team holds: read twice.
 __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, const TkPrep *__restrict__ table, int nprep, int uniform_m) {
   __shared__ TkPrepShared sh;
   int rowi;
@@ -2146,12 +2145,12 @@ __global__ __launch_bounds__(TK_WG) void tk_prep_digits_kernel(TkPrep single, co
 #pragma unroll
       for (int x = 0; x < 16; ++x) v[x] = 0.0f;
     }
-    emit_digits<STRICT>(pp, tok, pc, v, shift, sums, counts);
+    emit_digits<false>(pp, tok, pc, v, shift, sums, counts);
     pc += TK_WG;
   });
   int six[6] = {sums[0], sums[1], sums[2], sums[3], counts[0], counts[1]};
   team_sums<TK_WG, 6>(six, sh.sums);
-  const bool narrow = token_narrow<TK_WG, STRICT>(six[4], six[5], shift, sh, each);
+  const bool narrow = token_narrow<TK_WG, false>(six[4], six[5], shift, sh, each);
   if (tid == 0) {
     *(TK_GLOBAL v4i *)(pp.rowsum + tok * 4) = v4i{six[0], six[1], six[2], six[3]};
     pp.exps[tok] = -shift;
@@ -2709,8 +2708,8 @@ hipError_t tk_launch_prep(hipStream_t s, int kind, const TkPrep *single, const T
   switch (kind) {
     case TK_PREP_A8: hipLaunchKernelGGL(tk_prep_a8_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m); break;
     case TK_PREP_DIGITS:
-      if (strict) hipLaunchKernelGGL(tk_prep_digits_kernel<true>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
-      else hipLaunchKernelGGL(tk_prep_digits_kernel<false>, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
+      if (strict) return hipErrorInvalidValue;  // (rows of at most 9,984 elements: a team holds them)
+      hipLaunchKernelGGL(tk_prep_digits_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m);
       break;
     case TK_PREP_I8: hipLaunchKernelGGL(tk_prep_i8_kernel, dim3(rows), dim3(TK_WG), 0, s, sg, table, nprep, uniform_m); break;
     default: return hipErrorInvalidValue;
