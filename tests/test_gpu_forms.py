@@ -663,11 +663,10 @@ def test_prefill_kernel_k_split(backend, oracle, slices, m, n, k, planes, tiles)
 @pytest.mark.parametrize("k,m,copies", [(256, 1, 40), (2048, 4, 10), (2560, 2, 20), (6912, 3, 12), (17408, 1, 3), (6912, 40, 1),
                                           (2000, 2, 20)])
 def test_activation_prep_forms_agree(backend, oracle, mode, k, m, copies):
-    """The quantization / digit-split launch has three forms: a wave per token, a workgroup per token (both in
-    a straight-line variant for rows of whole K blocks, up to 8 pieces held per thread), and the general
-    workgroup-per-token kernels. Forced either way through the knob, a grouped launch of `copies` members must
-    give the same bits, and the int8 contract the oracle's (rows with NaN, Inf, all zeros and a single
-    non-zero element included; K=2000 is not whole blocks: the general kernels)."""
+    """The quantization / digit-split launch keeps a token in the registers of a wave or of a workgroup (each with straight-line
+    loads for rows of whole K blocks, up to 8 pieces per thread; K=2000 is not whole blocks). Forced either way through the knob, a
+    grouped launch of `copies` members must give the same bits, and the int8 contract the oracle's (rows with NaN, Inf, all zeros and a
+    single non-zero element included). Longer rows: test_activation_prep_of_long_rows_places_every_element."""
     print("case prep-forms", mode, k, m, copies, flush=True)
     if mode == 0 and m * 4 > 64:
         pytest.skip("float groups take at most 16 tokens")
@@ -772,8 +771,8 @@ def test_narrow_groups_of_several_row_tiles_take_the_prefill_kernel(backend, ora
 @pytest.mark.parametrize("m", [40, 400])
 def test_prep_of_rows_aligned_like_an_element(backend, oracle, m, k, dtype):
     """Rows whose starts are aligned like one element only (odd K, a base one element into a buffer): the vector loads of the
-    quantization against the oracle, and the digit split's two forms (a workgroup or a wave per token) against each other where
-    there are two: rows of 65 to 256 pieces of 16 elements (257 has one piece per lane and keeps the wave, 4099 the workgroup)."""
+    quantization against the oracle, and the digit split's two forms (a workgroup, which launches of this size take, and a wave per token)
+    against each other."""
     print("case ragged prep", m, k, dtype, flush=True)
     rng = np.random.default_rng(m + k)
     n = 40
@@ -790,7 +789,7 @@ def test_prep_of_rows_aligned_like_an_element(backend, oracle, m, k, dtype):
     backend.linear_a8(layer, moved, m, o)
     assert same_bits(o.to_host(), oracle.cpu_linear_a8_planes([packed], FMT_TQ2_0, [sc], act, m, n, k))
     backend.linear_float(layer, moved, m, o)
-    backend.set_prep_team_rows(0 if m == 40 else 1000)
+    backend.set_prep_team_rows(0)
     try:
         backend.linear_float(layer, moved, m, o2)
     finally:
@@ -834,6 +833,60 @@ def test_activation_prep_of_ragged_rows_places_every_element(backend, oracle, k,
     top = np.abs(seen).max(axis=1, keepdims=True)
     assert (np.abs(got - want) <= top * 2.0 ** -29 + np.abs(want) * 2e-7 + 1e-44)[plain].all()
     for x in (act, out):
+        x.free()
+    layer.free()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("k,m,team_rows", [(1283, 40, 0), (2560, 40, 0), (3001, 40, 0), (6001, 40, 0), (8191, 40, 0),       # a wave per token, 2 / 4 / 8 pieces a lane
+                                           (4099, 4, 384), (9001, 4, 384), (17001, 4, 384), (32767, 4, 384), (32768, 4, 384),   # a workgroup
+                                           (32769, 4, 384), (33024, 4, 384), (50001, 4, 384)])                                  # read twice
+def test_activation_prep_of_long_rows_places_every_element(backend, oracle, k, m, team_rows, dt):
+    """As the test of ragged rows above, for rows whose threads hold several pieces each and for rows that no team holds: outputs
+    of one non-zero trit at both ends of every K block's neighbourhood of a round of the team (1024 or 4096 elements), at the row's end
+    and in between; the same bounds. Quantized rows besides: row-major int8 values, scales and flags against the oracle's."""
+    print("case long-prep", k, m, team_rows, dt, flush=True)
+    rng = np.random.default_rng(k + m)
+    at = sorted({e for r in range(0, k + 1024, 1024) for e in (r - 129, r - 1, r, r + 1, r + 31, r + 32) if 0 <= e < k}
+                | set(range(max(0, k - 260), k)) | set(rng.integers(0, k, 40).tolist()))
+    n = len(at)
+    w = np.zeros((n, k), np.int8)
+    w[np.arange(n), at] = rng.choice([-1, 1], n)
+    packed, ones = T.pack_rows(w, n, k), np.ones(n, np.float32)
+    layer = backend.linear([packed], [ones], n, k)
+    a = (rng.standard_normal((m, k)) * 10.0 ** rng.integers(-3, 3, (m, 1))).astype(np.float32)
+    a[0] = rng.choice(np.float32([1e-37, -1e-37, 0.0, 3e-38, -2e-38]), k)
+    a[1, k - 2] = np.nan
+    a[2] = 0.0
+    a[3, k - 1] = np.abs(a[3]).max() * np.float32(1.5)  # the last element is the largest
+    host = f32_to_bf16_bits(a) if dt == "bf16" else a
+    seen = bf16_bits_to_f32(host).reshape(m, k) if dt == "bf16" else a
+    act, out = backend.to_device(host, dt), backend.empty(m * n, "f32")
+    q, qs, nonfinite = backend.empty(m * k, "i8"), backend.empty(m, "f32"), backend.empty(m, "i32")
+    backend.set_prep_team_rows(team_rows)
+    try:
+        backend.linear_a8(layer, act, m, out)
+        got = out.to_host().reshape(m, n)
+        backend.linear_float(layer, act, m, out)
+    finally:
+        backend.set_prep_team_rows(384)
+    # one trit per output: the oracle's quantized element itself, which is then multiplied by the token's scale
+    quant, scale = oracle.quantize_act_int8(seen, m, k)
+    picked = w[np.arange(n), at].astype(np.float32)
+    want = quant[:, at] * picked * scale[:, None]
+    fin = ~np.isnan(want)
+    assert (np.isnan(got) == ~fin).all() and (got[fin] == want[fin]).all()
+    got = out.to_host().reshape(m, n)
+    want = seen[:, at].astype(np.float64) * picked
+    plain = np.arange(m) != 1
+    top = np.abs(seen).max(axis=1, keepdims=True)
+    assert (np.abs(got - want) <= top * 2.0 ** -29 + np.abs(want) * 2e-7 + 1e-44)[plain].all()
+    nan = np.isnan(want[1])
+    assert (np.isnan(got[1]) == nan).all() and same_bits(got[1][~nan], want[1][~nan])  # in the reference's order: the element itself
+    backend.act_quant_i8(act, m, k, q, qs, nonfinite)
+    assert same_bits(qs.to_host(), scale) and (nonfinite.to_host() == [0, 1, 0, 0] + [0] * (m - 4)).all()
+    assert (q.to_host().reshape(m, k)[2:] == quant[2:].astype(np.int8)).all()
+    for x in (act, out, q, qs, nonfinite):
         x.free()
     layer.free()
 
