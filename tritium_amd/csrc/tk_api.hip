@@ -986,10 +986,10 @@ static int flow_run_tiles(const tk_ctx *ctx, unsigned total_tiles, int planes, i
   // where two workgroups share a CU: a CU's time follows the number of workgroups it is handed (two planes K=5120 N=5120
   // 16 rows, 32 copies, runs of 1 / 2 / 4 / 8: 86 / 94 / 77 / 123 us, rule: 2; three planes N=17408 370 / 364 / 387 / 425,
   // rule: 4).
-  // The 32x32x32 form in eight-wave workgroups (25..32 rows of up to 64 KiB; its registers leave a CU one workgroup): likewise. 32 digit rows
-  // of eight float tokens / 32 int8 rows, two planes K=2048 N=8192, 48 copies, runs of 1 / 2 / 4 / 6 pairs: 84 / 82.7 / 86 / 112 and 95 / 92 / 99 /
-  // 136 us (4 fill one and a half rounds); 128 copies 209 / 206 / 201 / 209 (4: four rounds; the rule's and the model's choice); one plane
-  // N=6912, 48 copies 44.5 / 41.6 / 41.9 / -.
+  // The 32x32x32 form in eight-wave workgroups (25..32 rows of up to 64 KiB; its registers leave a CU one workgroup):
+  // likewise. 32 digit rows of eight float tokens / 32 int8 rows, two planes K=2048 N=8192, 48 copies, runs of 1 / 2 / 4 / 6
+  // pairs: 84 / 82.7 / 86 / 112 and 95 / 92 / 99 / 136 us (4 fill one and a half rounds); 128 copies 209 / 206 / 201 / 209
+  // (4: four rounds; the rule's and the model's choice); one plane N=6912, 48 copies 44.5 / 41.6 / 41.9 / -.
   bool use_model = !b3 && waves >= 8 && (rt == 1 || (rt >= 2 && (wide || lds_bytes > kLdsFlowMax / 2)));
   if (use_model && rt > 2) {
     const double wgs = (double)((total_tiles + per_s * s - 1) / (per_s * s)), cus = (double)ctx->info.compute_units;

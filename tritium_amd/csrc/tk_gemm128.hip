@@ -18,12 +18,14 @@
 // SIMD a single one to hide its loads behind (gemm128_eight_waves in tk_api.hip).
 //
 // Bound: in long launches the chip's power -- registers full of gaussian int8 rows and codes, nothing but matrix instructions,
-// hold 4.0 POPS of the 5.0 that all-zero operands reach (and 3.5 with the weights as the first operand: so activations go first),
-// and interleaving the expansion with the matrix instructions one by one changed nothing. Otherwise the number of workgroups
-// on the CU that has most (gemm128_pays in tk_api.hip). Calls incl. quantization, 64 rows -> 128: 4096 tokens K=5120 N=17408 three
-// planes 759 -> 738 us, 1024 tokens K=5120 N=5120 79 -> 72, 200 tokens N=17408 73 -> 65; 768 tokens K=6144 N=20480 one plane
-// 98 -> 83, two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 -> 41.1 (35.7 with the
-// epilogue and the digit split of now). One workgroup alone on a CU runs its loop at 0.58 of the matrix rate, two at 0.70.
+// hold 4.0 to 4.2 POPS of the 5.0 that all-zero operands reach (3.5 with the weights as the first operand: so activations go
+// first), and interleaving the expansion with the matrix instructions one by one changed nothing. Otherwise the number of
+// workgroups on the CU that has most (gemm128_pays in tk_api.hip). Calls incl. quantization, 64 rows -> 128: 4096 tokens K=5120
+// N=17408 three planes 759 -> 738 us, 1024 tokens K=5120 N=5120 79 -> 72, 200 tokens N=17408 73 -> 65; 768 tokens K=6144
+// N=20480 one plane 98 -> 83, two planes (N=10240) 87 -> 81; float contract 333 f32 tokens K=2050 N=5003 two planes 43.2 ->
+// 41.1 (35.7 with the epilogue and the digit split of now). Counters: the matrix pipes work for 0.77 of a long launch's cycles
+// with three planes, 0.72 with two, 0.69 with one; with one workgroup per CU (1024 tokens K=6912 N=6912) for 0.45 on four waves
+// and 0.48 on eight.
 
 #include <type_traits>
 
@@ -289,9 +291,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W / 2, W
     if (esz == 2) staged(std::integral_constant<int, 2>{});
     else staged(std::integral_constant<int, 4>{});
   } else if (!int8_in && !hot.residual && !wg_flag) {
-    // float contract: token 8 rt + 2 q + kappa of the workgroup, one output per accumulator quad; a store is 32 adjacent columns of
-    // two tokens (straight-line: one address per column, stepped by two tokens, where flow_epilogue decides per output: 333 f32 tokens K=2050 N=5003
-    // two planes, call 37.3 -> 35.7 us)
+    // float contract: token 8 rt + 2 q + kappa of the workgroup, one output per accumulator quad; a store is 32 adjacent
+    // columns of two tokens (straight-line: one address per column, stepped by two tokens, where flow_epilogue decides per
+    // output: 333 f32 tokens K=2050 N=5003 two planes, call 37.3 -> 35.7 us)
     auto plain = [&](auto esz_c) {
       constexpr int ESZ = decltype(esz_c)::value;
       const size_t step = (size_t)hot.n * (2 * ESZ);

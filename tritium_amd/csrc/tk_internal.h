@@ -226,16 +226,16 @@ hipError_t tk_launch_salt_seq(hipStream_t s, const TkProblem *single);
 hipError_t tk_launch_salt_gemm(hipStream_t s, const TkProblem *single, int compute_units);
 hipError_t tk_launch_gemm(hipStream_t s, const TkProblem *single, const TkProblem *table, const int *wg_prob,
                           const TkLaunchCfg &cfg);
-// 128-row prefill kernel (tk_gemm128.hip): one to three planes of int8 rows, two and three of float digit rows, planes of less than
-// 4 GiB of codes and at least one K block; grid from the problem's XCD split over blocks of tk_gemm128_rows operand rows x tk_gemm128_tiles tiles.
-// eight_waves: the form of one plane with eight waves per workgroup
+// 128-row prefill kernel (tk_gemm128.hip): one to three planes of int8 rows, two and three of float digit rows, planes of less
+// than 4 GiB of codes and at least one K block; grid from the problem's XCD split over blocks of tk_gemm128_rows operand rows x
+// tk_gemm128_tiles tiles. eight_waves: the form of one plane with eight waves per workgroup
 int tk_gemm128_rows(int planes);
 int tk_gemm128_tiles(int planes);
 hipError_t tk_launch_gemm128(hipStream_t s, const TkProblem *single, bool eight_waves);
-// 256 x 224 prefill kernel (tk_gemm256.hip): one plane, int8 contract, f32 / bf16 rows of whole 16-byte pieces, no residual; the weight tile is expanded to
-// int8 once per workgroup, in LDS. form 0: four waves of 64 rows over the whole column block (224 outputs); 1: eight
-// waves of 32 rows; 2: four waves over a part of the column block (128 or 96 outputs), two workgroups per CU. Grid from
-// the problem's XCD split over 256-row x 14-tile blocks.
+// 256 x 224 prefill kernel (tk_gemm256.hip): one plane, int8 contract, f32 / bf16 rows of whole 16-byte pieces, no residual;
+// the weight tile is expanded to int8 once per workgroup, in LDS. form 0: four waves of 64 rows over the whole column block
+// (224 outputs); 1: eight waves of 32 rows; 2: four waves over a part of the column block (128 or 96 outputs), two workgroups
+// per CU. Grid from the problem's XCD split over 256-row x 14-tile blocks.
 int tk_gemm256_lds_bytes(int form);
 hipError_t tk_launch_gemm256(hipStream_t s, const TkProblem *single, int form);
 hipError_t tk_launch_seq(hipStream_t s, const TkProblem *single);

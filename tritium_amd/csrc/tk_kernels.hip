@@ -41,9 +41,10 @@ __global__ __launch_bounds__(TK_WG) void tk_skinny_kernel(TkProblem single, cons
   static_assert(!FUSED || RT == 1, "the fused form: one row tile");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tile = blockIdx.x;
-  // The problem is read through a pointer to constant memory, from the kernel arguments or the table alike, so that its fields come by
-  // scalar loads. (A pointer that may be either as the compiler saw it made each field a vector load of its own, one trip to
-  // memory behind the other: decoder layer of hidden 2560, one token 28.2 -> 27.1 us, one token of K=2560 N=2560 4.99 -> 4.94.)
+  // The problem is read through a pointer to constant memory, from the kernel arguments or the table alike, so that its fields
+  // come by scalar loads. (A pointer that may be either as the compiler saw it made each field a vector load of its own, one
+  // trip to memory behind the other: decoder layer of hidden 2560, one token 28.2 -> 27.1 us, one token of K=2560 N=2560 4.99
+  // -> 4.94.)
   typedef const __attribute__((address_space(4))) TkProblem *ConstProblem;
   auto ka = __builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(ka));
@@ -1260,9 +1261,9 @@ __device__ __forceinline__ void tk_gemm32_epilogue(const TkProblem &pr, const Tk
     }
   } else if (hot.mode != TK_MODE_INT8 && !hot.residual && !wg_flag) {
     // Float contract, the common case: one output per accumulator quad, and a store is 32 adjacent columns of two tokens, whole
-    // lines of f32 as it is -- no staging, one address per column stepped by two tokens. (Staged with the decisions per output below,
-    // or through flow_epilogue, call before -> now: 64 bf16 tokens K=2560 N=6912 15.3 -> 14.7 us, 256 29.0 -> 27.7, 512 f32 tokens 48.8 -> 46.5,
-    // 100 tokens of three planes 29.7 -> 28.7, 200 f32 tokens K=1500 N=4001 two planes 19.1 -> 18.4.)
+    // lines of f32 as it is -- no staging, one address per column stepped by two tokens. (Staged with the decisions per output
+    // below, or through flow_epilogue, call before -> now: 64 bf16 tokens K=2560 N=6912 15.3 -> 14.7 us, 256 29.0 -> 27.7, 512
+    // f32 tokens 48.8 -> 46.5, 100 tokens of three planes 29.7 -> 28.7, 200 f32 tokens K=1500 N=4001 two planes 19.1 -> 18.4.)
     auto plain = [&](auto esz_c) {
       constexpr int ESZ = decltype(esz_c)::value;
       const size_t step = (size_t)hot.n * (2 * ESZ);
@@ -1489,18 +1490,20 @@ __global__ void tk_decode_trits_kernel(const uint8_t *__restrict__ codes, size_t
 }
 
 // ------------------------------------------------------------------------------------------
-// activation prep. A thread builds whole 16-byte operand pieces and keeps them in registers between the pass that finds the
-// row maximum and the pass that quantizes, so that a row is read once. These launches are a token's chain -- load, maximum,
+// activation prep. A thread builds whole 16-byte operand pieces and keeps them in registers between the pass that finds the row
+// maximum and the pass that quantizes, so that a row is read once. These launches are a token's chain -- load, maximum,
 // reduction, quantization, stores -- on few waves, so the instructions of the chain and the trips to memory in it are what they
 // cost: every load of a token is issued before the first is used (a piece past the row's end re-reads the last one), the
-// maximum is an integer one on the magnitude bits (which shows NaN and Inf as well), a rounding to an integer is one add
-// (1.5 * 2^23 leaves the int8 in the low byte), the four balanced digits of a float are one add and one exclusive or, bytes
-// are gathered by v_perm and summed by v_dot4, and reductions go through DPP and lane swaps instead of LDS.
-// About 6 vector instructions per element of the int8 quantization and 17 of the digit split (17 and 40 element by element). Kernels, before
-// -> now: digit split of 128 bf16 tokens K=2048 with block sums 7.5 -> 4.9 us, of 333 f32 tokens K=2050 11.9 -> 7.2; quantization of 32
-// bf16 tokens K=2560 4.1 -> 3.4, K=6912 4.8 -> 4.0, behind an RMSNorm 5.5 -> 4.5; of 2048 tokens K=2560 9.9 -> 9.5, which is near the
-// rate of a copy (15.7 MB; 4096 tokens K=5120 move 3.7 TB/s in 20.6 us). There, eight tokens to a workgroup with token = lane % 8, so that a
-// store fills whole lines, was no faster (2048 tokens K=2560, call with N=64 17.8 us either way; 400 tokens 14.1 -> 15.6).
+// maximum is an integer one on the magnitude bits (which shows NaN and Inf as well), a rounding to an integer is one add (1.5 *
+// 2^23 leaves the int8 in the low byte), the four balanced digits of a float are one add and one exclusive or, bytes are
+// gathered by v_perm and summed by v_dot4, and reductions go through DPP and lane swaps instead of LDS.
+// About 6 vector instructions per element of the int8 quantization and 17 of the digit split (17 and 40 element by element).
+// Kernels, before -> now: digit split of 128 bf16 tokens K=2048 with block sums 7.5 -> 4.9 us, of 333 f32 tokens K=2050 11.9 ->
+// 7.2; quantization of 32 bf16 tokens K=2560 4.1 -> 3.4, K=6912 4.8 -> 4.0, behind an RMSNorm 5.5 -> 4.5; of 2048 tokens K=2560
+// between products 9.9 -> 9.5. From 512 tokens on a launch is 3.4 us (K=2560; 4.0 K=5120) and a slope of 4.3 to 4.5 TB/s, about
+// a copy's rate: 2048 tokens K=2560 back to back 7.4 us (2.1 TB/s), 4096 tokens K=5120 18 us (3.5). There, eight tokens to a
+// workgroup with token = lane % 8, so that a store fills whole lines, was no faster (2048 tokens K=2560, call with N=64 17.8 us
+// either way; 400 tokens 14.1 -> 15.6).
 // ------------------------------------------------------------------------------------------
 
 // ---- reductions: every lane receives the result ----
@@ -1803,9 +1806,9 @@ __device__ __forceinline__ void load_piece(const void *act, int dtype, size_t ba
     load_piece_ragged<TK_F32>(act, base, (unsigned)e0, (unsigned)k, v);
   }
 }
-// The pieces lane, lane + TEAM, ... of a row. FAST: rows of whole K blocks, 16-byte aligned, of one element type (1 = f32, 2 = bf16),
-// and at least one block: in a row without any, the piece that a lane past the end re-reads does not exist (the host's rules keep K = 0 off
-// every kernel that loads this way; FAST = 0 reads nothing of such a row).
+// The pieces lane, lane + TEAM, ... of a row. FAST: rows of whole K blocks, 16-byte aligned, of one element type (1 = f32, 2 =
+// bf16), and at least one block: in a row without any, the piece that a lane past the end re-reads does not exist (the host's
+// rules keep K = 0 off every kernel that loads this way; FAST = 0 reads nothing of such a row).
 template <int HELD, int FAST, int TEAM>
 __device__ __forceinline__ void load_held(const void *act, int dtype, size_t base, size_t k, int npieces, int lane,
                                           float (&held)[HELD][16]) {

@@ -202,22 +202,23 @@ __global__ __launch_bounds__(64) void tk_salt_v2_forward_kernel(TkSaltV2 t, cons
 // product (a trit times a float), and v_mfma_f32_16x16x4_f32 adds its four terms in ascending order with one rounding each,
 // denormals kept. So 16 weight rows x 16 tokens fold on the f32 matrix pipe in the pinned order; a zero trit adds +-0, which
 // changes no accumulator that started at +0. (A non-finite activation fails the call, so 0 * inf does not count.)
-// A workgroup owns 16 rows x 16 tokens; its 16 waves take every sixteenth segment: each lane recodes a quarter of the
-// segment of one row to 2-bit codes (whatever the codec), four lanes exchange them, and a step of four columns is one
-// conversion and one matrix instruction. The scaled terms of up to SV2_SLOTS segments meet in LDS (as many as fit, so that the
-// waves drift apart and one's loads hide behind another's folds), where one thread per output adds them in the pinned order. Plane counts differ by tile: a row without a plane folds its last one again and drops the term.
-// Floor: the f32 matrix pipe, 32 cycles per 16 x 16 x 4 (7 us at the size below); the recoding and the latency of the loads add to it.
-// 4096 x 4096, two planes, kernels, 8 tokens of B3: 64 us (fold with a lane per row, terms through memory) + 12 us (their sum) ->
-// 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 35 / 37 / 38 us, one token 57 / 69 / 66 -> 33 / 36 / 37, 64 tokens 302 / 389 / 353 ->
-// 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory); up to 16 tokens of moderate size, whose results
-// need no launch that commits them, 35 / 37 -> 32 / 34 (D2 / B3, 8 tokens). A segment's codes and activations requested ahead of the
-// fold before it: 38.8 against 35.5 for B3. With the activations as 32 four-byte loads per lane and the codes as single bytes the
-// kernel took 52 us: the loads of 16 rows a few KiB apart were the bound.
+// A workgroup owns 16 rows x 16 tokens; its 16 waves take every sixteenth segment: each lane recodes a quarter of the segment
+// of one row to 2-bit codes (whatever the codec), four lanes exchange them, and a step of four columns is one conversion and
+// one matrix instruction. The scaled terms of up to SV2_SLOTS segments meet in LDS (as many as fit, so that the waves drift
+// apart and one's loads hide behind another's folds), where one thread per output adds them in the pinned order. Plane counts
+// differ by tile: a row without a plane folds its last one again and drops the term.
+// Floor: the f32 matrix pipe, 32 cycles per 16 x 16 x 4 (7 us at the size below); the recoding and the latency of the loads add
+// to it. 4096 x 4096, two planes, kernels, 8 tokens of B3: 64 us (fold with a lane per row, terms through memory) + 12 us
+// (their sum) -> 26 us; call, D2 / B3 / S34: 84 / 98 / 93 -> 35 / 37 / 38 us, one token 57 / 69 / 66 -> 33 / 36 / 37, 64 tokens
+// 302 / 389 / 353 -> 99 / 109 / 113 (12 us of the first two from the verdict through pinned memory); up to 16 tokens of
+// moderate size, whose results need no launch that commits them, 35 / 37 -> 32 / 34 (D2 / B3, 8 tokens). A segment's codes and
+// activations requested ahead of the fold before it: 38.8 against 35.5 for B3. With the activations as 32 four-byte loads per
+// lane and the codes as single bytes the kernel took 52 us: the loads of 16 rows a few KiB apart were the bound.
 constexpr int SV2_WAVES = 16, SV2_SLOTS = 48, SV2_HEAD = 528;
 // out (null: not asked for): a call of one block of tokens writes its results there at once if none of its activations exceeds
-// SV2_TAME in magnitude, else to tmp, and says so in *spill. With finite scales (the host's condition) results of such activations are below
-// 3 k * SV2_TAME * 2^16, which is finite for every k that is staged, and every workgroup reads all activations: none can
-// refuse the call once one has written.
+// SV2_TAME in magnitude, else to tmp, and says so in *spill. With finite scales (the host's condition) results of such
+// activations are below 3 k * SV2_TAME * 2^16, which is finite for every k that is staged, and every workgroup reads all
+// activations: none can refuse the call once one has written.
 constexpr float SV2_TAME = 18446744073709551616.0f;  // 2^64
 template <int G>
 __global__ __launch_bounds__(SV2_WAVES * 64) void tk_salt_v2_exact_kernel(TkSaltV2 t, const float *__restrict__ act, unsigned m,
